@@ -481,7 +481,7 @@ static const char* kNames[K_COUNT] = {"join_count", "join_expand", "copy_expand"
 struct Group {
     std::map<u32, std::unique_ptr<DBuf>> seq;  // per intern tag: nb counters
     // order-preserving value dictionary for packed sort keys
-    DBuf dict;
+    DBuf dict, dict_vals;                    // value -> rank table; value of each rank
     u64 dict_cap = 0, dict_n = 0;
     int dict_state = 0, dict_rebuilds = 0;   // state: 0 stale, 1 valid, 2 disabled
     u64 dict_gen = 0;                        // dictionary builds so far
@@ -1257,6 +1257,8 @@ static void build_dictionary(pra_ctx* c, int gi)
     pra_launch_fill_u64(c->st, G.dict.as<u64>(), cap * 2, 0);
     pra_launch_dict_insert(c->st, V.d(), V.n, G.dict.as<u64>(), cap, c->dflags());
     check_launch("dict_insert");
+    G.dict_vals.reserve(V.n * 8, c->st);
+    HIPCHK(hipMemcpyAsync(G.dict_vals.p, V.d(), V.n * 8, hipMemcpyDeviceToDevice, c->st));
     sync_check(c);
     G.dict_cap = cap;
     G.dict_n = V.n;
@@ -1264,10 +1266,77 @@ static void build_dictionary(pra_ctx* c, int gi)
     G.dict_gen++;
 }
 
+// Order an interned relation's full version through its membership bitmap
+// (k_bm_place): one read and one write of the rows, where the byte-pass sort
+// moves them once per varying byte of (bucket, columns).  Taken when the
+// bitmap holds exactly the keys of full -- current for the dictionary, keyed
+// on every column, no delta, as many set bits as rows -- and a row's bucket is
+// a function of column 0 (one bucket, or one join column).  The bitmap and
+// the buckets' runs are read once more, so a rank space of more than 64 words
+// a row, or a run table of more than 4 words a row, is left to the sort.
+// Measured on the 150x150 grid (128 M rows of 24 bytes, 8 buckets), solve and
+// ordered result: 132.0 ms with the 26 byte passes, 63.8 ms this way; a
+// 20,000-vertex random graph on one bucket (72 M rows) 66.3 -> 30.3 ms.
+// False when the version is not of that kind.
+static bool order_by_bitmap(pra_ctx* c, pra_rel* R)
+{
+    Group& G = grp(c, R->group);
+    Rows& r = R->ver[PRA_FULL];
+    const u64 n = r.n, D = G.dict_n, nb = (u64)c->nb;
+    const int kw = R->bm_kw;
+    if (!R->bm_valid || R->bm_gen != G.dict_gen || !G.dict_vals.p || kw != R->arity || R->ver[PRA_DELTA].n ||
+        n < 2 || n >= (1ULL << 32) || (nb > 1 && R->jcc != 1))
+        return false;
+    u64 S = 1;
+    for (int i = 1; i < kw; i++) S *= D;
+    const u64 words = (S * D + 63) / 64, nblk = (words * 64 + PRA_BM_BITS - 1) / PRA_BM_BITS;
+    if (words > 64 * n + 4096 || (nb > 1 && nb * D > 4 * n + 16384)) return false;
+    try {
+        c->tmp64a.reserve((nblk + 2) * 4, c->st);
+        if (nb > 1) {
+            c->tmp64b.reserve((nb * D + 2) * 4, c->st);
+            c->tmp64c.reserve(D * 4, c->st);
+        }
+    } catch (const PraError& e) {
+        // no room for the prefix: the sort needs less
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        for (DBuf* b : {&c->tmp64a, &c->tmp64b, &c->tmp64c}) b->release();
+        return false;
+    }
+    u32* prefix = c->tmp64a.as<u32>();
+    const u64* bm = R->bm.as<u64>();
+    pra_launch_bm_count(c->st, bm, words, nblk, prefix);
+    scan_u32(c, prefix, prefix, nblk, prefix + nblk);
+    if ((u32)readback(c, prefix + nblk, 1)[0] != (u32)n) return false;
+    u32* adj = nullptr;
+    if (nb > 1) {
+        u32* runs = c->tmp64b.as<u32>();
+        adj = c->tmp64c.as<u32>();
+        R->bnd[PRA_FULL].reserve((nb + 1) * 8, c->st);
+        pra_launch_bm_runs(c->st, bm, words, prefix, G.dict_vals.as<u64>(), D, S, nb, runs);
+        scan_u32(c, runs, runs, nb * D, runs + nb * D);
+        pra_launch_bm_adjust(c->st, bm, words, prefix, G.dict_vals.as<u64>(), D, S, nb, n, runs, adj,
+                             R->bnd[PRA_FULL].as<u64>());
+    }
+    c->sort_tmp.reserve(n * R->w * 8, c->st);
+    {
+        Prof p(c, K_GATHER, 16.0 * n * R->w);
+        pra_launch_bm_place(c->st, r.d(), n, R->w, kw, G.dict.as<u64>(), G.dict_cap, D, S, bm, words, prefix, adj,
+                            c->sort_tmp.as<u64>());
+        check_launch("bm_place");
+    }
+    r.buf.swap(c->sort_tmp);
+    r.sorted = true;
+    R->touched(PRA_FULL);
+    R->bnd_valid[PRA_FULL] = nb > 1;
+    return true;
+}
+
 static void ensure_sorted(pra_ctx* c, pra_rel* R, int v)
 {
     Rows& r = R->ver[v];
     if (r.sorted) return;
+    if (v == PRA_FULL && order_by_bitmap(c, R)) return;
     sort_rows(c, r, R->w, R->jcc, R->w);
     R->touched(v);
 }

@@ -1678,6 +1678,85 @@ __global__ void k_dense_build(const u64* rows, u64 n, int w, const u64* dict, u6
     atomicOr(&bitmap[x >> 5], 1u << (x & 31));
 }
 
+// Trie order of a relation from its membership bitmap.  Bit x of the bitmap is
+// the key of rank index x, and rank indexes order as the columns do, so a
+// key's place among all keys is the number of set bits below x: the exclusive
+// prefix of the 256-bit blocks' counts, plus the bits below x in its block.
+// With several buckets (the bucket a function of column 0), column-0 value r0
+// owns the bits [r0 * S, (r0 + 1) * S), S = D^(kw-1), and its rows move as one
+// run: adj[r0] = (rows of earlier runs in bucket order) - (set bits below
+// r0 * S), added modulo 2^32.
+#define PRA_BM_BLOCK_WORDS 4   // u64 words per counted block
+
+// set bits below bit x; nblk blocks of u64 words, prefix[nblk] the total
+__device__ __forceinline__ u32 pra_bm_rank(const u64* bm, u64 words, const u32* prefix, u64 x)
+{
+    const u64 b = x >> 8, w0 = b * PRA_BM_BLOCK_WORDS;
+    u32 r = prefix[b];
+    if (w0 >= words) return r;
+    const u32 bit = (u32)(x & 255), wi = bit >> 6;
+    u64 v[PRA_BM_BLOCK_WORDS];
+#pragma unroll
+    for (u32 k = 0; k < PRA_BM_BLOCK_WORDS; k++) v[k] = w0 + k < words ? bm[w0 + k] : 0;
+#pragma unroll
+    for (u32 k = 0; k < PRA_BM_BLOCK_WORDS; k++) {
+        const u64 m = k < wi ? ~0ULL : k == wi ? (1ULL << (bit & 63)) - 1 : 0;
+        r += (u32)__popcll(v[k] & m);
+    }
+    return r;
+}
+
+__global__ void k_bm_count(const u64* bm, u64 words, u64 nblk, u32* cnt)
+{
+    const u64 b = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nblk) return;
+    u32 c = 0;
+#pragma unroll
+    for (u32 k = 0; k < PRA_BM_BLOCK_WORDS; k++) {
+        const u64 i = b * PRA_BM_BLOCK_WORDS + k;
+        c += i < words ? (u32)__popcll(bm[i]) : 0;
+    }
+    cnt[b] = c;
+}
+
+// runs[b * D + r0] = rows of column-0 value r0 when it falls in bucket b, else 0
+__global__ void k_bm_runs(const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S, u64 nb,
+                          u32* runs)
+{
+    const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r0 >= D) return;
+    const u64 mine = pra_fnv_word(PRA_FNV_OFFSET, vals[r0]) % nb;
+    const u32 c = pra_bm_rank(bm, words, prefix, (r0 + 1) * S) - pra_bm_rank(bm, words, prefix, r0 * S);
+    for (u64 b = 0; b < nb; b++) runs[b * D + r0] = b == mine ? c : 0u;
+}
+
+// the runs' adjustments and the bucket bounds, from the exclusive scan of runs
+__global__ void k_bm_adjust(const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S, u64 nb, u64 n,
+                            const u32* scan, u32* adj, u64* bnd)
+{
+    const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r0 <= nb) bnd[r0] = r0 < nb ? (u64)scan[r0 * D] : n;
+    if (r0 >= D) return;
+    const u64 mine = pra_fnv_word(PRA_FNV_OFFSET, vals[r0]) % nb;
+    adj[r0] = scan[mine * D + r0] - pra_bm_rank(bm, words, prefix, r0 * S);
+}
+
+// Every row (all of them members) to its place.  Bound by the rows' own
+// bytes and by the lines of 24-byte writes: runs of a delta log walk the
+// bitmap in order, so its words, the prefix and the dictionary hit in cache.
+template <int KW>
+__global__ void k_bm_place(const u64* rows, u64 n, int w, const u64* dict, u64 dcap, u64 D, u64 S, const u64* bm,
+                           u64 words, const u32* prefix, const u32* adj, u64* out)
+{
+    const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    u64 x;
+    if (!pra_dense_index<KW>(rows + i * w, dict, dcap, D, &x)) return;
+    u32 pos = pra_bm_rank(bm, words, prefix, x);
+    if (adj) pos += adj[KW == 1 ? x : x / S];
+    if (pos < n) pra_copy_row(out + (u64)pos * w, rows + i * w, w);
+}
+
 // Combine the PRA_NREP replicas of the scatter summaries and reset them to
 // their identity values for the next scatter.  Part 0 (packed keys): the
 // top-byte bin counters, whose exclusive offsets go to kgofs and whose
@@ -2837,6 +2916,33 @@ void pra_launch_dense_build(hipStream_t st, const u64* rows, u64 n, int w, int k
     case 3: hipLaunchKernelGGL(k_dense_build<3>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
     default: hipLaunchKernelGGL(k_dense_build<4>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
     }
+}
+
+void pra_launch_bm_count(hipStream_t st, const u64* bm, u64 words, u64 nblk, u32* cnt)
+{
+    hipLaunchKernelGGL(k_bm_count, dim3(grid_for(nblk)), dim3(PRA_BLOCK), 0, st, bm, words, nblk, cnt);
+}
+
+void pra_launch_bm_runs(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
+                        u64 nb, u32* runs)
+{
+    hipLaunchKernelGGL(k_bm_runs, dim3(grid_for(D)), dim3(PRA_BLOCK), 0, st, bm, words, prefix, vals, D, S, nb, runs);
+}
+
+void pra_launch_bm_adjust(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
+                          u64 nb, u64 n, const u32* scan, u32* adj, u64* bnd)
+{
+    hipLaunchKernelGGL(k_bm_adjust, dim3(grid_for(std::max<u64>(D, nb + 1))), dim3(PRA_BLOCK), 0, st, bm, words,
+                       prefix, vals, D, S, nb, n, scan, adj, bnd);
+}
+
+void pra_launch_bm_place(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
+                         u64 S, const u64* bm, u64 words, const u32* prefix, const u32* adj, u64* out)
+{
+    if (!n) return;
+    const dim3 g(grid_for(n)), b(PRA_BLOCK);
+    auto k = kw == 1 ? k_bm_place<1> : kw == 2 ? k_bm_place<2> : kw == 3 ? k_bm_place<3> : k_bm_place<4>;
+    hipLaunchKernelGGL(k, g, b, 0, st, rows, n, w, dict, dict_cap, D, S, bm, words, prefix, adj, out);
 }
 
 void pra_launch_dense_table_clear(hipStream_t st, u64* table, u64 cap) { pra_launch_fill_u64(st, table, cap, 0); }

@@ -398,6 +398,18 @@ void pra_launch_dense_many(hipStream_t st, const DenseArgs* jobs, int njobs, int
                            u32 decide_blocks, u32* flags);
 void pra_launch_dense_build(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
                             u32* bitmap, u64* miss);
+// trie order of a version from its membership bitmap (k_bm_count .. k_bm_place
+// in pra_kernels.hip): 256-bit block counts (scanned by the caller into
+// prefix, prefix[nblk] = total), the runs of column-0 values by bucket, their
+// adjustments and the bucket bounds, and the placement of the rows
+#define PRA_BM_BITS 256
+void pra_launch_bm_count(hipStream_t st, const u64* bm, u64 words, u64 nblk, u32* cnt);
+void pra_launch_bm_runs(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
+                        u64 nb, u32* runs);
+void pra_launch_bm_adjust(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
+                          u64 nb, u64 n, const u32* scan, u32* adj, u64* bnd);
+void pra_launch_bm_place(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
+                         u64 S, const u64* bm, u64 words, const u32* prefix, const u32* adj, u64* out);
 void pra_launch_dense_table_clear(hipStream_t st, u64* table, u64 cap);
 // batched forms of k_bin_sort (256 blocks per job), k_scan_small (u32, one
 // block per job of at most PRA_SMALL_SCAN elements), D2D copies (job table
