@@ -18,11 +18,8 @@ typedef uint32_t u32;
 #define PRA_TILE (PRA_BLOCK * PRA_ITEMS)
 // packed-key sort bins: rows per bin sorted in LDS by one block
 #define PRA_BIN_BLOCK 1024
-// one-block LDS sort of small inputs: rows, key words per row at that many rows
-// (n x key words must fit PRA_SMALL_SORT x PRA_SMALL_SORT_KW), threads
+// rows of the one-block LDS sort
 #define PRA_SMALL_SORT 2048
-#define PRA_SMALL_SORT_KW 8
-#define PRA_SMALL_SORT_BLOCK 1024
 // one-block LSD sort (all passes in one launch) of up to this many rows
 #define PRA_BLOCK_SORT 16384
 // threads of the dedup decision and of the newt scatter per PRA_TILE candidates
@@ -83,6 +80,16 @@ __device__ inline u64 pra_fnv(const u64* t, int n)
     return h;
 }
 
+// h % nb for a bucket count nb <= 256: a mask for powers of two, else 32-bit
+// remainders of the two halves (a 64-bit remainder costs several times more)
+__device__ inline u32 pra_bucket(u64 h, u64 nbuckets)
+{
+    const u32 nb = (u32)nbuckets;
+    if ((nb & (nb - 1)) == 0) return (u32)h & (nb - 1);
+    const u32 c = (0u - nb) % nb;   // 2^32 % nb
+    return ((u32)(h >> 32) % nb * c + (u32)h % nb) % nb;
+}
+
 __host__ __device__ inline u64 pra_mix64(u64 x)
 {
     x ^= x >> 33;
@@ -137,13 +144,36 @@ struct PassList {
     DigitSpec p[PRA_MAXPASS];
 };
 
+// Sort key of a row: the bits of these fields, most significant first (col -1:
+// the bucket, FNV(row[0:jcc]) % nb).
+// A field with `rank` is the column's dictionary rank instead of its bits.
+struct KeyField {
+    signed char col;
+    unsigned char shift, bits, rank;
+};
+struct KeyLayout {
+    int nf, bits, jcc, pad;
+    u64 nb, dict_cap;
+    const u64* dict;
+    KeyField f[PRA_MAXW + 1];
+};
+__host__ __device__ inline void pra_key_field(KeyLayout& L, int col, int shift, int bits, int rank = 0)
+{
+    L.f[L.nf].rank = (unsigned char)rank;
+    L.f[L.nf].col = (signed char)col;
+    L.f[L.nf].shift = (unsigned char)shift;
+    L.f[L.nf].bits = (unsigned char)bits;
+    L.nf++;
+    L.bits += bits;
+}
+
 __device__ inline u32 pra_digit(const u64* row, const DigitSpec& ds)
 {
     u64 v;
     if (ds.col >= 0)
         v = row[ds.col];
     else
-        v = pra_fnv(row, ds.jcc) % ds.nb;
+        v = pra_bucket(pra_fnv(row, ds.jcc), ds.nb);
     return (u32)((v >> ds.shift) & (PRA_RADIX - 1));
 }
 

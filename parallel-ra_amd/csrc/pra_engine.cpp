@@ -352,7 +352,7 @@ struct DBuf {
         st = s;
         big = nbig;
     }
-    template <typename T> T* as() { return static_cast<T*>(p); }
+    template <typename T> T* as() const { return static_cast<T*>(p); }
     void swap(DBuf& o)
     {
         std::swap(p, o.p);
@@ -910,18 +910,124 @@ static u32 next_sort_epoch(pra_ctx* c)
     return c->sort_epoch;
 }
 
+// Keyed sort of rows (more than one block holds): the varying bits of (bucket,
+// columns) as a multi-word key, one or two counting passes over (word 0, row
+// index) pairs, then an LDS sort and row gather per segment.  A pass moves 24
+// bytes a row instead of 16 w, and there are two or three instead of one per
+// varying byte.  False, with r untouched, when a segment is too large for one
+// block (skewed keys) or there is no room for the pairs: the byte passes take
+// any keys in no more than the rows' own bytes.  With bnd (bucketed), the
+// bucket bounds are written too.
+// One counting pass up to 2^18 rows (segments of at most 1,024 on average, 256
+// blocks), two beyond.
+// With a dictionary (G), keys of more than one word take the data columns'
+// ranks instead of their bits when that makes them one word (a value without a
+// rank: false).
+// *dup (nullable): whether two rows' keys may be equal.
+static bool sort_rows_keyed(pra_ctx* c, Rows& r, int w, int jcc, int keycols, const u64* orm, bool bucketed, u64* bnd,
+                            const Group* G, bool* dup)
+{
+    const u64 n = r.n;
+    KeyLayout L;
+    memset(&L, 0, sizeof(L));
+    L.jcc = jcc;
+    L.nb = (u64)c->nb;
+    auto bits_of = [](u64 x) { return x ? 64 - __builtin_clzll(x) : 0; };
+    auto layout = [&](int rbits) {   // rbits: bits of a rank (0: no ranks)
+        L.nf = L.bits = 0;
+        if (bucketed) pra_key_field(L, -1, 0, bits_of(L.nb - 1));
+        for (int col = 0; col < keycols; col++) {
+            const u64 vary = (orm && col < 16) ? (orm[col] ^ orm[16 + col]) : ~0ULL;
+            if (!vary) continue;
+            const int lo = __builtin_ctzll(vary), bits = bits_of(vary) - lo;
+            if (rbits && col < w - 1 && rbits < bits)
+                pra_key_field(L, col, 0, rbits, 1);
+            else
+                pra_key_field(L, col, lo, bits);
+        }
+    };
+    layout(0);
+    if (L.bits > 64 && G && G->dict_state == 1 && G->dict_n > 1) {
+        layout(bits_of(G->dict_n - 1));
+        L.dict = G->dict.as<u64>();
+        L.dict_cap = G->dict_cap;
+        if (L.bits > 64) layout(0);
+    }
+    const int np = n <= (1ULL << 18) ? 1 : 2;
+    const int sb = np == 1 ? 8 : std::min(16, std::max(9, bits_of((n - 1) / 2048)));
+    const u32 nseg = 1u << sb;
+    const int top = 64 - sb;
+    DBuf *ka = &c->tmp64a, *kb = &c->ktmp;
+    try {
+        prepare_lookback(c, n);
+        for (DBuf* b : {ka, kb}) b->reserve(n * 8, c->st);
+        for (DBuf* b : {&c->idxa, &c->idxb}) b->reserve(n * 4, c->st);
+        c->segb.reserve(((size_t)nseg + 5) * 8 + (size_t)nseg * 4, c->st);
+        c->sort_tmp.reserve(n * w * 8, c->st);
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        for (DBuf* b : {ka, kb, &c->idxa, &c->idxb}) b->release();
+        return false;
+    }
+    u64* seg = c->segb.as<u64>();
+    u64* stat = seg + nseg + 1;   // largest segment, larger segments listed, overflow or missing rank, equal keys
+    u32* list = (u32*)(seg + nseg + 5);
+    pra_launch_fill_u64(c->st, c->ghist.as<u64>(), np * PRA_RADIX / 2, 0);
+    pra_launch_fill_u64(c->st, stat, 4, 0);
+    {
+        Prof p(c, K_RADIX_HIST, 8.0 * n * (w + 1));
+        pra_launch_sort_keys(c->st, r.d(), n, w, L, np, ka->as<u64>(), c->ghist.as<u32>(), stat + 2);
+        check_launch("sort_keys");
+    }
+    pra_launch_sort_scan(c->st, c->ghist.as<u32>(), np, c->gofs.as<u32>(), nullptr, (u32)c->nb, n);
+    check_launch("sort_scan");
+    for (int i = 0; i < np; i++) {
+        const u32 ep = next_sort_epoch(c);
+        Prof p(c, K_RADIX_SCATTER, 24.0 * n);
+        pra_launch_sort_scatter(c->st, ka->as<u64>(), kb->as<u64>(), n, 1,
+                                DigitSpec{0, np == 2 && i == 0 ? 48 : 56, 0, 0, 0},
+                                c->gofs.as<u32>() + (size_t)i * PRA_RADIX, c->lb_status.as<u64>(),
+                                c->lb_ctr.as<u32>() + i, ep, c->dflags(), i ? c->idxa.as<u32>() : nullptr,
+                                c->idxb.as<u32>());
+        check_launch("key_sort_scatter");
+        std::swap(ka, kb);
+        c->idxa.swap(c->idxb);
+    }
+    if (np == 2) {
+        pra_launch_seg_bounds(c->st, ka->as<u64>(), n, top, nseg, seg, stat, list);
+        check_launch("seg_bounds");
+    }
+    {
+        Prof p(c, K_BLOCK_SORT, 12.0 * n + 16.0 * n * w);
+        pra_launch_keyseg_sort(c->st, ka->as<u64>(), c->idxa.as<u32>(), np == 2 ? seg : nullptr,
+                               c->gofs.as<u32>(), nseg, list, stat, top, n, r.d(), w, L, c->sort_tmp.as<u64>(), bnd,
+                               stat + 2);
+        check_launch("keyseg_sort");
+    }
+    const u64* status = readback(c, stat + 2, 2);
+    if (status[0]) return false;
+    if (dup) *dup = status[1] != 0;
+    r.buf.swap(c->sort_tmp);
+    r.sorted = true;
+    return true;
+}
+
 // One-sweep LSD radix sort of rows by (bucket, col0 .. col[keycols-1]).
 // `orm` holds the OR (words 0..15) and AND (16..31) of the first 16 key
 // columns: digits equal in every row are skipped.  When the bucket digit is
 // sorted and nb <= 256, the bucket bounds are written to `bnd` (nb+1 words)
 // and true is returned.
+// G (nullable): the instance whose dictionary may shorten the keys.  dup
+// (nullable): receives whether the sorted rows may hold equal keys.
 // With `defer`, a sort that takes the one-block path is not launched: its job
 // (into `defer_out`, which the caller swaps with r's buffer once the batch
 // has been launched) is returned in *defer, with defer->n = 0 otherwise.
 static bool sort_rows_masked(pra_ctx* c, Rows& r, int w, int jcc, int keycols, const u64* orm, u64* bnd,
-                             bool by_bucket = true, SmallSortJob* defer = nullptr, DBuf* defer_out = nullptr)
+                             bool by_bucket = true, SmallSortJob* defer = nullptr, DBuf* defer_out = nullptr,
+                             const Group* G = nullptr, bool* dup = nullptr)
 {
     if (defer) defer->n = 0;
+    if (dup) *dup = r.n > 1;
     u64 n = r.n;
     if (n <= 1) {
         r.sorted = true;
@@ -943,10 +1049,9 @@ static bool sort_rows_masked(pra_ctx* c, Rows& r, int w, int jcc, int keycols, c
         r.sorted = true;
         return false;
     }
-    // small inputs with several varying bytes: one block sorts them in LDS
+    // small inputs: one block sorts them in LDS
     const bool bucketed = c->nb > 1 && by_bucket;
-    const int kw = keycols + (bucketed ? 1 : 0);
-    if (n <= PRA_SMALL_SORT && n * kw <= (u64)PRA_SMALL_SORT * PRA_SMALL_SORT_KW && passes.size() >= 2) {
+    if (n <= PRA_SMALL_SORT) {
         u64* bout = (bnd && bucketed && bucket_last) ? bnd : nullptr;
         if (defer) {
             defer_out->reserve(n * w * 8, c->st);
@@ -955,15 +1060,27 @@ static bool sort_rows_masked(pra_ctx* c, Rows& r, int w, int jcc, int keycols, c
             return bout != nullptr;
         }
         c->sort_tmp.reserve(n * w * 8, c->st);
+        u64* dup_dev = nullptr;
+        if (dup) {
+            c->orand.reserve(32 * 8, c->st);
+            dup_dev = c->orand.as<u64>();
+            pra_launch_fill_u64(c->st, dup_dev, 1, 0);
+        }
         {
-            Prof p(c, K_SMALL_SORT, 8.0 * n * kw + 16.0 * n * w);
+            Prof p(c, K_SMALL_SORT, 8.0 * n * (keycols + 1) + 16.0 * n * w);
             pra_launch_small_sort(c->st, r.d(), n, w, jcc, keycols, (u64)c->nb, bucketed ? 1 : 0,
-                                  c->sort_tmp.as<u64>(), bout);
+                                  c->sort_tmp.as<u64>(), bout, dup_dev);
             check_launch("small_sort");
         }
         r.buf.swap(c->sort_tmp);
         r.sorted = true;
+        if (dup) *dup = readback(c, dup_dev, 1)[0] != 0;
         return bout != nullptr;
+    }
+    // the keyed sort, from two passes saved on
+    if (n < (1ULL << 32) && passes.size() >= 4) {
+        u64* bout = (bnd && bucketed && bucket_last) ? bnd : nullptr;
+        if (sort_rows_keyed(c, r, w, jcc, keycols, orm, bucketed, bout, G, dup)) return bout != nullptr;
     }
     // up to PRA_BLOCK_SORT rows: one block runs every pass in one launch
     if (n <= PRA_BLOCK_SORT && passes.size() >= 2 && passes.size() <= PRA_MAXPASS) {
@@ -1016,10 +1133,17 @@ static bool sort_rows_masked(pra_ctx* c, Rows& r, int w, int jcc, int keycols, c
     return wrote_bnd;
 }
 
-static void sort_rows(pra_ctx* c, Rows& r, int w, int jcc, int keycols, bool by_bucket = true)
+static void sort_rows(pra_ctx* c, Rows& r, int w, int jcc, int keycols, bool by_bucket = true,
+                      const Group* G = nullptr, bool* dup = nullptr)
 {
     if (r.n <= 1) {
         r.sorted = true;
+        if (dup) *dup = false;
+        return;
+    }
+    // the one-block sort collects the columns' varying bits itself
+    if (r.n <= PRA_SMALL_SORT) {
+        sort_rows_masked(c, r, w, jcc, keycols, nullptr, nullptr, by_bucket, nullptr, nullptr, G, dup);
         return;
     }
     int kc = std::min(keycols, 16);
@@ -1032,7 +1156,7 @@ static void sort_rows(pra_ctx* c, Rows& r, int w, int jcc, int keycols, bool by_
     u64* h = readback(c, om, 32);
     u64 m[32];
     std::copy(h, h + 32, m);
-    sort_rows_masked(c, r, w, jcc, keycols, m, nullptr, by_bucket);
+    sort_rows_masked(c, r, w, jcc, keycols, m, nullptr, by_bucket, nullptr, nullptr, G, dup);
 }
 
 static int ceil_log2(u64 x);
@@ -1337,7 +1461,7 @@ static void ensure_sorted(pra_ctx* c, pra_rel* R, int v)
     Rows& r = R->ver[v];
     if (r.sorted) return;
     if (v == PRA_FULL && order_by_bitmap(c, R)) return;
-    sort_rows(c, r, R->w, R->jcc, R->w);
+    sort_rows(c, r, R->w, R->jcc, R->w, true, &grp(c, R->group));
     R->touched(v);
 }
 
@@ -2360,7 +2484,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             a.fold = f;
             // column masks only pick the sort passes of outputs too large for
             // the one-block sort, which compares whole key words
-            a.summarize = C > PRA_SMALL_SORT || C * (u64)(R->w + 1) > (u64)PRA_SMALL_SORT * PRA_SMALL_SORT_KW;
+            a.summarize = C > PRA_SMALL_SORT;
             if (phase == 3 && nblocks < PRA_SCATTER_WIDE_TILES) {
                 // narrow partitions of a batched iteration go out together
                 scatter_jobs[pk ? 1 : 0].push_back(a);
@@ -2829,7 +2953,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         if (packed[oi] && !in_rounds[oi] && G.dict_state == 1) G.dict_state = ++G.dict_rebuilds > 3 ? 2 : 0;
         SmallSortJob job;
         bnd_ok[oi] = sort_rows_masked(c, NT, R->w, R->jcc, out_intern[oi] ? R->arity : R->w, masks, bnd, true, &job,
-                                      &R->ver[PRA_DELTA].buf);
+                                      &R->ver[PRA_DELTA].buf, &G);
         if (job.n) {
             ssb.job[ss_out.size()] = job;
             ss_out.push_back(oi);
@@ -3407,13 +3531,16 @@ int pra_rel_load_rows(pra_rel* rel, const uint64_t* rows, uint64_t nrows, int ve
     API_BEGIN(rel->ctx)
     pra_ctx* c = rel->ctx;
     if (nrows) {
-        DBuf tmp;
-        tmp.reserve(nrows * rel->w * 8, c->st);
-        HIPCHK(hipMemcpyAsync(tmp.p, rows, nrows * rel->w * 8, hipMemcpyHostToDevice, c->st));
-        append_rows(c, rel, version, tmp.as<u64>(), nrows);
         Rows& r = rel->ver[version];
-        sort_rows(c, r, rel->w, rel->jcc, rel->w);
-        unique_rows(c, r, rel->w);
+        const size_t used = (size_t)r.n * rel->w * 8, bytes = (size_t)nrows * rel->w * 8;
+        r.buf.reserve(used + bytes, c->st, used);
+        HIPCHK(hipMemcpyAsync(r.buf.as<char>() + used, rows, bytes, hipMemcpyHostToDevice, c->st));
+        r.n += nrows;
+        r.sorted = false;
+        rel->touched(version);
+        bool dup = false;   // a sort that saw no equal rows leaves none to remove
+        sort_rows(c, r, rel->w, rel->jcc, rel->w, true, nullptr, &dup);
+        if (dup) unique_rows(c, r, rel->w);
         HIPCHK(hipStreamSynchronize(c->st));
         rel->touched(version);
         rel->mt_valid = false;

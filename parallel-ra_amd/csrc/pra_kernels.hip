@@ -216,80 +216,558 @@ __global__ void k_sort_scatter(const u64* in, u64* out, u64 n, int w, DigitSpec 
     }
 }
 
-// One block sorts n <= PRA_SMALL_SORT rows, whose key words (n x kw) fit the
-// PRA_SMALL_SORT x PRA_SMALL_SORT_KW words of LDS, by (bucket, col0 .. col[kc-1])
-// (the bucket FNV(row[0:jcc]) % nb leads when `bucketed`; columns compare as
-// unsigned words) with a bitonic network over row indices in LDS, then
-// gathers the rows into `out`.  Unstable: rows with equal keys are equal.
-// With bnd (bucketed), bnd[s] = first row of bucket s, bnd[nb] = n.
-__device__ inline void pra_small_sort_block(const u64* rows, u64 n, int w, int jcc, int kc, u64 nb, int bucketed,
-                                            u64* out, u64* bnd)
+// ------------------------------------------------------ value dictionary ---
+//
+// An order-preserving dictionary of the values in the relations' key columns
+// (rank(a) < rank(b) iff a < b) lets a newt row's sort key
+// (bucket, col0, .., col[a-1]) be packed into one u64: the bucket and the
+// column ranks as digits of radix D (the dictionary size), which the sort
+// then orders in a few byte passes.
+// Slots: [value, rank + 1]; rank + 1 == 0 marks an empty slot.
+
+__device__ inline u64 pra_dict_slot(u64 v, u64 cap) { return pra_mix64(v ^ 0x5851F42D4C957F2DULL) & (cap - 1); }
+
+__device__ inline bool pra_dict_rank(const u64* tab, u64 cap, u64 v, u64* rank)
 {
-    __shared__ u64 key[PRA_SMALL_SORT * PRA_SMALL_SORT_KW];
-    __shared__ u32 idx[PRA_SMALL_SORT];
-    const int kw = kc + (bucketed ? 1 : 0);
-    const u32 m = (u32)n;
-    for (u32 i = threadIdx.x; i < m; i += PRA_SMALL_SORT_BLOCK) {
-        const u64* r = rows + (u64)i * w;
-        u64* k = key + (u64)i * kw;
-        int o = 0;
-        if (bucketed) k[o++] = pra_fnv(r, jcc) % nb;
-        for (int c = 0; c < kc; c++) k[o++] = r[c];
-    }
-    u32 N = 2;
-    while (N < m) N <<= 1;
-    for (u32 i = threadIdx.x; i < N; i += PRA_SMALL_SORT_BLOCK) idx[i] = i;   // i >= m: past every row
-    __syncthreads();
-    for (u32 k = 2; k <= N; k <<= 1)
-        for (u32 j = k >> 1; j > 0; j >>= 1) {
-            for (u32 i = threadIdx.x; i < N; i += PRA_SMALL_SORT_BLOCK) {
-                const u32 l = i ^ j;
-                if (l <= i) continue;
-                const u32 a = idx[i], b = idx[l];
-                bool gt;
-                if (a >= m || b >= m) {
-                    gt = a >= m && (b < m || a > b);
-                } else {
-                    const u64* ka = key + (u64)a * kw;
-                    const u64* kb = key + (u64)b * kw;
-                    int c = 0;
-                    while (c < kw && ka[c] == kb[c]) c++;
-                    gt = c < kw && ka[c] > kb[c];
-                }
-                if (((i & k) == 0) == gt) {
-                    idx[i] = b;
-                    idx[l] = a;
-                }
-            }
-            __syncthreads();
+    u64 m = cap - 1, s = pra_dict_slot(v, cap);
+    for (u64 q = 0; q < cap; q++) {
+        const u64* sl = tab + 2 * s;
+        u64 r = sl[1];
+        if (r == 0) return false;
+        if (sl[0] == v) {
+            *rank = r - 1;
+            return true;
         }
-    for (u32 i = threadIdx.x; i < m; i += PRA_SMALL_SORT_BLOCK) {
-        const u64* src = rows + (u64)idx[i] * w;
-        u64* dst = out + (u64)i * w;
-        pra_copy_row(dst, src, w);
+        s = (s + 1) & m;
     }
-    if (bnd && bucketed) {
-        for (u32 i = threadIdx.x; i <= m; i += PRA_SMALL_SORT_BLOCK) {
+    return false;
+}
+
+// ---------------------------------------------------------- LDS sorts ------
+
+// LDS of a block that sorts up to BLOCK * IT (key, index) pairs
+template <int BLOCK, int IT>
+struct SortLds {
+    u64 key[BLOCK * IT];
+    u32 idx[BLOCK * IT];
+    u32 wh[BLOCK / 64][PRA_RADIX];
+    u32 wsum[PRA_RADIX / 64];
+};
+
+// One stable counting pass of the block's m pairs by the 8 key bits from
+// `shift` up; thread t holds its pairs as items k of positions wave * 64 * IT
+// + k * 64 + lane, before and after.  Leaves digit d's first position in
+// L.wh[0][d] and the pairs in L.key / L.idx.
+template <int BLOCK, int IT>
+__device__ __forceinline__ void pra_lds_pass(SortLds<BLOCK, IT>& L, u64 (&key)[IT], u32 (&id)[IT], u32 m, int shift)
+{
+    constexpr int WAVES = BLOCK / 64;
+    constexpr u32 PER_WAVE = 64 * IT;
+    static_assert(BLOCK >= PRA_RADIX, "the digit scan takes a thread per digit");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const u64 lt = pra_lanemask_lt();
+    {
+        for (int i = threadIdx.x; i < WAVES * PRA_RADIX; i += BLOCK) (&L.wh[0][0])[i] = 0;
+        __syncthreads();
+        // stable rank of every pair among the pairs of its digit: wave-local
+        // counts in element order, then a scan over waves and digits
+        u32 dg[IT], lc[IT];
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
+            bool valid = i < m;
+            dg[k] = 0;
+            lc[k] = 0;
+            // a wave skips the ranking of item rows wholly past the pairs
+            if ((u32)wave * PER_WAVE + (u32)k * 64 >= m) continue;
+            u32 d = valid ? (u32)(key[k] >> shift) & 255u : 0u;
+            u64 peers = pra_match<PRA_RADIX_BITS>(d, __ballot(valid));
+            dg[k] = d;
+            if (valid) {
+                u32 before = L.wh[wave][d];
+                lc[k] = before + (u32)__popcll(peers & lt);
+                if ((peers >> lane) == 1ULL) L.wh[wave][d] = before + (u32)__popcll(peers);
+            }
+        }
+        __syncthreads();
+        const int d = threadIdx.x;   // digit of this thread in the scan (threads < PRA_RADIX)
+        u32 acc = 0;
+        if (d < PRA_RADIX)
+            for (int v = 0; v < WAVES; v++) {
+                u32 t = L.wh[v][d];
+                L.wh[v][d] = acc;
+                acc += t;
+            }
+        u32 x = acc;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            u32 y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (d < PRA_RADIX && lane == 63) L.wsum[wave] = x;
+        __syncthreads();
+        if (d < PRA_RADIX) {
+            u32 base = x - acc;
+            for (int v = 0; v < wave; v++) base += L.wsum[v];
+            for (int v = 0; v < WAVES; v++) L.wh[v][d] += base;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
+            if (i < m) {
+                u32 pos = L.wh[wave][dg[k]] + lc[k];
+                L.key[pos] = key[k];
+                L.idx[pos] = id[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
+            if (i < m) {
+                key[k] = L.key[i];
+                id[k] = L.idx[i];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Pairs equal in the sixteen highest varying key bits are put in order by
+// comparing each with its neighbours, up to this many to either side; a larger
+// group leaves the block to LSD passes.
+#define PRA_GROUP_MAX 32
+
+// Stable LSD passes over the bytes set in `bytes` (bit p = byte p)
+template <int BLOCK, int IT>
+__device__ __forceinline__ void pra_lds_lsd(SortLds<BLOCK, IT>& L, u64 (&key)[IT], u32 (&id)[IT], u32 m, u32 bytes)
+{
+#pragma unroll 1
+    for (int p = 0; p < 8; p++)
+        if ((bytes >> p) & 1u) pra_lds_pass<BLOCK, IT>(L, key, id, m, 8 * p);
+}
+
+// The block's m pairs into key order, given the key bits in which they may
+// differ: two counting passes over the sixteen highest of them, then every
+// pair's place among its neighbours that share those bits (before(j, i): index
+// j sorts before index i, their keys being equal).  The pairs of a block
+// are few beside 2^16 digits, so most have no such neighbour: two passes (each
+// five barriers and a digit scan, about 3 us) where LSD passes take one for
+// each varying byte.  False, with the pairs permuted, when a group is over
+// PRA_GROUP_MAX.
+template <int BLOCK, int IT, typename F>
+__device__ __forceinline__ bool pra_lds_group_sort(SortLds<BLOCK, IT>& L, u64 (&key)[IT], u32 (&id)[IT], u32 m,
+                                                   u64 vary, u32* s_far, F before)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int hb = vary ? 63 - __clzll(vary) : 0, shift = hb > 15 ? hb - 15 : 0;
+    if (threadIdx.x == 0) *s_far = 0;
+    pra_lds_pass<BLOCK, IT>(L, key, id, m, shift);
+    if (hb - shift >= 8) pra_lds_pass<BLOCK, IT>(L, key, id, m, shift + 8);
+    int pos[IT];
+    u32 far = 0, moved = 0;
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const int i = wave * 64 * IT + k * 64 + lane;
+        pos[k] = i;
+        if ((u32)i >= m) continue;
+        const u64 g = key[k] >> shift;
+        int r = i, steps = 0;
+        for (int j = i - 1; j >= 0 && steps <= PRA_GROUP_MAX; j--, steps++) {
+            const u64 kj = L.key[j];
+            if ((kj >> shift) != g) break;
+            if (kj > key[k] || (kj == key[k] && !before(L.idx[j], id[k], true))) r--;
+        }
+        far |= steps > PRA_GROUP_MAX;
+        steps = 0;
+        for (int j = i + 1; j < (int)m && steps <= PRA_GROUP_MAX; j++, steps++) {
+            const u64 kj = L.key[j];
+            if ((kj >> shift) != g) break;
+            if (kj < key[k] || (kj == key[k] && before(L.idx[j], id[k], false))) r++;
+        }
+        far |= steps > PRA_GROUP_MAX;
+        moved |= r != i;
+        pos[k] = r;
+    }
+    if (far || moved) atomicOr(s_far, far ? 3u : 1u);
+    __syncthreads();
+    const u32 st = *s_far;
+    if (st & 2) return false;
+    if (!st) return true;
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const int i = wave * 64 * IT + k * 64 + lane;
+        if ((u32)i < m) {
+            L.key[pos[k]] = key[k];
+            L.idx[pos[k]] = id[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const int i = wave * 64 * IT + k * 64 + lane;
+        if ((u32)i < m) {
+            key[k] = L.key[i];
+            id[k] = L.idx[i];
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
+// Row sort keys: the varying bits of (bucket, col0, col1, ..) concatenated,
+// most significant first, and cut into 64-bit words (word 0 the leading one,
+// the last one padded with zeros below).  Comparing the words orders rows as
+// comparing (bucket, columns) does, since the bits left out are the same in
+// every row.
+__device__ __forceinline__ u64 pra_key_word(const u64* row, const KeyLayout& L, int q, bool* miss)
+{
+    u64 out = 0;
+    int at = 0;
+    for (int j = 0; j < L.nf && at < 64 * (q + 1); j++) {
+        const int bits = L.f[j].bits, end = at + bits - 64 * q;
+        if (end > 0) {
+            u64 v;
+            if (L.f[j].col < 0)
+                v = pra_bucket(pra_fnv(row, L.jcc), L.nb);
+            else if (!L.f[j].rank)
+                v = row[L.f[j].col] >> L.f[j].shift;
+            else if (!pra_dict_rank(L.dict, L.dict_cap, row[L.f[j].col], &v))
+                *miss = true;
+            if (bits < 64) v &= (1ULL << bits) - 1;
+            out |= end <= 64 ? v << (64 - end) : v >> (end - 64);
+        }
+        at += bits;
+    }
+    return out;
+}
+
+// bits in which the block's m keys differ
+template <int BLOCK, int IT>
+__device__ __forceinline__ u64 pra_block_vary(const u64 (&key)[IT], u32 m, u64* s_or, u64* s_and)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    u64 o = 0, a = ~0ULL;
+#pragma unroll
+    for (int k = 0; k < IT; k++)
+        if ((u32)wave * 64 * IT + (u32)k * 64 + lane < m) {
+            o |= key[k];
+            a &= key[k];
+        }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        o |= __shfl_xor(o, d, 64);
+        a &= __shfl_xor(a, d, 64);
+    }
+    __syncthreads();
+    if (lane == 0) {
+        s_or[wave] = o;
+        s_and[wave] = a;
+    }
+    __syncthreads();
+    o = 0;
+    a = ~0ULL;
+    for (int v = 0; v < BLOCK / 64; v++) {
+        o |= s_or[v];
+        a &= s_and[v];
+    }
+    return m > 1 ? o ^ a : 0;
+}
+
+__device__ __forceinline__ u32 pra_vary_bytes(u64 vary)
+{
+    u32 bytes = 0;
+    for (int p = 0; p < 8; p++)
+        if ((vary >> (8 * p)) & 255) bytes |= 1u << p;
+    return bytes;
+}
+
+// The block's m pairs (key word 0, row index) into the order of the rows'
+// whole keys: by groups of word 0 when they are small, rows that share word 0
+// compared by their later words; else by LSD passes over every word, the last
+// word first.
+// (later, when not null: words 1 .. nlater of row i's key at later[(q - 1) *
+// BLOCK * IT + i]).  *dup, when not null, is set when two rows' keys are equal,
+// and where the LSD passes did not look.
+template <int BLOCK, int IT>
+__device__ __forceinline__ void pra_lds_sort_rows(SortLds<BLOCK, IT>& S, const KeyLayout& L, const u64* rows, int w,
+                                                  u64 (&key)[IT], u32 (&id)[IT], u32 m, u64* s_or, u64* s_and,
+                                                  u32* s_max, u64* dup, const u64* later = nullptr, int nlater = 0)
+{
+    if (m < 2) return;
+    bool same = false;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int words = (L.bits + 63) / 64;
+    bool miss = false;   // ranks are used in keys of one word only
+    const u64 vary = pra_block_vary<BLOCK, IT>(key, m, s_or, s_and);
+    if (pra_lds_group_sort<BLOCK, IT>(S, key, id, m, vary, s_max, [&](u32 idj, u32 idi, bool equal_order) {
+            for (int q = 1; q < words; q++) {
+                const bool held = q <= nlater;
+                const u64 a = held ? later[(q - 1) * BLOCK * IT + idj] : pra_key_word(rows + (u64)idj * w, L, q, &miss);
+                const u64 b = held ? later[(q - 1) * BLOCK * IT + idi] : pra_key_word(rows + (u64)idi * w, L, q, &miss);
+                if (a != b) return a < b;
+            }
+            same = true;
+            return equal_order;   // equal rows keep their places
+        })) {
+        if (dup && same) *dup = 1;
+        return;
+    }
+    if (dup && threadIdx.x == 0) *dup = 1;
+    for (int q = words - 1; q >= 0; q--) {
+        if (q || words > 1) {
+#pragma unroll
+            for (int k = 0; k < IT; k++)
+                if ((u32)wave * 64 * IT + (u32)k * 64 + lane < m) key[k] = pra_key_word(rows + (u64)id[k] * w, L, q, &miss);
+        }
+        pra_lds_lsd<BLOCK, IT>(S, key, id, m, pra_vary_bytes(pra_block_vary<BLOCK, IT>(key, m, s_or, s_and)));
+    }
+}
+
+// One block sorts n <= PRA_SMALL_SORT rows by (bucket, col0 .. col[kc-1]) (the
+// bucket FNV(row[0:jcc]) % nb leads when `bucketed`; columns compare as
+// unsigned words) and gathers them into `out`.  The key layout comes from the
+// columns' varying bits, which the block collects first; equal rows keep
+// their order.  With bnd (bucketed), bnd[s] = first row of bucket s, bnd[nb]
+// = n.  BLOCK threads hold up to 2 * BLOCK rows.  Bound by barriers and the
+// latency of a single block, so it takes two counting passes and a look at the
+// neighbours instead of a network's log^2 steps, and 256 threads where they
+// hold the rows.  1,300 edges of random 64-bit values in 8 buckets: 68 us as a
+// bitonic network over multi-word keys, 32 us; 60 edges 16 -> 14 us.
+template <int BLOCK>
+__device__ __forceinline__ void pra_small_sort_block(const u64* rows, u64 n, int w, int jcc, int kc, u64 nb,
+                                                     int bucketed, u64* out, u64* bnd, u64* dup)
+{
+    constexpr int IT = 2, LATER = 2;
+    __shared__ SortLds<BLOCK, IT> S;
+    __shared__ u64 later[LATER * BLOCK * IT];
+    __shared__ KeyLayout L;
+    __shared__ u64 s_or[BLOCK / 64], s_and[BLOCK / 64];
+    __shared__ unsigned long long c_or[PRA_MAXW], c_and[PRA_MAXW];
+    __shared__ u32 s_max;
+    const u32 m = (u32)n;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x < PRA_MAXW) {
+        c_or[threadIdx.x] = 0;
+        c_and[threadIdx.x] = ~0ULL;
+    }
+    __syncthreads();
+    for (int c = 0; c < kc; c++) {
+        u64 o = 0, a = ~0ULL;
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+            if (i < m) {
+                const u64 v = rows[(u64)i * w + c];
+                o |= v;
+                a &= v;
+            }
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            o |= __shfl_xor(o, d, 64);
+            a &= __shfl_xor(a, d, 64);
+        }
+        if (lane == 0) {
+            atomicOr(&c_or[c], (unsigned long long)o);
+            atomicAnd(&c_and[c], (unsigned long long)a);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        L.nb = nb;
+        L.jcc = jcc;
+        L.nf = L.bits = 0;
+        if (bucketed) pra_key_field(L, -1, 0, 64 - __clzll(nb - 1));
+        for (int c = 0; c < kc; c++) {
+            const u64 vary = c_or[c] ^ c_and[c];
+            if (vary && m > 1) pra_key_field(L, c, __ffsll((long long)vary) - 1, 65 - __clzll(vary) - __ffsll((long long)vary));
+        }
+    }
+    __syncthreads();
+    u64 key[IT];
+    u32 id[IT];
+    bool miss = false;
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+        key[k] = i < m ? pra_key_word(rows + (u64)i * w, L, 0, &miss) : 0;
+        id[k] = i;
+    }
+    const int nlater = min(LATER, (L.bits + 63) / 64 - 1);
+    for (int q = 1; q <= nlater; q++)
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+            if (i < m) later[(q - 1) * BLOCK * IT + i] = pra_key_word(rows + (u64)i * w, L, q, &miss);
+        }
+    __syncthreads();
+    pra_lds_sort_rows<BLOCK, IT>(S, L, rows, w, key, id, m, s_or, s_and, &s_max, dup, later, nlater);
+    __syncthreads();
+    const bool bounds = bnd && bucketed;
+    const int bsh = 64 - (bucketed ? L.f[0].bits : 0);
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+        if (i < m) {
+            pra_copy_row(out + (u64)i * w, rows + (u64)id[k] * w, w);
+            if (bounds) S.key[i] = key[k];
+        }
+    }
+    if (bounds) {
+        __syncthreads();
+        for (u32 i = threadIdx.x; i <= m; i += BLOCK) {
             // buckets (prev, cur] start at row i
-            const u64 prev = i == 0 ? 0 : key[(u64)idx[i - 1] * kw] + 1;
-            const u64 cur = i == m ? nb : key[(u64)idx[i] * kw];
+            const u64 prev = i == 0 ? 0 : (S.key[i - 1] >> bsh) + 1;
+            const u64 cur = i == m ? nb : S.key[i] >> bsh;
             for (u64 s = prev; s <= cur && s <= nb; s++) bnd[s] = i;
         }
     }
 }
 
-__global__ __launch_bounds__(PRA_SMALL_SORT_BLOCK) void k_small_sort(const u64* rows, u64 n, int w, int jcc, int kc,
-                                                                     u64 nb, int bucketed, u64* out, u64* bnd)
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_small_sort(const u64* rows, u64 n, int w, int jcc, int kc, u64 nb,
+                                                      int bucketed, u64* out, u64* bnd, u64* dup)
 {
-    pra_small_sort_block(rows, n, w, jcc, kc, nb, bucketed, out, bnd);
+    pra_small_sort_block<BLOCK>(rows, n, w, jcc, kc, nb, bucketed, out, bnd, dup);
 }
 
 // Independent small sorts (one per output relation of an iteration), one
 // block each.
-__global__ __launch_bounds__(PRA_SMALL_SORT_BLOCK) void k_small_sort_many(SmallSortBatch b)
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_small_sort_many(SmallSortBatch b)
 {
     const SmallSortJob& j = b.job[blockIdx.x];
-    pra_small_sort_block(j.rows, j.n, j.w, j.jcc, j.kc, b.nb, j.bucketed, j.out, j.bnd);
+    pra_small_sort_block<BLOCK>(j.rows, j.n, j.w, j.jcc, j.kc, b.nb, j.bucketed, j.out, j.bnd, nullptr);
+}
+
+// ------------------------------------------------------ keyed row sort -----
+//
+// Rows too many for one block: word 0 of every row's key and its index go
+// through one or two counting passes over the key's top bytes, then each
+// segment of equal top bits is sorted in LDS by its whole keys and its rows
+// gathered.  A row is read once for its key and once by the gather (and again
+// for later key words where rows of a segment share word 0), where byte
+// passes over whole rows read and write it once per varying byte.  2 M rows of
+// 4 words (19 varying bytes, 8 buckets): 1.77 ms of byte passes and
+// histogram, 0.30 ms this way; 13,000 edges: 275 us in one block, 60 us.
+
+// word 0 of the rows' keys, and the digit counts of its top np bytes (hist:
+// np x 256, the pass over the lower byte first); a column value without a
+// dictionary rank sets *missing
+__global__ void k_sort_keys(const u64* rows, u64 n, int w, KeyLayout L, int np, u64* keys, u32* hist, u64* missing)
+{
+    bool miss = false;
+    __shared__ u32 sh[2 * PRA_RADIX];
+    for (int i = threadIdx.x; i < np * PRA_RADIX; i += PRA_BLOCK) sh[i] = 0;
+    __syncthreads();
+    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    const u64 step = (u64)gridDim.x * blockDim.x;
+    for (; i < n; i += step) {
+        const u64 k = pra_key_word(rows + i * w, L, 0, &miss);
+        keys[i] = k;
+        atomicAdd(&sh[(np - 1) * PRA_RADIX + (u32)(k >> 56)], 1u);
+        if (np == 2) atomicAdd(&sh[(u32)(k >> 48) & 255u], 1u);
+    }
+    if (miss) *missing = 1;
+    __syncthreads();
+    for (int j = threadIdx.x; j < np * PRA_RADIX; j += PRA_BLOCK)
+        if (sh[j]) atomicAdd(&hist[j], sh[j]);
+}
+
+// Segment b of the pairs (seg: the segments' first positions, as
+// k_seg_bounds leaves them, or the top byte's 256 digit offsets when seg is
+// null) by a block of BLOCK threads.
+template <int BLOCK>
+__device__ __forceinline__ void pra_keyseg_sort(const u64* keys, const u32* idx, u64 start, u64 end, u64 n,
+                                                const u64* rows, int w, const KeyLayout& L, u64* out, u64* bnd,
+                                                u64* dup, const u32 b, const int top)
+{
+    constexpr int IT = PRA_BIN_ITEMS;
+    __shared__ SortLds<BLOCK, IT> S;
+    __shared__ u64 s_or[BLOCK / 64], s_and[BLOCK / 64];
+    __shared__ u32 s_max, below;
+    const int bbits = bnd ? L.f[0].bits : 0;
+    const u64 nb = bnd ? L.nb : 1;
+    if (bnd && b == 0 && threadIdx.x == 0) {
+        bnd[0] = 0;
+        bnd[nb] = n;
+    }
+    if (end <= start) {
+        for (u64 s = 1 + threadIdx.x; s < nb; s += BLOCK)
+            if (((s << (64 - bbits)) >> top) == b) bnd[s] = start;
+        return;
+    }
+    const u32 m = (u32)(end - start);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    u64 key[IT];
+    u32 id[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+        key[k] = 0;
+        id[k] = 0;
+        if (i < m) {
+            key[k] = keys[start + i];
+            id[k] = idx[start + i];
+        }
+    }
+    pra_lds_sort_rows<BLOCK, IT>(S, L, rows, w, key, id, m, s_or, s_and, &s_max, dup);
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u32 i = (u32)wave * 64 * IT + (u32)k * 64 + lane;
+        if (i < m) pra_copy_row(out + (start + i) * w, rows + (u64)id[k] * w, w);
+    }
+    for (u64 s = 1; s < nb; s++) {
+        const u64 T = s << (64 - bbits);
+        if ((T >> top) != b) continue;
+        __syncthreads();
+        if (threadIdx.x == 0) below = 0;
+        __syncthreads();
+        u32 cnt = 0;
+#pragma unroll
+        for (int k = 0; k < IT; k++)
+            if ((u32)wave * 64 * IT + (u32)k * 64 + lane < m && key[k] < T) cnt++;
+        if (cnt) atomicAdd(&below, cnt);
+        __syncthreads();
+        if (threadIdx.x == 0) bnd[s] = start + below;
+    }
+    __syncthreads();
+}
+
+// one block of 256 threads per segment of at most PRA_SEG_SMALL pairs
+__global__ __launch_bounds__(PRA_BLOCK) void k_keyseg_small(const u64* keys, const u32* idx, const u64* seg,
+                                                            const u32* gofs, int top, u64 n, const u64* rows, int w,
+                                                            KeyLayout L, u64* out, u64* bnd, u64* status)
+{
+    const u32 b = blockIdx.x;
+    const u64 start = seg ? seg[b] : gofs[b];
+    const u64 end = seg ? seg[b + 1] : b + 1 < PRA_RADIX ? (u64)gofs[b + 1] : n;
+    if (end - start > PRA_SEG_SMALL) return;
+    pra_keyseg_sort<PRA_BLOCK>(keys, idx, start, end, n, rows, w, L, out, bnd, status + 1, b, top);
+}
+
+// the larger segments, by blocks that take every gridDim.x-th of them (list
+// and count from k_seg_bounds; every segment in turn when seg is null); one
+// over PRA_BIN_CAP pairs sets status[0] and is left unsorted
+__global__ __launch_bounds__(PRA_BIN_BLOCK) void k_keyseg_large(const u64* keys, const u32* idx, const u64* seg,
+                                                                const u32* gofs, const u32* list, const u64* stat,
+                                                                int top, u64 n, const u64* rows, int w, KeyLayout L,
+                                                                u64* out, u64* bnd, u64* status)
+{
+    const u64 cnt = seg ? stat[1] : PRA_RADIX;
+    for (u64 i = blockIdx.x; i < cnt; i += gridDim.x) {
+        const u32 b = seg ? list[i] : (u32)i;
+        const u64 start = seg ? seg[b] : gofs[b];
+        const u64 end = seg ? seg[b + 1] : b + 1 < PRA_RADIX ? (u64)gofs[b + 1] : n;
+        if (end - start <= PRA_SEG_SMALL) continue;
+        if (end - start > PRA_BIN_CAP) {
+            if (threadIdx.x == 0) status[0] = 1;
+            continue;
+        }
+        pra_keyseg_sort<PRA_BIN_BLOCK>(keys, idx, start, end, n, rows, w, L, out, bnd, status + 1, b, top);
+    }
 }
 
 // One block sorts n <= PRA_BLOCK_SORT rows with all the LSD passes of `pl`
@@ -383,8 +861,8 @@ __global__ __launch_bounds__(PRA_BIN_BLOCK) void k_block_sort(const u64* rows, u
     if (bnd) {
         // buckets (bucket of row i-1, bucket of row i] start at row i
         for (u32 i = threadIdx.x; i <= m; i += PRA_BIN_BLOCK) {
-            const u64 prev = i == 0 ? 0 : pra_fnv(rows + (u64)sidx[i - 1] * w, jcc) % nb + 1;
-            const u64 cur = i == m ? nb : pra_fnv(rows + (u64)sidx[i] * w, jcc) % nb;
+            const u64 prev = i == 0 ? 0 : pra_bucket(pra_fnv(rows + (u64)sidx[i - 1] * w, jcc), nb) + 1;
+            const u64 cur = i == m ? nb : pra_bucket(pra_fnv(rows + (u64)sidx[i] * w, jcc), nb);
             for (u64 s = prev; s <= cur && s <= nb; s++) bnd[s] = i;
         }
     }
@@ -413,32 +891,7 @@ __global__ void k_col_orand2(const u64* rows, u64 n, int w, u64* out /* [0..15] 
     }
 }
 
-// ------------------------------------------------------ value dictionary ---
-//
-// An order-preserving dictionary of the values in the relations' key columns
-// (rank(a) < rank(b) iff a < b) lets a newt row's sort key
-// (bucket, col0, .., col[a-1]) be packed into one u64: the bucket and the
-// column ranks as digits of radix D (the dictionary size), which the sort
-// then orders in a few byte passes.
-// Slots: [value, rank + 1]; rank + 1 == 0 marks an empty slot.
-
-__device__ inline u64 pra_dict_slot(u64 v, u64 cap) { return pra_mix64(v ^ 0x5851F42D4C957F2DULL) & (cap - 1); }
-
-__device__ inline bool pra_dict_rank(const u64* tab, u64 cap, u64 v, u64* rank)
-{
-    u64 m = cap - 1, s = pra_dict_slot(v, cap);
-    for (u64 q = 0; q < cap; q++) {
-        const u64* sl = tab + 2 * s;
-        u64 r = sl[1];
-        if (r == 0) return false;
-        if (sl[0] == v) {
-            *rank = r - 1;
-            return true;
-        }
-        s = (s + 1) & m;
-    }
-    return false;
-}
+// ------------------------------------------------- dictionary and views ---
 
 __global__ void k_collect_cols(const u64* rows, u64 n, int w, int ncols, u64* out)
 {
@@ -454,7 +907,7 @@ __global__ void k_view_keep(const u64* rows, u64 n, int w, int ja, int jb, u64 n
     u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const u64* r = rows + i * w;
-    keep[i] = (pra_fnv(r, ja) % nb) == (pra_fnv(r, jb) % nb) ? 1u : 0u;
+    keep[i] = pra_bucket(pra_fnv(r, ja), nb) == pra_bucket(pra_fnv(r, jb), nb) ? 1u : 0u;
 }
 
 // the kept rows, in order, at their exclusive-prefix positions
@@ -520,11 +973,7 @@ __device__ __forceinline__ void pra_bin_sort_range(const u64* keys, const u32* i
     constexpr u32 CAP = BLOCK * PRA_BIN_ITEMS;
     constexpr int WAVES = BLOCK / 64;
     constexpr u32 PER_WAVE = CAP / WAVES;
-    static_assert(BLOCK >= PRA_RADIX, "the digit scan takes a thread per digit");
-    __shared__ u64 skey[CAP];
-    __shared__ u32 sidx[CAP];
-    __shared__ u32 wh[WAVES][PRA_RADIX];
-    __shared__ u32 wsum[PRA_RADIX / 64];
+    __shared__ SortLds<BLOCK, IT> L;
     __shared__ u32 below;
     if (b == 0 && threadIdx.x == 0) {
         bnd[0] = 0;
@@ -541,7 +990,6 @@ __device__ __forceinline__ void pra_bin_sort_range(const u64* keys, const u32* i
     }
     const u32 m = (u32)(end - start);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const u64 lt = pra_lanemask_lt();
     u64 key[IT];
     u32 id[IT];
 #pragma unroll
@@ -554,74 +1002,7 @@ __device__ __forceinline__ void pra_bin_sort_range(const u64* keys, const u32* i
             id[k] = idx[i];
         }
     }
-#pragma unroll 1
-    for (int p = 0; p < 8; p++) {
-        if (!((bytes >> p) & 1u)) continue;
-        for (int i = threadIdx.x; i < WAVES * PRA_RADIX; i += BLOCK) (&wh[0][0])[i] = 0;
-        __syncthreads();
-        // stable rank of every pair among the pairs of its digit: wave-local
-        // counts in element order, then a scan over waves and digits
-        u32 dg[IT], lc[IT];
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
-            bool valid = i < m;
-            dg[k] = 0;
-            lc[k] = 0;
-            // a wave skips the ranking of item rows wholly past the bin
-            if ((u32)wave * PER_WAVE + (u32)k * 64 >= m) continue;
-            u32 d = valid ? (u32)(key[k] >> (8 * p)) & 255u : 0u;
-            u64 peers = pra_match<PRA_RADIX_BITS>(d, __ballot(valid));
-            dg[k] = d;
-            if (valid) {
-                u32 before = wh[wave][d];
-                lc[k] = before + (u32)__popcll(peers & lt);
-                if ((peers >> lane) == 1ULL) wh[wave][d] = before + (u32)__popcll(peers);
-            }
-        }
-        __syncthreads();
-        const int d = threadIdx.x;   // digit of this thread in the scan (threads < PRA_RADIX)
-        u32 acc = 0;
-        if (d < PRA_RADIX)
-            for (int v = 0; v < WAVES; v++) {
-                u32 t = wh[v][d];
-                wh[v][d] = acc;
-                acc += t;
-            }
-        u32 x = acc;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            u32 y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (d < PRA_RADIX && lane == 63) wsum[wave] = x;
-        __syncthreads();
-        if (d < PRA_RADIX) {
-            u32 base = x - acc;
-            for (int v = 0; v < wave; v++) base += wsum[v];
-            for (int v = 0; v < WAVES; v++) wh[v][d] += base;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
-            if (i < m) {
-                u32 pos = wh[wave][dg[k]] + lc[k];
-                skey[pos] = key[k];
-                sidx[pos] = id[k];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            u32 i = (u32)wave * PER_WAVE + (u32)k * 64 + lane;
-            if (i < m) {
-                key[k] = skey[i];
-                id[k] = sidx[i];
-            }
-        }
-        __syncthreads();
-    }
+    pra_lds_lsd<BLOCK, IT>(L, key, id, m, bytes);
     for (u64 s = 1; s < nb; s++) {
         const u64 T = (s * bmul) << ls;
         if ((T >> top) != b) continue;
@@ -776,7 +1157,7 @@ __global__ void k_bucket_bounds(const u64* rows, u64 n, int w, int jcc, u64 nb, 
     u64 lo = 0, hi = n;
     while (lo < hi) {
         u64 mid = (lo + hi) >> 1;
-        u64 b = pra_fnv(rows + mid * w, jcc) % nb;
+        u64 b = pra_bucket(pra_fnv(rows + mid * w, jcc), nb);
         if (b < s) lo = mid + 1; else hi = mid;
     }
     bstart[s] = lo;
@@ -872,7 +1253,7 @@ __device__ inline int pra_row_cmp(const u64* a, const u64* b, int n)
 __device__ inline u64 pra_sorted_run(const u64* key, int jcc, const u64* inner, int wi, const u64* ibnd, u64 nb,
                                      u64* first_out)
 {
-    u64 b = nb == 1 ? 0 : pra_fnv(key, jcc) % nb;
+    u64 b = nb == 1 ? 0 : pra_bucket(pra_fnv(key, jcc), nb);
     u64 lo = ibnd[b], hi = ibnd[b + 1];
     u64 a = lo, z = hi;   // first row >= key
     while (a < z) {
@@ -1017,7 +1398,7 @@ __device__ __forceinline__ void pra_join_expand_block(const JoinExpandArgs& a, u
         }
         const u64* d = a.outer + i * a.wo;
         const u64* f = a.inner + (a.istart[i] + (o - a.off[i])) * a.wi;
-        u64 s = a.nb == 1 ? 0 : pra_fnv(d, a.jcc) % a.nb;
+        u64 s = a.nb == 1 ? 0 : pra_bucket(pra_fnv(d, a.jcc), a.nb);
         u64 pos = a.posadj[s] + o;
         u64* dst = a.cand + pos * a.cw;
         // the destination bucket hashes the output's first out_jcc columns
@@ -1033,7 +1414,7 @@ __device__ __forceinline__ void pra_join_expand_block(const JoinExpandArgs& a, u
             dst[c] = v;
             if (c < a.out_jcc) h = pra_fnv_word(h, v);
         }
-        a.dest[pos] = a.nb == 1 ? 0u : (u32)(h % a.nb);
+        a.dest[pos] = a.nb == 1 ? 0u : pra_bucket(h, a.nb);
     }
 }
 
@@ -1090,7 +1471,7 @@ __device__ __forceinline__ void pra_copy_expand_row(const CopyExpandArgs& a, u64
     if (i >= a.n) return;
     if (a.off[i + 1] == a.off[i]) return;
     const u64* r = a.rows + i * a.w;
-    u64 s = a.nb == 1 ? 0 : pra_fnv(r, a.in_jcc) % a.nb;
+    u64 s = a.nb == 1 ? 0 : pra_bucket(pra_fnv(r, a.in_jcc), a.nb);
     u64 pos = a.posadj[s] + a.off[i];
     u64* dst = a.cand + pos * a.cw;
     u64 h = PRA_FNV_OFFSET;
@@ -1099,7 +1480,7 @@ __device__ __forceinline__ void pra_copy_expand_row(const CopyExpandArgs& a, u64
         dst[c] = v;
         if (c < a.out_jcc) h = pra_fnv_word(h, v);
     }
-    a.dest[pos] = a.nb == 1 ? 0u : (u32)(h % a.nb);
+    a.dest[pos] = a.nb == 1 ? 0u : pra_bucket(h, a.nb);
 }
 
 __global__ void k_copy_expand(CopyExpandArgs a)
@@ -1725,7 +2106,7 @@ __global__ void k_bm_runs(const u64* bm, u64 words, const u32* prefix, const u64
 {
     const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (r0 >= D) return;
-    const u64 mine = pra_fnv_word(PRA_FNV_OFFSET, vals[r0]) % nb;
+    const u64 mine = pra_bucket(pra_fnv_word(PRA_FNV_OFFSET, vals[r0]), nb);
     const u32 c = pra_bm_rank(bm, words, prefix, (r0 + 1) * S) - pra_bm_rank(bm, words, prefix, r0 * S);
     for (u64 b = 0; b < nb; b++) runs[b * D + r0] = b == mine ? c : 0u;
 }
@@ -1737,7 +2118,7 @@ __global__ void k_bm_adjust(const u64* bm, u64 words, const u32* prefix, const u
     const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (r0 <= nb) bnd[r0] = r0 < nb ? (u64)scan[r0 * D] : n;
     if (r0 >= D) return;
-    const u64 mine = pra_fnv_word(PRA_FNV_OFFSET, vals[r0]) % nb;
+    const u64 mine = pra_bucket(pra_fnv_word(PRA_FNV_OFFSET, vals[r0]), nb);
     adj[r0] = scan[mine * D + r0] - pra_bm_rank(bm, words, prefix, r0 * S);
 }
 
@@ -2770,16 +3151,43 @@ void pra_launch_bin_sort(hipStream_t st, const u64* bin_keys, const u32* bin_idx
 #undef PRA_BIN_SORT
 }
 
-void pra_launch_small_sort(hipStream_t st, const u64* rows, u64 n, int w, int jcc, int kc, u64 nb, int bucketed,
-                           u64* out, u64* bnd)
+void pra_launch_sort_keys(hipStream_t st, const u64* rows, u64 n, int w, const KeyLayout& L, int np, u64* keys, u32* hist,
+                          u64* missing)
 {
-    hipLaunchKernelGGL(k_small_sort, dim3(1), dim3(PRA_SMALL_SORT_BLOCK), 0, st, rows, n, w, jcc, kc, nb, bucketed, out,
-                       bnd);
+    hipLaunchKernelGGL(k_sort_keys, dim3(std::min<unsigned>(grid_for(n), 2048)), dim3(PRA_BLOCK), 0, st, rows, n, w, L,
+                       np, keys, hist, missing);
+}
+
+void pra_launch_keyseg_sort(hipStream_t st, const u64* keys, const u32* idx, const u64* seg, const u32* gofs, u32 nseg,
+                            const u32* list, const u64* stat, int top, u64 n, const u64* rows, int w,
+                            const KeyLayout& L, u64* out, u64* bnd, u64* status)
+{
+    hipLaunchKernelGGL(k_keyseg_small, dim3(nseg), dim3(PRA_BLOCK), 0, st, keys, idx, seg, gofs, top, n, rows, w, L,
+                       out, bnd, status);
+    hipLaunchKernelGGL(k_keyseg_large, dim3(std::min<u32>(nseg, 256)), dim3(PRA_BIN_BLOCK), 0, st, keys, idx, seg, gofs,
+                       list, stat, top, n, rows, w, L, out, bnd, status);
+}
+
+void pra_launch_small_sort(hipStream_t st, const u64* rows, u64 n, int w, int jcc, int kc, u64 nb, int bucketed,
+                           u64* out, u64* bnd, u64* dup)
+{
+    if (n <= 2 * PRA_BLOCK)
+        hipLaunchKernelGGL(k_small_sort<PRA_BLOCK>, dim3(1), dim3(PRA_BLOCK), 0, st, rows, n, w, jcc, kc, nb, bucketed,
+                           out, bnd, dup);
+    else
+        hipLaunchKernelGGL(k_small_sort<PRA_SMALL_SORT / 2>, dim3(1), dim3(PRA_SMALL_SORT / 2), 0, st, rows, n, w, jcc,
+                           kc, nb, bucketed, out, bnd, dup);
 }
 
 void pra_launch_small_sort_many(hipStream_t st, const SmallSortBatch& b, int njobs)
 {
-    if (njobs > 0) hipLaunchKernelGGL(k_small_sort_many, dim3(njobs), dim3(PRA_SMALL_SORT_BLOCK), 0, st, b);
+    if (njobs <= 0) return;
+    u64 most = 0;
+    for (int k = 0; k < njobs; k++) most = std::max(most, b.job[k].n);
+    if (most <= 2 * PRA_BLOCK)
+        hipLaunchKernelGGL(k_small_sort_many<PRA_BLOCK>, dim3(njobs), dim3(PRA_BLOCK), 0, st, b);
+    else
+        hipLaunchKernelGGL(k_small_sort_many<PRA_SMALL_SORT / 2>, dim3(njobs), dim3(PRA_SMALL_SORT / 2), 0, st, b);
 }
 
 void pra_launch_block_sort(hipStream_t st, const u64* rows, u64 n, int w, const PassList& pl, u64* out, u64* bnd,

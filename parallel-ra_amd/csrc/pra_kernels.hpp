@@ -351,8 +351,22 @@ void pra_launch_view_compact(hipStream_t st, const u64* rows, u64 n, int w, cons
 void pra_launch_dict_insert(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* flags);
 void pra_launch_gather_rows(hipStream_t st, const u64* in, const u32* idx, u64 n, int w, u64* out);
 void pra_launch_key_bounds(hipStream_t st, const u64* keys, u64 n, u64 bmul, int ls, u64 nb, u64* bnd);
+// Keyed row sort of more rows than one block holds: word 0 of every row's key
+// (and the digit counts of its top np bytes), the caller's counting passes
+// over (keys, idx), then the segments of equal top bits, each sorted in LDS by
+// its whole keys with its rows gathered into out.  seg / list / stat: from
+// pra_launch_seg_bounds, or null: the segments are the top byte's, first
+// positions gofs.  bnd (nullable; field 0 is the bucket): the bucket bounds.
+// A value without the rank its field asks for sets *missing, a segment over
+// PRA_BIN_CAP pairs status[0]; the result is then of no use.  status[1]: set
+// when two rows' keys are equal (or may be).  The caller zeroes them.
+void pra_launch_sort_keys(hipStream_t st, const u64* rows, u64 n, int w, const KeyLayout& L, int np, u64* keys, u32* hist,
+                          u64* missing);
+void pra_launch_keyseg_sort(hipStream_t st, const u64* keys, const u32* idx, const u64* seg, const u32* gofs, u32 nseg,
+                            const u32* list, const u64* stat, int top, u64 n, const u64* rows, int w,
+                            const KeyLayout& L, u64* out, u64* bnd, u64* status);
 void pra_launch_small_sort(hipStream_t st, const u64* rows, u64 n, int w, int jcc, int kc, u64 nb, int bucketed,
-                           u64* out, u64* bnd);
+                           u64* out, u64* bnd, u64* dup = nullptr);
 void pra_launch_small_sort_many(hipStream_t st, const SmallSortBatch& b, int njobs);
 void pra_launch_block_sort(hipStream_t st, const u64* rows, u64 n, int w, const PassList& pl, u64* out, u64* bnd,
                            int jcc, u64 nb);

@@ -31,7 +31,7 @@ constexpr int kScanBlock = 1024;
 
 __device__ inline u32 part_bucket(const u64* __restrict__ rows, u64 i, int w, int jcc, u32 nb)
 {
-    return (u32)(pra_fnv(rows + i * (u64)w, jcc) % nb);
+    return pra_bucket(pra_fnv(rows + i * (u64)w, jcc), nb);
 }
 
 __global__ __launch_bounds__(kPartBlock) void k_part_hist(const u64* __restrict__ rows, u64 n, int w, int jcc,
