@@ -202,14 +202,18 @@ void small_flush(hipStream_t st)
 
 // Autotuned knobs, per device and band of log2(work): the dense claim
 // table's size (2, 4 or 8 slots per candidate of capacity, so a load of at
-// most 1/2, 1/4 or 1/8) and the newt scatter's block width (256 or 1,024
-// threads).  Neither changes a result: which arrival wins a key, and where
+// most 1/2, 1/4 or 1/8), the newt scatter's block width (256 or 1,024
+// threads), and whether a dense output takes the claim table (0) or ranked
+// membership (1).  None changes a result: which arrival wins a key, and where
 // every row and id goes, are the same under every variant.  Variants are
 // timed with events on single-output iterations, per candidate.
-enum { TUNE_DENSE_LOAD, TUNE_SCATTER_WIDE, TUNE_KNOBS };
-const char* const kTuneNames[TUNE_KNOBS] = {"dense_table_slots_log2_minus_1", "newt_scatter_wide"};
-const int kTuneVariants[TUNE_KNOBS] = {3, 2};
+enum { TUNE_DENSE_LOAD, TUNE_SCATTER_WIDE, TUNE_RANKED, TUNE_KNOBS };
+const char* const kTuneNames[TUNE_KNOBS] = {"dense_table_slots_log2_minus_1", "newt_scatter_wide", "ranked_membership"};
+const int kTuneVariants[TUNE_KNOBS] = {3, 2, 2};
 constexpr u64 kTuneMinCandidates = 1ULL << 16;
+// capacity from which a dense output takes ranked membership beside outputs of
+// the general table
+constexpr u64 kMixedRankedCandidates = 1ULL << 18;
 pra::Tuner g_tune(3);
 
 // Tuning cache: with PRA_AUTOTUNE_FILE set, the settled choices are read from
@@ -396,6 +400,11 @@ struct pra_rel {
     // kept current by the iterations that take the dense path; the
     // per-iteration claim table (empty between iterations)
     DBuf bm, dtab;
+    // ranked membership: the new keys' bitmap (zero between iterations), its
+    // superblocks' flags and prefixes, its lines' prefixes
+    DBuf fresh, dirty, sbpre, linep;
+    u64 fresh_sbs = 0;   // superblocks of the zeroed bitmap (0: none)
+    u64 sbs_use = 0;     // of them, those of the current rank space
     u64 bm_gen = ~0ULL, dtab_cap = 0, dtab_use = 0;   // slots allocated, slots in use this iteration
     int dtab_eb = -1;      // epoch bits of the claim table's slots (0: winners empty their slots)
     u32 dtab_epoch = 0;    // this iteration's epoch (slots of any other count as empty)
@@ -414,6 +423,7 @@ struct pra_rel {
     // bucket bounds per version
     DBuf bnd[2];
     bool bnd_valid[2] = {false, false};
+    DBuf next_bnd;   // the new rows' bounds, until they become the delta
     // set while an SCC runs: the relation is produced by one of its rules
     // (changes every iteration), and its full version is read by one of them
     // (so it is kept sorted by merging each delta into it)
@@ -465,12 +475,13 @@ struct KStat {
 enum {
     K_JOIN_COUNT, K_JOIN_EXPAND, K_COPY_EXPAND, K_DEDUP_CLAIM, K_DEDUP_DECIDE, K_DEDUP_VERIFY, K_DEDUP_SCATTER,
     K_RADIX_HIST, K_RADIX_SCATTER, K_TABLE_BUILD, K_INDEX_BUILD, K_SCAN, K_GATHER, K_MERGE, K_BIN_SORT, K_SMALL_SORT,
-    K_BLOCK_SORT, K_COUNT
+    K_BLOCK_SORT, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE, K_COUNT
 };
 static const char* kNames[K_COUNT] = {"join_count", "join_expand", "copy_expand", "dedup_claim", "dedup_decide",
                                       "dedup_verify_hist", "dedup_scatter", "radix_hist", "radix_scatter",
                                       "table_build", "index_build", "scan", "gather_rows", "merge_full",
-                                      "bin_sort", "small_sort", "block_sort"};
+                                      "bin_sort", "small_sort", "block_sort", "rank_scan", "rank_first",
+                                      "rank_place"};
 
 } // namespace
 
@@ -479,9 +490,15 @@ static const char* kNames[K_COUNT] = {"join_count", "join_expand", "copy_expand"
 // has its own intern counters (the reference keeps them per LIE,
 // src/lie/lie.h:36), value dictionary, join-pair count and iteration count.
 struct Group {
-    std::map<u32, std::unique_ptr<DBuf>> seq;  // per intern tag: nb counters
+    // per intern tag: nb counters in two copies, of which `now` is current (a
+    // ranked iteration reads one and writes the other)
+    struct Seq {
+        DBuf buf;
+        int now = 0;
+    };
+    std::map<u32, std::unique_ptr<Seq>> seq;
     // order-preserving value dictionary for packed sort keys
-    DBuf dict, dict_vals;                    // value -> rank table; value of each rank
+    DBuf dict, rank_of;                      // value -> rank table; rank by bucket-major rank
     u64 dict_cap = 0, dict_n = 0;
     int dict_state = 0, dict_rebuilds = 0;   // state: 0 stale, 1 valid, 2 disabled
     u64 dict_gen = 0;                        // dictionary builds so far
@@ -511,7 +528,7 @@ struct pra_scc {
 // are staged between a publication and its wait, so they alternate between
 // two slots, and the wait of the iteration in between covers each copy.
 enum { JOB_EXPAND, JOB_SCATTER, JOB_DENSE, JOB_SCAN, JOB_FOLD, JOB_SORT, JOB_EARLY_APPEND, JOB_EARLY_APPEND2,
-       JOB_APPEND, JOB_PLAN, PRA_JOB_SLOTS };
+       JOB_APPEND, JOB_PLAN, JOB_RANK, PRA_JOB_SLOTS };
 
 struct pra_ctx {
     int device = 0, nb = 1;
@@ -527,6 +544,8 @@ struct pra_ctx {
     // scratch
     DBuf hist, offs, sort_tmp, flags_buf, stage, stage2, orand, tmp64a, tmp64b, tmp64c;
     DBuf cand, dest, slot_of, keep;
+    DBuf first;              // ranked membership: earliest arrival per new key, all ones between iterations
+    size_t first_words = 0;  // u32 words of it known to hold that
     DBuf ghist, gofs, lb_status, lb_ctr;
     DBuf part_scratch;   // pra_partition_rows
     // order-preserving value dictionary for packed sort keys
@@ -552,6 +571,17 @@ struct pra_ctx {
         u64 cap;
     };
     std::vector<TuneSample> tune_pending;
+    // a claim-table sample of the ranked-membership choice still to be joined
+    // by its sort (ranked membership needs none): its time so far, then the
+    // sort's events
+    struct LateSample {
+        int band;
+        size_t oi;
+        u64 n;
+        double ms;
+        hipEvent_t a, b;
+    };
+    std::vector<LateSample> tune_late;
     size_t lb_zeroed = 0;        // words of lb_status known to be zero-initialised
     u32 sort_epoch = 0;
     u64 dedup_epoch = 0;
@@ -582,12 +612,15 @@ struct pra_ctx {
         if (st) (void)hipStreamSynchronize(st);
         groups.clear();
         for (DBuf* b : {&hist, &offs, &sort_tmp, &flags_buf, &stage, &stage2, &orand, &tmp64a, &tmp64b,
-                        &tmp64c, &cand, &dest, &slot_of, &keep, &ghist, &gofs, &lb_status, &lb_ctr, &ktmp,
+                        &tmp64c, &cand, &dest, &slot_of, &keep, &first, &ghist, &gofs, &lb_status, &lb_ctr, &ktmp,
                         &idxa, &idxb, &posadj_dev, &rep_words, &rctl, &ttab, &kp, &part_scratch, &segb})
             b->release();
         for (DBuf& b : jobtab) b.release();
         if (st) small_flush(st);   // the small blocks kept for this stream, freed on it
         if (st) (void)hipStreamSynchronize(st);
+        for (auto& t : tune_late)
+            for (hipEvent_t e : {t.a, t.b})
+                if (e) evpool.push_back(e);
         for (auto e : evpool) (void)hipEventDestroy(e);
         if (st) {
             stream_idle(st);
@@ -1381,8 +1414,16 @@ static void build_dictionary(pra_ctx* c, int gi)
     pra_launch_fill_u64(c->st, G.dict.as<u64>(), cap * 2, 0);
     pra_launch_dict_insert(c->st, V.d(), V.n, G.dict.as<u64>(), cap, c->dflags());
     check_launch("dict_insert");
-    G.dict_vals.reserve(V.n * 8, c->st);
-    HIPCHK(hipMemcpyAsync(G.dict_vals.p, V.d(), V.n * 8, hipMemcpyDeviceToDevice, c->st));
+    if (c->nb > 1) {
+        c->sort_tmp.reserve(V.n * 8, c->st);
+        c->orand.reserve((size_t)(c->nb + 1) * 8, c->st);
+        c->part_scratch.reserve(pra_partition_scratch_words(V.n, (u32)c->nb) * 4 + 256, c->st);
+        pra_launch_partition(c->st, V.d(), V.n, 1, 1, (u32)c->nb, c->sort_tmp.as<u64>(), c->orand.as<u64>(),
+                             c->part_scratch.as<u32>());
+        G.rank_of.reserve(V.n * 4, c->st);
+        pra_launch_dict_bucket_rank(c->st, c->sort_tmp.as<u64>(), V.n, G.dict.as<u64>(), cap, G.rank_of.as<u32>());
+        check_launch("dict_bucket_rank");
+    }
     sync_check(c);
     G.dict_cap = cap;
     G.dict_n = V.n;
@@ -1390,41 +1431,49 @@ static void build_dictionary(pra_ctx* c, int gi)
     G.dict_gen++;
 }
 
+// The bits of a dense output's rank indexes put rows in trie order when a
+// row's bucket is a function of its first column (their leading digit is then
+// the bucket-major rank); with more join columns and several buckets they put
+// them in column order.
+static bool by_bucket(const pra_ctx* c, const pra_rel* R) { return c->nb > 1 && R->jcc == 1; }
+static bool bits_in_trie_order(const pra_ctx* c, const pra_rel* R) { return c->nb == 1 || R->jcc == 1; }
+
+// r's rows, in column order, into trie order: a stable partition by bucket;
+// bnd receives the bucket bounds
+static void bucket_rows(pra_ctx* c, const u64* rows, u64 n, int w, int jcc, u64* out, u64* bnd)
+{
+    c->part_scratch.reserve(pra_partition_scratch_words(n, (u32)c->nb) * 4 + 256, c->st);
+    pra_launch_partition(c->st, rows, n, w, jcc, (u32)c->nb, out, bnd, c->part_scratch.as<u32>());
+    check_launch("bucket_rows");
+}
+
 // Order an interned relation's full version through its membership bitmap
-// (k_bm_place): one read and one write of the rows, where the byte-pass sort
-// moves them once per varying byte of (bucket, columns).  Taken when the
-// bitmap holds exactly the keys of full -- current for the dictionary, keyed
-// on every column, no delta, as many set bits as rows -- and a row's bucket is
-// a function of column 0 (one bucket, or one join column).  The bitmap and
-// the buckets' runs are read once more, so a rank space of more than 64 words
-// a row, or a run table of more than 4 words a row, is left to the sort.
+// (k_bm_place): one read and one write of the rows, where a sort moves them
+// several times.  Taken when the bitmap holds exactly the keys of full --
+// current for the dictionary, keyed on every column, no delta, as many set
+// bits as rows.  The bitmap is read once more, so a rank space of more than 64
+// words a row is left to the sort.
 // Measured on the 150x150 grid (128 M rows of 24 bytes, 8 buckets), solve and
-// ordered result: 132.0 ms with the 26 byte passes, 63.8 ms this way; a
-// 20,000-vertex random graph on one bucket (72 M rows) 66.3 -> 30.3 ms.
-// False when the version is not of that kind.
+// ordered result: 132.0 ms with 26 byte passes over the rows, 63.8 ms this way;
+// a 20,000-vertex random graph on one bucket (72 M rows) 66.3 -> 30.3 ms.
+// False when the version is not of that kind, or there is no room.
 static bool order_by_bitmap(pra_ctx* c, pra_rel* R)
 {
     Group& G = grp(c, R->group);
     Rows& r = R->ver[PRA_FULL];
-    const u64 n = r.n, D = G.dict_n, nb = (u64)c->nb;
+    const u64 n = r.n, D = G.dict_n;
     const int kw = R->bm_kw;
-    if (!R->bm_valid || R->bm_gen != G.dict_gen || !G.dict_vals.p || kw != R->arity || R->ver[PRA_DELTA].n ||
-        n < 2 || n >= (1ULL << 32) || (nb > 1 && R->jcc != 1))
+    if (!R->bm_valid || R->bm_gen != G.dict_gen || kw != R->arity || R->ver[PRA_DELTA].n || n < 2 || n >= (1ULL << 32))
         return false;
-    u64 S = 1;
-    for (int i = 1; i < kw; i++) S *= D;
-    const u64 words = (S * D + 63) / 64, nblk = (words * 64 + PRA_BM_BITS - 1) / PRA_BM_BITS;
-    if (words > 64 * n + 4096 || (nb > 1 && nb * D > 4 * n + 16384)) return false;
+    u64 bits = 1;
+    for (int i = 0; i < kw; i++) bits *= D;
+    const u64 words = (bits + 63) / 64, nblk = (words * 64 + PRA_BM_BITS - 1) / PRA_BM_BITS;
+    if (words > 64 * n + 4096) return false;
     try {
         c->tmp64a.reserve((nblk + 2) * 4, c->st);
-        if (nb > 1) {
-            c->tmp64b.reserve((nb * D + 2) * 4, c->st);
-            c->tmp64c.reserve(D * 4, c->st);
-        }
     } catch (const PraError& e) {
-        // no room for the prefix: the sort needs less
         if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
-        for (DBuf* b : {&c->tmp64a, &c->tmp64b, &c->tmp64c}) b->release();
+        c->tmp64a.release();
         return false;
     }
     u32* prefix = c->tmp64a.as<u32>();
@@ -1432,27 +1481,22 @@ static bool order_by_bitmap(pra_ctx* c, pra_rel* R)
     pra_launch_bm_count(c->st, bm, words, nblk, prefix);
     scan_u32(c, prefix, prefix, nblk, prefix + nblk);
     if ((u32)readback(c, prefix + nblk, 1)[0] != (u32)n) return false;
-    u32* adj = nullptr;
-    if (nb > 1) {
-        u32* runs = c->tmp64b.as<u32>();
-        adj = c->tmp64c.as<u32>();
-        R->bnd[PRA_FULL].reserve((nb + 1) * 8, c->st);
-        pra_launch_bm_runs(c->st, bm, words, prefix, G.dict_vals.as<u64>(), D, S, nb, runs);
-        scan_u32(c, runs, runs, nb * D, runs + nb * D);
-        pra_launch_bm_adjust(c->st, bm, words, prefix, G.dict_vals.as<u64>(), D, S, nb, n, runs, adj,
-                             R->bnd[PRA_FULL].as<u64>());
-    }
     c->sort_tmp.reserve(n * R->w * 8, c->st);
     {
         Prof p(c, K_GATHER, 16.0 * n * R->w);
-        pra_launch_bm_place(c->st, r.d(), n, R->w, kw, G.dict.as<u64>(), G.dict_cap, D, S, bm, words, prefix, adj,
-                            c->sort_tmp.as<u64>());
+        pra_launch_bm_place(c->st, r.d(), n, R->w, kw, G.dict.as<u64>(), G.dict_cap, D, by_bucket(c, R), bm, words,
+                            prefix, c->sort_tmp.as<u64>());
         check_launch("bm_place");
     }
-    r.buf.swap(c->sort_tmp);
-    r.sorted = true;
     R->touched(PRA_FULL);
-    R->bnd_valid[PRA_FULL] = nb > 1;
+    if (bits_in_trie_order(c, R)) {
+        r.buf.swap(c->sort_tmp);
+    } else {
+        R->bnd[PRA_FULL].reserve((size_t)(c->nb + 1) * 8, c->st);
+        bucket_rows(c, c->sort_tmp.as<u64>(), n, R->w, R->jcc, r.d(), R->bnd[PRA_FULL].as<u64>());
+        R->bnd_valid[PRA_FULL] = true;
+    }
+    r.sorted = true;
     return true;
 }
 
@@ -1569,11 +1613,11 @@ static void ensure_member_table(pra_ctx* c, pra_rel* R, int kw, u64 incoming)
 
 // Dense membership of interned output R keyed on kw columns: the bitmap of
 // full u delta for the current dictionary (rebuilt when the dictionary or the
-// relation changed since it was built) and a claim table of at least 2C
-// slots.  False when the output does not allow it: more than 4 key columns, a
-// rank space over 2^35 bits, 2^28 or more candidates, or a value of full u
-// delta without a rank.
-static bool ensure_dense(pra_ctx* c, pra_rel* R, int kw, u64 C, u64 slots_per_candidate)
+// relation changed since it was built); *bits receives its rank space.  False
+// when the output does not allow it: more than 4 key columns, a rank space
+// over 2^35 bits, 2^28 or more candidates, or a value of full u delta without
+// a rank.
+static bool ensure_bitmap(pra_ctx* c, pra_rel* R, int kw, u64 C, u64* bits_out)
 {
     Group& G = grp(c, R->group);
     if (!c->dense_on || G.dict_state != 1 || kw < 1 || kw > 4 || G.dict_n == 0 || C >= (1ULL << PRA_DENSE_PBITS))
@@ -1583,27 +1627,90 @@ static bool ensure_dense(pra_ctx* c, pra_rel* R, int kw, u64 C, u64 slots_per_ca
         bits *= G.dict_n;
         if (bits > ((unsigned __int128)1 << 35)) return false;
     }
+    *bits_out = (u64)bits;
     if (!R->bm_valid || R->bm_gen != G.dict_gen || R->bm_kw != kw) {
         const u64 words = ((u64)bits + 63) / 64;
         Prof p(c, K_TABLE_BUILD, 8.0 * words + 8.0 * kw * (R->ver[PRA_FULL].n + R->ver[PRA_DELTA].n));
         R->bm.reserve(words * 8, c->st);
         pra_launch_fill_u64(c->st, R->bm.as<u64>(), words, 0);
-        c->orand.reserve(32 * 8, c->st);
-        pra_launch_fill_u64(c->st, c->orand.as<u64>(), 1, 0);
-        for (int v : {PRA_FULL, PRA_DELTA}) {
-            Rows& r = R->ver[v];
-            pra_launch_dense_build(c->st, r.d(), r.n, R->w, kw, G.dict.as<u64>(), G.dict_cap, G.dict_n,
-                                   R->bm.as<u32>(), c->orand.as<u64>());
-            check_launch("dense_build");
-        }
-        if (readback(c, c->orand.p, 1)[0]) {
-            R->bm_valid = false;
-            return false;
+        if (R->ver[PRA_FULL].n + R->ver[PRA_DELTA].n) {
+            c->orand.reserve(32 * 8, c->st);
+            pra_launch_fill_u64(c->st, c->orand.as<u64>(), 1, 0);
+            for (int v : {PRA_FULL, PRA_DELTA}) {
+                Rows& r = R->ver[v];
+                pra_launch_dense_build(c->st, r.d(), r.n, R->w, kw, G.dict.as<u64>(), G.dict_cap, G.dict_n,
+                                       by_bucket(c, R), R->bm.as<u32>(), c->orand.as<u64>());
+                check_launch("dense_build");
+            }
+            if (readback(c, c->orand.p, 1)[0]) {
+                R->bm_valid = false;
+                return false;
+            }
         }
         R->bm_valid = true;
         R->bm_gen = G.dict_gen;
         R->bm_kw = kw;
     }
+    return true;
+}
+
+// c->first with room for `words` new keys, every word at rest
+static void reserve_first(pra_ctx* c, u64 words)
+{
+    if (c->first_words >= words) return;
+    c->first_words = 0;
+    c->first.reserve(words * 4, c->st);
+    const size_t w64 = c->first.cap / 8;
+    pra_launch_fill_u64(c->st, c->first.as<u64>(), w64, ~0ULL);
+    c->first_words = 2 * w64;
+}
+
+// Ranked membership over a bitmap of `bits` rank indexes, for up to C
+// candidates whose words of c->first begin at `base`: the new keys' bitmap
+// and its tables, at rest.  grow: c->first may move (no other output of the
+// iteration points into it yet).  False when there is no room (the claim
+// table needs less).
+static bool ensure_ranked(pra_ctx* c, pra_rel* R, u64 bits, u64 base, u64 C, bool grow)
+{
+    if (!grow && c->first_words < base + C) return false;
+    const u64 sbs = (bits + (1ULL << PRA_SB_BITS) - 1) >> PRA_SB_BITS;
+    try {
+        if (R->fresh_sbs < sbs) {
+            R->fresh_sbs = 0;
+            const u64 room = (sbs + 1) & ~1ULL;   // whole words of flags
+            R->fresh.reserve((room << PRA_SB_BITS) / 8, c->st);
+            R->dirty.reserve(room * 4, c->st);
+            R->sbpre.reserve(room * 4, c->st);
+            R->linep.reserve((room << (PRA_SB_BITS - PRA_LINE_BITS)) * 2, c->st);
+            pra_launch_fill_u64(c->st, R->fresh.as<u64>(), (room << PRA_SB_BITS) / 64, 0);
+            pra_launch_fill_u64(c->st, R->dirty.as<u64>(), room / 2, 0);
+            R->fresh_sbs = room;
+        }
+        R->sbs_use = sbs;
+        reserve_first(c, base + C);
+        prepare_lookback(c, C);
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        for (DBuf* b : {&R->fresh, &R->dirty, &R->sbpre, &R->linep}) b->release();
+        R->fresh_sbs = 0;
+        return false;
+    }
+    check_launch("ranked");
+    return true;
+}
+
+// the ranked tables of R back at rest, after claims that stopped at a
+// dictionary miss
+static void reset_ranked(pra_ctx* c, pra_rel* R)
+{
+    pra_launch_fill_u64(c->st, R->fresh.as<u64>(), (R->fresh_sbs << PRA_SB_BITS) / 64, 0);
+    pra_launch_fill_u64(c->st, R->dirty.as<u64>(), R->fresh_sbs / 2, 0);
+    check_launch("reset_ranked");
+}
+
+// A claim table of at least 2C slots over a bitmap of `bits` rank indexes.
+static void ensure_claims(pra_ctx* c, pra_rel* R, u64 bits, u64 C, u64 slots_per_candidate)
+{
     // slots in use: a power of two of at least slots_per_candidate x C; the
     // table is allocated for the largest use so far, and every slot is empty
     // between iterations, so a smaller use is a prefix of it
@@ -1613,7 +1720,7 @@ static bool ensure_dense(pra_ctx* c, pra_rel* R, int kw, u64 C, u64 slots_per_ca
     // the next epoch, so the slots of earlier ones count as empty, and the
     // table is filled with zeros only when the epochs wrap
     int kbits = 0;
-    while (kbits < 36 && ((unsigned __int128)1 << kbits) <= bits) kbits++;
+    while (kbits < 36 && (1ULL << kbits) <= bits) kbits++;
     const int eb = std::min(c->dense_epoch_bits, 36 - kbits);
     bool clear = false;
     if (cap > R->dtab_cap) {
@@ -1633,19 +1740,18 @@ static bool ensure_dense(pra_ctx* c, pra_rel* R, int kw, u64 C, u64 slots_per_ca
     }
     if (eb > 0) R->dtab_epoch++;
     R->dtab_use = cap;
-    return true;
 }
 
-static DBuf& seq_counters(pra_ctx* c, int gi, u32 tag)
+static Group::Seq& seq_counters(pra_ctx* c, int gi, u32 tag)
 {
     Group& G = grp(c, gi);
     auto it = G.seq.find(tag);
     if (it != G.seq.end()) return *it->second;
-    std::unique_ptr<DBuf> b(new DBuf());
-    b->reserve((size_t)c->nb * 8, c->st);
-    pra_launch_fill_u64(c->st, b->as<u64>(), (u64)c->nb, 0);
-    DBuf& ref = *b;
-    G.seq[tag] = std::move(b);
+    std::unique_ptr<Group::Seq> q(new Group::Seq());
+    q->buf.reserve((size_t)c->nb * 16, c->st);
+    pra_launch_fill_u64(c->st, q->buf.as<u64>(), 2 * (u64)c->nb, 0);
+    Group::Seq& ref = *q;
+    G.seq[tag] = std::move(q);
     return ref;
 }
 
@@ -2128,6 +2234,16 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                      packed_layout((u64)nb, G.dict_n, outs[oi]->arity, &pk_mul[oi], &pk_ls[oi]);
     }
 
+    // some output of the iteration takes the general membership table
+    bool mixed = false;
+    for (size_t oi = 0; oi < no; oi++) {
+        if (!cap[oi]) continue;
+        unsigned __int128 bits = packed[oi] && outs[oi]->arity <= 4 ? 1 : (unsigned __int128)1 << 36;
+        for (int i = 0; packed[oi] && i < outs[oi]->arity && bits < ((unsigned __int128)1 << 36); i++)
+            bits *= grp(c, outs[oi]->group).dict_n;
+        mixed = mixed || bits > ((unsigned __int128)1 << 35);
+    }
+
     // 3+4. per output: arrival plan, emit candidates, deduplicate, partition
     //      and intern, summaries for the sort
     // rs == nullptr: the iteration's whole emission; else one threshold round
@@ -2164,6 +2280,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     std::vector<char> use_dense(no, 0), dense_off(no, 0);
     std::vector<ScanJob> scan_jobs;
     std::vector<std::pair<DenseArgs, size_t>> dense_jobs;
+    std::vector<std::pair<RankArgs, size_t>> rank_jobs;
     // phase 0: one output start to end; 1: up to its candidates, 2: its
     // histogram scan, 3: from its partition on
     // kept counts on (the claims and decisions in between batched over the
@@ -2180,24 +2297,53 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         Rows& NT = R->ver[PRA_NEWT];
         u64* st2o = c->stage2.as<u64>() + oi * SW;
         u64* ctl = st2o + 4;
-        // dense claim table size: tuned (timed) on single-output iterations
-        // of at least kTuneMinCandidates candidates of capacity, the settled
-        // choice (or 2 slots per candidate) elsewhere
-        int dvar = 0;
-        bool dtime = false;
-        if (c->tune_on && !rs && C >= kTuneMinCandidates) {
-            if (phase == 0) {
-                dvar = g_tune.pick(c->device, TUNE_DENSE_LOAD, band_of(C), kTuneVariants[TUNE_DENSE_LOAD]);
-                dtime = g_tune.settled(c->device, TUNE_DENSE_LOAD, band_of(C)) < 0;
-            } else {
-                dvar = std::max(0, g_tune.settled(c->device, TUNE_DENSE_LOAD, band_of(C)));
+        // dense membership unless the output was redone the general way in
+        // this iteration, or this is a threshold round.  Ranked membership
+        // moves each candidate through four light launches and needs no sort;
+        // the claim table needs less memory.  From kTuneMinCandidates
+        // candidates of capacity on, single-output iterations time both (the
+        // claim table's sizes first) and the band's cheaper one is kept; below
+        // that, and untimed, ranked (150x150 grid, 846 K candidates an
+        // iteration: membership, new rows and their sort 118 us by the claim
+        // table, 88 us ranked).
+        int dvar = 0, mode = use_dense[oi];
+        bool dtime = false, rtime = false;
+        hipEvent_t tr = nullptr;   // opens the claim table's share of the choice
+        if (phase < 2) {
+            u64 bits = 0;
+            mode = 0;
+            if (!rs && !dense_off[oi] && packed[oi] && ensure_bitmap(c, R, kw, C, &bits)) {
+                mode = 2;
+                if (c->tune_on && C >= kTuneMinCandidates) {
+                    const int band = band_of(C), load = g_tune.settled(c->device, TUNE_DENSE_LOAD, band);
+                    dvar = std::max(0, load);
+                    if (phase != 0) {
+                        // outputs of a batched iteration share their launches
+                        // and are not timed
+                    } else if (load < 0) {
+                        dvar = g_tune.pick(c->device, TUNE_DENSE_LOAD, band, kTuneVariants[TUNE_DENSE_LOAD]);
+                        dtime = true;
+                        mode = 1;
+                    } else {
+                        mode = 1 + g_tune.pick(c->device, TUNE_RANKED, band, kTuneVariants[TUNE_RANKED]);
+                        rtime = g_tune.settled(c->device, TUNE_RANKED, band) < 0;
+                    }
+                }
+                // next to outputs that take the general table, the claim table
+                // shares the partition and sort launches they need anyway: two
+                // launches more, where ranked membership is four (points-to
+                // analysis, 62 iterations: 15.04 against 15.60 ms)
+                if (phase == 1 && mixed && C < kMixedRankedCandidates) mode = 1;
+                if (mode == 2 && !ensure_ranked(c, R, bits, rg.rb, C, phase == 0)) {
+                    mode = 1;
+                    rtime = false;
+                }
+                if (mode == 1) ensure_claims(c, R, bits, C, 2ULL << dvar);
             }
         }
-        // dense membership unless the output was redone the general way in
-        // this iteration, or this is a threshold round
-        const bool dn = phase < 2 ? (!rs && !dense_off[oi] && packed[oi] && ensure_dense(c, R, kw, C, 2ULL << dvar))
-                                   : use_dense[oi] != 0;
-        use_dense[oi] = dn;
+        const bool dn = mode != 0, ranked = mode == 2;
+        use_dense[oi] = (char)mode;
+        if (phase >= 2 && ranked) return;   // its new rows are in place
         if (dn)
             R->mt_valid = false;   // the general table is not kept current meanwhile
         else
@@ -2328,6 +2474,58 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                     check_launch("copy_expand");
                 }
             }
+            if (ranked) {
+                RankArgs ra;
+                memset(&ra, 0, sizeof(ra));
+                Group& G = grp(c, R->group);
+                Group::Seq& sq = seq_counters(c, R->group, R->tag);
+                ra.cand = cand0;
+                ra.ctl = ctl;
+                ra.xs = slot0;
+                ra.pos = keep0;
+                ra.dest = dest0;
+                ra.dict = G.dict.as<u64>();
+                ra.dict_cap = G.dict_cap;
+                ra.D = G.dict_n;
+                ra.member = R->bm.as<u32>();
+                ra.fresh = R->fresh.as<u32>();
+                ra.dirty = R->dirty.as<u32>();
+                ra.sbpre = R->sbpre.as<u32>();
+                ra.linep = R->linep.as<unsigned short>();
+                ra.first = c->first.as<u32>() + rg.rb;
+                ra.newt = NT.d();
+                if (bits_in_trie_order(c, R)) {
+                    R->next_bnd.reserve((size_t)(nb + 1) * 8, c->st);
+                    ra.bnd = R->next_bnd.as<u64>();
+                }
+                ra.stat = st2o;
+                ra.seq = sq.buf.as<u64>() + sq.now * nb;
+                ra.seq_next = sq.buf.as<u64>() + (sq.now ^ 1) * nb;
+                ra.sbs = (u32)R->sbs_use;
+                ra.chunks = std::min<u32>(PRA_SCAN_CHUNKS, (ra.sbs + 15) / 16);
+                ra.nb = (u32)nb;
+                ra.tag = R->tag;
+                ra.cw = cw;
+                ra.kw = kw;
+                ra.wn = R->w;
+                ra.by_bucket = by_bucket(c, R);
+                if (phase == 1) {
+                    // launched after the batched expansions
+                    rank_jobs.emplace_back(ra, oi);
+                    return;
+                }
+                hipEvent_t ta = c->tune_begin(rtime);
+                static const int kind[4] = {K_DEDUP_CLAIM, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE};
+                const double bytes[4] = {8.0 * (kw + 1), 0.0, 16.0, 8.0 * cw + 8.0 * R->w + 12.0};
+                for (int step = 0; step < 4; step++) {
+                    const u32 ep = next_sort_epoch(c);
+                    ProfPerCand p(c, kind[step], bytes[step], oi);
+                    pra_launch_rank(c->st, step, ra, C, c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
+                    check_launch("rank");
+                }
+                c->tune_end(ta, TUNE_RANKED, band_of(C), 1, oi, C);
+                return;
+            }
             if (dn) {
                 DenseArgs da;
                 memset(&da, 0, sizeof(da));
@@ -2353,11 +2551,16 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 da.nb = (u32)nb;
                 da.cw = cw;
                 da.kw = kw;
+                da.by_bucket = by_bucket(c, R);
+                da.rank_of = G.rank_of.as<u32>();
+                da.lead = 1;
+                for (int i = 1; i < kw; i++) da.lead *= G.dict_n;
                 if (phase == 1) {
                     // launched after the batched expansions
                     dense_jobs.emplace_back(da, oi);
                     return;
                 }
+                tr = c->tune_begin(rtime);
                 hipEvent_t ta = c->tune_begin(dtime);
                 {
                     ProfPerCand p(c, K_DEDUP_CLAIM, 8.0 * (kw + 1), oi);
@@ -2409,7 +2612,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             return;
         }
         if (phase == 0 && nblocks > 1) scan_u32(c, hist0, offs0, (u64)nb * nblocks, total_dev);
-        DBuf* sq = intern ? &seq_counters(c, R->group, R->tag) : nullptr;
+        Group::Seq* sq = intern ? &seq_counters(c, R->group, R->tag) : nullptr;
+        u64* seq_now = sq ? sq->buf.as<u64>() + sq->now * nb : nullptr;
         R->kgofs.reserve(PRA_RADIX * 4, c->st);
         NewtFoldArgs f;   // bin_cur: set with the scatter's bins
         memset(&f, 0, sizeof(f));
@@ -2419,7 +2623,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         f.ctl = ctl;
         f.stat = st2o;
         f.kgofs = R->kgofs.as<u32>();
-        f.seqbase = sq ? sq->as<u64>() : nullptr;
+        f.seqbase = seq_now;
         f.offs = offs0;
         f.total = total_dev;
         f.nblocks = nblocks;
@@ -2437,7 +2641,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             a.keep = keep0;
             a.dest = dest0;
             a.offs = offs0;
-            a.seqbase = sq ? sq->as<u64>() : nullptr;
+            a.seqbase = seq_now;
             a.newt = NT.d() + nt_base * R->w;
             a.nblocks = nblocks;
             a.nb = (u32)nb;
@@ -2509,6 +2713,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 pra_launch_dedup_scatter(c->st, a, wide);
                 check_launch("dedup_scatter");
                 c->tune_end(ta, TUNE_SCATTER_WIDE, sband, wide, oi, C);
+                c->tune_end(tr, TUNE_RANKED, band_of(C), 0, oi, C);
             }
         }
         if (!fold_here && planned && oi == last_oi) {
@@ -2603,6 +2808,11 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         c->keep.reserve(rt * 4, c->st);
         c->hist.reserve(ht * 4, c->st);
         c->offs.reserve(ht * 4 + 8, c->st);
+        try {
+            reserve_first(c, rt);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        }
         for (size_t oi = 0; oi < no; oi++)
             if (cap[oi]) run_output(oi, nullptr, true, 1);
         // the expansions of all rules: job tables through pinned staging into
@@ -2640,6 +2850,43 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                     pra_launch_expand_many(c->st, dv + jb, (int)cexp_jobs.size(), nbk, false);
                     check_launch("copy_expand_many");
                 }
+            }
+        }
+        // the ranked outputs: one table through pinned staging, one launch a step
+        if (!rank_jobs.empty()) {
+            const size_t n = rank_jobs.size();
+            std::vector<char> t(n * sizeof(RankArgs) + 3 * (n + 1) * 4);
+            RankArgs* J = (RankArgs*)t.data();
+            u32* base[3];
+            for (int q = 0; q < 3; q++) {
+                base[q] = (u32*)(t.data() + n * sizeof(RankArgs)) + q * (n + 1);
+                base[q][0] = 0;
+            }
+            for (size_t k = 0; k < n; k++) {
+                const u64 C = cap[rank_jobs[k].second];
+                J[k] = rank_jobs[k].first;
+                base[0][k + 1] = base[0][k] + (u32)((C + PRA_BLOCK - 1) / PRA_BLOCK);
+                base[1][k + 1] = base[1][k] + J[k].chunks;
+                base[2][k + 1] = base[2][k] + pra_tiles(C);
+            }
+            prepare_lookback(c, std::max<u64>(base[2][n], (base[1][n] + PRA_RADIX - 1) / PRA_RADIX) * PRA_TILE);
+            const RankArgs* d = (const RankArgs*)stage_table(c, JOB_RANK, t.data(), t.size());
+            static const int kind[4] = {K_DEDUP_CLAIM, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE};
+            for (int step = 0; step < 4; step++) {
+                const u32 ep = next_sort_epoch(c);
+                const size_t before = c->pending.size();
+                {
+                    Prof p(c, kind[step], 0.0);
+                    pra_launch_rank_many(c->st, step, d, (int)n, base[step == PRA_RANK_SCAN ? 1 : step == PRA_RANK_PLACE ? 2 : 0][n],
+                                         c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
+                    check_launch("rank_many");
+                }
+                if (c->pending.size() == before + 1)
+                    for (auto& j : rank_jobs) {
+                        const RankArgs& a = j.first;
+                        const double per[4] = {8.0 * (a.kw + 1), 0.0, 16.0, 8.0 * a.cw + 8.0 * a.wn + 12.0};
+                        c->per_candidate.emplace_back(before, per[step], j.second);
+                    }
             }
         }
         // the dense claims and decisions: one table per key width through
@@ -2839,8 +3086,12 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             if (st2[oi * SW + 5] == 3) {
                 // claims that stopped at the miss left slots behind
                 pra_rel* R = outs[oi];
-                pra_launch_dense_table_clear(c->st, R->dtab.as<u64>(), R->dtab_cap);
-                check_launch("dense_table_clear");
+                if (use_dense[oi] == 2) {
+                    reset_ranked(c, R);
+                } else {
+                    pra_launch_dense_table_clear(c->st, R->dtab.as<u64>(), R->dtab_cap);
+                    check_launch("dense_table_clear");
+                }
                 dense_off[oi] = 1;
             }
             cap[oi] = st2[oi * SW + 4];
@@ -2863,10 +3114,22 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     c->per_candidate.clear();
     // tuned launches: cost per candidate; a launch whose candidates passed
     // its capacity did part of the work and is not counted
+    for (auto& t : c->tune_late) {
+        float ms = 0;
+        if (t.b && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess &&
+            g_tune.record(c->device, TUNE_RANKED, t.band, 0, (t.ms + ms) / (double)t.n, kTuneVariants[TUNE_RANKED]))
+            tune_save();
+        for (hipEvent_t e : {t.a, t.b})
+            if (e) c->evpool.push_back(e);
+    }
+    c->tune_late.clear();
     for (auto& t : c->tune_pending) {
         const u64 n = st2[t.oi * SW + 4];
         float ms = 0;
-        if (n > 0 && n <= t.cap && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess &&
+        const bool timed = n > 0 && n <= t.cap && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess;
+        if (timed && t.knob == TUNE_RANKED && t.var == 0)
+            c->tune_late.push_back({t.band, t.oi, n, (double)ms, nullptr, nullptr});
+        else if (timed &&
             g_tune.record(c->device, t.knob, t.band, t.var, (double)ms / (double)n, kTuneVariants[t.knob]))
             tune_save();
         c->evpool.push_back(t.a);
@@ -2879,6 +3142,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         R->jhint = cap[oi] ? st2[oi * SW + 4] : 0;
         R->ver[PRA_NEWT].n = cnt;
         R->ver[PRA_NEWT].sorted = false;
+        // the counters a ranked iteration advanced are the current ones now
+        if (cap[oi] && use_dense[oi] == 2 && !in_rounds[oi]) seq_counters(c, R->group, R->tag).now ^= 1;
         if (!in_rounds[oi]) R->mt_entries += cnt;   // rounds count their own
     }
 
@@ -2914,7 +3179,10 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     std::vector<size_t> bin_out;
     u64 bins_max = 0;   // the largest bin of the deferred bin sorts
     size_t n_packed_sorts = 0;
-    for (size_t oi = 0; oi < no; oi++) n_packed_sorts += packed[oi] && !in_rounds[oi] && st2[oi * SW + 3] == 0;
+    // outputs whose new rows are in place already
+    auto placed = [&](size_t oi) { return cap[oi] && use_dense[oi] == 2 && !in_rounds[oi]; };
+    for (size_t oi = 0; oi < no; oi++)
+        n_packed_sorts += packed[oi] && !placed(oi) && !in_rounds[oi] && st2[oi * SW + 3] == 0;
     auto flush_small_sorts = [&]() {
         if (ss_out.empty()) return;
         double bytes = 0;
@@ -2935,14 +3203,29 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         Rows& NT = R->ver[PRA_NEWT];
         R->bnd[PRA_DELTA].reserve((size_t)(nb + 1) * 8, c->st);
         u64* bnd = R->bnd[PRA_DELTA].as<u64>();
+        if (placed(oi)) {
+            if (bits_in_trie_order(c, R)) {
+                R->bnd[PRA_DELTA].swap(R->next_bnd);
+            } else {
+                c->sort_tmp.reserve(NT.n * R->w * 8, c->st);
+                bucket_rows(c, NT.d(), NT.n, R->w, R->jcc, c->sort_tmp.as<u64>(), bnd);
+                NT.buf.swap(c->sort_tmp);
+            }
+            bnd_ok[oi] = 1;
+            continue;
+        }
         if (packed[oi] && !in_rounds[oi] && st2[oi * SW + 3] == 0) {
             BinSortJob job;
+            auto late = std::find_if(c->tune_late.begin(), c->tune_late.end(),
+                                     [&](const pra_ctx::LateSample& t) { return t.oi == oi && !t.a; });
+            if (late != c->tune_late.end()) late->a = c->tune_begin(true);
             if (sort_by_packed_key(c, R, st2[oi * SW + 1], st2[oi * SW + 2], st2[oi * SW + 6], pk_mul[oi], pk_ls[oi],
                                    bnd, n_packed_sorts > 1 ? &job : nullptr, &R->ver[PRA_DELTA].buf)) {
                 bin_jobs.push_back(job);
                 bin_out.push_back(oi);
                 bins_max = std::max<u64>(bins_max, st2[oi * SW + 6]);
             }
+            if (late != c->tune_late.end()) late->b = c->tune_begin(true);
             bnd_ok[oi] = 1;
             continue;
         }
@@ -3407,7 +3690,7 @@ int pra_ctx_group_status(pra_ctx* ctx, int group, int* done, uint64_t* iteration
         for (pra_rel* R : ctx->rels) {
             if (R->group != group) continue;
             for (auto& v : R->ver) b += v.buf.cap;
-            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
+            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
                                   &R->bin_keys, &R->bin_idx, &R->bin_cur, &R->bnd[0], &R->bnd[1]})
                 b += d->cap;
         }
@@ -3465,8 +3748,9 @@ int pra_ctx_trim(pra_ctx* ctx)
     // work already enqueued
     for (DBuf* b : {&ctx->sort_tmp, &ctx->stage, &ctx->stage2, &ctx->tmp64a, &ctx->tmp64b, &ctx->tmp64c, &ctx->cand,
                     &ctx->dest, &ctx->slot_of, &ctx->keep, &ctx->hist, &ctx->offs, &ctx->ktmp, &ctx->idxa, &ctx->idxb,
-                    &ctx->posadj_dev, &ctx->ttab, &ctx->kp, &ctx->lb_status})
+                    &ctx->posadj_dev, &ctx->ttab, &ctx->kp, &ctx->lb_status, &ctx->first})
         b->release();
+    ctx->first_words = 0;
     ctx->lb_zeroed = 0;   // look-back words are zeroed again on next use
     API_END
 }

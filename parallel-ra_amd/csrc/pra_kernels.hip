@@ -223,24 +223,30 @@ __global__ void k_sort_scatter(const u64* in, u64* out, u64 n, int w, DigitSpec 
 // (bucket, col0, .., col[a-1]) be packed into one u64: the bucket and the
 // column ranks as digits of radix D (the dictionary size), which the sort
 // then orders in a few byte passes.
-// Slots: [value, rank + 1]; rank + 1 == 0 marks an empty slot.
+// Slots: [value, bucket-major rank << 32 | rank + 1]; 0 marks an empty slot.
+// The bucket-major rank orders the values by (bucket of the value alone,
+// value): as the leading digit of a relation keyed on its first column it puts
+// rows in trie order, bucket first.
 
 __device__ inline u64 pra_dict_slot(u64 v, u64 cap) { return pra_mix64(v ^ 0x5851F42D4C957F2DULL) & (cap - 1); }
 
-__device__ inline bool pra_dict_rank(const u64* tab, u64 cap, u64 v, u64* rank)
+// the slot word of a value, 0 when it has none
+__device__ __forceinline__ u64 pra_dict_find(const u64* tab, u64 cap, u64 v)
 {
     u64 m = cap - 1, s = pra_dict_slot(v, cap);
     for (u64 q = 0; q < cap; q++) {
-        const u64* sl = tab + 2 * s;
-        u64 r = sl[1];
-        if (r == 0) return false;
-        if (sl[0] == v) {
-            *rank = r - 1;
-            return true;
-        }
+        const ulonglong2 sl = *(const ulonglong2*)(tab + 2 * s);
+        if (sl.y == 0 || sl.x == v) return sl.y;
         s = (s + 1) & m;
     }
-    return false;
+    return 0;
+}
+
+__device__ inline bool pra_dict_rank(const u64* tab, u64 cap, u64 v, u64* rank)
+{
+    const u64 e = pra_dict_find(tab, cap, v);
+    *rank = (u32)e - 1;
+    return e != 0;
 }
 
 // ---------------------------------------------------------- LDS sorts ------
@@ -936,6 +942,24 @@ __global__ void k_dict_insert(const u64* vals, u64 n, u64* tab, u64 cap, u32* fl
         s = (s + 1) & m;
     }
     atomicOr(flags, PRA_FLAG_TABLE_FULL);
+}
+
+// vals: the dictionary's values by (bucket, value); their places into the
+// slots' high halves, and each place's rank into rank_of
+__global__ void k_dict_bucket_rank(const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of)
+{
+    const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const u64 v = vals[i], m = cap - 1;
+    u64 s = pra_dict_slot(v, cap);
+    for (u64 q = 0; q < cap && tab[2 * s + 1]; q++) {
+        if (tab[2 * s] == v) {
+            rank_of[i] = (u32)tab[2 * s + 1] - 1;
+            tab[2 * s + 1] |= i << 32;
+            return;
+        }
+        s = (s + 1) & m;
+    }
 }
 
 // out[i] = in[idx[i]] for rows of w words
@@ -1868,22 +1892,37 @@ __global__ __launch_bounds__(PRA_DECIDE_BLOCK) void k_dedup_decide_many(DecideBa
 
 // ----------------------------------------------------- dense membership ---
 
-// rank index of a key of KW words, false when a value has no dictionary rank
+// rank index of a key of KW words (its leading digit the bucket-major rank
+// when by_bucket), false when a value has no dictionary rank
 template <int KW>
-__device__ __forceinline__ bool pra_dense_index(const u64* key, const u64* dict, u64 dcap, u64 D, u64* idx)
+__device__ __forceinline__ bool pra_dense_index(const u64* key, const u64* dict, u64 dcap, u64 D, int by_bucket,
+                                                u64* idx)
 {
-    u64 v[KW];
+    u64 v[KW], e[KW];
 #pragma unroll
     for (int c = 0; c < KW; c++) v[c] = key[c];
+#pragma unroll
+    for (int c = 0; c < KW; c++) e[c] = pra_dict_find(dict, dcap, v[c]);
     u64 x = 0;
+    bool ok = true;
 #pragma unroll
     for (int c = 0; c < KW; c++) {
-        u64 r;
-        if (!pra_dict_rank(dict, dcap, v[c], &r)) return false;
-        x = x * D + r;
+        ok = ok && e[c] != 0;
+        x = x * D + (c == 0 && by_bucket ? e[c] >> 32 : (u64)((u32)e[c] - 1));
     }
     *idx = x;
-    return true;
+    return ok;
+}
+
+__device__ __forceinline__ bool pra_dense_index_n(int kw, const u64* key, const u64* dict, u64 dcap, u64 D,
+                                                  int by_bucket, u64* idx)
+{
+    switch (kw) {
+    case 1: return pra_dense_index<1>(key, dict, dcap, D, by_bucket, idx);
+    case 2: return pra_dense_index<2>(key, dict, dcap, D, by_bucket, idx);
+    case 3: return pra_dense_index<3>(key, dict, dcap, D, by_bucket, idx);
+    default: return pra_dense_index<4>(key, dict, dcap, D, by_bucket, idx);
+    }
 }
 
 // a slot written in this iteration (the others count as empty)
@@ -1899,7 +1938,7 @@ template <int KW>
 __device__ __forceinline__ void pra_dense_claim_one(const DenseArgs& a, u64 p, u32* flags)
 {
     u64 x;
-    if (!pra_dense_index<KW>(a.cand + p * a.cw, a.dict, a.dict_cap, a.D, &x)) {
+    if (!pra_dense_index<KW>(a.cand + p * a.cw, a.dict, a.dict_cap, a.D, a.by_bucket, &x)) {
         atomicCAS((unsigned long long*)(a.ctl + 1), 0ULL, 3ULL);
         return;
     }
@@ -2002,8 +2041,9 @@ __device__ __forceinline__ void pra_dense_decide_tile(const DenseArgs& a, u64 n,
                     const u64 x = ((v & ~a.emask) >> PRA_DENSE_PBITS) - 1;
                     atomicOr(&a.bitmap[x >> 5], 1u << (x & 31));
                     if (!a.emask) *slot = 0;
-                    // the rank index, for the newt scatter's packed key
-                    a.slot_of[p] = x;
+                    // the rank index, for the newt scatter's packed key (which
+                    // leads with the bucket, so its digits are plain ranks)
+                    a.slot_of[p] = a.by_bucket ? a.rank_of[x / a.lead] * a.lead + x % a.lead : x;
                 }
             }
             a.keep[p] = kp;
@@ -2047,26 +2087,23 @@ __global__ __launch_bounds__(PRA_DECIDE_BLOCK) void k_dense_decide_many(const De
 
 // the membership bits of n rows (key = their first kw columns)
 template <int KW>
-__global__ void k_dense_build(const u64* rows, u64 n, int w, const u64* dict, u64 dcap, u64 D, u32* bitmap, u64* miss)
+__global__ void k_dense_build(const u64* rows, u64 n, int w, const u64* dict, u64 dcap, u64 D, int by_bucket, u32* bitmap,
+                              u64* miss)
 {
     const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     u64 x;
-    if (!pra_dense_index<KW>(rows + i * w, dict, dcap, D, &x)) {
+    if (!pra_dense_index<KW>(rows + i * w, dict, dcap, D, by_bucket, &x)) {
         atomicAdd((unsigned long long*)miss, 1ULL);
         return;
     }
     atomicOr(&bitmap[x >> 5], 1u << (x & 31));
 }
 
-// Trie order of a relation from its membership bitmap.  Bit x of the bitmap is
-// the key of rank index x, and rank indexes order as the columns do, so a
-// key's place among all keys is the number of set bits below x: the exclusive
-// prefix of the 256-bit blocks' counts, plus the bits below x in its block.
-// With several buckets (the bucket a function of column 0), column-0 value r0
-// owns the bits [r0 * S, (r0 + 1) * S), S = D^(kw-1), and its rows move as one
-// run: adj[r0] = (rows of earlier runs in bucket order) - (set bits below
-// r0 * S), added modulo 2^32.
+// Order of a relation from its membership bitmap.  Bit x of the bitmap is the
+// key of rank index x, and rank indexes order as the rows do, so a key's place
+// among all keys is the number of set bits below x: the exclusive prefix of
+// the 256-bit blocks' counts, plus the bits below x in its block.
 #define PRA_BM_BLOCK_WORDS 4   // u64 words per counted block
 
 // set bits below bit x; nblk blocks of u64 words, prefix[nblk] the total
@@ -2100,42 +2137,418 @@ __global__ void k_bm_count(const u64* bm, u64 words, u64 nblk, u32* cnt)
     cnt[b] = c;
 }
 
-// runs[b * D + r0] = rows of column-0 value r0 when it falls in bucket b, else 0
-__global__ void k_bm_runs(const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S, u64 nb,
-                          u32* runs)
-{
-    const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r0 >= D) return;
-    const u64 mine = pra_bucket(pra_fnv_word(PRA_FNV_OFFSET, vals[r0]), nb);
-    const u32 c = pra_bm_rank(bm, words, prefix, (r0 + 1) * S) - pra_bm_rank(bm, words, prefix, r0 * S);
-    for (u64 b = 0; b < nb; b++) runs[b * D + r0] = b == mine ? c : 0u;
-}
-
-// the runs' adjustments and the bucket bounds, from the exclusive scan of runs
-__global__ void k_bm_adjust(const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S, u64 nb, u64 n,
-                            const u32* scan, u32* adj, u64* bnd)
-{
-    const u64 r0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r0 <= nb) bnd[r0] = r0 < nb ? (u64)scan[r0 * D] : n;
-    if (r0 >= D) return;
-    const u64 mine = pra_bucket(pra_fnv_word(PRA_FNV_OFFSET, vals[r0]), nb);
-    adj[r0] = scan[mine * D + r0] - pra_bm_rank(bm, words, prefix, r0 * S);
-}
-
 // Every row (all of them members) to its place.  Bound by the rows' own
 // bytes and by the lines of 24-byte writes: runs of a delta log walk the
 // bitmap in order, so its words, the prefix and the dictionary hit in cache.
 template <int KW>
-__global__ void k_bm_place(const u64* rows, u64 n, int w, const u64* dict, u64 dcap, u64 D, u64 S, const u64* bm,
-                           u64 words, const u32* prefix, const u32* adj, u64* out)
+__global__ void k_bm_place(const u64* rows, u64 n, int w, const u64* dict, u64 dcap, u64 D, int by_bucket,
+                           const u64* bm, u64 words, const u32* prefix, u64* out)
 {
     const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     u64 x;
-    if (!pra_dense_index<KW>(rows + i * w, dict, dcap, D, &x)) return;
-    u32 pos = pra_bm_rank(bm, words, prefix, x);
-    if (adj) pos += adj[KW == 1 ? x : x / S];
+    if (!pra_dense_index<KW>(rows + i * w, dict, dcap, D, by_bucket, &x)) return;
+    const u32 pos = pra_bm_rank(bm, words, prefix, x);
     if (pos < n) pra_copy_row(out + (u64)pos * w, rows + i * w, w);
+}
+
+// Exclusive prefix of `tile` over its predecessors' published values (digit
+// 0 of the status words, `stride` apart), walked by the 64 lanes of one wave: each step reads
+// the 64 nearest unconsumed predecessors at once and adds the ready ones up to
+// the nearest inclusive prefix.  Every lane returns the same value.
+__device__ inline u64 pra_lookback_wave(const u64* status, u32 tile, u32 epoch, u32* flags, u32 stride = PRA_RADIX)
+{
+    constexpr u64 VAL = (1ULL << 46) - 1;
+    const int lane = __lane_id();
+    u64 excl = 0;
+    long long t = (long long)tile - 1;
+    u32 spins = 0;
+    while (t >= 0) {
+        long long j = t - lane;
+        u64 v = j >= 0 ? __hip_atomic_load(status + (u64)j * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                       : st_pack(epoch, PRA_ST_INC, 0);
+        u64 fl = (v >> 46) & 3ULL;
+        bool ready = (u32)(v >> 48) == epoch && fl != 0;
+        u64 notready = __ballot(!ready);
+        u64 inc = __ballot(ready && fl == PRA_ST_INC);
+        int first_nr = notready ? __ffsll((unsigned long long)notready) - 1 : 64;
+        int first_inc = inc ? __ffsll((unsigned long long)inc) - 1 : 64;
+        bool stop = first_inc < first_nr;
+        int take = stop ? first_inc + 1 : first_nr;
+        u64 x = lane < take ? (v & VAL) : 0;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d, 64);
+        excl += x;
+        if (stop) break;
+        t -= take;
+        if (take == 0 && ++spins > PRA_LOOKBACK_SPIN_LIMIT) {
+            if (lane == 0) atomicOr(flags, PRA_FLAG_SORT_STALL);
+            break;
+        }
+    }
+    return excl;
+}
+
+// ---------------------------------------------------- ranked membership ---
+//
+// The whole newt step of a dense output without a hash slot or a sort.  A
+// candidate that is no member sets its key's bit in a second bitmap, `fresh`;
+// the fresh keys' places are the numbers of fresh bits below them, so each
+// fresh key has a word of the dense array `first`, where the earliest arrival
+// wins by atomicMin, and each kept row goes straight to its sorted place.
+//   claim   rank index, member bit, fresh bit         (xs[p], fresh, dirty)
+//   scan    fresh bits per line and superblock, scanned over the dirty
+//           superblocks                               (linep, sbpre)
+//   first   place of the key, earliest arrival        (pos[p], first)
+//   place   kept rows counted by bucket in arrival order (look-back), ids, rows
+//           at their places; fresh, dirty and first are left as they were
+// Why: scattered atomics run at about 23 G/s on the device whatever they do
+// (36 us for 846 K of them), but lanes that share a cache line share the
+// transaction (14 us), and keys of neighbouring candidates are neighbours in
+// a bitmap and in `first`, while their hash slots are not.  The hash form
+// (claim, decision, scan, scatter and bin sort of the 150x150 grid, 846 K
+// candidates an iteration) took 118 us, this form 88 us.
+
+// fresh bits below bit x
+__device__ __forceinline__ u32 pra_fresh_rank(const RankArgs& a, u64 x)
+{
+    u32 r = a.sbpre[x >> PRA_SB_BITS] + a.linep[x >> PRA_LINE_BITS];
+    const ulonglong2* line = (const ulonglong2*)a.fresh + (x >> PRA_LINE_BITS) * 4;
+    const u32 bit = (u32)(x & ((1u << PRA_LINE_BITS) - 1)), wi = bit >> 6;
+    ulonglong2 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = line[k];
+#pragma unroll
+    for (u32 k = 0; k < 8; k++) {
+        const u64 m = k < wi ? ~0ULL : k == wi ? (1ULL << (bit & 63)) - 1 : 0;
+        r += (u32)__popcll((k & 1 ? v[k >> 1].y : v[k >> 1].x) & m);
+    }
+    return r;
+}
+
+__device__ __forceinline__ void pra_rank_claim_one(const RankArgs& a, u64 p)
+{
+    u64 x;
+    if (!pra_dense_index_n(a.kw, a.cand + p * a.cw, a.dict, a.dict_cap, a.D, a.by_bucket, &x)) {
+        atomicCAS((unsigned long long*)(a.ctl + 1), 0ULL, 3ULL);
+        return;
+    }
+    const u32 bit = 1u << (x & 31);
+    if (a.member[x >> 5] & bit) {
+        a.xs[p] = ~0ULL;
+        return;
+    }
+    a.xs[p] = x;
+    if (!(a.fresh[x >> 5] & bit)) {
+        atomicOr(a.fresh + (x >> 5), bit);
+        u32* d = a.dirty + (x >> PRA_SB_BITS);
+        if (!*d) *d = 1;
+    }
+}
+
+__global__ void k_rank_claim(RankArgs a)
+{
+    if (a.ctl[1]) return;
+    const u64 p = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < a.ctl[0]) pra_rank_claim_one(a, p);
+}
+
+// Chunk `chunk` of the scan: an equal share of the superblocks, a wave to each
+// dirty one, a lane to each of its 512-bit lines.  A clean superblock costs its
+// flag, so large rank spaces with few new keys stay cheap; there are at most
+// PRA_SCAN_CHUNKS chunks, since the tickets of a launch are atomics on one
+// word (about 10 ns each) and a look-back step reads 64 of them.
+__device__ __forceinline__ void pra_rank_scan_chunk(const RankArgs& a, u64* status, u32 chunk, u32 epoch, u32* flags)
+{
+    constexpr int SB = PRA_SCAN_BLOCK, SW = SB / 64, PER = 4, MAX = PRA_SCAN_CHUNK_MAX / SB;
+    __shared__ u32 cnt[PRA_SCAN_CHUNK_MAX];
+    __shared__ unsigned short list[PRA_SCAN_CHUNK_MAX];
+    __shared__ u32 lds[SW + 1], s_n, s_excl;
+    const u32 per = (a.sbs + a.chunks - 1) / a.chunks;
+    const u32 c0 = chunk * per, size = c0 < a.sbs ? min(per, a.sbs - c0) : 0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < size; i += SB) {
+        cnt[i] = 0;
+        if (a.dirty[c0 + i]) {
+            list[atomicAdd(&s_n, 1u)] = (unsigned short)i;
+            a.dirty[c0 + i] = 0;
+        }
+    }
+    __syncthreads();
+    const u32 nd = s_n;
+    for (u32 j0 = (u32)wave * PER; j0 < nd; j0 += SW * PER) {
+        u32 c[PER];
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            c[q] = 0;
+            if (j0 + q < nd) {
+                const u64 sb = c0 + list[j0 + q];
+                const ulonglong2* line = (const ulonglong2*)a.fresh + (sb * 64 + lane) * 4;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const ulonglong2 v = line[k];
+                    c[q] += (u32)(__popcll(v.x) + __popcll(v.y));
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            if (j0 + q >= nd) break;
+            u32 x = c[q];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const u32 y = __shfl_up(x, d, 64);
+                if (lane >= d) x += y;
+            }
+            const u32 i = list[j0 + q];
+            a.linep[(u64)(c0 + i) * 64 + lane] = (unsigned short)(x - c[q]);
+            if (lane == 63) cnt[i] = x;
+        }
+    }
+    __syncthreads();
+    // MAX consecutive superblocks a thread
+    u32 v[MAX], sum = 0, tot;
+#pragma unroll
+    for (int k = 0; k < MAX; k++) {
+        const u32 i = threadIdx.x * MAX + k;
+        v[k] = i < size ? cnt[i] : 0;
+        sum += v[k];
+    }
+    const u32 ex = block_exclusive_scan<u32, SW>(sum, lds, &tot);
+    if (wave == 0) {
+        u64 excl = 0;
+        if (lane == 0)
+            __hip_atomic_store(status + chunk, st_pack(epoch, chunk == 0 ? PRA_ST_INC : PRA_ST_AGG, tot),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (chunk != 0) {
+            excl = pra_lookback_wave(status, chunk, epoch, flags, 1);
+            if (lane == 0)
+                __hip_atomic_store(status + chunk, st_pack(epoch, PRA_ST_INC, excl + tot), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (lane == 0) s_excl = (u32)excl;
+    }
+    __syncthreads();
+    u32 run = s_excl + ex;
+#pragma unroll
+    for (int k = 0; k < MAX; k++) {
+        const u32 i = threadIdx.x * MAX + k;
+        if (i < size) a.sbpre[c0 + i] = run;
+        run += v[k];
+    }
+}
+
+// a block's place in launch order among the `takers` blocks that take one; the
+// block taking the last returns the counter to zero
+__device__ __forceinline__ u32 pra_ticket(u32* ctr, u32 takers)
+{
+    __shared__ u32 s_ticket;
+    if (threadIdx.x == 0) {
+        const u32 t = atomicAdd(ctr, 1u);
+        if (t == takers - 1) atomicExch(ctr, 0u);
+        s_ticket = t;
+    }
+    __syncthreads();
+    return s_ticket;
+}
+
+__global__ __launch_bounds__(PRA_SCAN_BLOCK) void k_rank_scan(RankArgs a, u64* status, u32* ctr, u32 epoch,
+                                                              u32* flags)
+{
+    const u32 t = pra_ticket(ctr, gridDim.x);
+    if (a.ctl[1]) return;
+    pra_rank_scan_chunk(a, status, t, epoch, flags);
+}
+
+__device__ __forceinline__ void pra_rank_first_one(const RankArgs& a, u64 p)
+{
+    const u64 x = a.xs[p];
+    u32 r = ~0u;
+    if (x != ~0ULL) {
+        r = pra_fresh_rank(a, x);
+        if (a.first[r] > (u32)p) atomicMin(a.first + r, (u32)p);
+    }
+    a.pos[p] = r;
+}
+
+__global__ void k_rank_first(RankArgs a)
+{
+    if (a.ctl[1]) return;
+    const u64 p = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < a.ctl[0]) pra_rank_first_one(a, p);
+}
+
+// Tile `tile` of the placement (PRA_TILE candidates by PRA_PLACE_BLOCK
+// threads).  The tile of the last candidate also writes the output's totals:
+// its new tuples, the advanced seq counters (into the copy the next iteration
+// reads) and the bucket bounds of the new rows.
+__device__ __forceinline__ void pra_rank_place_tile(const RankArgs& a, u64* status, u32 tile, u32 epoch, u32* flags)
+{
+    constexpr int SB = PRA_PLACE_BLOCK, SW = SB / 64, IT = PRA_TILE / SB;
+    __shared__ u32 wh[SW][PRA_RADIX];
+    __shared__ u32 s_base[PRA_RADIX];
+    __shared__ u32 lds[SW + 1];
+    const u64 n = a.ctl[0];
+    const u32 last = n ? (u32)((n - 1) / PRA_TILE) : 0;
+    const u32 nb = a.nb;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const u64 lt = pra_lanemask_lt();
+    const u64 base = (u64)tile * PRA_TILE + (u64)wave * 64 * IT;
+    u32 pos[IT], dg[IT], lc[IT];
+    bool kept[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u64 p = base + (u64)k * 64 + lane;
+        pos[k] = p < n ? a.pos[p] : ~0u;
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++)
+        kept[k] = pos[k] != ~0u && a.first[pos[k]] == (u32)(base + (u64)k * 64 + lane);
+    // what the kept rows need, loaded before the barriers (rows of up to PW words)
+    constexpr int PW = 2;
+    u64 x[IT], row[IT][PW];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u64 p = base + (u64)k * 64 + lane;
+        dg[k] = kept[k] && nb > 1 ? a.dest[p] : 0u;
+        x[k] = kept[k] ? a.xs[p] : 0;
+        if (kept[k] && a.cw <= PW)
+#pragma unroll
+            for (int c = 0; c < PW; c++)
+                if (c < a.cw) row[k][c] = a.cand[p * a.cw + c];
+    }
+    for (u32 i = lane; i < nb; i += 64) wh[wave][i] = 0;
+    // (a wave counts in its own row of wh, in lane order within each item)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const u64 act = __ballot(kept[k]);
+        const u64 peers = nb > 1 ? pra_match<PRA_RADIX_BITS>(dg[k], act) : act;
+        lc[k] = 0;
+        if (kept[k]) {
+            const u32 before = wh[wave][dg[k]];
+            lc[k] = before + (u32)__popcll(peers & lt);
+            if ((peers >> lane) == 1ULL) wh[wave][dg[k]] = before + (u32)__popcll(peers);
+        }
+    }
+    __syncthreads();
+    u32 acc = 0;
+    const u32 d0 = threadIdx.x;
+    if (d0 < nb) {
+        for (int v = 0; v < SW; v++) {
+            const u32 t = wh[v][d0];
+            wh[v][d0] = acc;
+            acc += t;
+        }
+        __hip_atomic_store(status + (u64)tile * PRA_RADIX + d0, st_pack(epoch, tile == 0 ? PRA_ST_INC : PRA_ST_AGG, acc),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (nb <= 2 * SW) {
+        // few buckets: a wave looks back for each, 64 tiles a step
+        for (u32 d = wave; d < nb; d += SW) {
+            const u32 e = tile ? (u32)pra_lookback_wave(status + d, tile, epoch, flags) : 0u;
+            if (lane == 0) s_base[d] = e;
+        }
+    } else if (d0 < nb) {
+        s_base[d0] = tile ? (u32)pra_lookback(status, tile, (int)d0, epoch, flags) : 0u;
+    }
+    __syncthreads();
+    if (d0 < nb && tile)
+        __hip_atomic_store(status + (u64)tile * PRA_RADIX + d0, st_pack(epoch, PRA_ST_INC, (u64)s_base[d0] + acc),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        if (!kept[k]) continue;
+        const u64 p = base + (u64)k * 64 + lane;
+        const u32 d = dg[k];
+        const u64 seq = a.seq[d] + s_base[d] + wh[wave][d] + lc[k];
+        u64* dst = a.newt + (u64)pos[k] * a.wn;
+        if (a.cw <= PW) {
+#pragma unroll
+            for (int c = 0; c < PW; c++)
+                if (c < a.cw) dst[c] = row[k][c];
+        } else {
+            pra_copy_row(dst, a.cand + p * a.cw, a.cw);
+        }
+        dst[a.cw] = ((u64)a.tag << 46) | ((u64)d << 28) | seq;
+        atomicOr(a.member + (x[k] >> 5), 1u << (x[k] & 31));
+        // back to the state between iterations: the word's fresh bits are all
+        // of this iteration, and no other arrival equals ~0
+        a.fresh[x[k] >> 5] = 0;
+        a.first[pos[k]] = ~0u;
+    }
+    if (tile != last) return;
+    u32 tot;
+    const u32 mine = d0 < nb ? s_base[d0] + acc : 0u;
+    const u32 ex = block_exclusive_scan<u32, SW>(mine, lds, &tot);
+    if (d0 < nb) {
+        a.seq_next[d0] = a.seq[d0] + mine;
+        if (a.bnd) a.bnd[d0] = ex;
+    }
+    if (d0 == 0) {
+        if (a.bnd) a.bnd[nb] = tot;
+        a.stat[0] = tot;
+    }
+}
+
+__global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place(RankArgs a, u64* status, u32* ctr, u32 epoch,
+                                                                u32* flags)
+{
+    // only the blocks that have candidates (and the first) take a ticket
+    const u64 n = a.ctl[1] ? 0 : a.ctl[0];
+    const u32 tiles = n ? (u32)((n + PRA_TILE - 1) / PRA_TILE) : 1;
+    if (blockIdx.x >= tiles) return;
+    const u32 t = pra_ticket(ctr, tiles);
+    if (a.ctl[1]) return;
+    pra_rank_place_tile(a, status, t, epoch, flags);
+}
+
+// Several outputs in one launch each: `jobs` (device memory) holds njobs
+// RankArgs, then three tables of njobs + 1 first blocks (claim and first, scan,
+// place).
+__global__ void k_rank_claim_many(const RankArgs* jobs, int njobs)
+{
+    const u32* base = (const u32*)(jobs + njobs);
+    const int k = pra_job_of(base, njobs, blockIdx.x);
+    const RankArgs* jp = jobs + k;
+    const u64 p = (u64)(blockIdx.x - base[k]) * blockDim.x + threadIdx.x;
+    if (jp->ctl[1] || p >= jp->ctl[0]) return;
+    pra_rank_claim_one(*jp, p);
+}
+
+__global__ __launch_bounds__(PRA_SCAN_BLOCK) void k_rank_scan_many(const RankArgs* jobs, int njobs, u64* status,
+                                                                   u32* ctr, u32 epoch, u32* flags)
+{
+    const u32* base = (const u32*)(jobs + njobs) + njobs + 1;
+    const u32 t = pra_ticket(ctr, gridDim.x);
+    const int k = pra_job_of(base, njobs, t);
+    const RankArgs* jp = jobs + k;
+    if (jp->ctl[1]) return;
+    pra_rank_scan_chunk(*jp, status + base[k], t - base[k], epoch, flags);
+}
+
+__global__ void k_rank_first_many(const RankArgs* jobs, int njobs)
+{
+    const u32* base = (const u32*)(jobs + njobs);
+    const int k = pra_job_of(base, njobs, blockIdx.x);
+    const RankArgs* jp = jobs + k;
+    const u64 p = (u64)(blockIdx.x - base[k]) * blockDim.x + threadIdx.x;
+    if (jp->ctl[1] || p >= jp->ctl[0]) return;
+    pra_rank_first_one(*jp, p);
+}
+
+__global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place_many(const RankArgs* jobs, int njobs, u64* status,
+                                                                     u32* ctr, u32 epoch, u32* flags)
+{
+    const u32* base = (const u32*)(jobs + njobs) + 2 * (njobs + 1);
+    const u32 t = pra_ticket(ctr, gridDim.x);
+    const int k = pra_job_of(base, njobs, t);
+    const RankArgs a = jobs[k];
+    const u32 tile = t - base[k];
+    if (a.ctl[1] || (tile && (u64)tile * PRA_TILE >= a.ctl[0])) return;
+    pra_rank_place_tile(a, status + (u64)base[k] * PRA_RADIX, tile, epoch, flags);
 }
 
 // Combine the PRA_NREP replicas of the scatter summaries and reset them to
@@ -2313,7 +2726,7 @@ __device__ __forceinline__ void pra_scatter_block(NewtScatterArgs& a, const u32 
                     if ((kept >> k) & 1u) {
                         u64 r = 0;
                         if (r1[k] != 0 && e[k] == v[k])
-                            r = r1[k] - 1;
+                            r = (u32)r1[k] - 1;
                         else if (!pra_dict_rank(a.dict, a.dict_cap, v[k], &r))
                             kmiss = 1;
                         K[k] = K[k] * a.rank_radix + r;
@@ -2643,43 +3056,6 @@ __global__ void k_copy_many(const CopyJob* jobs, int njobs)
 #pragma unroll
     for (int q = 0; q < 8; q++)
         if (i0 + q < j.words) j.dst[i0 + q] = t[q];
-}
-
-// Exclusive prefix of `tile` over its predecessors' published values (digit
-// 0 of the status words), walked by the 64 lanes of one wave: each step reads
-// the 64 nearest unconsumed predecessors at once and adds the ready ones up to
-// the nearest inclusive prefix.  Every lane returns the same value.
-__device__ inline u64 pra_lookback_wave(const u64* status, u32 tile, u32 epoch, u32* flags)
-{
-    constexpr u64 VAL = (1ULL << 46) - 1;
-    const int lane = __lane_id();
-    u64 excl = 0;
-    long long t = (long long)tile - 1;
-    u32 spins = 0;
-    while (t >= 0) {
-        long long j = t - lane;
-        u64 v = j >= 0 ? __hip_atomic_load(status + (u64)j * PRA_RADIX, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                       : st_pack(epoch, PRA_ST_INC, 0);
-        u64 fl = (v >> 46) & 3ULL;
-        bool ready = (u32)(v >> 48) == epoch && fl != 0;
-        u64 notready = __ballot(!ready);
-        u64 inc = __ballot(ready && fl == PRA_ST_INC);
-        int first_nr = notready ? __ffsll((unsigned long long)notready) - 1 : 64;
-        int first_inc = inc ? __ffsll((unsigned long long)inc) - 1 : 64;
-        bool stop = first_inc < first_nr;
-        int take = stop ? first_inc + 1 : first_nr;
-        u64 x = lane < take ? (v & VAL) : 0;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d, 64);
-        excl += x;
-        if (stop) break;
-        t -= take;
-        if (take == 0 && ++spins > PRA_LOOKBACK_SPIN_LIMIT) {
-            if (lane == 0) atomicOr(flags, PRA_FLAG_SORT_STALL);
-            break;
-        }
-    }
-    return excl;
 }
 
 // One-pass exclusive scan: tiles of PRA_TILE elements are taken in ticket
@@ -3314,15 +3690,50 @@ void pra_launch_dense_decide(hipStream_t st, const DenseArgs& a, u32*)
 }
 
 void pra_launch_dense_build(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
-                            u32* bitmap, u64* miss)
+                            int by_bucket, u32* bitmap, u64* miss)
 {
     if (!n) return;
     const dim3 g(grid_for(n)), b(PRA_BLOCK);
     switch (kw) {
-    case 1: hipLaunchKernelGGL(k_dense_build<1>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
-    case 2: hipLaunchKernelGGL(k_dense_build<2>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
-    case 3: hipLaunchKernelGGL(k_dense_build<3>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
-    default: hipLaunchKernelGGL(k_dense_build<4>, g, b, 0, st, rows, n, w, dict, dict_cap, D, bitmap, miss); break;
+    case 1: hipLaunchKernelGGL(k_dense_build<1>, g, b, 0, st, rows, n, w, dict, dict_cap, D, by_bucket, bitmap, miss); break;
+    case 2: hipLaunchKernelGGL(k_dense_build<2>, g, b, 0, st, rows, n, w, dict, dict_cap, D, by_bucket, bitmap, miss); break;
+    case 3: hipLaunchKernelGGL(k_dense_build<3>, g, b, 0, st, rows, n, w, dict, dict_cap, D, by_bucket, bitmap, miss); break;
+    default: hipLaunchKernelGGL(k_dense_build<4>, g, b, 0, st, rows, n, w, dict, dict_cap, D, by_bucket, bitmap, miss); break;
+    }
+}
+
+void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of)
+{
+    if (n) hipLaunchKernelGGL(k_dict_bucket_rank, dim3(grid_for(n)), dim3(PRA_BLOCK), 0, st, vals, n, tab, cap, rank_of);
+}
+
+void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* status, u32* ctr, u32 epoch, u32* flags)
+{
+    switch (step) {
+    case PRA_RANK_CLAIM: hipLaunchKernelGGL(k_rank_claim, dim3(grid_for(cap)), dim3(PRA_BLOCK), 0, st, a); break;
+    case PRA_RANK_SCAN:
+        hipLaunchKernelGGL(k_rank_scan, dim3(a.chunks), dim3(PRA_SCAN_BLOCK), 0, st, a, status, ctr, epoch, flags);
+        break;
+    case PRA_RANK_FIRST: hipLaunchKernelGGL(k_rank_first, dim3(grid_for(cap)), dim3(PRA_BLOCK), 0, st, a); break;
+    default:
+        hipLaunchKernelGGL(k_rank_place, dim3(pra_tiles(cap)), dim3(PRA_PLACE_BLOCK), 0, st, a, status, ctr, epoch,
+                           flags);
+    }
+}
+
+void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,
+                          u32 epoch, u32* flags)
+{
+    switch (step) {
+    case PRA_RANK_CLAIM: hipLaunchKernelGGL(k_rank_claim_many, dim3(blocks), dim3(PRA_BLOCK), 0, st, jobs, njobs); break;
+    case PRA_RANK_SCAN:
+        hipLaunchKernelGGL(k_rank_scan_many, dim3(blocks), dim3(PRA_SCAN_BLOCK), 0, st, jobs, njobs, status, ctr, epoch,
+                           flags);
+        break;
+    case PRA_RANK_FIRST: hipLaunchKernelGGL(k_rank_first_many, dim3(blocks), dim3(PRA_BLOCK), 0, st, jobs, njobs); break;
+    default:
+        hipLaunchKernelGGL(k_rank_place_many, dim3(blocks), dim3(PRA_PLACE_BLOCK), 0, st, jobs, njobs, status, ctr,
+                           epoch, flags);
     }
 }
 
@@ -3331,26 +3742,13 @@ void pra_launch_bm_count(hipStream_t st, const u64* bm, u64 words, u64 nblk, u32
     hipLaunchKernelGGL(k_bm_count, dim3(grid_for(nblk)), dim3(PRA_BLOCK), 0, st, bm, words, nblk, cnt);
 }
 
-void pra_launch_bm_runs(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
-                        u64 nb, u32* runs)
-{
-    hipLaunchKernelGGL(k_bm_runs, dim3(grid_for(D)), dim3(PRA_BLOCK), 0, st, bm, words, prefix, vals, D, S, nb, runs);
-}
-
-void pra_launch_bm_adjust(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
-                          u64 nb, u64 n, const u32* scan, u32* adj, u64* bnd)
-{
-    hipLaunchKernelGGL(k_bm_adjust, dim3(grid_for(std::max<u64>(D, nb + 1))), dim3(PRA_BLOCK), 0, st, bm, words,
-                       prefix, vals, D, S, nb, n, scan, adj, bnd);
-}
-
 void pra_launch_bm_place(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
-                         u64 S, const u64* bm, u64 words, const u32* prefix, const u32* adj, u64* out)
+                         int by_bucket, const u64* bm, u64 words, const u32* prefix, u64* out)
 {
     if (!n) return;
     const dim3 g(grid_for(n)), b(PRA_BLOCK);
     auto k = kw == 1 ? k_bm_place<1> : kw == 2 ? k_bm_place<2> : kw == 3 ? k_bm_place<3> : k_bm_place<4>;
-    hipLaunchKernelGGL(k, g, b, 0, st, rows, n, w, dict, dict_cap, D, S, bm, words, prefix, adj, out);
+    hipLaunchKernelGGL(k, g, b, 0, st, rows, n, w, dict, dict_cap, D, by_bucket, bm, words, prefix, out);
 }
 
 void pra_launch_dense_table_clear(hipStream_t st, u64* table, u64 cap) { pra_launch_fill_u64(st, table, cap, 0); }

@@ -197,7 +197,50 @@ struct DenseArgs {
     u64 emask, stamp;    // the slots' epoch bits and this iteration's epoch in them
     u32 nblocks, nb;
     int cw, kw;
+    int by_bucket;       // the leading digit of x is the bucket-major rank
+    const u32* rank_of;  // by_bucket: the rank of each bucket-major rank
+    u64 lead;            // by_bucket: D^(kw-1), the leading digit's weight
 };
+
+// Ranked membership of a dense output (k_rank_claim .. k_rank_place): bitmaps
+// in 512-bit lines and superblocks of 64 lines, the latter scanned in at most
+// PRA_SCAN_CHUNKS chunks (2^35 bits: 4,096 superblocks each).
+#define PRA_LINE_BITS 9
+#define PRA_SB_BITS 15
+#define PRA_SCAN_BLOCK 1024
+#define PRA_SCAN_CHUNKS 256
+#define PRA_SCAN_CHUNK_MAX 4096
+#define PRA_PLACE_BLOCK 1024
+struct RankArgs {
+    const u64* cand;
+    u64* ctl;
+    u64* xs;              // per candidate: its rank index, ~0 for members
+    u32* pos;             // per candidate: its key's place among the new keys
+    const u32* dest;
+    const u64* dict;
+    u64 dict_cap, D;
+    u32 *member, *fresh;  // fresh: all zero between iterations
+    u32* dirty;           // per superblock: holds fresh bits (all zero between iterations)
+    u32* sbpre;           // per superblock: fresh bits before it
+    unsigned short* linep;   // per line of a dirty superblock: its fresh bits before the line
+    u32* first;           // per new key: earliest arrival (all ones between iterations)
+    u64* newt;
+    u64* bnd;             // bucket bounds of the new rows (null: not wanted)
+    u64* stat;
+    const u64* seq;       // per-bucket seq counters, and their values after this iteration
+    u64* seq_next;
+    u32 sbs, chunks, nb, tag;   // superblocks, and the chunks they are scanned in
+    int cw, kw, wn, by_bucket;
+};
+enum { PRA_RANK_CLAIM, PRA_RANK_SCAN, PRA_RANK_FIRST, PRA_RANK_PLACE };
+// one step of one output; status: look-back words of its tiles (one a tile for
+// the scan, PRA_RADIX for the placement)
+void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* status, u32* ctr, u32 epoch,
+                     u32* flags);
+// the step of several outputs: jobs (device) = njobs RankArgs, then three
+// tables of njobs + 1 first blocks (claim / first, scan, place)
+void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,
+                          u32 epoch, u32* flags);
 
 // job tables (device memory) of the batched launches of a lock-step iteration
 struct BinSortJob {
@@ -349,6 +392,9 @@ void pra_launch_collect_cols(hipStream_t st, const u64* rows, u64 n, int w, int 
 void pra_launch_view_keep(hipStream_t st, const u64* rows, u64 n, int w, int ja, int jb, u64 nb, u32* keep);
 void pra_launch_view_compact(hipStream_t st, const u64* rows, u64 n, int w, const u32* keep, const u32* pos, u64* out);
 void pra_launch_dict_insert(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* flags);
+// bucket-major ranks (vals: the n dictionary values by (bucket, value)) into
+// the dictionary's slots
+void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of);
 void pra_launch_gather_rows(hipStream_t st, const u64* in, const u32* idx, u64 n, int w, u64* out);
 void pra_launch_key_bounds(hipStream_t st, const u64* keys, u64 n, u64 bmul, int ls, u64 nb, u64* bnd);
 // Keyed row sort of more rows than one block holds: word 0 of every row's key
@@ -411,19 +457,13 @@ void pra_launch_dense_decide(hipStream_t st, const DenseArgs& a, u32* flags);
 void pra_launch_dense_many(hipStream_t st, const DenseArgs* jobs, int njobs, int kw, u32 claim_blocks,
                            u32 decide_blocks, u32* flags);
 void pra_launch_dense_build(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
-                            u32* bitmap, u64* miss);
-// trie order of a version from its membership bitmap (k_bm_count .. k_bm_place
-// in pra_kernels.hip): 256-bit block counts (scanned by the caller into
-// prefix, prefix[nblk] = total), the runs of column-0 values by bucket, their
-// adjustments and the bucket bounds, and the placement of the rows
+                            int by_bucket, u32* bitmap, u64* miss);
+// order of a version by its membership bitmap: 256-bit block counts (scanned
+// by the caller into prefix, prefix[nblk] = total), then the rows' placement
 #define PRA_BM_BITS 256
 void pra_launch_bm_count(hipStream_t st, const u64* bm, u64 words, u64 nblk, u32* cnt);
-void pra_launch_bm_runs(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
-                        u64 nb, u32* runs);
-void pra_launch_bm_adjust(hipStream_t st, const u64* bm, u64 words, const u32* prefix, const u64* vals, u64 D, u64 S,
-                          u64 nb, u64 n, const u32* scan, u32* adj, u64* bnd);
 void pra_launch_bm_place(hipStream_t st, const u64* rows, u64 n, int w, int kw, const u64* dict, u64 dict_cap, u64 D,
-                         u64 S, const u64* bm, u64 words, const u32* prefix, const u32* adj, u64* out);
+                         int by_bucket, const u64* bm, u64 words, const u32* prefix, u64* out);
 void pra_launch_dense_table_clear(hipStream_t st, u64* table, u64 cap);
 // batched forms of k_bin_sort (256 blocks per job), k_scan_small (u32, one
 // block per job of at most PRA_SMALL_SCAN elements), D2D copies (job table
