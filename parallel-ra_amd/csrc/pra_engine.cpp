@@ -214,6 +214,8 @@ constexpr u64 kTuneMinCandidates = 1ULL << 16;
 // capacity from which a dense output takes ranked membership beside outputs of
 // the general table
 constexpr u64 kMixedRankedCandidates = 1ULL << 18;
+// longest run of inner rows that an emission in digits walks in one thread
+constexpr u64 kEmitRun = 32;
 pra::Tuner g_tune(3);
 
 // Tuning cache: with PRA_AUTOTUNE_FILE set, the settled choices are read from
@@ -405,6 +407,15 @@ struct pra_rel {
     DBuf fresh, dirty, sbpre, linep;
     u64 fresh_sbs = 0;   // superblocks of the zeroed bitmap (0: none)
     u64 sbs_use = 0;     // of them, those of the current rank space
+    // rank indexes of the delta rows (valid for dictionary generation dx_gen)
+    // and of the new rows
+    DBuf dx, nx;
+    u64 dx_gen = ~0ULL;
+    // per version: the dictionary words of the rows' columns and the first row
+    // of every leading digit (valid for dictionary generation rk_gen)
+    DBuf rk_words[2], rk_first[2];
+    u64 rk_gen[2] = {~0ULL, ~0ULL};
+    bool rk_no[2] = {false, false};   // rows without ranks, or no room
     u64 bm_gen = ~0ULL, dtab_cap = 0, dtab_use = 0;   // slots allocated, slots in use this iteration
     int dtab_eb = -1;      // epoch bits of the claim table's slots (0: winners empty their slots)
     u32 dtab_epoch = 0;    // this iteration's epoch (slots of any other count as empty)
@@ -442,6 +453,9 @@ struct pra_rel {
         if (v == PRA_DELTA || v == PRA_FULL) {
             idx_valid[v] = false;
             bnd_valid[v] = false;
+            rk_gen[v] = ~0ULL;
+            rk_no[v] = false;
+            if (v == PRA_DELTA) dx_gen = ~0ULL;
             gen[v]++;
         }
     }
@@ -475,12 +489,12 @@ struct KStat {
 enum {
     K_JOIN_COUNT, K_JOIN_EXPAND, K_COPY_EXPAND, K_DEDUP_CLAIM, K_DEDUP_DECIDE, K_DEDUP_VERIFY, K_DEDUP_SCATTER,
     K_RADIX_HIST, K_RADIX_SCATTER, K_TABLE_BUILD, K_INDEX_BUILD, K_SCAN, K_GATHER, K_MERGE, K_BIN_SORT, K_SMALL_SORT,
-    K_BLOCK_SORT, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE, K_COUNT
+    K_BLOCK_SORT, K_RANK_EMIT, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE, K_COUNT
 };
 static const char* kNames[K_COUNT] = {"join_count", "join_expand", "copy_expand", "dedup_claim", "dedup_decide",
                                       "dedup_verify_hist", "dedup_scatter", "radix_hist", "radix_scatter",
                                       "table_build", "index_build", "scan", "gather_rows", "merge_full",
-                                      "bin_sort", "small_sort", "block_sort", "rank_scan", "rank_first",
+                                      "bin_sort", "small_sort", "block_sort", "rank_emit", "rank_scan", "rank_first",
                                       "rank_place"};
 
 } // namespace
@@ -498,7 +512,9 @@ struct Group {
     };
     std::map<u32, std::unique_ptr<Seq>> seq;
     // order-preserving value dictionary for packed sort keys
-    DBuf dict, rank_of;                      // value -> rank table; rank by bucket-major rank
+    // value -> rank table; the values by rank; with several buckets, the values
+    // by bucket-major rank, its maps to and from ranks, and its bucket
+    DBuf dict, vals, lead_vals, rank_of, lead_of, lead_bucket;
     u64 dict_cap = 0, dict_n = 0;
     int dict_state = 0, dict_rebuilds = 0;   // state: 0 stale, 1 valid, 2 disabled
     u64 dict_gen = 0;                        // dictionary builds so far
@@ -873,12 +889,16 @@ static void sync_check(pra_ctx* c) { readback(c, nullptr, 0); }
 // kernel reports errors, and after a while the host falls back to a blocking
 // wait on it.
 // fold: a newt fold still to run, done by the publishing kernel itself
-static u64* publish_begin(pra_ctx* c, const u64* src, size_t words, const NewtFoldArgs* fold = nullptr)
+// by_place: the placement of the iteration's one ranked output publishes (as
+// sequence number pub_seq + 1), and this call only takes note of it
+static u64* publish_begin(pra_ctx* c, const u64* src, size_t words, const NewtFoldArgs* fold = nullptr,
+                          bool by_place = false)
 {
     // mailbox word 0: the sequence number; the summary and flags after it
     u64* h = c->mailbox_buf(words + 2) + 1;
     const u64 seq = ++c->pub_seq;
-    if (fold)
+    if (by_place) {
+    } else if (fold)
         pra_launch_newt_fold_publish(c->st, *fold, src, words, c->flags_buf.as<u32>(), h, seq);
     else
         pra_launch_publish(c->st, src, words, c->flags_buf.as<u32>(), h, seq);
@@ -1385,6 +1405,15 @@ static void unique_rows(pra_ctx* c, Rows& r, int w)
     r.n = h[0];
 }
 
+// rows in column order into trie order: a stable partition by bucket; bnd
+// receives the bucket bounds
+static void bucket_rows(pra_ctx* c, const u64* rows, u64 n, int w, int jcc, u64* out, u64* bnd)
+{
+    c->part_scratch.reserve(pra_partition_scratch_words(n, (u32)c->nb) * 4 + 256, c->st);
+    pra_launch_partition(c->st, rows, n, w, jcc, (u32)c->nb, out, bnd, c->part_scratch.as<u32>());
+    check_launch("bucket_rows");
+}
+
 // (Re)build instance gi's value dictionary from the key columns of every
 // relation of that instance.
 static void build_dictionary(pra_ctx* c, int gi)
@@ -1414,14 +1443,17 @@ static void build_dictionary(pra_ctx* c, int gi)
     pra_launch_fill_u64(c->st, G.dict.as<u64>(), cap * 2, 0);
     pra_launch_dict_insert(c->st, V.d(), V.n, G.dict.as<u64>(), cap, c->dflags());
     check_launch("dict_insert");
+    G.vals.reserve(V.n * 8, c->st);
+    HIPCHK(hipMemcpyAsync(G.vals.p, V.d(), V.n * 8, hipMemcpyDeviceToDevice, c->st));
     if (c->nb > 1) {
-        c->sort_tmp.reserve(V.n * 8, c->st);
-        c->orand.reserve((size_t)(c->nb + 1) * 8, c->st);
-        c->part_scratch.reserve(pra_partition_scratch_words(V.n, (u32)c->nb) * 4 + 256, c->st);
-        pra_launch_partition(c->st, V.d(), V.n, 1, 1, (u32)c->nb, c->sort_tmp.as<u64>(), c->orand.as<u64>(),
-                             c->part_scratch.as<u32>());
+        G.lead_vals.reserve(V.n * 8, c->st);
         G.rank_of.reserve(V.n * 4, c->st);
-        pra_launch_dict_bucket_rank(c->st, c->sort_tmp.as<u64>(), V.n, G.dict.as<u64>(), cap, G.rank_of.as<u32>());
+        G.lead_of.reserve(V.n * 4, c->st);
+        G.lead_bucket.reserve(V.n, c->st);
+        c->tmp64a.reserve((size_t)(c->nb + 1) * 8, c->st);
+        bucket_rows(c, V.d(), V.n, 1, 1, G.lead_vals.as<u64>(), c->tmp64a.as<u64>());
+        pra_launch_dict_bucket_rank(c->st, G.lead_vals.as<u64>(), V.n, G.dict.as<u64>(), cap, G.rank_of.as<u32>(),
+                                    G.lead_of.as<u32>(), (u64)c->nb, G.lead_bucket.as<unsigned char>());
         check_launch("dict_bucket_rank");
     }
     sync_check(c);
@@ -1437,15 +1469,6 @@ static void build_dictionary(pra_ctx* c, int gi)
 // them in column order.
 static bool by_bucket(const pra_ctx* c, const pra_rel* R) { return c->nb > 1 && R->jcc == 1; }
 static bool bits_in_trie_order(const pra_ctx* c, const pra_rel* R) { return c->nb == 1 || R->jcc == 1; }
-
-// r's rows, in column order, into trie order: a stable partition by bucket;
-// bnd receives the bucket bounds
-static void bucket_rows(pra_ctx* c, const u64* rows, u64 n, int w, int jcc, u64* out, u64* bnd)
-{
-    c->part_scratch.reserve(pra_partition_scratch_words(n, (u32)c->nb) * 4 + 256, c->st);
-    pra_launch_partition(c->st, rows, n, w, jcc, (u32)c->nb, out, bnd, c->part_scratch.as<u32>());
-    check_launch("bucket_rows");
-}
 
 // Order an interned relation's full version through its membership bitmap
 // (k_bm_place): one read and one write of the rows, where a sort moves them
@@ -1568,6 +1591,37 @@ static void ensure_index(pra_ctx* c, pra_rel* R, int v)
     R->idx_valid[v] = true;
 }
 
+// The dictionary words of a sorted version's columns and the first row of each
+// leading digit, for emissions in digits.  False when a value has no rank or
+// there is no room for 8 bytes a column.
+static bool ensure_rank_rows(pra_ctx* c, pra_rel* R, int v)
+{
+    const Group& G = grp(c, R->group);
+    Rows& r = R->ver[v];
+    if (R->rk_gen[v] == G.dict_gen) return true;
+    if (R->rk_no[v] || R->jcc != 1 || !r.sorted || r.n >= (1ULL << 32)) return false;
+    try {
+        R->rk_words[v].reserve(r.n * (u64)R->arity * 8, c->st);
+        R->rk_first[v].reserve((G.dict_n + 1) * 4, c->st);
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        R->rk_words[v].release();
+        R->rk_no[v] = true;
+        return false;
+    }
+    c->orand.reserve(32 * 8, c->st);
+    pra_launch_fill_u64(c->st, c->orand.as<u64>(), 1, 0);
+    pra_launch_rank_rows(c->st, r.d(), r.n, R->w, R->arity, G.dict.as<u64>(), G.dict_cap, G.dict_n, c->nb > 1,
+                         R->rk_words[v].as<u64>(), R->rk_first[v].as<u32>(), c->orand.as<u64>());
+    check_launch("rank_rows");
+    if (readback(c, c->orand.p, 1)[0]) {
+        R->rk_no[v] = true;
+        return false;
+    }
+    R->rk_gen[v] = G.dict_gen;
+    return true;
+}
+
 // membership table of full u delta keyed on kw leading columns, with room for
 // `incoming` more keys at load factor <= 1/2
 static void ensure_member_table(pra_ctx* c, pra_rel* R, int kw, u64 incoming)
@@ -1688,6 +1742,7 @@ static bool ensure_ranked(pra_ctx* c, pra_rel* R, u64 bits, u64 base, u64 C, boo
         }
         R->sbs_use = sbs;
         reserve_first(c, base + C);
+        R->nx.reserve(C * 8, c->st);
         prepare_lookback(c, C);
     } catch (const PraError& e) {
         if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
@@ -2105,69 +2160,9 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             if (ra.active) ensure_sorted(c, ra.outer, ra.outer_v);
         }
     }
+    for (auto& ra : S->ras) ra.n_outer = ra.active ? ra.outer->ver[ra.outer_v].n : 0;
 
-    // 1. per-RA output counts and their exclusive offsets (the arrival plan
-    //    reads them at the source-bucket bounds)
-    c->stage.reserve((size_t)std::max(1, nra) * 2 * nb * 8, c->st);
-    CountScanBatch csb;
-    memset(&csb, 0, sizeof(csb));
-    double cs_bytes = 0;
-    auto flush_count_scans = [&]() {
-        if (!csb.njobs) return;
-        prepare_lookback(c, (u64)csb.tile_base[csb.njobs] * PRA_TILE);
-        const u32 ep = next_sort_epoch(c);
-        {
-            Prof p(c, K_JOIN_COUNT, cs_bytes);
-            pra_launch_count_scan_many(c->st, csb, c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
-            check_launch("count_scan_many");
-        }
-        memset(&csb, 0, sizeof(csb));
-        cs_bytes = 0;
-    };
-    for (int r = 0; r < nra; r++) {
-        RADesc& ra = S->ras[r];
-        Rows& O = ra.outer->ver[ra.outer_v];
-        u64 n = O.n;
-        ra.n_outer = ra.active ? n : 0;
-        if (!ra.active) continue;
-        ra.off.reserve((n + 1) * 8, c->st);
-        ra.istart.reserve(std::max<u64>(1, n) * 8, c->st);
-        if (n == 0) {
-            pra_launch_fill_u64(c->st, ra.off.as<u64>(), 1, 0);
-        } else {
-            // the counts and their offsets in one pass, batched over rules
-            CountScanJob& j = csb.job[csb.njobs];
-            memset(&j, 0, sizeof(j));
-            j.outer = O.d();
-            j.n = n;
-            j.wo = ra.outer->w;
-            j.off = ra.off.as<u64>();
-            const bool join = ra.type == RA_JOIN;
-            j.kind = !join ? PRA_CS_FILTER : ra.sorted_probe ? PRA_CS_SORTED : PRA_CS_INDEX;
-            if (join) {
-                j.inner = ra.inner->ver[ra.inner_v].d();
-                j.wi = ra.inner->w;
-                j.jcc = ra.in0->jcc;
-                j.istart = ra.istart.as<u64>();
-                if (ra.sorted_probe) {
-                    j.ibnd = ra.inner->bnd[ra.inner_v].as<u64>();
-                    j.nb = (u64)nb;
-                } else {
-                    j.table = ra.inner->idx[ra.inner_v].as<u64>();
-                    j.cap = ra.inner->idx_cap[ra.inner_v];
-                }
-            } else {
-                j.op = ra.type == RA_COPY_FILTER ? ra.op : PRA_F_TRUE;
-            }
-            csb.tile_base[csb.njobs + 1] = csb.tile_base[csb.njobs] + pra_tiles(n);
-            cs_bytes += 8.0 * n * ra.outer->w + (join ? 24.0 : 8.0) * n;
-            if (++csb.njobs == PRA_CS_JOBS) flush_count_scans();
-        }
-        bucket_bounds(c, ra.outer, ra.outer_v);
-    }
-    flush_count_scans();
-
-    // 2. output relations, their rule kinds, and candidate capacities: the
+    // 1. output relations, their rule kinds, and candidate capacities: the
     //    previous iteration's count with headroom, else an upper bound from the
     //    outer sizes and the inner index's longest key run.  No host
     //    synchronization: the arrival plan is computed on the device and an
@@ -2244,6 +2239,183 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         mixed = mixed || bits > ((unsigned __int128)1 << 35);
     }
 
+    size_t nactive = 0;
+    for (size_t oi = 0; oi < no; oi++) nactive += cap[oi] ? 1 : 0;
+    // per output: its rows (dest, slot_of, keep), candidate words and
+    // histogram words in the shared buffers when its claim and decision are
+    // batched with other outputs
+    struct OutRegion {
+        u64 rb = 0, cb = 0, hb = 0;
+    };
+    std::vector<OutRegion> reg(no);
+    u64 region_rows = 0;
+    if (nactive >= 2)
+        for (size_t oi = 0; oi < no; oi++) {
+            reg[oi].rb = region_rows;
+            region_rows += cap[oi];
+        }
+
+    // dense membership of an output with C candidates of capacity: 0 = the
+    // general table, 1 = the claim table, 2 = ranked.  Ranked membership
+    // moves each candidate through a few light launches and needs no sort;
+    // the claim table needs less memory.  From kTuneMinCandidates candidates
+    // of capacity on, single-output iterations time both (the claim table's
+    // sizes first) and the band's cheaper one is kept; below that, and
+    // untimed, ranked (150x150 grid, 846 K candidates an iteration:
+    // membership, new rows and their sort 118 us by the claim table, 88 us
+    // ranked).
+    struct Choice {
+        int mode = 0, dvar = 0;
+        bool dtime = false, rtime = false;
+    };
+    std::vector<char> dense_off(no, 0);   // redone the general way in this iteration
+    auto decide = [&](size_t oi, u64 C, int phase, u64 rb) {
+        Choice ch;
+        pra_rel* R = outs[oi];
+        u64 bits = 0;
+        if (dense_off[oi] || !packed[oi] || !ensure_bitmap(c, R, R->arity, C, &bits)) return ch;
+        ch.mode = 2;
+        if (c->tune_on && C >= kTuneMinCandidates) {
+            const int band = band_of(C), load = g_tune.settled(c->device, TUNE_DENSE_LOAD, band);
+            ch.dvar = std::max(0, load);
+            if (phase != 0) {
+                // outputs of a batched iteration share their launches and are
+                // not timed
+            } else if (load < 0) {
+                ch.dvar = g_tune.pick(c->device, TUNE_DENSE_LOAD, band, kTuneVariants[TUNE_DENSE_LOAD]);
+                ch.dtime = true;
+                ch.mode = 1;
+            } else {
+                ch.mode = 1 + g_tune.pick(c->device, TUNE_RANKED, band, kTuneVariants[TUNE_RANKED]);
+                ch.rtime = g_tune.settled(c->device, TUNE_RANKED, band) < 0;
+            }
+        }
+        // next to outputs that take the general table, the claim table
+        // shares the partition and sort launches they need anyway: two
+        // launches more, where ranked membership is four (points-to
+        // analysis, 62 iterations: 15.04 against 15.60 ms)
+        if (phase == 1 && mixed && C < kMixedRankedCandidates) ch.mode = 1;
+        if (ch.mode == 2 && !ensure_ranked(c, R, bits, rb, C, phase == 0)) {
+            ch.mode = 1;
+            ch.rtime = false;
+        }
+        if (ch.mode == 1) ensure_claims(c, R, bits, C, 2ULL << ch.dvar);
+        return ch;
+    };
+    // the rule of a ranked output that can be emitted in digits (k_rank_emit):
+    // its only active one, a join on one column of a delta whose rank indexes
+    // are at hand with an inner version that stays as it is, projecting data
+    // columns.  A thread walks its row's matches, so joins with a run of more
+    // than kEmitRun inner rows take the expansion that balances outputs.
+    // -1: none.
+    std::vector<char> emit_off(no, 0);
+    auto emit_rule_of = [&](size_t oi) {
+        pra_rel* R = outs[oi];
+        if (emit_off[oi] || !bits_in_trie_order(c, R)) return -1;
+        int rule = -1;
+        for (int r = 0; r < nra; r++)
+            if (S->ras[r].active && S->ras[r].out == R) {
+                if (rule >= 0) return -1;
+                rule = r;
+            }
+        if (rule < 0) return -1;
+        RADesc& ra = S->ras[rule];
+        const Group& G = grp(c, R->group);
+        if (ra.type != RA_JOIN || ra.sorted_probe || ra.outer_v != PRA_DELTA || ra.outer->dx_gen != G.dict_gen ||
+            ra.outer->jcc != 1 || ra.inner->jcc != 1 || ra.outer->arity > 4 || ra.inner->view_of || ra.outer->view_of ||
+            ra.inner->idx_maxlen[ra.inner_v] > kEmitRun || ra.n_outer >= (1ULL << 32))
+            return -1;
+        for (int m : ra.map) {
+            const int first = ra.left ? ra.outer->w : ra.inner->w;
+            const int w = m < first ? first : ra.left ? ra.inner->w : ra.outer->w;
+            const int col = m < first ? m : ra.in0->jcc + (m - first);
+            if (col >= w - 1) return -1;   // an intern id
+        }
+        return ensure_rank_rows(c, ra.inner, ra.inner_v) ? rule : -1;
+    };
+    // taken per output; the rule an output emits (-1: the general expansions);
+    // an emission that stopped left fresh bits that only another would set
+    std::vector<Choice> choice(no);
+    std::vector<int> emit_rule(no, -1);
+    std::vector<char> use_dense(no, 0), fresh_left(no, 0);
+    if (nactive >= 2) {
+        try {
+            reserve_first(c, region_rows);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        }
+    }
+    for (size_t oi = 0; oi < no; oi++) {
+        if (!cap[oi]) continue;
+        choice[oi] = decide(oi, cap[oi], nactive >= 2 ? 1 : 0, reg[oi].rb);
+        if (choice[oi].mode == 2) emit_rule[oi] = emit_rule_of(oi);
+    }
+
+    // 2. per-RA output counts and their exclusive offsets (the arrival plan
+    //    reads them at the source-bucket bounds); an output that emits in
+    //    digits counts its rule itself
+    c->stage.reserve((size_t)std::max(1, nra) * 2 * nb * 8, c->st);
+    CountScanBatch csb;
+    memset(&csb, 0, sizeof(csb));
+    double cs_bytes = 0;
+    auto flush_count_scans = [&]() {
+        if (!csb.njobs) return;
+        prepare_lookback(c, (u64)csb.tile_base[csb.njobs] * PRA_TILE);
+        const u32 ep = next_sort_epoch(c);
+        {
+            Prof p(c, K_JOIN_COUNT, cs_bytes);
+            pra_launch_count_scan_many(c->st, csb, c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
+            check_launch("count_scan_many");
+        }
+        memset(&csb, 0, sizeof(csb));
+        cs_bytes = 0;
+    };
+    std::vector<char> counted((size_t)nra, 0);
+    auto count_rule = [&](int r) {
+        RADesc& ra = S->ras[r];
+        if (!ra.active || counted[(size_t)r]) return;
+        counted[(size_t)r] = 1;
+        Rows& O = ra.outer->ver[ra.outer_v];
+        u64 n = O.n;
+        ra.off.reserve((n + 1) * 8, c->st);
+        ra.istart.reserve(std::max<u64>(1, n) * 8, c->st);
+        if (n == 0) {
+            pra_launch_fill_u64(c->st, ra.off.as<u64>(), 1, 0);
+        } else {
+            // the counts and their offsets in one pass, batched over rules
+            CountScanJob& j = csb.job[csb.njobs];
+            memset(&j, 0, sizeof(j));
+            j.outer = O.d();
+            j.n = n;
+            j.wo = ra.outer->w;
+            j.off = ra.off.as<u64>();
+            const bool join = ra.type == RA_JOIN;
+            j.kind = !join ? PRA_CS_FILTER : ra.sorted_probe ? PRA_CS_SORTED : PRA_CS_INDEX;
+            if (join) {
+                j.inner = ra.inner->ver[ra.inner_v].d();
+                j.wi = ra.inner->w;
+                j.jcc = ra.in0->jcc;
+                j.istart = ra.istart.as<u64>();
+                if (ra.sorted_probe) {
+                    j.ibnd = ra.inner->bnd[ra.inner_v].as<u64>();
+                    j.nb = (u64)nb;
+                } else {
+                    j.table = ra.inner->idx[ra.inner_v].as<u64>();
+                    j.cap = ra.inner->idx_cap[ra.inner_v];
+                }
+            } else {
+                j.op = ra.type == RA_COPY_FILTER ? ra.op : PRA_F_TRUE;
+            }
+            csb.tile_base[csb.njobs + 1] = csb.tile_base[csb.njobs] + pra_tiles(n);
+            cs_bytes += 8.0 * n * ra.outer->w + (join ? 24.0 : 8.0) * n;
+            if (++csb.njobs == PRA_CS_JOBS) flush_count_scans();
+        }
+        bucket_bounds(c, ra.outer, ra.outer_v);
+    };
+    for (int r = 0; r < nra; r++)
+        if (emit_rule[std::find(outs.begin(), outs.end(), S->ras[r].out) - outs.begin()] != r) count_rule(r);
+    flush_count_scans();
+
     // 3+4. per output: arrival plan, emit candidates, deduplicate, partition
     //      and intern, summaries for the sort
     // rs == nullptr: the iteration's whole emission; else one threshold round
@@ -2265,19 +2437,19 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     std::vector<CopyExpandArgs> cexp_jobs;
     std::vector<u32> cexp_blocks;
     double cexp_bytes = 0;
-    // planned: the arrival plan was made by the iteration's batched plan
-    // per output: its rows (dest, slot_of, keep), candidate words and
-    // histogram words in the shared buffers when its claim and decision are
-    // batched with other outputs
-    struct OutRegion {
-        u64 rb = 0, cb = 0, hb = 0;
+    static const int rank_kind[PRA_RANK_STEPS] = {K_RANK_EMIT, K_DEDUP_CLAIM, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE};
+    auto rank_bytes = [](int step, int kw) {   // per candidate
+        return step == PRA_RANK_EMIT    ? 24.0
+               : step == PRA_RANK_CLAIM ? 8.0 * (kw + 1)
+               : step == PRA_RANK_FIRST ? 16.0
+               : step == PRA_RANK_PLACE ? 8.0 * (kw + 2) + 12.0
+                                        : 0.0;
     };
-    std::vector<OutRegion> reg(no);
+    // an iteration of one ranked output: its placement publishes the summary
+    const bool place_publishes = no == 1 && nactive == 1 && choice[0].mode == 2;
+    // planned: the arrival plan was made by the iteration's batched plan
     std::vector<ClaimJob> claim_jobs(no);
     std::vector<DecideJob> decide_jobs(no);
-    // dense membership: taken per output, switched off for the rest of the
-    // iteration by a dictionary miss; the dense claims of a batched iteration
-    std::vector<char> use_dense(no, 0), dense_off(no, 0);
     std::vector<ScanJob> scan_jobs;
     std::vector<std::pair<DenseArgs, size_t>> dense_jobs;
     std::vector<std::pair<RankArgs, size_t>> rank_jobs;
@@ -2297,65 +2469,47 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         Rows& NT = R->ver[PRA_NEWT];
         u64* st2o = c->stage2.as<u64>() + oi * SW;
         u64* ctl = st2o + 4;
-        // dense membership unless the output was redone the general way in
-        // this iteration, or this is a threshold round.  Ranked membership
-        // moves each candidate through four light launches and needs no sort;
-        // the claim table needs less memory.  From kTuneMinCandidates
-        // candidates of capacity on, single-output iterations time both (the
-        // claim table's sizes first) and the band's cheaper one is kept; below
-        // that, and untimed, ranked (150x150 grid, 846 K candidates an
-        // iteration: membership, new rows and their sort 118 us by the claim
-        // table, 88 us ranked).
-        int dvar = 0, mode = use_dense[oi];
-        bool dtime = false, rtime = false;
+        // dense membership: the first pass as decided above, a re-run anew, a
+        // threshold round by the general table
+        Choice ch;
+        if (phase >= 2)
+            ch.mode = use_dense[oi];
+        else if (planned)
+            ch = choice[oi];
+        else if (!rs)
+            ch = decide(oi, C, 0, 0);
+        const int mode = ch.mode, dvar = ch.dvar;
+        const bool dtime = ch.dtime, rtime = ch.rtime;
         hipEvent_t tr = nullptr;   // opens the claim table's share of the choice
-        if (phase < 2) {
-            u64 bits = 0;
-            mode = 0;
-            if (!rs && !dense_off[oi] && packed[oi] && ensure_bitmap(c, R, kw, C, &bits)) {
-                mode = 2;
-                if (c->tune_on && C >= kTuneMinCandidates) {
-                    const int band = band_of(C), load = g_tune.settled(c->device, TUNE_DENSE_LOAD, band);
-                    dvar = std::max(0, load);
-                    if (phase != 0) {
-                        // outputs of a batched iteration share their launches
-                        // and are not timed
-                    } else if (load < 0) {
-                        dvar = g_tune.pick(c->device, TUNE_DENSE_LOAD, band, kTuneVariants[TUNE_DENSE_LOAD]);
-                        dtime = true;
-                        mode = 1;
-                    } else {
-                        mode = 1 + g_tune.pick(c->device, TUNE_RANKED, band, kTuneVariants[TUNE_RANKED]);
-                        rtime = g_tune.settled(c->device, TUNE_RANKED, band) < 0;
-                    }
-                }
-                // next to outputs that take the general table, the claim table
-                // shares the partition and sort launches they need anyway: two
-                // launches more, where ranked membership is four (points-to
-                // analysis, 62 iterations: 15.04 against 15.60 ms)
-                if (phase == 1 && mixed && C < kMixedRankedCandidates) mode = 1;
-                if (mode == 2 && !ensure_ranked(c, R, bits, rg.rb, C, phase == 0)) {
-                    mode = 1;
-                    rtime = false;
-                }
-                if (mode == 1) ensure_claims(c, R, bits, C, 2ULL << dvar);
-            }
-        }
         const bool dn = mode != 0, ranked = mode == 2;
         use_dense[oi] = (char)mode;
         if (phase >= 2 && ranked) return;   // its new rows are in place
+        const int er = !ranked ? -1 : planned ? emit_rule[oi] : emit_rule_of(oi);
+        if (phase < 2 && fresh_left[oi]) {
+            if (er < 0) reset_ranked(c, R);
+            fresh_left[oi] = 0;
+        }
+        if (!planned && er < 0) {
+            for (int r = 0; r < nra; r++)
+                if (S->ras[r].out == R) count_rule(r);
+            flush_count_scans();
+        }
         if (dn)
             R->mt_valid = false;   // the general table is not kept current meanwhile
         else
             R->bm_valid = false, ensure_member_table(c, R, kw, C);
-        c->cand.reserve(C * cw * 8, c->st);
-        c->dest.reserve(C * 4, c->st);
+        if (er < 0) {
+            c->cand.reserve(C * cw * 8, c->st);
+            c->dest.reserve(C * 4, c->st);
+        }
         c->slot_of.reserve(C * 8, c->st);
         c->keep.reserve(C * 4, c->st);
         NT.buf.reserve((nt_base + C) * R->w * 8, c->st, nt_base * R->w * 8);
         const u32 nblocks = pra_tiles(C);
-        c->hist.reserve((size_t)nb * nblocks * 4, c->st);
-        c->offs.reserve((size_t)nb * nblocks * 4 + 8, c->st);
+        if (!ranked) {
+            c->hist.reserve((size_t)nb * nblocks * 4, c->st);
+            c->offs.reserve((size_t)nb * nblocks * 4 + 8, c->st);
+        }
         u64* cand0 = c->cand.as<u64>() + rg.cb;
         u32* dest0 = c->dest.as<u32>() + rg.rb;
         u64* slot0 = c->slot_of.as<u64>() + rg.rb;
@@ -2363,7 +2517,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         u32* hist0 = c->hist.as<u32>() + rg.hb;
         u32* offs0 = c->offs.as<u32>() + rg.hb;
         if (phase < 2) {
-            if (!planned) {
+            if (!planned && er < 0) {
                 PlanArgs pa;
                 memset(&pa, 0, sizeof(pa));
                 pa.srcoff = c->stage.as<u64>();
@@ -2403,7 +2557,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             }
             for (int r = 0; r < nra; r++) {
                 RADesc& ra = S->ras[r];
-                if (ra.out != R || !ra.active) continue;
+                if (ra.out != R || !ra.active || er >= 0) continue;
                 size_t k = 0;   // position in the round's rule list
                 if (rs) {
                     while (k < rs->ras.size() && rs->ras[k] != r) k++;
@@ -2479,6 +2633,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 memset(&ra, 0, sizeof(ra));
                 Group& G = grp(c, R->group);
                 Group::Seq& sq = seq_counters(c, R->group, R->tag);
+                const bool lead = by_bucket(c, R);
                 ra.cand = cand0;
                 ra.ctl = ctl;
                 ra.xs = slot0;
@@ -2487,16 +2642,21 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 ra.dict = G.dict.as<u64>();
                 ra.dict_cap = G.dict_cap;
                 ra.D = G.dict_n;
+                ra.inv = 1.0 / (double)G.dict_n;
                 ra.member = R->bm.as<u32>();
                 ra.fresh = R->fresh.as<u32>();
                 ra.dirty = R->dirty.as<u32>();
                 ra.sbpre = R->sbpre.as<u32>();
                 ra.linep = R->linep.as<unsigned short>();
                 ra.first = c->first.as<u32>() + rg.rb;
+                ra.vals = G.vals.as<u64>();
+                ra.lead_vals = (lead ? G.lead_vals : G.vals).as<u64>();
+                ra.bucket = G.lead_bucket.as<unsigned char>();
                 ra.newt = NT.d();
                 if (bits_in_trie_order(c, R)) {
                     R->next_bnd.reserve((size_t)(nb + 1) * 8, c->st);
                     ra.bnd = R->next_bnd.as<u64>();
+                    ra.nx = R->nx.as<u64>();
                 }
                 ra.stat = st2o;
                 ra.seq = sq.buf.as<u64>() + sq.now * nb;
@@ -2505,25 +2665,59 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 ra.chunks = std::min<u32>(PRA_SCAN_CHUNKS, (ra.sbs + 15) / 16);
                 ra.nb = (u32)nb;
                 ra.tag = R->tag;
-                ra.cw = cw;
                 ra.kw = kw;
                 ra.wn = R->w;
-                ra.by_bucket = by_bucket(c, R);
+                ra.by_bucket = lead;
+                if (planned && place_publishes) {
+                    ra.host = c->mailbox_buf(no * SW + 2) + 1;
+                    ra.host_seq = c->pub_seq + 1;
+                    ra.host_words = (u32)(no * SW);
+                    ra.err = c->dflags();
+                }
+                if (er >= 0) {
+                    RADesc& rule = S->ras[er];
+                    EmitArgs& em = ra.emit;
+                    em.dx = rule.outer->dx.as<u64>();
+                    em.n = rule.n_outer;
+                    em.cap = C;
+                    em.thresh = c->threshold;
+                    em.joined = G.joined.as<u64>();
+                    em.first = rule.inner->rk_first[rule.inner_v].as<u32>();
+                    em.words = rule.inner->rk_words[rule.inner_v].as<u64>();
+                    em.rank_of = G.rank_of.as<u32>();
+                    em.lead_of = G.lead_of.as<u32>();
+                    em.inv = ra.inv;
+                    em.kwo = rule.outer->arity;
+                    em.ia = rule.inner->arity;
+                    for (int i = 0; i < kw; i++) {
+                        const int m = rule.map[i], first = rule.left ? rule.outer->w : rule.inner->w;
+                        const bool outer = (m < first) == (rule.left != 0);
+                        const int col = m < first ? m : rule.in0->jcc + (m - first);
+                        em.side[i] = outer ? 0 : 1;
+                        em.col[i] = (signed char)col;
+                        // outer digits: the first is a leading digit (with
+                        // several buckets), the others are ranks
+                        const bool have = outer && nb > 1 && col == 0, want = i == 0 && lead;
+                        em.conv[i] = !outer || have == want ? 0 : have ? 1 : 2;
+                    }
+                }
                 if (phase == 1) {
                     // launched after the batched expansions
                     rank_jobs.emplace_back(ra, oi);
                     return;
                 }
+                const u64 etiles = er >= 0 ? (ra.emit.n + PRA_EMIT_BLOCK - 1) / PRA_EMIT_BLOCK : 0;
+                prepare_lookback(c, std::max<u64>(C, (etiles + PRA_RADIX - 1) / PRA_RADIX * PRA_TILE));
                 hipEvent_t ta = c->tune_begin(rtime);
-                static const int kind[4] = {K_DEDUP_CLAIM, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE};
-                const double bytes[4] = {8.0 * (kw + 1), 0.0, 16.0, 8.0 * cw + 8.0 * R->w + 12.0};
-                for (int step = 0; step < 4; step++) {
+                for (int step = 0; step < PRA_RANK_STEPS; step++) {
+                    if (step == (er >= 0 ? PRA_RANK_CLAIM : PRA_RANK_EMIT)) continue;
                     const u32 ep = next_sort_epoch(c);
-                    ProfPerCand p(c, kind[step], bytes[step], oi);
+                    ProfPerCand p(c, rank_kind[step], rank_bytes(step, kw), oi);
                     pra_launch_rank(c->st, step, ra, C, c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
                     check_launch("rank");
                 }
                 c->tune_end(ta, TUNE_RANKED, band_of(C), 1, oi, C);
+                fresh_left[oi] = er >= 0;
                 return;
             }
             if (dn) {
@@ -2736,12 +2930,12 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         std::vector<PlanOut> pouts;
         for (int r = 0; r < nra; r++) {
             RADesc& ra = S->ras[r];
-            if (ra.active)
+            if (ra.active && counted[(size_t)r])
                 rules[(size_t)r] = PlanRule{ra.off.as<u64>(), ra.outer->bnd[ra.outer_v].as<u64>(),
                                             ra.type == RA_JOIN ? 1u : 0u, 0u};
         }
         for (size_t oi = 0; oi < no; oi++) {
-            if (!cap[oi]) continue;
+            if (!cap[oi] || emit_rule[oi] >= 0) continue;
             PlanOut po{cap[oi], grp(c, outs[oi]->group).joined.as<u64>(), (u32)ids.size(), 0, (u32)oi, 0};
             for (int r = 0; r < nra; r++)
                 if (S->ras[r].active && S->ras[r].out == outs[oi]) ids.push_back((u32)r);
@@ -2757,7 +2951,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         const char* d = stage_table(c, JOB_PLAN, t.data(), t.size());
         PlanTabArgs pa{c->stage.as<u64>(), c->posadj_dev.as<u64>(), c->stage2.as<u64>(), c->threshold, nb, (int)SW,
                        (const PlanRule*)d, (const u32*)(d + rb), (const PlanOut*)(d + rb + ib)};
-        pra_launch_plan_tab(c->st, pa, (int)pouts.size());
+        if (!pouts.empty()) pra_launch_plan_tab(c->st, pa, (int)pouts.size());
         check_launch("plan_tab");
     } else {
         PlanAllArgs pl;
@@ -2773,12 +2967,12 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         int nblk = 0;
         for (size_t oi = 0; oi < no; oi++) {
             pl.cap[oi] = cap[oi];
-            if (cap[oi]) pl.outs[nblk++] = (unsigned char)oi;
+            if (cap[oi] && emit_rule[oi] < 0) pl.outs[nblk++] = (unsigned char)oi;
         }
         for (int r = 0; r < nra; r++) {
             RADesc& ra = S->ras[r];
             pl.rout[r] = 0xFF;
-            if (!ra.active) continue;
+            if (!ra.active || !counted[(size_t)r]) continue;
             const size_t oi = std::find(outs.begin(), outs.end(), ra.out) - outs.begin();
             pl.rout[r] = (unsigned char)oi;
             pl.is_join[r] = ra.type == RA_JOIN;
@@ -2788,31 +2982,24 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         pra_launch_plan_all(c->st, pl, nblk);
         check_launch("plan_all");
     }
-    size_t nactive = 0;
-    for (size_t oi = 0; oi < no; oi++) nactive += cap[oi] ? 1 : 0;
     if (plan_all && nactive >= 2) {
         // every output's candidates in its own region; their claims and
         // decisions batched by key width
-        u64 rt = 0, ct = 0, ht = 0;
+        u64 ct = 0, ht = 0;
         for (size_t oi = 0; oi < no; oi++) {
             if (!cap[oi]) continue;
             const int cwo = out_intern[oi] == 1 ? outs[oi]->arity : outs[oi]->arity + 1;
-            reg[oi] = OutRegion{rt, ct, ht};
-            rt += cap[oi];
-            ct += cap[oi] * (u64)cwo;
-            ht += (u64)nb * pra_tiles(cap[oi]) + 2;
+            reg[oi].cb = ct;
+            reg[oi].hb = ht;
+            if (emit_rule[oi] < 0) ct += cap[oi] * (u64)cwo;
+            if (choice[oi].mode != 2) ht += (u64)nb * pra_tiles(cap[oi]) + 2;
         }
-        c->cand.reserve(ct * 8, c->st);
-        c->dest.reserve(rt * 4, c->st);
-        c->slot_of.reserve(rt * 8, c->st);
-        c->keep.reserve(rt * 4, c->st);
+        c->cand.reserve(std::max<u64>(ct, 1) * 8, c->st);
+        c->dest.reserve(region_rows * 4, c->st);
+        c->slot_of.reserve(region_rows * 8, c->st);
+        c->keep.reserve(region_rows * 4, c->st);
         c->hist.reserve(ht * 4, c->st);
         c->offs.reserve(ht * 4 + 8, c->st);
-        try {
-            reserve_first(c, rt);
-        } catch (const PraError& e) {
-            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
-        }
         for (size_t oi = 0; oi < no; oi++)
             if (cap[oi]) run_output(oi, nullptr, true, 1);
         // the expansions of all rules: job tables through pinned staging into
@@ -2855,38 +3042,40 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         // the ranked outputs: one table through pinned staging, one launch a step
         if (!rank_jobs.empty()) {
             const size_t n = rank_jobs.size();
-            std::vector<char> t(n * sizeof(RankArgs) + 3 * (n + 1) * 4);
+            std::vector<char> t(n * sizeof(RankArgs) + PRA_RANK_STEPS * (n + 1) * 4);
             RankArgs* J = (RankArgs*)t.data();
-            u32* base[3];
-            for (int q = 0; q < 3; q++) {
+            u32* base[PRA_RANK_STEPS];
+            for (int q = 0; q < PRA_RANK_STEPS; q++) {
                 base[q] = (u32*)(t.data() + n * sizeof(RankArgs)) + q * (n + 1);
                 base[q][0] = 0;
             }
             for (size_t k = 0; k < n; k++) {
-                const u64 C = cap[rank_jobs[k].second];
+                const size_t oi = rank_jobs[k].second;
+                const u64 C = cap[oi];
                 J[k] = rank_jobs[k].first;
-                base[0][k + 1] = base[0][k] + (u32)((C + PRA_BLOCK - 1) / PRA_BLOCK);
-                base[1][k + 1] = base[1][k] + J[k].chunks;
-                base[2][k + 1] = base[2][k] + pra_tiles(C);
+                const bool em = emit_rule[oi] >= 0;
+                const u32 cb = (u32)((C + PRA_BLOCK - 1) / PRA_BLOCK);
+                const u32 blocks[PRA_RANK_STEPS] = {
+                    em ? (u32)((J[k].emit.n + PRA_EMIT_BLOCK - 1) / PRA_EMIT_BLOCK) : 0, em ? 0 : cb, J[k].chunks, cb,
+                    pra_tiles(C)};
+                for (int q = 0; q < PRA_RANK_STEPS; q++) base[q][k + 1] = base[q][k] + blocks[q];
+                fresh_left[oi] = em;
             }
-            prepare_lookback(c, std::max<u64>(base[2][n], (base[1][n] + PRA_RADIX - 1) / PRA_RADIX) * PRA_TILE);
+            const u64 words = std::max(base[PRA_RANK_EMIT][n], base[PRA_RANK_SCAN][n]);
+            prepare_lookback(c, std::max<u64>(base[PRA_RANK_PLACE][n], (words + PRA_RADIX - 1) / PRA_RADIX) * PRA_TILE);
             const RankArgs* d = (const RankArgs*)stage_table(c, JOB_RANK, t.data(), t.size());
-            static const int kind[4] = {K_DEDUP_CLAIM, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE};
-            for (int step = 0; step < 4; step++) {
+            for (int step = 0; step < PRA_RANK_STEPS; step++) {
+                if (!base[step][n]) continue;
                 const u32 ep = next_sort_epoch(c);
                 const size_t before = c->pending.size();
                 {
-                    Prof p(c, kind[step], 0.0);
-                    pra_launch_rank_many(c->st, step, d, (int)n, base[step == PRA_RANK_SCAN ? 1 : step == PRA_RANK_PLACE ? 2 : 0][n],
-                                         c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
+                    Prof p(c, rank_kind[step], 0.0);
+                    pra_launch_rank_many(c->st, step, d, (int)n, base[step][n], c->lb_status.as<u64>(),
+                                         c->lb_ctr.as<u32>(), ep, c->dflags());
                     check_launch("rank_many");
                 }
                 if (c->pending.size() == before + 1)
-                    for (auto& j : rank_jobs) {
-                        const RankArgs& a = j.first;
-                        const double per[4] = {8.0 * (a.kw + 1), 0.0, 16.0, 8.0 * a.cw + 8.0 * a.wn + 12.0};
-                        c->per_candidate.emplace_back(before, per[step], j.second);
-                    }
+                    for (auto& j : rank_jobs) c->per_candidate.emplace_back(before, rank_bytes(step, j.first.kw), j.second);
             }
         }
         // the dense claims and decisions: one table per key width through
@@ -3062,7 +3251,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     // sized exactly) or whose dense claims met a value without a dictionary
     // rank (now the general way); pass 2 the few that needed both
     for (int pass = 0; pass < 3; pass++) {
-        u64* h = publish_begin(c, c->stage2.as<u64>(), no * SW, pass == 0 && have_last_fold ? &last_fold : nullptr);
+        u64* h = publish_begin(c, c->stage2.as<u64>(), no * SW, pass == 0 && have_last_fold ? &last_fold : nullptr,
+                               pass == 0 && place_publishes);
         if (pass == 0) {
             std::vector<CopyJob> appends;
             for (size_t i = 0; i < S->rels.size(); i++) {
@@ -3078,7 +3268,9 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         for (size_t oi = 0; oi < no; oi++) {
             if (!cap[oi]) continue;
             std::copy(h + oi * SW, h + (oi + 1) * SW, st2.begin() + oi * SW);
-            if (st2[oi * SW + 5] == 1 || st2[oi * SW + 5] == 3) redo.push_back(oi);
+            const u64 state = st2[oi * SW + 5];
+            if (state == 1 || state == 3 || state == 4) redo.push_back(oi);
+            if (state == 0) fresh_left[oi] = 0;
         }
         if (redo.empty()) break;
         if (pass == 2) throw PraError(PRA_E_HIP, "candidate capacity overflow after resizing");
@@ -3094,6 +3286,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 }
                 dense_off[oi] = 1;
             }
+            // an emission over the join threshold: by the arrival plan
+            if (st2[oi * SW + 5] == 4) emit_off[oi] = 1;
             cap[oi] = st2[oi * SW + 4];
             run_output(oi, nullptr);
         }
@@ -3273,7 +3467,12 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         R->ver[PRA_NEWT].n = 0;
         R->touched(PRA_DELTA);
         auto it = std::find(outs.begin(), outs.end(), R);
-        if (it != outs.end() && bnd_ok[it - outs.begin()]) R->bnd_valid[PRA_DELTA] = true;
+        if (it == outs.end()) continue;
+        if (bnd_ok[it - outs.begin()]) R->bnd_valid[PRA_DELTA] = true;
+        if (placed((size_t)(it - outs.begin())) && bits_in_trie_order(c, R)) {
+            R->dx.swap(R->nx);
+            R->dx_gen = grp(c, R->group).dict_gen;
+        }
     }
     for (pra_scc* m : members) grp(c, m->group).iterations++;
 }
@@ -3690,7 +3889,8 @@ int pra_ctx_group_status(pra_ctx* ctx, int group, int* done, uint64_t* iteration
         for (pra_rel* R : ctx->rels) {
             if (R->group != group) continue;
             for (auto& v : R->ver) b += v.buf.cap;
-            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
+            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->dx, &R->nx,
+                                  &R->rk_words[0], &R->rk_words[1], &R->rk_first[0], &R->rk_first[1], &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
                                   &R->bin_keys, &R->bin_idx, &R->bin_cur, &R->bnd[0], &R->bnd[1]})
                 b += d->cap;
         }

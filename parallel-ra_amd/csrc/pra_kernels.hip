@@ -945,21 +945,54 @@ __global__ void k_dict_insert(const u64* vals, u64 n, u64* tab, u64 cap, u32* fl
 }
 
 // vals: the dictionary's values by (bucket, value); their places into the
-// slots' high halves, and each place's rank into rank_of
-__global__ void k_dict_bucket_rank(const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of)
+// slots' high halves, the maps between places and ranks, and the places'
+// buckets
+__global__ void k_dict_bucket_rank(const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of, u32* lead_of, u64 nb,
+                                   unsigned char* bucket)
 {
     const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const u64 v = vals[i], m = cap - 1;
+    bucket[i] = (unsigned char)pra_bucket(pra_fnv_word(PRA_FNV_OFFSET, v), nb);
     u64 s = pra_dict_slot(v, cap);
     for (u64 q = 0; q < cap && tab[2 * s + 1]; q++) {
         if (tab[2 * s] == v) {
-            rank_of[i] = (u32)tab[2 * s + 1] - 1;
+            const u32 r = (u32)tab[2 * s + 1] - 1;
+            rank_of[i] = r;
+            lead_of[r] = (u32)i;
             tab[2 * s + 1] |= i << 32;
             return;
         }
         s = (s + 1) & m;
     }
+}
+
+// The slot words of the rows' first a columns (a words a row), and, rows
+// sorted by their leading digit, the first row of every digit value (D + 1
+// words); a value without a rank is counted in *miss.
+__global__ void k_rank_rows(const u64* rows, u64 n, int w, int a, const u64* dict, u64 dcap, u64 D, int by_bucket,
+                            u64* words, u32* first, u64* miss)
+{
+    const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    bool ok = true;
+    u64 e0 = 0;
+    for (int c = 0; c < a; c++) {
+        const u64 e = pra_dict_find(dict, dcap, rows[i * w + c]);
+        ok = ok && e != 0;
+        words[i * a + c] = e;
+        if (c == 0) e0 = e;
+    }
+    const u64 p0 = i ? pra_dict_find(dict, dcap, rows[(i - 1) * w]) : 0;
+    if (!ok || (i && !p0)) {
+        atomicAdd((unsigned long long*)miss, 1ULL);
+        return;
+    }
+    const u64 mine = by_bucket ? e0 >> 32 : (u64)((u32)e0 - 1);
+    const u64 prev = !i ? 0 : 1 + (by_bucket ? p0 >> 32 : (u64)((u32)p0 - 1));
+    for (u64 d = prev; d <= mine; d++) first[d] = (u32)i;
+    if (i + 1 == n)
+        for (u64 d = mine + 1; d <= D; d++) first[d] = (u32)n;
 }
 
 // out[i] = in[idx[i]] for rows of w words
@@ -2226,13 +2259,8 @@ __device__ __forceinline__ u32 pra_fresh_rank(const RankArgs& a, u64 x)
     return r;
 }
 
-__device__ __forceinline__ void pra_rank_claim_one(const RankArgs& a, u64 p)
+__device__ __forceinline__ void pra_rank_claim_key(const RankArgs& a, u64 p, u64 x)
 {
-    u64 x;
-    if (!pra_dense_index_n(a.kw, a.cand + p * a.cw, a.dict, a.dict_cap, a.D, a.by_bucket, &x)) {
-        atomicCAS((unsigned long long*)(a.ctl + 1), 0ULL, 3ULL);
-        return;
-    }
     const u32 bit = 1u << (x & 31);
     if (a.member[x >> 5] & bit) {
         a.xs[p] = ~0ULL;
@@ -2243,6 +2271,146 @@ __device__ __forceinline__ void pra_rank_claim_one(const RankArgs& a, u64 p)
         atomicOr(a.fresh + (x >> 5), bit);
         u32* d = a.dirty + (x >> PRA_SB_BITS);
         if (!*d) *d = 1;
+    }
+}
+
+__device__ __forceinline__ void pra_rank_claim_one(const RankArgs& a, u64 p)
+{
+    u64 x;
+    if (!pra_dense_index_n(a.kw, a.cand + p * a.kw, a.dict, a.dict_cap, a.D, a.by_bucket, &x))
+        atomicCAS((unsigned long long*)(a.ctl + 1), 0ULL, 3ULL);
+    else
+        pra_rank_claim_key(a, p, x);
+}
+
+// digits of a rank index x < 2^35 in radix D < 2^32: x = q * D + rest
+__device__ __forceinline__ void pra_digit_split(u64 x, u64 D, double inv, u64* q, u32* rest)
+{
+    u64 k = (u64)((double)x * inv);   // within one of the quotient
+    long long r = (long long)(x - k * D);
+    if (r < 0) {
+        k--;
+        r += (long long)D;
+    } else if (r >= (long long)D) {
+        k++;
+        r -= (long long)D;
+    }
+    *q = k;
+    *rest = (u32)r;
+}
+
+// Emission and claims of a ranked output with one rule, a join of a delta
+// whose rows' rank indexes are known with a static inner relation whose rows
+// are ranked (RankArgs::EmitArgs), in one launch: tiles of outer rows in ticket
+// order find their offsets by look-back over the tiles' match counts, and each
+// match's rank index is put together from digits, without a hash, a value or
+// a candidate row.  With one rule the arrival position of an output is its
+// emission offset.  The last tile leaves the candidate count, the capacity
+// flag (1: over the capacity; 4: over the join threshold, so the arrival plan
+// decides) and the join pairs.  A tile past the capacity claims nothing; the
+// bits of the tiles before it are those the re-run sets again.
+// Why: count, plan, expansion and claim as four launches took 69 us on the
+// 150x150 grid's 430 K rows and 846 K matches, mostly key hashes, dictionary
+// probes and candidate rows written and read back; this takes 30 us, bound by
+// the lines of the two bitmaps (63 MB each).
+#define PRA_EMIT_MLP 4   // 1, 2, 4: 10,000-vertex graph 6.03, 5.91, 5.84 ms, 150x150 grid 41.6, 42.2, 42.1 ms
+__device__ __forceinline__ void pra_rank_emit_tile(const RankArgs& a, u64* status, u32 tile, u32 ntiles, u32 epoch,
+                                                   u32* flags)
+{
+    constexpr int SW = PRA_EMIT_BLOCK / 64;
+    __shared__ u32 lds[SW + 1];
+    __shared__ u64 s_excl;
+    const EmitArgs& em = a.emit;
+    const u64 i = (u64)tile * PRA_EMIT_BLOCK + threadIdx.x;
+    u32 digit[4] = {0, 0, 0, 0};
+    u32 i0 = 0, cnt = 0;
+    if (i < em.n) {
+        u64 x = em.dx[i];
+#pragma unroll
+        for (int c = 3; c > 0; c--)
+            if (c < em.kwo) pra_digit_split(x, a.D, em.inv, &x, &digit[c]);
+        digit[0] = (u32)x;
+        i0 = em.first[digit[0]];
+        cnt = em.first[digit[0] + 1] - i0;
+    }
+    u32 tot;
+    const u32 ex = block_exclusive_scan<u32, SW>(cnt, lds, &tot);
+    if (threadIdx.x < 64) {
+        u64 excl = 0;
+        if (threadIdx.x == 0)
+            __hip_atomic_store(status + tile, st_pack(epoch, tile == 0 ? PRA_ST_INC : PRA_ST_AGG, tot), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        if (tile != 0) {
+            excl = pra_lookback_wave(status, tile, epoch, flags, 1);
+            if (threadIdx.x == 0)
+                __hip_atomic_store(status + tile, st_pack(epoch, PRA_ST_INC, excl + tot), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (threadIdx.x == 0) {
+            s_excl = excl;
+            if (tile == ntiles - 1) {
+                const u64 total = excl + tot;
+                const u64 st = total > em.cap ? 1 : (long long)total > em.thresh ? 4 : 0;
+                a.ctl[0] = total;
+                a.ctl[1] = st;
+                if (!st && total) atomicAdd((unsigned long long*)em.joined, (unsigned long long)total);
+            }
+        }
+    }
+    __syncthreads();
+    if (s_excl + tot > em.cap) return;
+    // the digits that come from the outer row
+    u64 base = 0;
+    for (int c = 0; c < a.kw; c++) {
+        u32 d = 0;
+        if (em.side[c] == 0) {
+            const int q = em.col[c];
+            d = q == 0 ? digit[0] : q == 1 ? digit[1] : q == 2 ? digit[2] : digit[3];
+            if (em.conv[c] == 1) d = em.rank_of[d];        // leading digit -> rank
+            else if (em.conv[c] == 2) d = em.lead_of[d];   // rank -> leading digit
+        }
+        base = base * a.D + d;
+    }
+    // the row's matches, PRA_EMIT_MLP at a time with their loads in flight
+    // together (a match's chain is inner words, member word, fresh word, atomic)
+    const u64 p0 = s_excl + ex;
+    for (u32 j0 = 0; j0 < cnt; j0 += PRA_EMIT_MLP) {
+        u64 x[PRA_EMIT_MLP];
+        u32 mw[PRA_EMIT_MLP], fw[PRA_EMIT_MLP];
+#pragma unroll
+        for (int q = 0; q < PRA_EMIT_MLP; q++) {
+            x[q] = 0;
+            if (j0 + q < cnt)
+                for (int c = 0; c < a.kw; c++) {
+                    u32 d = 0;
+                    if (em.side[c] == 1) {
+                        const u64 e = em.words[(u64)(i0 + j0 + q) * em.ia + em.col[c]];
+                        d = c == 0 && a.by_bucket ? (u32)(e >> 32) : (u32)e - 1;
+                    }
+                    x[q] = x[q] * a.D + d;
+                }
+            x[q] += base;
+        }
+#pragma unroll
+        for (int q = 0; q < PRA_EMIT_MLP; q++) {
+            mw[q] = fw[q] = ~0u;
+            if (j0 + q < cnt) {
+                mw[q] = a.member[x[q] >> 5];
+                fw[q] = a.fresh[x[q] >> 5];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < PRA_EMIT_MLP; q++) {
+            if (j0 + q >= cnt) continue;
+            const u32 bit = 1u << (x[q] & 31);
+            const bool member = mw[q] & bit;
+            a.xs[p0 + j0 + q] = member ? ~0ULL : x[q];
+            if (!member && !(fw[q] & bit)) {
+                atomicOr(a.fresh + (x[q] >> 5), bit);
+                u32* d = a.dirty + (x[q] >> PRA_SB_BITS);
+                if (!*d) *d = 1;
+            }
+        }
     }
 }
 
@@ -2354,6 +2522,12 @@ __device__ __forceinline__ u32 pra_ticket(u32* ctr, u32 takers)
     return s_ticket;
 }
 
+__global__ __launch_bounds__(PRA_EMIT_BLOCK) void k_rank_emit(RankArgs a, u64* status, u32* ctr, u32 epoch, u32* flags)
+{
+    const u32 t = pra_ticket(ctr, gridDim.x);
+    pra_rank_emit_tile(a, status, t, gridDim.x, epoch, flags);
+}
+
 __global__ __launch_bounds__(PRA_SCAN_BLOCK) void k_rank_scan(RankArgs a, u64* status, u32* ctr, u32 epoch,
                                                               u32* flags)
 {
@@ -2378,6 +2552,18 @@ __global__ void k_rank_first(RankArgs a)
     if (a.ctl[1]) return;
     const u64 p = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     if (p < a.ctl[0]) pra_rank_first_one(a, p);
+}
+
+// The summary of an iteration of one ranked output, to the host as
+// pra_publish_words does it, by one thread: the words the host reads of it.
+__device__ __forceinline__ void pra_publish_ranked(const RankArgs& a, u64 new_rows)
+{
+    a.host[0] = new_rows;
+    a.host[4] = a.ctl[0];
+    a.host[5] = a.ctl[1];
+    a.host[a.host_words] = *a.err;
+    __threadfence_system();
+    __hip_atomic_store(a.host - 1, a.host_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Tile `tile` of the placement (PRA_TILE candidates by PRA_PLACE_BLOCK
@@ -2406,18 +2592,28 @@ __device__ __forceinline__ void pra_rank_place_tile(const RankArgs& a, u64* stat
 #pragma unroll
     for (int k = 0; k < IT; k++)
         kept[k] = pos[k] != ~0u && a.first[pos[k]] == (u32)(base + (u64)k * 64 + lane);
-    // what the kept rows need, loaded before the barriers (rows of up to PW words)
-    constexpr int PW = 2;
-    u64 x[IT], row[IT][PW];
+    // the kept rows' values, by their digits, and buckets (of the leading digit,
+    // or, with more join columns, the candidate's), loaded before the barriers
+    u64 x[IT], row[IT][4];
 #pragma unroll
     for (int k = 0; k < IT; k++) {
         const u64 p = base + (u64)k * 64 + lane;
-        dg[k] = kept[k] && nb > 1 ? a.dest[p] : 0u;
         x[k] = kept[k] ? a.xs[p] : 0;
-        if (kept[k] && a.cw <= PW)
+    }
 #pragma unroll
-            for (int c = 0; c < PW; c++)
-                if (c < a.cw) row[k][c] = a.cand[p * a.cw + c];
+    for (int k = 0; k < IT; k++) {
+        dg[k] = 0;
+        if (!kept[k]) continue;
+        u64 q = x[k];
+#pragma unroll
+        for (int c = 3; c > 0; c--)
+            if (c < a.kw) {
+                u32 d;
+                pra_digit_split(q, a.D, a.inv, &q, &d);
+                row[k][c] = a.vals[d];
+            }
+        row[k][0] = a.lead_vals[q];
+        if (nb > 1) dg[k] = a.by_bucket ? (u32)a.bucket[q] : a.dest[base + (u64)k * 64 + lane];
     }
     for (u32 i = lane; i < nb; i += 64) wh[wave][i] = 0;
     // (a wave counts in its own row of wh, in lane order within each item)
@@ -2461,18 +2657,14 @@ __device__ __forceinline__ void pra_rank_place_tile(const RankArgs& a, u64* stat
 #pragma unroll
     for (int k = 0; k < IT; k++) {
         if (!kept[k]) continue;
-        const u64 p = base + (u64)k * 64 + lane;
         const u32 d = dg[k];
         const u64 seq = a.seq[d] + s_base[d] + wh[wave][d] + lc[k];
         u64* dst = a.newt + (u64)pos[k] * a.wn;
-        if (a.cw <= PW) {
 #pragma unroll
-            for (int c = 0; c < PW; c++)
-                if (c < a.cw) dst[c] = row[k][c];
-        } else {
-            pra_copy_row(dst, a.cand + p * a.cw, a.cw);
-        }
-        dst[a.cw] = ((u64)a.tag << 46) | ((u64)d << 28) | seq;
+        for (int c = 0; c < 4; c++)
+            if (c < a.kw) dst[c] = row[k][c];
+        dst[a.kw] = ((u64)a.tag << 46) | ((u64)d << 28) | seq;
+        if (a.nx) a.nx[pos[k]] = x[k];
         atomicOr(a.member + (x[k] >> 5), 1u << (x[k] & 31));
         // back to the state between iterations: the word's fresh bits are all
         // of this iteration, and no other arrival equals ~0
@@ -2490,6 +2682,7 @@ __device__ __forceinline__ void pra_rank_place_tile(const RankArgs& a, u64* stat
     if (d0 == 0) {
         if (a.bnd) a.bnd[nb] = tot;
         a.stat[0] = tot;
+        if (a.host) pra_publish_ranked(a, tot);
     }
 }
 
@@ -2497,20 +2690,33 @@ __global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place(RankArgs a, u64*
                                                                 u32* flags)
 {
     // only the blocks that have candidates (and the first) take a ticket
-    const u64 n = a.ctl[1] ? 0 : a.ctl[0];
+    if (a.ctl[1]) {
+        if (a.host && blockIdx.x == 0 && threadIdx.x == 0) pra_publish_ranked(a, 0);
+        return;
+    }
+    const u64 n = a.ctl[0];
     const u32 tiles = n ? (u32)((n + PRA_TILE - 1) / PRA_TILE) : 1;
     if (blockIdx.x >= tiles) return;
     const u32 t = pra_ticket(ctr, tiles);
-    if (a.ctl[1]) return;
     pra_rank_place_tile(a, status, t, epoch, flags);
 }
 
 // Several outputs in one launch each: `jobs` (device memory) holds njobs
-// RankArgs, then three tables of njobs + 1 first blocks (claim and first, scan,
-// place).
+// RankArgs, then five tables of njobs + 1 first blocks, one a step (outputs
+// that emit have no claim blocks, the others no emission tiles).
+__global__ __launch_bounds__(PRA_EMIT_BLOCK) void k_rank_emit_many(const RankArgs* jobs, int njobs, u64* status,
+                                                                   u32* ctr, u32 epoch, u32* flags)
+{
+    const u32* base = (const u32*)(jobs + njobs) + PRA_RANK_EMIT * (njobs + 1);
+    const u32 t = pra_ticket(ctr, gridDim.x);
+    const int k = pra_job_of(base, njobs, t);
+    const RankArgs a = jobs[k];
+    pra_rank_emit_tile(a, status + base[k], t - base[k], base[k + 1] - base[k], epoch, flags);
+}
+
 __global__ void k_rank_claim_many(const RankArgs* jobs, int njobs)
 {
-    const u32* base = (const u32*)(jobs + njobs);
+    const u32* base = (const u32*)(jobs + njobs) + PRA_RANK_CLAIM * (njobs + 1);
     const int k = pra_job_of(base, njobs, blockIdx.x);
     const RankArgs* jp = jobs + k;
     const u64 p = (u64)(blockIdx.x - base[k]) * blockDim.x + threadIdx.x;
@@ -2521,7 +2727,7 @@ __global__ void k_rank_claim_many(const RankArgs* jobs, int njobs)
 __global__ __launch_bounds__(PRA_SCAN_BLOCK) void k_rank_scan_many(const RankArgs* jobs, int njobs, u64* status,
                                                                    u32* ctr, u32 epoch, u32* flags)
 {
-    const u32* base = (const u32*)(jobs + njobs) + njobs + 1;
+    const u32* base = (const u32*)(jobs + njobs) + PRA_RANK_SCAN * (njobs + 1);
     const u32 t = pra_ticket(ctr, gridDim.x);
     const int k = pra_job_of(base, njobs, t);
     const RankArgs* jp = jobs + k;
@@ -2531,7 +2737,7 @@ __global__ __launch_bounds__(PRA_SCAN_BLOCK) void k_rank_scan_many(const RankArg
 
 __global__ void k_rank_first_many(const RankArgs* jobs, int njobs)
 {
-    const u32* base = (const u32*)(jobs + njobs);
+    const u32* base = (const u32*)(jobs + njobs) + PRA_RANK_FIRST * (njobs + 1);
     const int k = pra_job_of(base, njobs, blockIdx.x);
     const RankArgs* jp = jobs + k;
     const u64 p = (u64)(blockIdx.x - base[k]) * blockDim.x + threadIdx.x;
@@ -2542,7 +2748,7 @@ __global__ void k_rank_first_many(const RankArgs* jobs, int njobs)
 __global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place_many(const RankArgs* jobs, int njobs, u64* status,
                                                                      u32* ctr, u32 epoch, u32* flags)
 {
-    const u32* base = (const u32*)(jobs + njobs) + 2 * (njobs + 1);
+    const u32* base = (const u32*)(jobs + njobs) + PRA_RANK_PLACE * (njobs + 1);
     const u32 t = pra_ticket(ctr, gridDim.x);
     const int k = pra_job_of(base, njobs, t);
     const RankArgs a = jobs[k];
@@ -3702,14 +3908,29 @@ void pra_launch_dense_build(hipStream_t st, const u64* rows, u64 n, int w, int k
     }
 }
 
-void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of)
+void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of, u32* lead_of,
+                                 u64 nb, unsigned char* bucket)
 {
-    if (n) hipLaunchKernelGGL(k_dict_bucket_rank, dim3(grid_for(n)), dim3(PRA_BLOCK), 0, st, vals, n, tab, cap, rank_of);
+    if (n)
+        hipLaunchKernelGGL(k_dict_bucket_rank, dim3(grid_for(n)), dim3(PRA_BLOCK), 0, st, vals, n, tab, cap, rank_of,
+                           lead_of, nb, bucket);
+}
+
+void pra_launch_rank_rows(hipStream_t st, const u64* rows, u64 n, int w, int a, const u64* dict, u64 dict_cap, u64 D,
+                          int by_bucket, u64* words, u32* first, u64* miss)
+{
+    if (n)
+        hipLaunchKernelGGL(k_rank_rows, dim3(grid_for(n)), dim3(PRA_BLOCK), 0, st, rows, n, w, a, dict, dict_cap, D,
+                           by_bucket, words, first, miss);
 }
 
 void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* status, u32* ctr, u32 epoch, u32* flags)
 {
     switch (step) {
+    case PRA_RANK_EMIT:
+        hipLaunchKernelGGL(k_rank_emit, dim3((unsigned)((a.emit.n + PRA_EMIT_BLOCK - 1) / PRA_EMIT_BLOCK)),
+                           dim3(PRA_EMIT_BLOCK), 0, st, a, status, ctr, epoch, flags);
+        break;
     case PRA_RANK_CLAIM: hipLaunchKernelGGL(k_rank_claim, dim3(grid_for(cap)), dim3(PRA_BLOCK), 0, st, a); break;
     case PRA_RANK_SCAN:
         hipLaunchKernelGGL(k_rank_scan, dim3(a.chunks), dim3(PRA_SCAN_BLOCK), 0, st, a, status, ctr, epoch, flags);
@@ -3724,7 +3945,12 @@ void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* 
 void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,
                           u32 epoch, u32* flags)
 {
+    if (!blocks) return;
     switch (step) {
+    case PRA_RANK_EMIT:
+        hipLaunchKernelGGL(k_rank_emit_many, dim3(blocks), dim3(PRA_EMIT_BLOCK), 0, st, jobs, njobs, status, ctr, epoch,
+                           flags);
+        break;
     case PRA_RANK_CLAIM: hipLaunchKernelGGL(k_rank_claim_many, dim3(blocks), dim3(PRA_BLOCK), 0, st, jobs, njobs); break;
     case PRA_RANK_SCAN:
         hipLaunchKernelGGL(k_rank_scan_many, dim3(blocks), dim3(PRA_SCAN_BLOCK), 0, st, jobs, njobs, status, ctr, epoch,

@@ -211,6 +211,24 @@ struct DenseArgs {
 #define PRA_SCAN_CHUNKS 256
 #define PRA_SCAN_CHUNK_MAX 4096
 #define PRA_PLACE_BLOCK 1024
+#define PRA_EMIT_BLOCK 1024   // outer rows of an emission tile, one a thread
+// A ranked output's own emission (k_rank_emit): its one rule, a join on one
+// column of a delta with a static inner relation, in digits.  Output column c
+// comes from the outer row (side 0) or the inner row (side 1), its column
+// col[c]; conv: 1 = the outer's leading digit to a rank, 2 = a rank to a
+// leading digit, 0 = as it is.
+struct EmitArgs {
+    const u64* dx;        // per outer row: its rank index (kwo digits)
+    u64 n, cap;
+    long long thresh;
+    u64* joined;
+    const u32* first;     // per leading digit: its first inner row
+    const u64* words;     // per inner row: the dictionary words of its ia columns
+    const u32 *rank_of, *lead_of;
+    double inv;           // 1 / D
+    int kwo, ia;
+    signed char side[4], col[4], conv[4];
+};
 struct RankArgs {
     const u64* cand;
     u64* ctl;
@@ -224,21 +242,32 @@ struct RankArgs {
     u32* sbpre;           // per superblock: fresh bits before it
     unsigned short* linep;   // per line of a dirty superblock: its fresh bits before the line
     u32* first;           // per new key: earliest arrival (all ones between iterations)
+    const u64 *vals, *lead_vals;   // value of each rank, and of each leading digit
+    const unsigned char* bucket;   // by_bucket: bucket of each leading digit
+    double inv;           // 1 / D
     u64* newt;
+    u64* nx;              // the new rows' rank indexes (null: not wanted)
     u64* bnd;             // bucket bounds of the new rows (null: not wanted)
     u64* stat;
+    u64* host;            // the summary goes to the host from the placement (null: it does not)
+    u64 host_seq;
+    const u32* err;       // the error flags that go with it, as word host_words
+    u32 host_words;
     const u64* seq;       // per-bucket seq counters, and their values after this iteration
     u64* seq_next;
     u32 sbs, chunks, nb, tag;   // superblocks, and the chunks they are scanned in
-    int cw, kw, wn, by_bucket;
+    int kw, wn, by_bucket;   // the candidates' rows are keys of kw words
+    EmitArgs emit;
 };
-enum { PRA_RANK_CLAIM, PRA_RANK_SCAN, PRA_RANK_FIRST, PRA_RANK_PLACE };
+// an output either emits (its own emission and claims) or claims (candidates
+// of the general expansions)
+enum { PRA_RANK_EMIT, PRA_RANK_CLAIM, PRA_RANK_SCAN, PRA_RANK_FIRST, PRA_RANK_PLACE, PRA_RANK_STEPS };
 // one step of one output; status: look-back words of its tiles (one a tile for
-// the scan, PRA_RADIX for the placement)
+// the emission and the scan, PRA_RADIX for the placement)
 void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* status, u32* ctr, u32 epoch,
                      u32* flags);
-// the step of several outputs: jobs (device) = njobs RankArgs, then three
-// tables of njobs + 1 first blocks (claim / first, scan, place)
+// the step of several outputs: jobs (device) = njobs RankArgs, then
+// PRA_RANK_STEPS tables of njobs + 1 first blocks
 void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,
                           u32 epoch, u32* flags);
 
@@ -393,8 +422,13 @@ void pra_launch_view_keep(hipStream_t st, const u64* rows, u64 n, int w, int ja,
 void pra_launch_view_compact(hipStream_t st, const u64* rows, u64 n, int w, const u32* keep, const u32* pos, u64* out);
 void pra_launch_dict_insert(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* flags);
 // bucket-major ranks (vals: the n dictionary values by (bucket, value)) into
-// the dictionary's slots
-void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of);
+// the dictionary's slots, with the maps to and from ranks and their buckets
+void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of, u32* lead_of,
+                                 u64 nb, unsigned char* bucket);
+// the dictionary words of rows' first a columns and the first row of every
+// leading digit (k_rank_rows)
+void pra_launch_rank_rows(hipStream_t st, const u64* rows, u64 n, int w, int a, const u64* dict, u64 dict_cap, u64 D,
+                          int by_bucket, u64* words, u32* first, u64* miss);
 void pra_launch_gather_rows(hipStream_t st, const u64* in, const u32* idx, u64 n, int w, u64* out);
 void pra_launch_key_bounds(hipStream_t st, const u64* keys, u64 n, u64 bmul, int ls, u64 nb, u64* bnd);
 // Keyed row sort of more rows than one block holds: word 0 of every row's key
