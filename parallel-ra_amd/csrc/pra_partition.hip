@@ -9,9 +9,7 @@
 //   k_part_hist     per tile, the rows of each bucket          -> H[b][tile]
 //   k_part_scan     per bucket, exclusive prefix over tiles    -> H, T[b]
 //   k_part_scatter  per tile, bucket starts (scan of T) + H, then every row to
-//                   its place: rows are taken in input order, 256 at a time,
-//                   ranked inside each wave by matching bucket ballots and
-//                   across the block's waves by their per-bucket counts.
+//                   its place, through LDS in bucket order.
 // Scratch: nb * tiles + nb u32 words (H then T); every word a call reads was
 // written earlier in the same call, so the scratch carries no state between
 // calls and needs no clearing.
@@ -28,10 +26,11 @@ namespace {
 constexpr int kPartBlock = 256;
 constexpr int kPartRounds = PRA_PART_TILE / kPartBlock;
 constexpr int kScanBlock = 1024;
+constexpr u32 kStreamRun = 1024;   // bytes
 
-__device__ inline u32 part_bucket(const u64* __restrict__ rows, u64 i, int w, int jcc, u32 nb)
+__device__ inline u32 part_bucket(const u64* __restrict__ row, int jcc, u32 nb)
 {
-    return pra_bucket(pra_fnv(rows + i * (u64)w, jcc), nb);
+    return pra_bucket(pra_fnv(row, jcc), nb);
 }
 
 __global__ __launch_bounds__(kPartBlock) void k_part_hist(const u64* __restrict__ rows, u64 n, int w, int jcc,
@@ -42,10 +41,17 @@ __global__ __launch_bounds__(kPartBlock) void k_part_hist(const u64* __restrict_
     h[tid] = 0;
     __syncthreads();
     const u64 base = (u64)tile * PRA_PART_TILE;
+    u32 b[kPartRounds];
 #pragma unroll
     for (int r = 0; r < kPartRounds; r++) {
         const u64 i = base + (u64)r * kPartBlock + tid;
-        if (i < n) atomicAdd(&h[part_bucket(rows, i, w, jcc, nb)], 1u);
+        b[r] = i < n ? part_bucket(rows + i * (u64)w, jcc, nb) : ~0u;
+    }
+#pragma unroll
+    for (int r = 0; r < kPartRounds; r++) {
+        // one LDS add per bucket and wave: a wave's lanes fall into few buckets
+        const u64 peers = pra_match<PRA_RADIX_BITS>(b[r], __ballot(b[r] != ~0u));
+        if (b[r] != ~0u && __lane_id() == (u32)(__ffsll((long long)peers) - 1)) atomicAdd(&h[b[r]], (u32)__popcll(peers));
     }
     __syncthreads();
     if (tid < nb) H[(u64)tid * ntiles + tile] = h[tid];
@@ -78,62 +84,126 @@ __global__ __launch_bounds__(kScanBlock) void k_part_scan(u32* __restrict__ H, u
     if (tid == kScanBlock - 1) T[blockIdx.x] = part[tid];
 }
 
-__global__ __launch_bounds__(kPartBlock) void k_part_scatter(const u64* __restrict__ rows, u64 n, int w, int jcc,
+// A tile's rows to their places, SUB rows at a time through LDS: the rows come
+// in as consecutive words, are ranked in input order (inside each wave by
+// matching bucket ballots, then over the waves), and go out in bucket order as
+// consecutive words again, so both sides move whole cache lines where each
+// lane's own row would touch several.  Tiles run from the last one back: the
+// rows the histogram read last are still in the last-level cache.
+// W: the row width, 0 = any (w).  NT: non-temporal stores.
+// 24 M rows of 3 words into 8 buckets: 488 -> 377 us; 12 M rows of 6 words into
+// 64: 738 -> 463; 30 M of 2 into 200: 801 -> 561, into 3: 361 -> 346.  With
+// the histogram's read these move 24 bytes a word at 4.6 TB/s of the card's
+// copy rate, so 375 us is the first one's bound.
+// NT against plain stores: 377 / 402 us (8 buckets, runs of 1.5 KB), 483 / 463
+// (64, 384 bytes), 854 / 561 (200, 41 bytes): kStreamRun lies in between.
+template <int W, int SUB, bool NT>
+__global__ __launch_bounds__(kPartBlock) void k_part_scatter(const u64* __restrict__ rows, u64 n, int w_, int jcc,
                                                               u32 nb, const u32* __restrict__ H,
                                                               const u32* __restrict__ T, u32 ntiles,
                                                               u64* __restrict__ out, u64* __restrict__ bounds)
 {
-    __shared__ u32 start[PRA_RADIX];
-    __shared__ u32 base[PRA_RADIX];
+    constexpr int IT = SUB / kPartBlock;
+    extern __shared__ u64 stage[];   // SUB rows
+    __shared__ u32 next[PRA_RADIX];        // where the bucket's next row goes
     __shared__ u32 wc[PRA_WAVES][PRA_RADIX];
-    const u32 tid = threadIdx.x, tile = blockIdx.x;
+    __shared__ u32 shift[PRA_RADIX];       // output row of a bucket's rows minus their place in the sub-tile
+    __shared__ unsigned short perm[SUB];   // row of each place of the sub-tile
+    __shared__ unsigned char pb[SUB];      // its bucket
+    __shared__ u32 wsum[PRA_WAVES];
+    const int w = W ? W : w_;
+    const u32 tid = threadIdx.x, tile = gridDim.x - 1 - blockIdx.x;
     const u32 wave = tid / 64, lane = __lane_id();
-    // bucket starts: exclusive scan of the bucket totals
-    const u32 tot = tid < nb ? T[tid] : 0;
-    start[tid] = tot;
-    __syncthreads();
-    for (u32 d = 1; d < PRA_RADIX; d <<= 1) {
-        const u32 v = tid >= d ? start[tid - d] : 0;
+    // exclusive scan over the buckets, a thread each
+    auto scan = [&](u32 v) {
+        u32 x = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const u32 y = __shfl_up(x, d, 64);
+            if (lane >= (u32)d) x += y;
+        }
+        if (lane == 63) wsum[wave] = x;
         __syncthreads();
-        start[tid] += v;
+        for (u32 q = 0; q < wave; q++) x += wsum[q];
         __syncthreads();
-    }
-    const u32 st = start[tid] - tot;
+        return x - v;
+    };
+    const u32 st = scan(tid < nb ? T[tid] : 0);
     if (tile == 0) {
         if (tid < nb) bounds[tid] = st;
         if (tid == 0) bounds[nb] = n;
     }
-    base[tid] = tid < nb ? st + H[(u64)tid * ntiles + tile] : 0;
+    next[tid] = tid < nb ? st + H[(u64)tid * ntiles + tile] : 0;
+    const u64 t0 = (u64)tile * PRA_PART_TILE;
+    const u32 trows = (u32)min((u64)PRA_PART_TILE, n - t0);
+    for (u32 s0 = 0; s0 < trows; s0 += SUB) {
+        const u32 m = min((u32)SUB, trows - s0);
+        const u64* src = rows + (t0 + s0) * (u64)w;
+        for (u32 i = tid; i < m * w; i += kPartBlock) stage[i] = src[i];
 #pragma unroll
-    for (int q = 0; q < PRA_WAVES; q++) wc[q][tid] = 0;
-    __syncthreads();
-    const u64 tbase = (u64)tile * PRA_PART_TILE;
-    for (int r = 0; r < kPartRounds; r++) {
-        const u64 i = tbase + (u64)r * kPartBlock + tid;
-        const bool valid = i < n;
-        const u32 b = valid ? part_bucket(rows, i, w, jcc, nb) : 0;
-        const u64 active = __ballot(valid);
-        const u64 peers = pra_match<PRA_RADIX_BITS>(b, active);
-        const u32 rank = (u32)__popcll(peers & pra_lanemask_lt());
-        if (valid && lane == (u32)(__ffsll((long long)peers) - 1)) wc[wave][b] = (u32)__popcll(peers);
+        for (int q = 0; q < PRA_WAVES; q++) wc[q][tid] = 0;
         __syncthreads();
-        if (valid) {
-            u32 off = base[b] + rank;
-            for (u32 q = 0; q < wave; q++) off += wc[q][b];
-            pra_copy_row(out + (u64)off * w, rows + i * (u64)w, w);
+        // rows in input order: wave v holds rows [v * 64 * IT, (v + 1) * 64 * IT)
+        u32 b[IT], rank[IT];
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const u32 i = wave * 64 * IT + k * 64 + lane;
+            const bool valid = i < m;
+            b[k] = valid ? part_bucket(stage + (size_t)i * w, jcc, nb) : 0;
+            const u64 peers = pra_match<PRA_RADIX_BITS>(b[k], __ballot(valid));
+            if (valid) {
+                const u32 before = wc[wave][b[k]];
+                rank[k] = before + (u32)__popcll(peers & pra_lanemask_lt());
+                if ((peers >> lane) == 1ULL) wc[wave][b[k]] = before + (u32)__popcll(peers);
+            }
         }
         __syncthreads();
-        if (tid < nb) {
-            u32 add = 0;
+        u32 tot = 0;
 #pragma unroll
-            for (int q = 0; q < PRA_WAVES; q++) {
-                add += wc[q][tid];
-                wc[q][tid] = 0;
+        for (int q = 0; q < PRA_WAVES; q++) {
+            const u32 v = wc[q][tid];
+            wc[q][tid] = tot;
+            tot += v;
+        }
+        const u32 start = scan(tot);
+        shift[tid] = next[tid] - start;
+        next[tid] += tot;
+#pragma unroll
+        for (int q = 0; q < PRA_WAVES; q++) wc[q][tid] += start;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const u32 i = wave * 64 * IT + k * 64 + lane;
+            if (i < m) {
+                const u32 p = wc[wave][b[k]] + rank[k];
+                perm[p] = (unsigned short)i;
+                pb[p] = (unsigned char)b[k];
             }
-            base[tid] += add;
+        }
+        __syncthreads();
+        for (u32 i = tid; i < m * w; i += kPartBlock) {
+            const u32 p = i / w, c = i - p * w;
+            u64* dst = &out[(u64)(shift[pb[p]] + p) * w + c];
+            const u64 v = stage[(u32)perm[p] * w + c];
+            if (NT)
+                __builtin_nontemporal_store(v, dst);
+            else
+                *dst = v;
         }
         __syncthreads();
     }
+}
+
+template <int W, int SUB>
+void launch_scatter(hipStream_t st, const u64* rows, u64 n, int w, int jcc, u32 nb, const u32* H, const u32* T, u32 ntiles,
+                    u64* out, u64* bounds)
+{
+    // a sub-tile's run of one bucket, at least kStreamRun bytes on average:
+    // the runs are mostly whole lines, which need not stay in the caches
+    const bool stream = (u64)SUB * w * 8 >= (u64)kStreamRun * nb;
+    auto k = stream ? k_part_scatter<W, SUB, true> : k_part_scatter<W, SUB, false>;
+    hipLaunchKernelGGL(k, dim3(ntiles), dim3(kPartBlock), (size_t)SUB * w * 8, st, rows, n, w, jcc, nb, H, T, ntiles, out,
+                       bounds);
 }
 
 __global__ void k_part_empty(u64* bounds, u32 nb)
@@ -168,8 +238,19 @@ void pra_launch_partition(hipStream_t st, const u64* rows, u64 n, int w, int jcc
     u32* T = scratch_words + (size_t)nb * ntiles;
     hipLaunchKernelGGL(k_part_hist, dim3(ntiles), dim3(kPartBlock), 0, st, rows, n, w, jcc, nb, H, ntiles);
     hipLaunchKernelGGL(k_part_scan, dim3(nb), dim3(kScanBlock), 0, st, H, ntiles, T);
-    hipLaunchKernelGGL(k_part_scatter, dim3(ntiles), dim3(kPartBlock), 0, st, rows, n, w, jcc, nb, H, T, ntiles, out,
-                       bounds);
+    // rows of a sub-tile: 512 (256, 1,024: 5 to 10 % slower at 2, 3 and 6
+    // words a row), fewer where they would not leave room for two blocks a CU
+    switch (w) {
+    case 1: launch_scatter<1, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    case 2: launch_scatter<2, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    case 3: launch_scatter<3, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    case 4: launch_scatter<4, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    default:
+        if (w <= 8)
+            launch_scatter<0, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds);
+        else
+            launch_scatter<0, 256>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds);
+    }
 }
 
 // Once per device, with that device current: the device address of this
