@@ -435,6 +435,7 @@ struct pra_rel {
     DBuf bnd[2];
     bool bnd_valid[2] = {false, false};
     DBuf next_bnd;   // the new rows' bounds, until they become the delta
+    DBuf merged;     // the other buffer of a full version kept sorted by merges
     // set while an SCC runs: the relation is produced by one of its rules
     // (changes every iteration), and its full version is read by one of them
     // (so it is kept sorted by merging each delta into it)
@@ -1827,40 +1828,88 @@ static void append_rows(pra_ctx* c, pra_rel* R, int v, const u64* src, u64 n, st
     R->touched(v);
 }
 
-// full <- full u delta keeping full sorted: both are sorted by (bucket,
-// columns) and disjoint, so each delta row's place is a binary search inside
-// its bucket and every row moves once (falls back to an append when either
-// side is unsorted)
-static void merge_into_full(pra_ctx* c, pra_rel* R)
-{
-    Rows& D = R->ver[PRA_DELTA];
-    Rows& F = R->ver[PRA_FULL];
-    if (D.n == 0) return;
-    if (F.n == 0 || !F.sorted || !D.sorted) {
-        bool sorted = F.n == 0 && D.sorted;
-        append_rows(c, R, PRA_FULL, D.d(), D.n);
-        F.sorted = sorted;
-        return;
-    }
-    const u64* fb = bucket_bounds(c, R, PRA_FULL);
-    const u64* db = bucket_bounds(c, R, PRA_DELTA);
-    u64 n = F.n + D.n;
-    c->tmp64a.reserve(D.n * 8, c->st);
-    c->sort_tmp.reserve(n * R->w * 8, c->st);
+// full <- full u delta keeping full sorted, for several relations: both sides
+// are sorted by (bucket, columns) and disjoint, so each delta row's place is a
+// search inside its bucket and every row moves once, into the relation's other
+// full buffer.  A relation whose sides are not both sorted is appended to; one
+// without room for a second buffer is merged by itself, through the scratch
+// that all share.
+struct Merges {
+    pra_ctx* c;
+    MergeBatch b;
+    std::vector<pra_rel*> rels;
+    u64 rank_words = 0;
+    double bytes = 0;
+    explicit Merges(pra_ctx* c_) : c(c_) { memset(&b, 0, sizeof(b)); }
+
+    void add(pra_rel* R)
     {
-        Prof p(c, K_MERGE, 16.0 * R->w * n);
-        // the merged bucket s holds full's and delta's rows of bucket s: the
-        // merge adds delta's bounds to full's
-        pra_launch_merge(c->st, F.d(), F.n, fb, D.d(), D.n, db, (u64)c->nb, R->w, c->tmp64a.as<u64>(),
-                         c->sort_tmp.as<u64>(), R->bnd[PRA_FULL].as<u64>());
-        check_launch("merge");
+        Rows &D = R->ver[PRA_DELTA], &F = R->ver[PRA_FULL];
+        if (D.n == 0) return;
+        if (F.n == 0 || !F.sorted || !D.sorted) {
+            bool sorted = F.n == 0 && D.sorted;
+            append_rows(c, R, PRA_FULL, D.d(), D.n);
+            F.sorted = sorted;
+            return;
+        }
+        bool own = true;
+        try {
+            R->merged.reserve((F.n + D.n) * R->w * 8, c->st);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+            R->merged.release();
+            own = false;
+            run();
+        }
+        MergeJob& m = b.job[b.njobs];
+        m.F = F.d();
+        m.nf = F.n;
+        m.fbnd = bucket_bounds(c, R, PRA_FULL);
+        m.add_to = R->bnd[PRA_FULL].as<u64>();
+        m.D = D.d();
+        m.nd = D.n;
+        m.dbnd = bucket_bounds(c, R, PRA_DELTA);
+        m.w = R->w;
+        m.rank = (u64*)rank_words;   // its offset until the scratch is sized
+        rank_words += D.n;
+        if (!own) c->sort_tmp.reserve((F.n + D.n) * R->w * 8, c->st);
+        m.out = (own ? R->merged : c->sort_tmp).as<u64>();
+        b.rank_base[b.njobs + 1] = b.rank_base[b.njobs] + (u32)((D.n + PRA_BLOCK - 1) / PRA_BLOCK);
+        b.scatter_base[b.njobs + 1] = b.scatter_base[b.njobs] + (u32)((F.n + D.n + PRA_BLOCK - 1) / PRA_BLOCK);
+        b.njobs++;
+        bytes += 16.0 * R->w * (F.n + D.n);
+        rels.push_back(R);
+        if (!own || b.njobs == PRA_MERGE_JOBS) run(own ? nullptr : &c->sort_tmp);
     }
-    F.buf.swap(c->sort_tmp);
-    F.n = n;
-    F.sorted = true;
-    R->touched(PRA_FULL);
-    R->bnd_valid[PRA_FULL] = true;
-}
+
+    // the merges so far; shared: the one job's output, in place of the
+    // relation's own second buffer
+    void run(DBuf* shared = nullptr)
+    {
+        if (!b.njobs) return;
+        c->tmp64a.reserve(rank_words * 8, c->st);
+        for (int k = 0; k < b.njobs; k++) b.job[k].rank = c->tmp64a.as<u64>() + (size_t)b.job[k].rank;
+        b.nb = (u64)c->nb;
+        {
+            Prof p(c, K_MERGE, bytes);
+            pra_launch_merge(c->st, b);
+            check_launch("merge");
+        }
+        for (pra_rel* R : rels) {
+            Rows& F = R->ver[PRA_FULL];
+            F.buf.swap(shared ? *shared : R->merged);
+            F.n += R->ver[PRA_DELTA].n;
+            F.sorted = true;
+            // the merged bucket s holds full's and delta's rows of bucket s
+            R->touched(PRA_FULL);
+            R->bnd_valid[PRA_FULL] = true;
+        }
+        rels.clear();
+        memset(&b, 0, sizeof(b));
+        rank_words = 0;
+        bytes = 0;
+    }
+};
 
 // The SCCs of one lock-step iteration seen as one: the rules of every member
 // in member order, then rule order, and every member's relations.  Members
@@ -2406,7 +2455,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             } else {
                 j.op = ra.type == RA_COPY_FILTER ? ra.op : PRA_F_TRUE;
             }
-            csb.tile_base[csb.njobs + 1] = csb.tile_base[csb.njobs] + pra_tiles(n);
+            csb.tile_base[csb.njobs + 1] =
+                csb.tile_base[csb.njobs] + (u32)((n + PRA_COUNT_SCAN_TILE - 1) / PRA_COUNT_SCAN_TILE);
             cs_bytes += 8.0 * n * ra.outer->w + (join ? 24.0 : 8.0) * n;
             if (++csb.njobs == PRA_CS_JOBS) flush_count_scans();
         }
@@ -3346,14 +3396,16 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     //    first: the newt sort writes the next delta's bucket bounds.
     {
         std::vector<CopyJob> appends;
+        Merges merges(c);
         for (size_t i = 0; i < S->rels.size(); i++) {
             pra_rel* R = S->rels[i];
             Rows& D = R->ver[PRA_DELTA];
             if (R->merge_full)
-                merge_into_full(c, R);
+                merges.add(R);
             else if (!early[i])
                 append_rows(c, R, PRA_FULL, D.d(), D.n, &appends);
         }
+        merges.run();
         copy_ranges(c, JOB_APPEND, appends);
         for (pra_rel* R : S->rels) {
             R->ver[PRA_DELTA].n = 0;
@@ -3577,6 +3629,7 @@ static void scc_end(pra_scc* S, bool check = true)
     if (!S->running) throw PraError(PRA_E_STATE, "SCC not started");
     for (pra_rel* R : S->rels) {
         delta_to_full(c, R);
+        R->merged.release();
         R->scc_changing = R->merge_full = R->full_read = false;
     }
     if (check) sync_check(c);
@@ -3889,7 +3942,7 @@ int pra_ctx_group_status(pra_ctx* ctx, int group, int* done, uint64_t* iteration
         for (pra_rel* R : ctx->rels) {
             if (R->group != group) continue;
             for (auto& v : R->ver) b += v.buf.cap;
-            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->dx, &R->nx,
+            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->merged, &R->dx, &R->nx,
                                   &R->rk_words[0], &R->rk_words[1], &R->rk_first[0], &R->rk_first[1], &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
                                   &R->bin_keys, &R->bin_idx, &R->bin_cur, &R->bnd[0], &R->bnd[1]})
                 b += d->cap;

@@ -1303,88 +1303,115 @@ __device__ inline int pra_row_cmp(const u64* a, const u64* b, int n)
     return 0;
 }
 
+// First row of the sorted rows [a, z) whose first n columns are >= key (upper:
+// > key).  Three probes a step, their loads in flight together, so a search
+// takes half the dependent loads of a binary one; rows that differ from the
+// key in column 0 need no more than that.  With one row a thread and runs
+// found by four parallel compares, the points-to analysis' counts took 21 us a
+// launch instead of 30.
+__device__ inline u64 pra_row_bound(const u64* rows, int w, const u64* key, int n, u64 a, u64 z, bool upper)
+{
+    const u64 k0 = key[0];
+    auto below = [&](u64 v, u64 m) {
+        if (v != k0) return v < k0;
+        const int c = n == 1 ? 0 : pra_row_cmp(rows + m * w + 1, key + 1, n - 1);
+        return upper ? c <= 0 : c < 0;
+    };
+    while (z - a >= 4) {
+        const u64 q = (z - a) / 4, m1 = a + q, m2 = m1 + q, m3 = m2 + q;
+        const u64 v1 = rows[m1 * w], v2 = rows[m2 * w], v3 = rows[m3 * w];
+        if (below(v2, m2)) {
+            if (below(v3, m3)) {
+                a = m3 + 1;
+            } else {
+                a = m2 + 1;
+                z = m3;
+            }
+        } else if (below(v1, m1)) {
+            a = m1 + 1;
+            z = m2;
+        } else {
+            z = m1;
+        }
+    }
+    while (a < z) {
+        const u64 m = (a + z) >> 1;
+        if (below(rows[m * w], m)) a = m + 1; else z = m;
+    }
+    return a;
+}
+
 // Run of inner rows matching an outer key, in an inner version kept sorted by
-// (bucket, columns): one run inside the key's bucket, found by a binary
-// search and a gallop (used for inner relations that change every iteration,
+// (bucket, columns): one run inside the key's bucket, found by two searches
+// (used for inner relations that change every iteration,
 // where a hash index would be rebuilt each time).  Returns its length.
 __device__ inline u64 pra_sorted_run(const u64* key, int jcc, const u64* inner, int wi, const u64* ibnd, u64 nb,
                                      u64* first_out)
 {
     u64 b = nb == 1 ? 0 : pra_bucket(pra_fnv(key, jcc), nb);
     u64 lo = ibnd[b], hi = ibnd[b + 1];
-    u64 a = lo, z = hi;   // first row >= key
-    while (a < z) {
-        u64 m = (a + z) >> 1;
-        if (pra_row_cmp(inner + m * wi, key, jcc) < 0) a = m + 1; else z = m;
-    }
-    u64 first = a;
-    // first row > key: gallop from the first match (key runs are short), then
-    // a binary search inside the last step
-    u64 step = 1;
-    z = first;
-    while (z < hi && pra_row_cmp(inner + z * wi, key, jcc) <= 0) {
-        a = z + 1;
-        z = first + step < hi ? first + step : hi;
-        step <<= 1;
-    }
-    while (a < z) {
-        u64 m = (a + z) >> 1;
-        if (pra_row_cmp(inner + m * wi, key, jcc) <= 0) a = m + 1; else z = m;
-    }
+    const u64 first = pra_row_bound(inner, wi, key, jcc, lo, hi, false);   // first row >= key
+    // first row > key: most runs end within four rows, whose loads go out
+    // together; the others are searched for
+    u32 eq = 0;
+#pragma unroll
+    for (u32 q = 0; q < 4; q++)
+        if (first + q < hi && pra_row_cmp(inner + (first + q) * wi, key, jcc) == 0) eq |= 1u << q;
+    const u64 a = eq != 15u ? first + (u64)__popc(eq) : pra_row_bound(inner, wi, key, jcc, first + 4, hi, true);
     *first_out = first;
     return a - first;
 }
 
-// Merge of a sorted delta into a sorted full (both ordered by (bucket, all w
-// columns), disjoint).  rank[j] = number of full rows before delta row j,
-// searched inside delta row j's bucket.
-__global__ void k_merge_rank(const u64* D, u64 nd, const u64* dbnd, const u64* F, const u64* fbnd, u64 nb, int w,
-                             u64* rank)
+// Merges of sorted deltas into sorted fulls (both ordered by (bucket, all w
+// columns), disjoint), several relations in one launch each: rank[j] = number
+// of full rows before delta row j, searched inside delta row j's bucket; then
+// delta row j goes to j + rank[j], and full row i after the delta rows ranked
+// at or before it (rank is non-decreasing).  Small merges are all launch and
+// search latency: the points-to analysis' 221 merges took 9.3 + 4.5 us each, in
+// 61 launches of each kernel 12.8 + 6.4 us.
+__device__ inline int pra_merge_job(const MergeBatch& b, const u32* base)
 {
-    u64 j = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nd) return;
-    u64 b = 0, bh = nb;   // bucket of row j: last b with dbnd[b] <= j
-    while (b + 1 < bh) {
-        u64 m = (b + bh) >> 1;
-        if (dbnd[m] <= j) b = m; else bh = m;
-    }
-    const u64* d = D + j * w;
-    u64 a = fbnd[b], z = fbnd[b + 1];
-    while (a < z) {
-        u64 m = (a + z) >> 1;
-        if (pra_row_cmp(F + m * w, d, w) < 0) a = m + 1; else z = m;
-    }
-    rank[j] = a;
+    int k = 0;
+    while (k + 1 < b.njobs && base[k + 1] <= blockIdx.x) k++;
+    return k;
 }
 
-// Place every row of the merge: delta row j at j + rank[j], full row i after
-// the delta rows ranked at or before it (rank is non-decreasing).
-// (with add_to: block 0 also adds delta's bucket bounds to full's, the
-// bounds of the merged version; k_merge_rank has read full's before)
-__global__ void k_merge_scatter(const u64* F, u64 nf, const u64* D, u64 nd, const u64* rank, int w, u64* out,
-                                u64* add_to, const u64* dbnd, u64 nbb)
+__global__ void k_merge_rank(MergeBatch b)
 {
-    if (add_to && blockIdx.x == 0)
-        for (u64 i = threadIdx.x; i < nbb; i += blockDim.x) add_to[i] += dbnd[i];
-    u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nf + nd) return;
+    const int k = pra_merge_job(b, b.rank_base);
+    const MergeJob& m = b.job[k];
+    const u64 j = (u64)(blockIdx.x - b.rank_base[k]) * blockDim.x + threadIdx.x;
+    if (j >= m.nd) return;
+    u64 lo = 0, hi = b.nb;   // bucket of row j: last b with dbnd[b] <= j
+    while (lo + 1 < hi) {
+        const u64 mid = (lo + hi) >> 1;
+        if (m.dbnd[mid] <= j) lo = mid; else hi = mid;
+    }
+    m.rank[j] = pra_row_bound(m.F, m.w, m.D + j * m.w, m.w, m.fbnd[lo], m.fbnd[lo + 1], false);
+}
+
+// (the first block of a job also adds delta's bucket bounds to full's, the
+// bounds of the merged version; k_merge_rank has read full's before)
+__global__ void k_merge_scatter(MergeBatch b)
+{
+    const int k = pra_merge_job(b, b.scatter_base);
+    const MergeJob& m = b.job[k];
+    const u32 bid = blockIdx.x - b.scatter_base[k];
+    if (bid == 0)
+        for (u64 i = threadIdx.x; i <= b.nb; i += blockDim.x) m.add_to[i] += m.dbnd[i];
+    const u64 t = (u64)bid * blockDim.x + threadIdx.x;
+    if (t >= m.nf + m.nd) return;
     const u64* src;
     u64 pos;
-    if (t < nf) {
-        u64 a = 0, z = nd;   // delta rows with rank <= t
-        while (a < z) {
-            u64 m = (a + z) >> 1;
-            if (rank[m] <= t) a = m + 1; else z = m;
-        }
-        src = F + t * w;
-        pos = t + a;
+    if (t < m.nf) {
+        src = m.F + t * m.w;
+        pos = t + pra_row_bound(m.rank, 1, &t, 1, 0, m.nd, true);   // delta rows with rank <= t
     } else {
-        u64 j = t - nf;
-        src = D + j * w;
-        pos = j + rank[j];
+        const u64 j = t - m.nf;
+        src = m.D + j * m.w;
+        pos = j + m.rank[j];
     }
-    u64* dst = out + pos * w;
-    pra_copy_row(dst, src, w);
+    pra_copy_row(m.out + pos * m.w, src, m.w);
 }
 
 // One thread per join pair: locate the outer row by binary search over the
@@ -2766,16 +2793,19 @@ __global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place_many(const RankA
 // the seq counters advance by the new tuples of each bucket (bucket d's rows
 // start at offs[d * nblocks]).  PRA_BLOCK threads; counters and replicas are
 // read by atomic exchange, so the scatter's own block may run it too.
+// NW waves, at least PRA_WAVES; threads past PRA_BLOCK only keep the barriers.
+template <int NW = PRA_WAVES>
 __device__ inline void pra_newt_fold_part(const NewtFoldArgs& a, u32 y, u32 t, u32* lds, u32* mx)
 {
     if (y == 0) {
         if (!a.packed) return;
-        const u32 v = atomicExch(&a.bin_cur[t], 0u);
+        const u32 v = t < PRA_BLOCK ? atomicExch(&a.bin_cur[t], 0u) : 0u;
         u32 tot;
-        a.kgofs[t] = block_exclusive_scan<u32>(v, lds, &tot);
+        const u32 ex = block_exclusive_scan<u32, NW>(v, lds, &tot);
+        if (t < PRA_BLOCK) a.kgofs[t] = ex;
         if (t == 0) *mx = 0;
         __syncthreads();
-        atomicMax(mx, v);
+        if (v) atomicMax(mx, v);
         __syncthreads();
         if (t == 0) a.stat[6] = *mx;
     } else if (y == 1) {
@@ -2801,13 +2831,14 @@ __device__ inline void pra_newt_fold_part(const NewtFoldArgs& a, u32 y, u32 t, u
 }
 
 // k_newt_fold's three parts in one block after the scatter of a single tile
+template <int NW>
 __device__ inline void pra_scatter_fold_tail(const NewtFoldArgs& f)
 {
-    __shared__ u32 flds[PRA_WAVES + 1];
+    __shared__ u32 flds[NW + 1];
     __shared__ u32 fmx;
     __syncthreads();
     for (u32 y = 0; y < 3; y++) {
-        pra_newt_fold_part(f, y, threadIdx.x, flds, &fmx);
+        pra_newt_fold_part<NW>(f, y, threadIdx.x, flds, &fmx);
         __syncthreads();
     }
 }
@@ -2824,7 +2855,7 @@ __device__ __forceinline__ void pra_scatter_block(NewtScatterArgs& a, const u32 
     a.n = a.ctl[0];
     // blocks past the candidates hold nothing; the summary reduce skips them
     if ((u64)bid * PRA_TILE >= a.n) {
-        if (SB == PRA_BLOCK && a.fold_here) pra_scatter_fold_tail(a.fold);
+        if (a.fold_here) pra_scatter_fold_tail<SW>(a.fold);
         return;
     }
     __shared__ u32 wh[SW][PRA_RADIX];
@@ -3032,7 +3063,7 @@ __device__ __forceinline__ void pra_scatter_block(NewtScatterArgs& a, const u32 
             if (!is_and && v != 0) atomicOr(dst, (unsigned long long)v);
         }
     }
-    if (SB == PRA_BLOCK && a.fold_here) pra_scatter_fold_tail(a.fold);
+    if (a.fold_here) pra_scatter_fold_tail<SW>(a.fold);
 }
 
 template <bool PACKED, int SB>
@@ -3041,12 +3072,13 @@ __global__ __launch_bounds__(SB) void k_dedup_scatter(NewtScatterArgs a)
     pra_scatter_block<PACKED, SB>(a, blockIdx.x);
 }
 
-// Partitions of several outputs' candidates in one launch (PRA_BLOCK-thread
-// blocks): the jobs' arguments and block ranges are read from device memory
+// Partitions of several outputs' candidates in one launch (tiles of few items a
+// thread: points-to analysis, 256 threads of 8 items 22.9 us a launch, 1,024 of
+// 2 items 15.5): the jobs' arguments and block ranges are read from device memory
 // (njobs arguments, then njobs + 1 block bases), a block serving the job whose
 // range holds it as k_dedup_scatter serves its one output.
 template <bool PACKED>
-__global__ __launch_bounds__(PRA_BLOCK) void k_dedup_scatter_many(const NewtScatterArgs* jobs, int njobs)
+__global__ __launch_bounds__(PRA_SCATTER_BLOCK) void k_dedup_scatter_many(const NewtScatterArgs* jobs, int njobs)
 {
     const u32* block_base = (const u32*)(jobs + njobs);
     // the job: the number of later jobs' block bases at or below this block,
@@ -3057,7 +3089,7 @@ __global__ __launch_bounds__(PRA_BLOCK) void k_dedup_scatter_many(const NewtScat
         k += __popcll(__ballot(j < njobs && block_base[j] <= blockIdx.x));
     }
     NewtScatterArgs a = jobs[k];
-    pra_scatter_block<PACKED, PRA_BLOCK>(a, blockIdx.x - block_base[k]);
+    pra_scatter_block<PACKED, PRA_SCATTER_BLOCK>(a, blockIdx.x - block_base[k]);
 }
 
 // The folds of several outputs in one launch: block b runs part b % 3 of job
@@ -3330,17 +3362,17 @@ __global__ void k_scan_lookback(const T* in, T* out, u64 n, u64* status, u32* ti
 // (join): a row's count is the length of its key's run of inner rows, found
 // in the static inner's key index (istart = the run's first row);
 // PRA_CS_SORTED (join): the same run searched in the inner's sorted rows;
-// PRA_CS_FILTER (copy, copy_filter): 1 for rows passing the filter `op`.  A tile holds PRA_TILE rows (PRA_TILE /
-// PRA_COUNT_SCAN_BLOCK consecutive rows per thread) and finds its offset by
+// PRA_CS_FILTER (copy, copy_filter): 1 for rows passing the filter `op`.  A tile holds PRA_COUNT_SCAN_TILE rows (one
+// a thread: a second one's search would wait for the first's) and finds its offset by
 // decoupled look-back over digit 0 of the status words, as k_scan_lookback
 // does; the last tile writes off[n] = total.
 template <int KIND>
 __device__ inline void pra_count_scan_tile(const CountScanArgs& a, u64* status, u32 tile, u32 ntiles, u32 epoch,
                                            u32* flags, u64* lds, u64* s_excl)
 {
-    constexpr int IT = PRA_TILE / PRA_COUNT_SCAN_BLOCK;
+    constexpr int IT = PRA_COUNT_SCAN_TILE / PRA_COUNT_SCAN_BLOCK;
     constexpr int NW = PRA_COUNT_SCAN_BLOCK / 64;
-    const u64 base = (u64)tile * PRA_TILE + (u64)threadIdx.x * IT;
+    const u64 base = (u64)tile * PRA_COUNT_SCAN_TILE + (u64)threadIdx.x * IT;
     u64 c[IT];
     if (KIND == PRA_CS_SORTED) {
 #pragma unroll
@@ -3635,9 +3667,9 @@ void pra_launch_dedup_scatter_many(hipStream_t st, const NewtScatterArgs* jobs, 
 {
     if (njobs <= 0 || !nblocks) return;
     if (packed)
-        hipLaunchKernelGGL(k_dedup_scatter_many<true>, dim3(nblocks), dim3(PRA_BLOCK), 0, st, jobs, njobs);
+        hipLaunchKernelGGL(k_dedup_scatter_many<true>, dim3(nblocks), dim3(PRA_SCATTER_BLOCK), 0, st, jobs, njobs);
     else
-        hipLaunchKernelGGL(k_dedup_scatter_many<false>, dim3(nblocks), dim3(PRA_BLOCK), 0, st, jobs, njobs);
+        hipLaunchKernelGGL(k_dedup_scatter_many<false>, dim3(nblocks), dim3(PRA_SCATTER_BLOCK), 0, st, jobs, njobs);
 }
 
 void pra_launch_table_insert_rows(hipStream_t st, const u64* rows, u64 n, int w, int kw, u64* table, u64 cap,
@@ -4068,13 +4100,11 @@ void pra_launch_newt_rep_init(hipStream_t st, u64* rep_words, int sets)
                            dim3(PRA_BLOCK), 0, st, rep_words + (size_t)k * PRA_NREP * PRA_PART_WORDS);
 }
 
-void pra_launch_merge(hipStream_t st, const u64* F, u64 nf, const u64* fbnd, const u64* D, u64 nd, const u64* dbnd,
-                      u64 nb, int w, u64* rank, u64* out, u64* add_to)
+void pra_launch_merge(hipStream_t st, const MergeBatch& b)
 {
-    if (!nd) return;
-    hipLaunchKernelGGL(k_merge_rank, dim3(grid_for(nd)), dim3(PRA_BLOCK), 0, st, D, nd, dbnd, F, fbnd, nb, w, rank);
-    hipLaunchKernelGGL(k_merge_scatter, dim3(grid_for(nf + nd)), dim3(PRA_BLOCK), 0, st, F, nf, D, nd, rank, w, out,
-                       add_to, dbnd, nb + 1);
+    if (b.njobs <= 0) return;
+    hipLaunchKernelGGL(k_merge_rank, dim3(b.rank_base[b.njobs]), dim3(PRA_BLOCK), 0, st, b);
+    hipLaunchKernelGGL(k_merge_scatter, dim3(b.scatter_base[b.njobs]), dim3(PRA_BLOCK), 0, st, b);
 }
 
 void pra_launch_rows_checksum(hipStream_t st, const u64* rows, u64 n, int w, u64* out)

@@ -513,7 +513,22 @@ void pra_launch_newt_fold_publish(hipStream_t st, const NewtFoldArgs& a, const u
 // `sets` consecutive replica sets (one per output of a batched partition)
 void pra_launch_newt_rep_init(hipStream_t st, u64* rep_words, int sets = 1);
 void pra_launch_rows_checksum(hipStream_t st, const u64* rows, u64 n, int w, u64* out);
-// merge of sorted delta into sorted full (out); add_to (nullable): full's
-// bucket bounds, which become the merged version's
-void pra_launch_merge(hipStream_t st, const u64* F, u64 nf, const u64* fbnd, const u64* D, u64 nd, const u64* dbnd,
-                      u64 nb, int w, u64* rank, u64* out, u64* add_to = nullptr);
+// merges of sorted deltas into sorted fulls: rank receives nd words, out the
+// merged rows, and delta's bucket bounds are added to full's (add_to = fbnd).
+// Blocks of PRA_BLOCK rows: rank_base over nd, scatter_base over nf + nd.
+struct MergeJob {
+    const u64 *F, *fbnd, *D, *dbnd;
+    u64 *rank, *out, *add_to;
+    u64 nf, nd;
+    int w, pad;
+};
+#define PRA_MERGE_JOBS 32
+struct MergeBatch {
+    MergeJob job[PRA_MERGE_JOBS];
+    u32 rank_base[PRA_MERGE_JOBS + 1], scatter_base[PRA_MERGE_JOBS + 1];
+    u64 nb;
+    int njobs;
+};
+static_assert(sizeof(MergeBatch) <= 4096, "merge batch exceeds the kernel arguments");
+void pra_launch_merge(hipStream_t st, const MergeBatch& b);
+
