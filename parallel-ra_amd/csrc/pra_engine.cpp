@@ -607,6 +607,8 @@ struct pra_ctx {
     u64* mailbox = nullptr;     // pinned, written by the publish kernel
     size_t mailbox_cap = 0;
     u64 pub_seq = 0;            // sequence number of the last publication
+    u64 pub_wait = 0;           // the one the host waits for
+    bool pub_open = false;      // a publication is under way: the mailbox is taken
     hipEvent_t pub_ev = nullptr;
     std::string err;
     // profiling
@@ -869,8 +871,17 @@ static void check_flags(u32 f)
 // Read back `words` u64 from device memory in one synchronization, together
 // with the device error flags.  Flags are sticky: kernels only ever set them
 // on a detected error, and every synchronization point checks them.
+// A few words are published (below): a kernel and a spin cost about 10 us
+// where two copies and a blocking wait cost about 25.
+constexpr size_t kPublishWords = 256;
+static u64* publish_readback(pra_ctx* c, const u64* src, size_t words);
 static u64* readback(pra_ctx* c, const void* src, size_t words)
 {
+    if (words <= kPublishWords && !c->pub_open) {
+        u64* h = publish_readback(c, (const u64*)src, words);
+        stream_idle(c->st);
+        return h;
+    }
     u64* h = c->host_buf(words + 1);
     if (words) HIPCHK(hipMemcpyAsync(h, src, words * 8, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipMemcpyAsync(h + words, c->flags_buf.p, 8, hipMemcpyDeviceToHost, c->st));
@@ -890,15 +901,25 @@ static void sync_check(pra_ctx* c) { readback(c, nullptr, 0); }
 // kernel reports errors, and after a while the host falls back to a blocking
 // wait on it.
 // fold: a newt fold still to run, done by the publishing kernel itself
-// by_place: the placement of the iteration's one ranked output publishes (as
-// sequence number pub_seq + 1), and this call only takes note of it
-static u64* publish_begin(pra_ctx* c, const u64* src, size_t words, const NewtFoldArgs* fold = nullptr,
-                          bool by_place = false)
+// by_kernel: a kernel given publish_take's mailbox publishes (the placement of
+// the iteration's one ranked output, a one-block build), and this call only
+// takes note of it
+static u64* publish_take(pra_ctx* c, size_t words, u64* seq)
 {
     // mailbox word 0: the sequence number; the summary and flags after it
     u64* h = c->mailbox_buf(words + 2) + 1;
-    const u64 seq = ++c->pub_seq;
-    if (by_place) {
+    *seq = ++c->pub_seq;
+    c->pub_open = true;
+    return h;
+}
+
+static u64* publish_begin(pra_ctx* c, const u64* src, size_t words, const NewtFoldArgs* fold = nullptr,
+                          bool by_kernel = false)
+{
+    u64 seq = c->pub_seq;
+    u64* h = by_kernel ? c->mailbox + 1 : publish_take(c, words, &seq);
+    c->pub_wait = seq;
+    if (by_kernel) {
     } else if (fold)
         pra_launch_newt_fold_publish(c->st, *fold, src, words, c->flags_buf.as<u32>(), h, seq);
     else
@@ -915,7 +936,7 @@ static u64* publish_wait(pra_ctx* c, u64* h, size_t words)
 {
     auto t0 = std::chrono::steady_clock::now();
     for (u32 k = 0;; k++) {
-        if (__atomic_load_n(h - 1, __ATOMIC_ACQUIRE) == c->pub_seq) break;
+        if (__atomic_load_n(h - 1, __ATOMIC_ACQUIRE) == c->pub_wait) break;
         if ((k & 63) == 63) {
             const hipError_t q = hipEventQuery(c->pub_ev);
             if (q != hipSuccess && q != hipErrorNotReady) HIPCHK(q);
@@ -925,6 +946,7 @@ static u64* publish_wait(pra_ctx* c, u64* h, size_t words)
             }
         }
     }
+    c->pub_open = false;
     check_flags((u32)h[words]);
     return h;
 }
@@ -1415,6 +1437,62 @@ static void bucket_rows(pra_ctx* c, const u64* rows, u64 n, int w, int jcc, u64*
     check_launch("bucket_rows");
 }
 
+// The same by one block, when at most PRA_DICT_SMALL_WORDS column values of at
+// most PRA_DICT_SMALL_RELS versions hold no more than PRA_DICT_SMALL distinct
+// ones: what one compute unit reads and sorts in the time of two or three of
+// the general build's dozen launches.  False when they do not, or there is no
+// room for tables of that many values.
+static bool build_small_dictionary(pra_ctx* c, int gi, u64 total)
+{
+    Group& G = grp(c, gi);
+    if (total > PRA_DICT_SMALL_WORDS || c->pub_open) return false;
+    DictSmallArgs a{};
+    for (pra_rel* R : c->rels)
+        for (int v : {PRA_FULL, PRA_DELTA}) {
+            Rows& r = R->ver[v];
+            if (R->group != gi || R->view_of || !r.n || !R->arity) continue;
+            if (a.k == PRA_DICT_SMALL_RELS) return false;
+            a.rows[a.k] = r.d();
+            a.n[a.k] = (u32)r.n;
+            a.w[a.k] = R->w;
+            a.arity[a.k++] = R->arity;
+        }
+    const u64 room = std::min<u64>(total, PRA_DICT_SMALL);
+    a.cap = pow2_at_least(std::max<u64>(64, 2 * room));
+    a.nb = (u64)c->nb;
+    try {
+        G.dict.reserve(a.cap * 16, c->st);
+        G.vals.reserve(room * 8, c->st);
+        if (c->nb > 1) {
+            G.lead_vals.reserve(room * 8, c->st);
+            G.rank_of.reserve(room * 4, c->st);
+            G.lead_of.reserve(room * 4, c->st);
+            G.lead_bucket.reserve(room, c->st);
+        }
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        for (DBuf* b : {&G.dict, &G.vals, &G.lead_vals, &G.rank_of, &G.lead_of, &G.lead_bucket}) b->release();
+        return false;
+    }
+    a.dict = G.dict.as<u64>();
+    a.vals = G.vals.as<u64>();
+    a.lead_vals = G.lead_vals.as<u64>();
+    a.rank_of = G.rank_of.as<u32>();
+    a.lead_of = G.lead_of.as<u32>();
+    a.lead_bucket = G.lead_bucket.as<unsigned char>();
+    a.err = c->dflags();
+    a.host = publish_take(c, 1, &a.seq);
+    pra_launch_dict_small(c->st, a);
+    check_launch("dict_small");
+    const u64 n = publish_wait(c, publish_begin(c, nullptr, 1, nullptr, true), 1)[0];
+    if (n == ~0ULL) return false;
+    G.dict_cap = a.cap;
+    G.dict_n = n;
+    G.dict_state = 1;
+    G.dict_gen++;
+    return true;
+}
+
 // (Re)build instance gi's value dictionary from the key columns of every
 // relation of that instance.
 static void build_dictionary(pra_ctx* c, int gi)
@@ -1425,6 +1503,7 @@ static void build_dictionary(pra_ctx* c, int gi)
         if (R->group == gi && !R->view_of)
             for (int v : {PRA_FULL, PRA_DELTA}) total += R->ver[v].n * (u64)R->arity;
     if (total == 0) return;
+    if (build_small_dictionary(c, gi, total)) return;
     Rows V;
     V.buf.reserve(total * 8, c->st);
     u64 off = 0;
@@ -1551,6 +1630,35 @@ static const u64* bucket_bounds(pra_ctx* c, pra_rel* R, int v)
     return R->bnd[v].as<u64>();
 }
 
+// The index of a version of at most PRA_INDEX_SMALL rows by one block; false
+// when it has more, or there is no room for a table of that many runs.
+static bool small_index(pra_ctx* c, pra_rel* R, int v)
+{
+    Rows& r = R->ver[v];
+    if (r.n > PRA_INDEX_SMALL || c->pub_open) return false;
+    try {
+        R->idx[v].reserve(pow2_at_least(std::max<u64>(64, 2 * r.n)) * 3 * 8, c->st);
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        return false;
+    }
+    IndexSmallArgs a{};
+    a.rows = r.d();
+    a.n = (u32)r.n;
+    a.w = R->w;
+    a.jcc = R->jcc;
+    a.table = R->idx[v].as<u64>();
+    a.err = c->dflags();
+    a.host = publish_take(c, 2, &a.seq);
+    pra_launch_index_small(c->st, a);
+    check_launch("index_small");
+    const u64* h = publish_wait(c, publish_begin(c, nullptr, 2, nullptr, true), 2);
+    R->idx_maxlen[v] = h[0];
+    R->idx_cap[v] = pow2_at_least(std::max<u64>(64, 2 * h[1]));
+    R->idx_valid[v] = true;
+    return true;
+}
+
 // (key -> first row, count) index over the sorted rows of a version
 static void ensure_index(pra_ctx* c, pra_rel* R, int v)
 {
@@ -1565,6 +1673,7 @@ static void ensure_index(pra_ctx* c, pra_rel* R, int v)
         return;
     }
     Prof p(c, K_INDEX_BUILD, 8.0 * n * R->jcc);
+    if (small_index(c, R, v)) return;
     c->tmp64a.reserve(n * 8, c->st);
     c->tmp64b.reserve((n + 1) * 8, c->st);
     c->tmp64c.reserve((n + 1) * 8, c->st);
@@ -2719,8 +2828,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 ra.wn = R->w;
                 ra.by_bucket = lead;
                 if (planned && place_publishes) {
-                    ra.host = c->mailbox_buf(no * SW + 2) + 1;
-                    ra.host_seq = c->pub_seq + 1;
+                    ra.host = publish_take(c, no * SW, &ra.host_seq);
                     ra.host_words = (u32)(no * SW);
                     ra.err = c->dflags();
                 }

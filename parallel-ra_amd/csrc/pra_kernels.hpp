@@ -421,6 +421,36 @@ void pra_launch_collect_cols(hipStream_t st, const u64* rows, u64 n, int w, int 
 void pra_launch_view_keep(hipStream_t st, const u64* rows, u64 n, int w, int ja, int jb, u64 nb, u32* keep);
 void pra_launch_view_compact(hipStream_t st, const u64* rows, u64 n, int w, const u32* keep, const u32* pos, u64* out);
 void pra_launch_dict_insert(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* flags);
+// a dictionary or a join index built by one block (k_dict_small,
+// k_index_small), whose host words follow host[-1] as in pra_launch_publish
+#define PRA_DICT_SMALL 4096          // distinct values
+#define PRA_DICT_SMALL_WORDS 32768   // column values read
+#define PRA_DICT_SMALL_RELS 16       // versions read
+#define PRA_INDEX_SMALL 4096         // rows
+struct DictSmallArgs {
+    const u64* rows[PRA_DICT_SMALL_RELS];
+    u32 n[PRA_DICT_SMALL_RELS];
+    int w[PRA_DICT_SMALL_RELS], arity[PRA_DICT_SMALL_RELS];
+    int k;
+    u64 nb, cap;
+    u64 *dict, *vals, *lead_vals;   // the last with the maps below: nb > 1
+    u32 *rank_of, *lead_of;
+    unsigned char* lead_bucket;
+    u32* err;
+    u64* host;
+    u64 seq;
+};
+void pra_launch_dict_small(hipStream_t st, const DictSmallArgs& a);
+struct IndexSmallArgs {
+    const u64* rows;
+    u32 n;
+    int w, jcc;
+    u64* table;   // room for the next power of two from max(64, 2 n) slots
+    u32* err;
+    u64* host;
+    u64 seq;
+};
+void pra_launch_index_small(hipStream_t st, const IndexSmallArgs& a);
 // bucket-major ranks (vals: the n dictionary values by (bucket, value)) into
 // the dictionary's slots, with the maps to and from ranks and their buckets
 void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of, u32* lead_of,
