@@ -107,12 +107,15 @@ void trim_pool(int dev)
     if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess && pool) (void)hipMemPoolTrimTo(pool, 0);
 }
 
+void small_idle_flush(int dev, hipStream_t st);
+
 void* big_get(size_t bytes, hipStream_t st, size_t* got)
 {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
     void* p = g_big.get(dev, st, bytes, got, kHipBlocks);
     if (!p) {
+        small_idle_flush(dev, st);
         HIPCHK(hipStreamSynchronize(st));
         g_big.idle(st);
         trim_pool(dev);
@@ -139,15 +142,39 @@ void stream_idle(hipStream_t st) { g_big.idle(st); }
 // runs after every earlier use of the block, so stream order alone makes the
 // reuse safe, and no hipFreeAsync / hipMallocAsync pair is paid per buffer
 // (about 0.1 ms of host time each).  At most kSmallKeep bytes are kept per
-// stream; the rest, and a stream's blocks when its context goes away or the
-// device runs out of memory, are freed on their stream.
+// stream; the rest, and a stream's blocks when the device runs out of memory,
+// are freed on their stream.  When a context goes away its stream has been
+// waited for, so its blocks are idle: up to kSmallIdle bytes a device stay for
+// whichever context asks next (a short-lived context used to spend more on
+// freeing its sixty blocks than on solving: 0.65 ms of 1.3 on 40 vertices),
+// and go back when the device runs out of memory.
 constexpr size_t kSmallKeep = 2ULL << 30;
+constexpr size_t kSmallIdle = 512ULL << 20;
 struct SmallFree {
     std::map<size_t, std::vector<void*>> by_class;
     size_t bytes = 0;
+
+    void* take(size_t cls)
+    {
+        auto c = by_class.find(cls);
+        if (c == by_class.end() || c->second.empty()) return nullptr;
+        void* p = c->second.back();
+        c->second.pop_back();
+        bytes -= cls;
+        return p;
+    }
+    bool put(size_t cls, void* p, size_t limit)
+    {
+        if (bytes + cls > limit) return false;
+        by_class[cls].push_back(p);
+        bytes += cls;
+        return true;
+    }
 };
 std::mutex g_small_mu;
 std::map<hipStream_t, SmallFree> g_small;
+std::map<int, SmallFree> g_small_idle;   // per device
+std::atomic<size_t> g_small_idle_limit{kSmallIdle};   // no more than the stream-ordered pool may keep
 
 size_t small_class(size_t bytes)
 {
@@ -160,14 +187,15 @@ size_t small_class(size_t bytes)
 
 void* small_take(hipStream_t st, size_t cls)
 {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
     std::lock_guard<std::mutex> lk(g_small_mu);
     auto it = g_small.find(st);
-    if (it == g_small.end()) return nullptr;
-    auto c = it->second.by_class.find(cls);
-    if (c == it->second.by_class.end() || c->second.empty()) return nullptr;
-    void* p = c->second.back();
-    c->second.pop_back();
-    it->second.bytes -= cls;
+    void* p = it == g_small.end() ? nullptr : it->second.take(cls);
+    if (!p) {
+        auto d = g_small_idle.find(dev);
+        if (d != g_small_idle.end()) p = d->second.take(cls);
+    }
     return p;
 }
 
@@ -175,19 +203,29 @@ void small_put(hipStream_t st, void* p, size_t cls)
 {
     {
         std::lock_guard<std::mutex> lk(g_small_mu);
-        SmallFree& f = g_small[st];
-        if (f.bytes + cls <= kSmallKeep) {
-            f.by_class[cls].push_back(p);
-            f.bytes += cls;
-            return;
-        }
+        if (g_small[st].put(cls, p, kSmallKeep)) return;
     }
     (void)hipFreeAsync(p, st);
 }
 
-// free the small blocks kept for a stream, on that stream
+// free, on a stream, the idle small blocks of its device
+void small_idle_flush(int dev, hipStream_t st)
+{
+    SmallFree f;
+    {
+        std::lock_guard<std::mutex> lk(g_small_mu);
+        std::swap(f, g_small_idle[dev]);
+    }
+    for (auto& c : f.by_class)
+        for (void* p : c.second) (void)hipFreeAsync(p, st);
+}
+
+// free the small blocks kept for a stream and the device's idle ones, on it
 void small_flush(hipStream_t st)
 {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    small_idle_flush(dev, st);
     SmallFree f;
     {
         std::lock_guard<std::mutex> lk(g_small_mu);
@@ -198,6 +236,110 @@ void small_flush(hipStream_t st)
     }
     for (auto& c : f.by_class)
         for (void* p : c.second) (void)hipFreeAsync(p, st);
+}
+
+// The small blocks of a stream that has been waited for and goes away become
+// idle.  Past the limit the largest idle blocks are freed first: a block costs
+// the same to free and to make again whatever its size.
+void small_retire(hipStream_t st)
+{
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const size_t limit = g_small_idle_limit;
+    std::vector<void*> drop;
+    {
+        std::lock_guard<std::mutex> lk(g_small_mu);
+        auto it = g_small.find(st);
+        if (it == g_small.end()) return;
+        SmallFree& idle = g_small_idle[dev];
+        for (auto& c : it->second.by_class)
+            for (void* p : c.second) {
+                while (idle.bytes + c.first > limit && !idle.by_class.empty() && idle.by_class.rbegin()->first > c.first) {
+                    if (void* q = idle.take(idle.by_class.rbegin()->first))
+                        drop.push_back(q);
+                    else
+                        idle.by_class.erase(std::prev(idle.by_class.end()));
+                }
+                if (!idle.put(c.first, p, limit)) drop.push_back(p);
+            }
+        g_small.erase(it);
+    }
+    for (void* p : drop) (void)hipFreeAsync(p, st);
+}
+
+// What a context needs of the driver beside device memory -- its stream and
+// pinned host blocks -- kept idle for the next context, a few of each: making
+// and freeing them costs from 0.05 to 0.4 ms apiece.
+constexpr size_t kIdleStreams = 8, kIdlePinned = 32;
+constexpr size_t kPinnedKeep = 256 << 10;   // larger pinned blocks are freed
+struct IdleHost {
+    std::map<int, std::vector<hipStream_t>> streams;         // per device
+    std::map<std::pair<size_t, unsigned>, std::vector<void*>> pinned;   // by bytes and allocation flags
+    size_t npinned = 0;
+};
+std::mutex g_idle_mu;
+IdleHost g_idle;
+
+hipStream_t stream_get(int dev)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        auto& v = g_idle.streams[dev];
+        if (!v.empty()) {
+            hipStream_t s = v.back();
+            v.pop_back();
+            return s;
+        }
+    }
+    hipStream_t s = nullptr;
+    HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    return s;
+}
+
+// ok: everything enqueued on the stream has completed without an error
+void stream_put(int dev, hipStream_t s, bool ok)
+{
+    if (ok) {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        auto& v = g_idle.streams[dev];
+        if (v.size() < kIdleStreams) {
+            v.push_back(s);
+            return;
+        }
+    }
+    (void)hipStreamDestroy(s);
+}
+
+void* pinned_get(size_t bytes, unsigned flags)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        auto it = g_idle.pinned.find({bytes, flags});
+        if (it != g_idle.pinned.end() && !it->second.empty()) {
+            void* p = it->second.back();
+            it->second.pop_back();
+            g_idle.npinned--;
+            return p;
+        }
+    }
+    void* p = nullptr;
+    HIPCHK(hipHostMalloc(&p, bytes, flags));
+    return p;
+}
+
+// ok: no work that was enqueued can still touch the block
+void pinned_put(void* p, size_t bytes, unsigned flags, bool ok)
+{
+    if (!p) return;
+    if (ok && bytes <= kPinnedKeep) {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        if (g_idle.npinned < kIdlePinned) {
+            g_idle.pinned[{bytes, flags}].push_back(p);
+            g_idle.npinned++;
+            return;
+        }
+    }
+    (void)hipHostFree(p);
 }
 
 // Autotuned knobs, per device and band of log2(work): the dense claim
@@ -635,8 +777,11 @@ struct pra_ctx {
                         &idxa, &idxb, &posadj_dev, &rep_words, &rctl, &ttab, &kp, &part_scratch, &segb})
             b->release();
         for (DBuf& b : jobtab) b.release();
-        if (st) small_flush(st);   // the small blocks kept for this stream, freed on it
-        if (st) (void)hipStreamSynchronize(st);
+        const bool ok = st && hipStreamSynchronize(st) == hipSuccess;
+        if (ok)
+            small_retire(st);
+        else if (st)
+            small_flush(st);
         for (auto& t : tune_late)
             for (hipEvent_t e : {t.a, t.b})
                 if (e) evpool.push_back(e);
@@ -647,11 +792,11 @@ struct pra_ctx {
             g_acct.erase(st);
         }
         if (host_stage) (void)hipHostFree(host_stage);
-        if (mailbox) (void)hipHostFree(mailbox);
-        for (char* js : job_stage)
-            if (js) (void)hipHostFree(js);
+        pinned_put(mailbox, mailbox_cap * sizeof(u64), hipHostMallocCoherent, ok);
+        for (size_t i = 0; i < sizeof(job_stage) / sizeof(job_stage[0]); i++)
+            pinned_put(job_stage[i], job_stage_cap[i], hipHostMallocDefault, ok);
         if (pub_ev) (void)hipEventDestroy(pub_ev);
-        if (st) (void)hipStreamDestroy(st);
+        if (st) stream_put(device, st, ok);
     }
 
     hipEvent_t ev()
@@ -736,11 +881,11 @@ struct pra_ctx {
         if (bytes > job_stage_cap[slot]) {
             if (job_stage[slot]) {
                 HIPCHK(hipStreamSynchronize(st));
-                HIPCHK(hipHostFree(job_stage[slot]));
+                pinned_put(job_stage[slot], job_stage_cap[slot], hipHostMallocDefault, true);
             }
             job_stage[slot] = nullptr;
             const size_t c = std::max<size_t>(bytes, 64 << 10);
-            HIPCHK(hipHostMalloc((void**)&job_stage[slot], c, hipHostMallocDefault));
+            job_stage[slot] = (char*)pinned_get(c, hipHostMallocDefault);
             job_stage_cap[slot] = c;
         }
         return job_stage[slot];
@@ -750,8 +895,9 @@ struct pra_ctx {
         if (words > mailbox_cap) {
             if (mailbox) HIPCHK(hipHostFree(mailbox));
             mailbox = nullptr;
+            mailbox_cap = 0;
             size_t c = std::max<size_t>(words, 1024);
-            HIPCHK(hipHostMalloc((void**)&mailbox, c * sizeof(u64), hipHostMallocCoherent));
+            mailbox = (u64*)pinned_get(c * sizeof(u64), hipHostMallocCoherent);
             memset(mailbox, 0, c * sizeof(u64));
             mailbox_cap = c;
         }
@@ -3864,13 +4010,14 @@ int pra_ctx_create(int device, int nbuckets, uint64_t hbm_budget, pra_ctx** out)
             const char* env = getenv("PRA_POOL_RELEASE_GB");   // bytes the pool keeps, in GiB
             if (env && *env) keep = (uint64_t)(atof(env) * (double)(1ULL << 30));
             HIPCHK(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
+            g_small_idle_limit = (size_t)std::min<uint64_t>(keep, kSmallIdle);
         }
-        HIPCHK(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking));
+        c->device = device;
+        c->st = stream_get(device);
         {
             std::lock_guard<std::mutex> lk(g_acct_mu);
             g_acct[c->st].budget = hbm_budget;
         }
-        c->device = device;
         c->nb = nbuckets;
         c->budget = hbm_budget;
         grp(c.get(), 0);

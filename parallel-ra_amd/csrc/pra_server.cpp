@@ -54,7 +54,8 @@ struct Request {
     std::vector<uint64_t> edges;
     uint64_t m = 0, est = 0;
     pra_request_result res{};
-    std::vector<uint64_t> rows;
+    std::unique_ptr<uint64_t[]> rows;   // nrows x 3 words, not cleared before they are written
+    uint64_t nrows = 0;
     bool done = false;
 };
 
@@ -186,9 +187,11 @@ struct pra_server {
         if (rc == PRA_OK) rc = pra_ctx_group_joined(ctx, g, &r->res.joined);
         if (rc == PRA_OK) rc = pra_ctx_group_status(ctx, g, nullptr, &r->res.iterations, nullptr);
         if (rc == PRA_OK && keep_rows) {
-            r->rows.resize(r->res.tuples * 3);
+            r->rows.reset(new uint64_t[r->res.tuples * 3]);
             uint64_t got = 0;
-            rc = pra_rel_download(s.T, PRA_FULL, r->rows.data(), r->res.tuples, &got);
+            rc = pra_rel_download(s.T, PRA_FULL, r->rows.get(), r->res.tuples, &got);
+            r->nrows = r->res.tuples;
+            if (rc != PRA_OK) std::fill_n(r->rows.get(), r->nrows * 3, 0);
         }
         if (rc != PRA_OK)
             std::fprintf(stderr, "pra_server: results of request %llu not read (%d): %s\n",
@@ -407,9 +410,9 @@ int pra_server_rows(pra_server* s, uint64_t ticket, uint64_t* rows, uint64_t cap
     auto it = s->all.find(ticket);
     if (it == s->all.end() || !it->second->done) return PRA_E_STATE;
     Request* r = it->second.get();
-    uint64_t n = r->rows.size() / 3;
+    uint64_t n = r->nrows;
     *nrows = n;
-    for (uint64_t i = 0; rows && i < std::min(n, cap) * 3; i++) rows[i] = r->rows[i];
+    if (rows && r->rows) std::copy(r->rows.get(), r->rows.get() + std::min(n, cap) * 3, rows);
     return PRA_OK;
 }
 

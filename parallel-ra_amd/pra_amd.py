@@ -172,8 +172,7 @@ class Context:
         self.sccs = []
         self.scc_rels = {}
         self.cur_group = 0
-        self._group_of = {}       # relation handle -> instance
-        self._scc_group = {}      # scc handle -> instance
+        self._made = {}           # instance -> its (relation, scc) handles
         self.set_batch_size(batch_size)
 
     def _chk(self, rc, what):
@@ -263,8 +262,11 @@ class Context:
     def release_group(self, g):
         """free instance g's relations and SCCs (their handles become invalid) and reset it"""
         self._chk(self.L.pra_ctx_release_group(self.c, int(g)), "release_group")
-        self.rels = [None if self._group_of.get(i) == g else r for i, r in enumerate(self.rels)]
-        self.sccs = [None if self._scc_group.get(i) == g else s for i, s in enumerate(self.sccs)]
+        rels, sccs = self._made.pop(int(g), ((), ()))
+        for r in rels:
+            self.rels[r] = None
+        for s in sccs:
+            self.sccs[s] = None
 
     def device_bytes(self):
         """(bytes held now, peak bytes held) on the device by this context"""
@@ -301,7 +303,7 @@ class Context:
         self.rels.append(h)
         r = len(self.rels) - 1
         self.arity[r] = arity
-        self._group_of[r] = self.cur_group
+        self._made.setdefault(self.cur_group, ([], []))[0].append(r)
         return r
 
     def load_rows(self, rel, rows, version=FULL):
@@ -342,7 +344,7 @@ class Context:
         self.sccs.append(h)
         s = len(self.sccs) - 1
         self.scc_rels[s] = []
-        self._scc_group[s] = self.cur_group
+        self._made.setdefault(self.cur_group, ([], []))[1].append(s)
         return s
 
     def scc_add_relation(self, scc, rel, move_full_to_delta):

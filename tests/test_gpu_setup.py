@@ -3,6 +3,8 @@ to a size and by the general kernels above it: value and row counts on both
 sides of those sizes and of a block's chunks, the value of all ones (the LDS
 table's empty mark), and more relations than one launch reads.  Rows, ids
 included, per-batch deltas and join pairs must equal the oracle's."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,32 @@ def test_many_relations(more):
         return T, fix
 
     check(build, 3)
+
+
+def test_contexts_that_come_and_go():
+    """contexts made, used and closed by three threads at once take over each
+    other's streams, pinned blocks and idle device blocks"""
+    want = {}
+    for n in (64, 700):
+        o = O.Oracle(3)
+        T, *_ = tc_program(o, layers(n, n + 20))
+        o.execute(1)
+        want[n] = o.rows(T)
+    bad = []
+
+    def user(k):
+        for i in range(12):
+            n = (64, 700)[(i + k) % 2]
+            g = pra_amd.Context(3, batch_size=1)
+            T, *_ = tc_program(g, layers(n, n + 20))
+            g.execute()
+            if not np.array_equal(g.rows(T), want[n]):
+                bad.append((k, i))
+            g.close()
+
+    users = [threading.Thread(target=user, args=(k,)) for k in range(3)]
+    for u in users:
+        u.start()
+    for u in users:
+        u.join()
+    assert not bad
