@@ -687,7 +687,7 @@ struct pra_scc {
 // are staged between a publication and its wait, so they alternate between
 // two slots, and the wait of the iteration in between covers each copy.
 enum { JOB_EXPAND, JOB_SCATTER, JOB_DENSE, JOB_SCAN, JOB_FOLD, JOB_SORT, JOB_EARLY_APPEND, JOB_EARLY_APPEND2,
-       JOB_APPEND, JOB_PLAN, JOB_RANK, PRA_JOB_SLOTS };
+       JOB_APPEND, JOB_PLAN, JOB_RANK, JOB_SETUP, PRA_JOB_SLOTS };
 
 struct pra_ctx {
     int device = 0, nb = 1;
@@ -1583,26 +1583,29 @@ static void bucket_rows(pra_ctx* c, const u64* rows, u64 n, int w, int jcc, u64*
     check_launch("bucket_rows");
 }
 
-// The same by one block, when at most PRA_DICT_SMALL_WORDS column values of at
-// most PRA_DICT_SMALL_RELS versions hold no more than PRA_DICT_SMALL distinct
-// ones: what one compute unit reads and sorts in the time of two or three of
-// the general build's dozen launches.  False when they do not, or there is no
-// room for tables of that many values.
-static bool build_small_dictionary(pra_ctx* c, int gi, u64 total)
+// The arguments of a one-block dictionary of instance gi, and its tables: when
+// at most PRA_DICT_SMALL_WORDS column values of at most PRA_DICT_SMALL_RELS
+// versions may hold no more than PRA_DICT_SMALL distinct ones, what one compute
+// unit reads and sorts in the time of two or three of the general build's dozen
+// launches.  False when they do not, or there is no room for tables of that
+// many values.
+static bool small_dictionary_args(pra_ctx* c, int gi, DictSmallArgs* args)
 {
     Group& G = grp(c, gi);
-    if (total > PRA_DICT_SMALL_WORDS || c->pub_open) return false;
     DictSmallArgs a{};
+    u64 total = 0;
     for (pra_rel* R : c->rels)
         for (int v : {PRA_FULL, PRA_DELTA}) {
             Rows& r = R->ver[v];
             if (R->group != gi || R->view_of || !r.n || !R->arity) continue;
-            if (a.k == PRA_DICT_SMALL_RELS) return false;
+            total += r.n * (u64)R->arity;
+            if (a.k == PRA_DICT_SMALL_RELS || total > PRA_DICT_SMALL_WORDS) return false;
             a.rows[a.k] = r.d();
             a.n[a.k] = (u32)r.n;
             a.w[a.k] = R->w;
             a.arity[a.k++] = R->arity;
         }
+    if (total == 0) return false;
     const u64 room = std::min<u64>(total, PRA_DICT_SMALL);
     a.cap = pow2_at_least(std::max<u64>(64, 2 * room));
     a.nb = (u64)c->nb;
@@ -1627,16 +1630,65 @@ static bool build_small_dictionary(pra_ctx* c, int gi, u64 total)
     a.lead_of = G.lead_of.as<u32>();
     a.lead_bucket = G.lead_bucket.as<unsigned char>();
     a.err = c->dflags();
-    a.host = publish_take(c, 1, &a.seq);
-    pra_launch_dict_small(c->st, a);
-    check_launch("dict_small");
-    const u64 n = publish_wait(c, publish_begin(c, nullptr, 1, nullptr, true), 1)[0];
-    if (n == ~0ULL) return false;
-    G.dict_cap = a.cap;
-    G.dict_n = n;
-    G.dict_state = 1;
-    G.dict_gen++;
+    *args = a;
     return true;
+}
+
+// Whether a one-block build of n words of results a job may publish them
+// itself: one job does, the results of several are read back together.
+static u64* small_jobs_host(pra_ctx* c, size_t njobs, size_t words, u64* seq)
+{
+    if (njobs == 1 && !c->pub_open) return publish_take(c, words, seq);
+    c->tmp64a.reserve(njobs * words * 8, c->st);
+    return nullptr;
+}
+
+static void build_dictionary(pra_ctx* c, int gi);
+
+// (Re)build the value dictionaries of some instances: the small ones by one
+// block each, in one launch.
+static void build_dictionaries(pra_ctx* c, const std::vector<int>& groups)
+{
+    std::vector<DictSmallArgs> jobs;
+    std::vector<int> of, general;
+    for (int gi : groups) {
+        DictSmallArgs a;
+        if (small_dictionary_args(c, gi, &a)) {
+            jobs.push_back(a);
+            of.push_back(gi);
+        } else {
+            general.push_back(gi);
+        }
+    }
+    if (!jobs.empty()) {
+        const u64* n;
+        u64 seq = 0;
+        if (u64* host = small_jobs_host(c, jobs.size(), 1, &seq)) {
+            jobs[0].host = host;
+            jobs[0].seq = seq;
+            pra_launch_dict_small(c->st, jobs[0]);
+            check_launch("dict_small");
+            n = publish_wait(c, publish_begin(c, nullptr, 1, nullptr, true), 1);
+        } else {
+            for (size_t k = 0; k < jobs.size(); k++) jobs[k].out = c->tmp64a.as<u64>() + k;
+            const char* d = stage_table(c, JOB_SETUP, jobs.data(), jobs.size() * sizeof(DictSmallArgs));
+            pra_launch_dict_small_many(c->st, (const DictSmallArgs*)d, (int)jobs.size());
+            check_launch("dict_small_many");
+            n = readback(c, c->tmp64a.p, jobs.size());
+        }
+        for (size_t k = 0; k < jobs.size(); k++) {
+            Group& G = grp(c, of[k]);
+            if (n[k] == ~0ULL) {
+                general.push_back(of[k]);
+                continue;
+            }
+            G.dict_cap = jobs[k].cap;
+            G.dict_n = n[k];
+            G.dict_state = 1;
+            G.dict_gen++;
+        }
+    }
+    for (int gi : general) build_dictionary(c, gi);
 }
 
 // (Re)build instance gi's value dictionary from the key columns of every
@@ -1649,7 +1701,6 @@ static void build_dictionary(pra_ctx* c, int gi)
         if (R->group == gi && !R->view_of)
             for (int v : {PRA_FULL, PRA_DELTA}) total += R->ver[v].n * (u64)R->arity;
     if (total == 0) return;
-    if (build_small_dictionary(c, gi, total)) return;
     Rows V;
     V.buf.reserve(total * 8, c->st);
     u64 off = 0;
@@ -1776,33 +1827,59 @@ static const u64* bucket_bounds(pra_ctx* c, pra_rel* R, int v)
     return R->bnd[v].as<u64>();
 }
 
-// The index of a version of at most PRA_INDEX_SMALL rows by one block; false
-// when it has more, or there is no room for a table of that many runs.
-static bool small_index(pra_ctx* c, pra_rel* R, int v)
+// The indexes of sorted versions of at most PRA_INDEX_SMALL rows that have none
+// yet, by one block each, in one launch; a version with more rows, or without
+// room for a table of that many runs, is left to ensure_index.
+static void small_indexes(pra_ctx* c, const std::vector<std::pair<pra_rel*, int>>& versions)
 {
-    Rows& r = R->ver[v];
-    if (r.n > PRA_INDEX_SMALL || c->pub_open) return false;
-    try {
-        R->idx[v].reserve(pow2_at_least(std::max<u64>(64, 2 * r.n)) * 3 * 8, c->st);
-    } catch (const PraError& e) {
-        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
-        return false;
+    std::vector<IndexSmallArgs> jobs;
+    std::vector<std::pair<pra_rel*, int>> of;
+    for (auto& rv : versions) {
+        pra_rel* R = rv.first;
+        const int v = rv.second;
+        Rows& r = R->ver[v];
+        if (R->idx_valid[v] || !r.sorted || !r.n || r.n > PRA_INDEX_SMALL) continue;
+        if (std::find(of.begin(), of.end(), rv) != of.end()) continue;
+        try {
+            R->idx[v].reserve(pow2_at_least(std::max<u64>(64, 2 * r.n)) * 3 * 8, c->st);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+            continue;
+        }
+        IndexSmallArgs a{};
+        a.rows = r.d();
+        a.n = (u32)r.n;
+        a.w = R->w;
+        a.jcc = R->jcc;
+        a.table = R->idx[v].as<u64>();
+        a.err = c->dflags();
+        jobs.push_back(a);
+        of.push_back(rv);
     }
-    IndexSmallArgs a{};
-    a.rows = r.d();
-    a.n = (u32)r.n;
-    a.w = R->w;
-    a.jcc = R->jcc;
-    a.table = R->idx[v].as<u64>();
-    a.err = c->dflags();
-    a.host = publish_take(c, 2, &a.seq);
-    pra_launch_index_small(c->st, a);
-    check_launch("index_small");
-    const u64* h = publish_wait(c, publish_begin(c, nullptr, 2, nullptr, true), 2);
-    R->idx_maxlen[v] = h[0];
-    R->idx_cap[v] = pow2_at_least(std::max<u64>(64, 2 * h[1]));
-    R->idx_valid[v] = true;
-    return true;
+    if (jobs.empty()) return;
+    Prof p(c, K_INDEX_BUILD, 8.0 * jobs[0].n * jobs[0].jcc);
+    const u64* h;
+    u64 seq = 0;
+    if (u64* host = small_jobs_host(c, jobs.size(), 2, &seq)) {
+        jobs[0].host = host;
+        jobs[0].seq = seq;
+        pra_launch_index_small(c->st, jobs[0]);
+        check_launch("index_small");
+        h = publish_wait(c, publish_begin(c, nullptr, 2, nullptr, true), 2);
+    } else {
+        for (size_t k = 0; k < jobs.size(); k++) jobs[k].out = c->tmp64a.as<u64>() + 2 * k;
+        const char* d = stage_table(c, JOB_SETUP, jobs.data(), jobs.size() * sizeof(IndexSmallArgs));
+        pra_launch_index_small_many(c->st, (const IndexSmallArgs*)d, (int)jobs.size());
+        check_launch("index_small_many");
+        h = readback(c, c->tmp64a.p, 2 * jobs.size());
+    }
+    for (size_t k = 0; k < jobs.size(); k++) {
+        pra_rel* R = of[k].first;
+        const int v = of[k].second;
+        R->idx_maxlen[v] = h[2 * k];
+        R->idx_cap[v] = pow2_at_least(std::max<u64>(64, 2 * h[2 * k + 1]));
+        R->idx_valid[v] = true;
+    }
 }
 
 // (key -> first row, count) index over the sorted rows of a version
@@ -1810,6 +1887,8 @@ static void ensure_index(pra_ctx* c, pra_rel* R, int v)
 {
     if (R->idx_valid[v]) return;
     ensure_sorted(c, R, v);
+    small_indexes(c, {{R, v}});
+    if (R->idx_valid[v]) return;
     Rows& r = R->ver[v];
     u64 n = r.n;
     if (n == 0) {
@@ -1819,7 +1898,6 @@ static void ensure_index(pra_ctx* c, pra_rel* R, int v)
         return;
     }
     Prof p(c, K_INDEX_BUILD, 8.0 * n * R->jcc);
-    if (small_index(c, R, v)) return;
     c->tmp64a.reserve(n * 8, c->st);
     c->tmp64b.reserve((n + 1) * 8, c->st);
     c->tmp64c.reserve((n + 1) * 8, c->st);
@@ -2441,6 +2519,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
 
     // 0. inputs ready: sorted versions, join indexes.  Rules whose outer (or
     //    inner) version is empty emit nothing and launch nothing.
+    std::vector<std::pair<pra_rel*, int>> indexed;
     for (auto& ra : S->ras) {
         if (ra.type == RA_JOIN) {
             if (ra.v0 == PRA_DELTA) {
@@ -2452,18 +2531,19 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             ra.sorted_probe = ra.inner->scc_changing;
             if (!ra.active) continue;
             ensure_sorted(c, ra.outer, ra.outer_v);
-            if (ra.sorted_probe) {
-                ensure_sorted(c, ra.inner, ra.inner_v);
+            ensure_sorted(c, ra.inner, ra.inner_v);
+            if (ra.sorted_probe)
                 bucket_bounds(c, ra.inner, ra.inner_v);
-            } else {
-                ensure_index(c, ra.inner, ra.inner_v);
-            }
+            else if (!ra.inner->idx_valid[ra.inner_v])
+                indexed.push_back({ra.inner, ra.inner_v});
         } else {
             ra.outer = ra.in0; ra.outer_v = ra.v0; ra.inner = nullptr; ra.left = 1;
             ra.active = ra.outer->ver[ra.outer_v].n > 0;
             if (ra.active) ensure_sorted(c, ra.outer, ra.outer_v);
         }
     }
+    small_indexes(c, indexed);
+    for (auto& rv : indexed) ensure_index(c, rv.first, rv.second);
     for (auto& ra : S->ras) ra.n_outer = ra.active ? ra.outer->ver[ra.outer_v].n : 0;
 
     // 1. output relations, their rule kinds, and candidate capacities: the
@@ -2521,9 +2601,14 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     }
     // packed sort keys need the instance's value dictionary (rebuilt after a
     // miss, given up after repeated misses)
-    for (size_t oi = 0; oi < no; oi++)
-        if (out_intern[oi] && ub[oi] && grp(c, outs[oi]->group).dict_state == 0)
-            build_dictionary(c, outs[oi]->group);
+    std::vector<int> stale;
+    for (size_t oi = 0; oi < no; oi++) {
+        const int gi = outs[oi]->group;
+        if (out_intern[oi] && ub[oi] && grp(c, gi).dict_state == 0 &&
+            std::find(stale.begin(), stale.end(), gi) == stale.end())
+            stale.push_back(gi);
+    }
+    build_dictionaries(c, stale);
     std::vector<char> packed(no, 0);
     std::vector<u64> pk_mul(no, 0);
     std::vector<int> pk_ls(no, 0);
@@ -3821,7 +3906,15 @@ static void delta_to_full(pra_ctx* c, pra_rel* R)
 {
     Rows& D = R->ver[PRA_DELTA];
     if (D.n == 0) return;
-    append_rows(c, R, PRA_FULL, D.d(), D.n);
+    Rows& F = R->ver[PRA_FULL];
+    if (F.n == 0) {   // the rows move, and stay in order
+        F.buf.swap(D.buf);
+        F.n = D.n;
+        F.sorted = D.sorted;
+        R->touched(PRA_FULL);
+    } else {
+        append_rows(c, R, PRA_FULL, D.d(), D.n);
+    }
     D.n = 0;
     R->touched(PRA_DELTA);
 }

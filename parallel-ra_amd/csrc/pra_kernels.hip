@@ -1295,7 +1295,11 @@ __global__ void k_index_insert(const u64* rows, int w, int jcc, const u64* gstar
 
 // ------------------------------------------------- setup in one block ------
 
-// Sort an array of P words (a power of two) in LDS, in place (bitonic network)
+// Sort an array of P words (a power of two) in LDS, in place (bitonic network).
+// Lane l of wave v exchanges within words 128 v .. 128 v + 127 (and the same
+// 2,048 further on, block after block) while the distance is below 128, so
+// only longer exchanges, and the step into one, meet at a barrier: 18 barriers
+// instead of 78 at 4,096 words.
 template <typename T>
 __device__ __forceinline__ void pra_lds_bitonic(T* a, u32 P)
 {
@@ -1309,8 +1313,14 @@ __device__ __forceinline__ void pra_lds_bitonic(T* a, u32 P)
                     a[o] = x;
                 }
             }
-            __syncthreads();
+            if (j >= 128 || (j == 1 && k >= 128)) {
+                __syncthreads();
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
+    __syncthreads();
 }
 
 __device__ __forceinline__ void pra_publish_words(const u64* src, u64 words, const u32* flags, u64* host, u64 seq);
@@ -1323,8 +1333,10 @@ __device__ __forceinline__ void pra_publish_words(const u64* src, u64 words, con
 // Bound by the latency of its LDS sorts; one compute unit works, but the
 // general build is a dozen dependent launches and two waits: with this, the
 // one-block index (k_index_small) and waits on published words, 60 programs of
-// 200-1,500 vertices in one context take 28.5 ms instead of 36.1.
-__global__ __launch_bounds__(1024) void k_dict_small(DictSmallArgs a)
+// 200-1,500 vertices in one context took 28.5 ms instead of 36.1; one block an
+// instance in one launch and one wait for all of them (k_dict_small_many,
+// k_index_small_many), 16.3.
+__device__ __forceinline__ void pra_dict_small(const DictSmallArgs& a)
 {
     __shared__ u64 tab[2 * PRA_DICT_SMALL];
     __shared__ u64 sv[PRA_DICT_SMALL];
@@ -1407,14 +1419,21 @@ __global__ __launch_bounds__(1024) void k_dict_small(DictSmallArgs a)
     }
     __threadfence();
     __syncthreads();
-    pra_publish_words(&result, 1, a.err, a.host, a.seq);
+    if (a.host)
+        pra_publish_words(&result, 1, a.err, a.host, a.seq);
+    else if (t == 0)
+        *a.out = result;
 }
+
+__global__ __launch_bounds__(1024) void k_dict_small(DictSmallArgs a) { pra_dict_small(a); }
+
+__global__ __launch_bounds__(1024) void k_dict_small_many(const DictSmallArgs* jobs) { pra_dict_small(jobs[blockIdx.x]); }
 
 // The join index of a sorted version of at most PRA_INDEX_SMALL rows in one
 // launch: the runs of equal keys, their longest, and the table, sized for the
 // runs as the general build sizes it (longest run and number of runs to the
 // host).  The general build is eight launches and two waits.
-__global__ __launch_bounds__(1024) void k_index_small(IndexSmallArgs a)
+__device__ __forceinline__ void pra_index_small(const IndexSmallArgs& a)
 {
     __shared__ u32 gstart[PRA_INDEX_SMALL + 1];
     __shared__ u32 wsum[16];
@@ -1476,7 +1495,17 @@ __global__ __launch_bounds__(1024) void k_index_small(IndexSmallArgs a)
         result[1] = ng;
     }
     __syncthreads();
-    pra_publish_words(result, 2, a.err, a.host, a.seq);
+    if (a.host)
+        pra_publish_words(result, 2, a.err, a.host, a.seq);
+    else if (t < 2)
+        a.out[t] = result[t];
+}
+
+__global__ __launch_bounds__(1024) void k_index_small(IndexSmallArgs a) { pra_index_small(a); }
+
+__global__ __launch_bounds__(1024) void k_index_small_many(const IndexSmallArgs* jobs)
+{
+    pra_index_small(jobs[blockIdx.x]);
 }
 
 // --------------------------------------------------------------- join ------
@@ -4023,6 +4052,16 @@ void pra_launch_dict_insert(hipStream_t st, const u64* vals, u64 n, u64* tab, u6
 void pra_launch_dict_small(hipStream_t st, const DictSmallArgs& a)
 {
     hipLaunchKernelGGL(k_dict_small, dim3(1), dim3(1024), 0, st, a);
+}
+
+void pra_launch_dict_small_many(hipStream_t st, const DictSmallArgs* jobs, int njobs)
+{
+    hipLaunchKernelGGL(k_dict_small_many, dim3(njobs), dim3(1024), 0, st, jobs);
+}
+
+void pra_launch_index_small_many(hipStream_t st, const IndexSmallArgs* jobs, int njobs)
+{
+    hipLaunchKernelGGL(k_index_small_many, dim3(njobs), dim3(1024), 0, st, jobs);
 }
 
 void pra_launch_index_small(hipStream_t st, const IndexSmallArgs& a)

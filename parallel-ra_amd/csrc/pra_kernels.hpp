@@ -437,20 +437,24 @@ struct DictSmallArgs {
     u32 *rank_of, *lead_of;
     unsigned char* lead_bucket;
     u32* err;
-    u64* host;
+    u64* host;   // null: the count to out
     u64 seq;
+    u64* out;
 };
 void pra_launch_dict_small(hipStream_t st, const DictSmallArgs& a);
+void pra_launch_dict_small_many(hipStream_t st, const DictSmallArgs* jobs, int njobs);   // jobs: device memory
 struct IndexSmallArgs {
     const u64* rows;
     u32 n;
     int w, jcc;
     u64* table;   // room for the next power of two from max(64, 2 n) slots
     u32* err;
-    u64* host;
+    u64* host;   // null: the two words to out
     u64 seq;
+    u64* out;
 };
 void pra_launch_index_small(hipStream_t st, const IndexSmallArgs& a);
+void pra_launch_index_small_many(hipStream_t st, const IndexSmallArgs* jobs, int njobs);
 // bucket-major ranks (vals: the n dictionary values by (bucket, value)) into
 // the dictionary's slots, with the maps to and from ranks and their buckets
 void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* tab, u64 cap, u32* rank_of, u32* lead_of,

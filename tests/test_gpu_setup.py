@@ -105,3 +105,25 @@ def test_contexts_that_come_and_go():
     for u in users:
         u.join()
     assert not bad
+
+
+@pytest.mark.parametrize("k", [1, 3])
+def test_instances_of_all_sizes(k):
+    """one launch for the small instances of a context, the general kernels for
+    the others"""
+    sizes = SIZES + [(64, 80)] * 5
+    g = pra_amd.Context(k, batch_size=1)
+    made = []
+    for i, (values, rows) in enumerate(sizes):
+        g.set_group(i)
+        T, _, fix, _ = tc_program(g, layers(values, rows))
+        made.append((T, fix))
+    g.execute()
+    for i, (values, rows) in enumerate(sizes):
+        o = O.Oracle(k)
+        T, _, fix, _ = tc_program(o, layers(values, rows))
+        o.execute(1)
+        np.testing.assert_array_equal(g.rows(made[i][0]), o.rows(T))
+        assert g.history(made[i][1]) == o.history(fix)
+        assert g.group_joined(i) == o.joined()
+    g.close()
