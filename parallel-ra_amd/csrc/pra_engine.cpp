@@ -547,6 +547,7 @@ struct pra_rel {
     // ranked membership: the new keys' bitmap (zero between iterations), its
     // superblocks' flags and prefixes, its lines' prefixes
     DBuf fresh, dirty, sbpre, linep;
+    DBuf places;         // whole iterations in one block: the new keys' places
     u64 fresh_sbs = 0;   // superblocks of the zeroed bitmap (0: none)
     u64 sbs_use = 0;     // of them, those of the current rank space
     // rank indexes of the delta rows (valid for dictionary generation dx_gen)
@@ -584,6 +585,8 @@ struct pra_rel {
     bool scc_changing = false, merge_full = false;
     // set while an SCC runs: a rule of it reads the relation's full version
     bool full_read = false;
+    // set while an SCC runs whose iterations one block can run (loop_rule)
+    bool loops = false;
     // changes of the delta and full versions so far
     u64 gen[2] = {0, 0};
     // a view: the rows of relation view_of that a join keyed on this
@@ -632,13 +635,13 @@ struct KStat {
 enum {
     K_JOIN_COUNT, K_JOIN_EXPAND, K_COPY_EXPAND, K_DEDUP_CLAIM, K_DEDUP_DECIDE, K_DEDUP_VERIFY, K_DEDUP_SCATTER,
     K_RADIX_HIST, K_RADIX_SCATTER, K_TABLE_BUILD, K_INDEX_BUILD, K_SCAN, K_GATHER, K_MERGE, K_BIN_SORT, K_SMALL_SORT,
-    K_BLOCK_SORT, K_RANK_EMIT, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE, K_COUNT
+    K_BLOCK_SORT, K_RANK_EMIT, K_RANK_SCAN, K_RANK_FIRST, K_RANK_PLACE, K_RANK_LOOP, K_COUNT
 };
 static const char* kNames[K_COUNT] = {"join_count", "join_expand", "copy_expand", "dedup_claim", "dedup_decide",
                                       "dedup_verify_hist", "dedup_scatter", "radix_hist", "radix_scatter",
                                       "table_build", "index_build", "scan", "gather_rows", "merge_full",
                                       "bin_sort", "small_sort", "block_sort", "rank_emit", "rank_scan", "rank_first",
-                                      "rank_place"};
+                                      "rank_place", "rank_loop"};
 
 } // namespace
 
@@ -678,6 +681,9 @@ struct pra_scc {
     std::vector<RADesc> ras;
     bool done = false, running = false;
     std::vector<u64> hist;
+    // delta rows at which an iteration last had too many candidates for one
+    // block (~0: none had)
+    u64 loop_stop = ~0ULL;
 };
 
 // Job-table staging slots.  A slot's pinned buffer is rewritten only after the
@@ -687,7 +693,7 @@ struct pra_scc {
 // are staged between a publication and its wait, so they alternate between
 // two slots, and the wait of the iteration in between covers each copy.
 enum { JOB_EXPAND, JOB_SCATTER, JOB_DENSE, JOB_SCAN, JOB_FOLD, JOB_SORT, JOB_EARLY_APPEND, JOB_EARLY_APPEND2,
-       JOB_APPEND, JOB_PLAN, JOB_RANK, JOB_SETUP, PRA_JOB_SLOTS };
+       JOB_APPEND, JOB_PLAN, JOB_RANK, JOB_SETUP, JOB_LOOP, JOB_LOOP_FULL, JOB_LOOP_DELTA, PRA_JOB_SLOTS };
 
 struct pra_ctx {
     int device = 0, nb = 1;
@@ -718,6 +724,7 @@ struct pra_ctx {
     int early_parity = 0;          // early appends' slot of the last iteration
     bool dense_on = true;        // dense membership for outputs that allow it
     bool tune_on = true;         // autotuned knobs (PRA_AUTOTUNE=0: the fixed defaults)
+    bool loop_on = true;         // whole iterations in one block for small outputs (PRA_RANK_LOOP=0: never)
     bool seg_sort_on = true;     // segmented sort of newts too large for the bins (PRA_SEG_SORT=0: byte passes)
     u64 bin_cap_test = 0;        // PRA_SORT_TEST_BIN_CAP: a lower bin capacity, so tests reach the large-newt paths
     int dense_epoch_bits = 16;   // PRA_DENSE_EPOCH_BITS: at most this many epoch bits in claim slots (0: none)
@@ -2019,7 +2026,7 @@ static bool ensure_bitmap(pra_ctx* c, pra_rel* R, int kw, u64 C, u64* bits_out)
     if (!R->bm_valid || R->bm_gen != G.dict_gen || R->bm_kw != kw) {
         const u64 words = ((u64)bits + 63) / 64;
         Prof p(c, K_TABLE_BUILD, 8.0 * words + 8.0 * kw * (R->ver[PRA_FULL].n + R->ver[PRA_DELTA].n));
-        R->bm.reserve(words * 8, c->st);
+        R->bm.reserve((words + 1) / 2 * 16, c->st);   // (one block reads and writes it by 16 bytes)
         pra_launch_fill_u64(c->st, R->bm.as<u64>(), words, 0);
         if (R->ver[PRA_FULL].n + R->ver[PRA_DELTA].n) {
             c->orand.reserve(32 * 8, c->st);
@@ -2507,6 +2514,53 @@ static void refresh_view(pra_ctx* c, pra_rel* V, int v)
     V->view_gen[v] = src->gen[v];
 }
 
+// whether a join's output columns are all data columns of its inputs
+static bool projects_data(const RADesc& ra)
+{
+    for (int m : ra.map) {
+        const int first = ra.left ? ra.outer->w : ra.inner->w;
+        const int w = m < first ? first : ra.left ? ra.inner->w : ra.outer->w;
+        const int col = m < first ? m : ra.in0->jcc + (m - first);
+        if (col >= w - 1) return false;
+    }
+    return true;
+}
+
+// the arguments of a join's emission in digits over its whole outer version
+static EmitArgs emit_args(pra_ctx* c, const RADesc& rule)
+{
+    Group& G = grp(c, rule.out->group);
+    const bool lead = by_bucket(c, rule.out);
+    EmitArgs em;
+    memset(&em, 0, sizeof(em));
+    em.dx = rule.outer->dx.as<u64>();
+    em.n = rule.outer->ver[rule.outer_v].n;
+    em.thresh = c->threshold;
+    em.joined = G.joined.as<u64>();
+    em.first = rule.inner->rk_first[rule.inner_v].as<u32>();
+    em.words = rule.inner->rk_words[rule.inner_v].as<u64>();
+    em.rank_of = G.rank_of.as<u32>();
+    em.lead_of = G.lead_of.as<u32>();
+    em.inv = 1.0 / (double)G.dict_n;
+    em.kwo = rule.outer->arity;
+    em.ia = rule.inner->arity;
+    for (int i = 0; i < rule.out->arity; i++) {
+        const int m = rule.map[i], first = rule.left ? rule.outer->w : rule.inner->w;
+        const bool outer = (m < first) == (rule.left != 0);
+        const int col = m < first ? m : rule.in0->jcc + (m - first);
+        em.side[i] = outer ? 0 : 1;
+        em.col[i] = (signed char)col;
+        // outer digits: the first is a leading digit (with several buckets),
+        // the others are ranks
+        const bool have = outer && c->nb > 1 && col == 0, want = i == 0 && lead;
+        em.conv[i] = !outer || have == want ? 0 : have ? 1 : 2;
+    }
+    return em;
+}
+
+// rank spaces that one block's superblock flags cover
+static bool loop_space(u64 bits) { return bits <= (u64)PRA_LOOP_SBS << PRA_SB_BITS; }
+
 static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
 {
     for (pra_scc* m : members)
@@ -2664,7 +2718,11 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         u64 bits = 0;
         if (dense_off[oi] || !packed[oi] || !ensure_bitmap(c, R, R->arity, C, &bits)) return ch;
         ch.mode = 2;
-        if (c->tune_on && C >= kTuneMinCandidates) {
+        // (an output that one block can run is not tuned: its iterations
+        // would go to the claim table, which that block does not know)
+        const bool small = phase == 0 && R->loops && loop_space(bits) && R->jhint <= PRA_LOOP_ROWS &&
+                           R->ver[PRA_DELTA].n <= PRA_LOOP_ROWS;
+        if (c->tune_on && C >= kTuneMinCandidates && !small) {
             const int band = band_of(C), load = g_tune.settled(c->device, TUNE_DENSE_LOAD, band);
             ch.dvar = std::max(0, load);
             if (phase != 0) {
@@ -2714,12 +2772,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             ra.outer->jcc != 1 || ra.inner->jcc != 1 || ra.outer->arity > 4 || ra.inner->view_of || ra.outer->view_of ||
             ra.inner->idx_maxlen[ra.inner_v] > kEmitRun || ra.n_outer >= (1ULL << 32))
             return -1;
-        for (int m : ra.map) {
-            const int first = ra.left ? ra.outer->w : ra.inner->w;
-            const int w = m < first ? first : ra.left ? ra.inner->w : ra.outer->w;
-            const int col = m < first ? m : ra.in0->jcc + (m - first);
-            if (col >= w - 1) return -1;   // an intern id
-        }
+        if (!projects_data(ra)) return -1;   // an intern id
         return ensure_rank_rows(c, ra.inner, ra.inner_v) ? rule : -1;
     };
     // taken per output; the rule an output emits (-1: the general expansions);
@@ -3064,31 +3117,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                     ra.err = c->dflags();
                 }
                 if (er >= 0) {
-                    RADesc& rule = S->ras[er];
-                    EmitArgs& em = ra.emit;
-                    em.dx = rule.outer->dx.as<u64>();
-                    em.n = rule.n_outer;
-                    em.cap = C;
-                    em.thresh = c->threshold;
-                    em.joined = G.joined.as<u64>();
-                    em.first = rule.inner->rk_first[rule.inner_v].as<u32>();
-                    em.words = rule.inner->rk_words[rule.inner_v].as<u64>();
-                    em.rank_of = G.rank_of.as<u32>();
-                    em.lead_of = G.lead_of.as<u32>();
-                    em.inv = ra.inv;
-                    em.kwo = rule.outer->arity;
-                    em.ia = rule.inner->arity;
-                    for (int i = 0; i < kw; i++) {
-                        const int m = rule.map[i], first = rule.left ? rule.outer->w : rule.inner->w;
-                        const bool outer = (m < first) == (rule.left != 0);
-                        const int col = m < first ? m : rule.in0->jcc + (m - first);
-                        em.side[i] = outer ? 0 : 1;
-                        em.col[i] = (signed char)col;
-                        // outer digits: the first is a leading digit (with
-                        // several buckets), the others are ranks
-                        const bool have = outer && nb > 1 && col == 0, want = i == 0 && lead;
-                        em.conv[i] = !outer || have == want ? 0 : have ? 1 : 2;
-                    }
+                    ra.emit = emit_args(c, S->ras[er]);
+                    ra.emit.cap = C;
                 }
                 if (phase == 1) {
                     // launched after the batched expansions
@@ -3875,6 +3905,223 @@ static u64 delta_sum(pra_scc* S)
     return d;
 }
 
+// ------------------------------------------- whole iterations in a block ---
+
+// The rule of an SCC whose iterations one block can run (k_rank_loop), by its
+// shape: its only rule, a join on one column of its own output's delta with
+// the full version of a relation that stays as it is, projecting data
+// columns, into an output whose full version is a log.  Null: none.
+static RADesc* loop_rule(pra_scc* S)
+{
+    if (!S->fixpoint || S->ras.size() != 1) return nullptr;
+    RADesc& ra = S->ras[0];
+    if (ra.type != RA_JOIN) return nullptr;
+    ra.left = ra.v0 == PRA_DELTA;
+    ra.outer = ra.left ? ra.in0 : ra.in1;
+    ra.inner = ra.left ? ra.in1 : ra.in0;
+    ra.outer_v = ra.left ? ra.v0 : ra.v1;
+    ra.inner_v = ra.left ? ra.v1 : ra.v0;
+    if (ra.outer != ra.out || ra.outer_v != PRA_DELTA || ra.inner == ra.out || ra.inner_v != PRA_FULL ||
+        ra.inner->view_of || ra.outer->jcc != 1 || ra.inner->jcc != 1 || ra.out->arity > 4 || ra.out->full_read ||
+        ra.out->merge_full || !projects_data(ra))
+        return nullptr;
+    return &ra;
+}
+
+// Whether S's next iterations can be run by one block now: the output ranked,
+// its delta's rank indexes at hand and small, and every table in place (the
+// general iterations before have made them).
+static bool loop_ready(pra_ctx* c, pra_scc* S, u32 max_cand)
+{
+    if (!c->loop_on || !S->running || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
+    RADesc* ra = loop_rule(S);
+    if (!ra) return false;
+    pra_rel* R = ra->out;
+    Group& G = grp(c, R->group);
+    const u64 n = R->ver[PRA_DELTA].n;
+    if (!n || n > max_cand || R->jhint > max_cand || n >= S->loop_stop) return false;
+    if (c->nb > 1 && G.dict_n > PRA_LOOP_LEADS) return false;
+    if (G.dict_state != 1 || R->dx_gen != G.dict_gen || !R->bm_valid || R->bm_gen != G.dict_gen ||
+        R->bm_kw != R->arity || !G.joined.p)
+        return false;
+    u64 bits = 1;
+    for (int i = 0; i < R->arity; i++) {
+        bits *= G.dict_n;
+        if (!loop_space(bits)) return false;
+    }
+    if (R->sbs_use != (bits + (1ULL << PRA_SB_BITS) - 1) >> PRA_SB_BITS || R->fresh_sbs < R->sbs_use) return false;
+    if (!ra->inner->idx_valid[PRA_FULL] || ra->inner->idx_maxlen[PRA_FULL] > kEmitRun || !ra->inner->ver[PRA_FULL].n ||
+        ra->inner->ver[PRA_FULL].n >= (1ULL << PRA_LOOP_RUN_SHIFT))
+        return false;
+    for (pra_rel* o : S->rels)
+        if (o != R && o->ver[PRA_DELTA].n) return false;
+    return ra->inner->rk_gen[PRA_FULL] == G.dict_gen;
+}
+
+// Up to `max` iterations of each of some SCCs that are ready for it, a block
+// each, in one launch; rows[k] receives the new rows of each iteration that
+// SCC k made (none: the general iteration takes its next one).
+// The full log takes the delta first and the new rows behind it, in place; the
+// last iteration's are copied out as the delta again.
+static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u32 max_cand,
+                      std::vector<std::vector<u32>>& rows)
+{
+    std::vector<LoopArgs> jobs;
+    std::vector<size_t> of;
+    std::vector<CopyJob> appends;
+    for (size_t k = 0; k < sccs.size(); k++) {
+        RADesc& ra = *loop_rule(sccs[k]);
+        pra_rel* R = ra.out;
+        Group& G = grp(c, R->group);
+        Rows &F = R->ver[PRA_FULL], &D = R->ver[PRA_DELTA];
+        LoopArgs a;
+        memset(&a, 0, sizeof(a));
+        // room for what the rank space can still hold, or as much again twice
+        // over; an iteration stops by its candidates, so their most on top
+        u64 bits = 1;
+        for (int i = 0; i < R->arity; i++) bits *= G.dict_n;
+        const u64 have = F.n + D.n;
+        a.room = std::min<u64>(bits - std::min(bits, have), std::max<u64>(1 << 18, 2 * have)) + PRA_LOOP_ROWS;
+        try {
+            F.buf.reserve((have + a.room) * R->w * 8, c->st, (size_t)F.n * R->w * 8);
+            R->dx.reserve(PRA_LOOP_ROWS * 8, c->st, D.n * 8);
+            R->places.reserve((R->sbs_use << (PRA_SB_BITS - 5)) * 8, c->st);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+            continue;
+        }
+        appends.push_back(CopyJob{D.d(), F.d() + F.n * R->w, D.n * (u64)R->w});
+        a.emit = emit_args(c, ra);
+        a.vals = G.vals.as<u64>();
+        a.lead_vals = (by_bucket(c, R) ? G.lead_vals : G.vals).as<u64>();
+        a.bucket = G.lead_bucket.as<unsigned char>();
+        a.member = R->bm.as<u32>();
+        a.fresh = R->fresh.as<u32>();
+        a.places = R->places.as<u64>();
+        a.rows = F.d() + have * R->w;
+        Group::Seq& sq = seq_counters(c, R->group, R->tag);
+        a.seq = sq.buf.as<u64>() + sq.now * c->nb;
+        a.D = G.dict_n;
+        a.inv = a.emit.inv;
+        a.sbs = (u32)R->sbs_use;
+        a.nb = (u32)c->nb;
+        a.tag = R->tag;
+        a.max_iters = std::min<u32>(max, PRA_LOOP_ITERS);
+        a.max_cand = max_cand;
+        a.kw = R->arity;
+        a.wn = R->w;
+        a.by_bucket = by_bucket(c, R);
+        jobs.push_back(a);
+        of.push_back(k);
+    }
+    if (jobs.empty()) return;
+    copy_ranges(c, JOB_LOOP_FULL, appends);
+    c->tmp64a.reserve(jobs.size() * PRA_LOOP_OUT * 8, c->st);
+    for (size_t k = 0; k < jobs.size(); k++) jobs[k].out = c->tmp64a.as<u64>() + k * PRA_LOOP_OUT;
+    const u64* out;
+    if (jobs.size() == 1 && !c->pub_open) {
+        LoopArgs& a = jobs[0];
+        a.host = publish_take(c, PRA_LOOP_OUT, &a.host_seq);
+        a.host_words = PRA_LOOP_OUT;
+        a.err = c->dflags();
+        {
+            Prof p(c, K_RANK_LOOP, 0.0);
+            pra_launch_rank_loop(c->st, a);
+            check_launch("rank_loop");
+        }
+        out = publish_wait(c, publish_begin(c, nullptr, PRA_LOOP_OUT, nullptr, true), PRA_LOOP_OUT);
+    } else {
+        const char* d = stage_table(c, JOB_LOOP, jobs.data(), jobs.size() * sizeof(LoopArgs));
+        {
+            Prof p(c, K_RANK_LOOP, 0.0);
+            pra_launch_rank_loop_many(c->st, (const LoopArgs*)d, (int)jobs.size());
+            check_launch("rank_loop_many");
+        }
+        out = readback(c, c->tmp64a.p, jobs.size() * PRA_LOOP_OUT);
+    }
+    std::vector<CopyJob> deltas;
+    for (size_t j = 0; j < jobs.size(); j++, out += PRA_LOOP_OUT) {
+        pra_scc* S = sccs[of[j]];
+        pra_rel* R = S->ras[0].out;
+        Group& G = grp(c, R->group);
+        Rows &F = R->ver[PRA_FULL], &D = R->ver[PRA_DELTA];
+        const u64 its = out[0], written = out[1], last = out[2];
+        if (out[3] >> 32) S->loop_stop = last;   // too many candidates for one block from this delta
+        if (!its) continue;
+        const u32* h = (const u32*)(out + 4);
+        rows[of[j]].assign(h, h + its);
+        F.n += D.n + written - last;
+        F.sorted = false;
+        R->touched(PRA_FULL);
+        D.n = last;
+        D.sorted = true;
+        R->touched(PRA_DELTA);
+        R->dx_gen = G.dict_gen;
+        if (last) {
+            D.buf.reserve((size_t)last * R->w * 8, c->st);
+            deltas.push_back(CopyJob{F.d() + F.n * R->w, D.d(), last * (u64)R->w});
+        }
+        R->jhint = (u32)out[3];
+        R->mt_entries += written;
+        G.iterations += its;
+    }
+    copy_ranges(c, JOB_LOOP_DELTA, deltas);
+}
+
+// The next iterations of some SCCs: all of them make up to `max` by one block
+// each when all are ready for that, else one together.  rows[k]: the new rows
+// of each iteration of SCC k (of the general one: its delta after it).
+// One block takes about 3 us and 3 us per 1,024 candidates an iteration, the
+// general launches 45 us for one SCC and 100 us for sixty.  So a few SCCs give
+// an iteration of more than 8,192 candidates to the general launches, four and
+// more only one of more than 16,384.  Transitive closure of random graphs,
+// general against one block of at most 4,096, 8,192, 16,384 candidates: 200
+// vertices 802 against 544, 541, 542 us, 1,000 vertices 2.27 against 1.84,
+// 1.70, 1.61 ms, 3,000 vertices 3.14 against 2.99, 3.03, 3.26 ms.  Sixty of
+// 200-1,500 vertices: 17.0 ms by the general launches, 15.3 with 8,192, 15.2
+// with 16,384; 17.1 when half of them being ready was enough (the others wait
+// meanwhile).
+static void advance(pra_ctx* c, const std::vector<pra_scc*>& members, u32 max, std::vector<std::vector<u64>>& rows)
+{
+    const u32 max_cand = members.size() < 4 ? PRA_LOOP_ROWS / 2 : PRA_LOOP_ROWS;
+    rows.assign(members.size(), {});
+    bool loops = max > 1;
+    for (size_t k = 0; loops && k < members.size(); k++) loops = loop_ready(c, members[k], max_cand);
+    if (loops) {
+        std::vector<std::vector<u32>> made(members.size());
+        run_loops(c, members, max, max_cand, made);
+        for (size_t k = 0; k < members.size(); k++) rows[k].assign(made[k].begin(), made[k].end());
+    }
+    std::vector<pra_scc*> rest;
+    for (size_t k = 0; k < members.size(); k++)
+        if (rows[k].empty()) rest.push_back(members[k]);
+    if (rest.empty()) return;
+    run_iteration(c, rest);
+    for (size_t k = 0; k < members.size(); k++)
+        if (rows[k].empty()) rows[k].push_back(delta_sum(members[k]));
+}
+
+// The batches that some iterations of S complete, *b of whose current batch
+// are made: records the delta after each.  True when S ends: after its one
+// iteration, or after a batch that leaves its delta at zero.  Iterations that
+// one block made end at an empty one, and those left of its batch would find
+// nothing either.
+static bool record(pra_scc* S, u32* b, const std::vector<u64>& rows)
+{
+    pra_ctx* c = S->ctx;
+    for (u64 n : rows) {
+        if (S->fixpoint && ++*b < c->batch_size) continue;
+        *b = 0;
+        S->hist.push_back(n);
+        if (!S->fixpoint || n == 0) return true;
+    }
+    if (*b == 0 || rows.back() != 0 || !S->ras[0].out->loops || S->ras.size() != 1) return false;
+    grp(c, S->group).iterations += c->batch_size - *b;
+    *b = 0;
+    S->hist.push_back(0);
+    return true;
+}
+
 // full -> delta at SCC start (src/relation/balanced_hash_relation.cpp:1152-1179)
 static void full_to_delta(pra_ctx* c, pra_rel* R)
 {
@@ -3952,6 +4199,9 @@ static void scc_begin(pra_scc* S, bool move_status)
         for (size_t i = 0; i < S->rels.size(); i++)
             if (S->status[i]) full_to_delta(c, S->rels[i]);
     S->running = true;
+    S->loop_stop = ~0ULL;
+    for (pra_rel* R : S->rels) R->loops = false;
+    if (RADesc* ra = c->loop_on ? loop_rule(S) : nullptr) ra->out->loops = true;
 }
 
 // one batch: a single iteration for an SCC that runs once, else batch_size
@@ -3977,7 +4227,7 @@ static void scc_end(pra_scc* S, bool check = true)
     for (pra_rel* R : S->rels) {
         delta_to_full(c, R);
         R->merged.release();
-        R->scc_changing = R->merge_full = R->full_read = false;
+        R->scc_changing = R->merge_full = R->full_read = R->loops = false;
     }
     if (check) sync_check(c);
     S->running = false;
@@ -3987,11 +4237,10 @@ static void scc_end(pra_scc* S, bool check = true)
 static void scc_run(pra_scc* S)
 {
     scc_begin(S, true);
-    if (!S->fixpoint)
-        scc_step(S);
-    else
-        while (scc_step(S) != 0) {
-        }
+    std::vector<std::vector<u64>> rows;
+    u32 b = 0;
+    do advance(S->ctx, {S}, PRA_LOOP_ITERS, rows);
+    while (!record(S, &b, rows[0]));
     scc_end(S);
 }
 
@@ -4015,7 +4264,8 @@ static pra_scc* one_runnable(pra_ctx* c, int g = -1)
 // progress, and each SCC records its batch and ends where its own LIE would:
 // after its one iteration, or after a batch that leaves its delta at zero.
 // Returns the instances with work left.
-static u64 lockstep_step(pra_ctx* c)
+// max > 1: an SCC that one block can run makes up to so many iterations.
+static u64 lockstep_step(pra_ctx* c, u32 max = 1)
 {
     std::vector<pra_scc*> members;
     for (size_t g = 0; g < c->groups.size(); g++) {
@@ -4030,18 +4280,14 @@ static u64 lockstep_step(pra_ctx* c)
         members.push_back(G.running);
     }
     if (members.empty()) return 0;
-    run_iteration(c, members);
+    std::vector<std::vector<u64>> rows;
+    advance(c, members, max, rows);
     u64 left = 0;
-    for (pra_scc* s : members) {
-        Group& G = grp(c, s->group);
-        if (!s->fixpoint || ++G.batch_it == c->batch_size) {
-            G.batch_it = 0;
-            const u64 d = delta_sum(s);
-            s->hist.push_back(d);
-            if (!s->fixpoint || d == 0) {
-                scc_end(s, false);
-                G.running = nullptr;
-            }
+    for (size_t k = 0; k < members.size(); k++) {
+        Group& G = grp(c, members[k]->group);
+        if (record(members[k], &G.batch_it, rows[k])) {
+            scc_end(members[k], false);
+            G.running = nullptr;
         }
     }
     for (size_t g = 0; g < c->groups.size(); g++)
@@ -4051,7 +4297,7 @@ static u64 lockstep_step(pra_ctx* c)
 
 static void execute_lockstep(pra_ctx* c)
 {
-    while (lockstep_step(c)) {
+    while (lockstep_step(c, PRA_LOOP_ITERS)) {
     }
     sync_check(c);
 }
@@ -4121,6 +4367,8 @@ int pra_ctx_create(int device, int nbuckets, uint64_t hbm_budget, pra_ctx** out)
         tune_init();
         const char* seg_env = getenv("PRA_SEG_SORT");             // "0": byte passes for newts over the bins
         c->seg_sort_on = !(seg_env && seg_env[0] == '0');
+        const char* loop_env = getenv("PRA_RANK_LOOP");
+        c->loop_on = !(loop_env && loop_env[0] == '0');
         const char* cap_env = getenv("PRA_SORT_TEST_BIN_CAP");
         c->bin_cap_test = cap_env ? strtoull(cap_env, nullptr, 10) : 0;
         const char* eb_env = getenv("PRA_DENSE_EPOCH_BITS");
@@ -4290,7 +4538,7 @@ int pra_ctx_group_status(pra_ctx* ctx, int group, int* done, uint64_t* iteration
         for (pra_rel* R : ctx->rels) {
             if (R->group != group) continue;
             for (auto& v : R->ver) b += v.buf.cap;
-            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->next_bnd, &R->merged, &R->dx, &R->nx,
+            for (const DBuf* d : {&R->mt, &R->bm, &R->dtab, &R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->places, &R->next_bnd, &R->merged, &R->dx, &R->nx,
                                   &R->rk_words[0], &R->rk_words[1], &R->rk_first[0], &R->rk_first[1], &R->idx[0], &R->idx[1], &R->nkeys, &R->kgofs,
                                   &R->bin_keys, &R->bin_idx, &R->bin_cur, &R->bnd[0], &R->bnd[1]})
                 b += d->cap;

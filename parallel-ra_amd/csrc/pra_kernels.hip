@@ -2943,6 +2943,423 @@ __global__ __launch_bounds__(PRA_PLACE_BLOCK) void k_rank_place(RankArgs a, u64*
     pra_rank_place_tile(a, status, t, epoch, flags);
 }
 
+// exclusive prefix of one value a thread over the block's SW waves; every wave
+// adds up the others' totals itself (two barriers)
+template <int SW>
+__device__ __forceinline__ u32 pra_block_prefix(u32 v, u32* lds, u32* total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    u32 x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const u32 y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) lds[wave] = x;
+    __syncthreads();
+    u32 w = lds[lane & (SW - 1)];
+#pragma unroll
+    for (int d = 1; d < SW; d <<= 1) {
+        const u32 y = __shfl_up(w, d, SW);
+        if ((lane & (SW - 1)) >= d) w += y;
+    }
+    *total = __shfl(w, SW - 1, SW);
+    const u32 before = wave ? __shfl(w, wave - 1, SW) : 0u;
+    __syncthreads();
+    return before + x - v;
+}
+
+// x = q * D + rest for x < 2^25: M = ceil(2^32 / D) puts the quotient at most
+// one too high (x * M / 2^32 < x / D + 2^-7)
+__device__ __forceinline__ u32 pra_split32(u32 x, u32 D, u32 M, u32* rest)
+{
+    u32 q = __umulhi(x, M), r = x - q * D;
+    if ((int)r < 0) {
+        q--;
+        r += D;
+    }
+    *rest = r;
+    return q;
+}
+
+// Whole iterations of a small ranked output that emits in digits from its own
+// delta, one after another, by one block: what k_rank_emit .. k_rank_place do,
+// with the delta's rank indexes, the candidates, the earliest arrivals and the
+// seq counters in LDS, so that an iteration has neither a launch nor a wait of
+// the host.  The loop ends at an empty iteration (the caller's fixed point),
+// after max_iters, or, with nothing of it done, before an iteration of more
+// than max_cand candidates, over the join threshold, or without room for its
+// rows; the general steps take that one.
+// A compute unit has one random access in flight after another (about three
+// cycles a lane), which bounds it, so a candidate costs two: it sets its bit
+// in the fresh bitmap without a look at the members, and finds its place in
+// `places`, a 64-bit word for each 32 bits of a dirty superblock (the bits that
+// are new, and their count before them).  One pass over the dirty superblocks
+// in between takes the members out, adds the new keys to them, clears the
+// fresh bits and leaves those words.  Digits are 32-bit here, and a row's
+// matches are spread over the block before anything is looked up.  New rows
+// are written in trie order, each iteration's after the last's, where the full
+// log will have them.
+// A closure of 1,000 vertices, 49 iterations of 3,700 rows and 4,400
+// candidates on average: 45 us an iteration by the general launches and the
+// readback, 24 us here (14 us of it the passes over bitmaps and `places`);
+// one of 40 vertices 45 against 9 us.
+__device__ __forceinline__ void pra_rank_loop(const LoopArgs& a)
+{
+    constexpr int SB = PRA_LOOP_BLOCK, SW = SB / 64, IT = PRA_LOOP_ROWS / SB, MLP = 4;
+    __shared__ u32 va[PRA_LOOP_ROWS];   // the delta's rank indexes; inner rows; earliest arrivals; the new rank indexes
+    __shared__ u32 vb[PRA_LOOP_ROWS];   // outer digits, then rank indexes of the candidates; the new rows' seq offsets
+    __shared__ u32 wh[SW][PRA_RADIX];
+    __shared__ u32 sbpre[PRA_LOOP_SBS];
+    __shared__ unsigned short list[PRA_LOOP_SBS];
+    __shared__ u32 dirty[PRA_LOOP_SBS / 32];
+    __shared__ u32 lds[SW], s_run[PRA_RADIX], s_nd;
+    __shared__ u64 s_seq[PRA_RADIX];
+    __shared__ unsigned char s_bucket[PRA_LOOP_LEADS];   // of each leading digit (several buckets)
+    const EmitArgs& em = a.emit;
+    const u32 t = threadIdx.x, nb = a.nb, D = (u32)a.D, M = 0xFFFFFFFFu / D + 1;
+    const int lane = t & 63, wave = t >> 6, kw = a.kw, wn = a.wn, ia = em.ia;
+    const u64 lt = pra_lanemask_lt();
+    const int dbits = nb > 1 ? 32 - __clz(nb - 1) : 0;
+    u64* const dx = (u64*)em.dx;
+    const u32* const first = em.first;
+    const u64 *const words = em.words, *const vals = a.vals, *const lead_vals = a.lead_vals;
+    const u32 *const rank_of = em.rank_of, *const lead_of = em.lead_of;
+    u32* const fresh = a.fresh;
+    u64* const places = a.places;
+    // what each digit of the outer row adds to an output's rank index: as it
+    // is, its leading digit as a rank, one of its ranks as a leading digit;
+    // and each column of the inner row
+    u32 wo[4] = {0, 0, 0, 0}, wrank = 0, wlead = 0, wi[4], ci[4];
+    int qlead = 0;
+    {
+        u32 w = 1;
+#pragma unroll
+        for (int c = 3; c >= 0; c--) {
+            wi[c] = 0;
+            ci[c] = 0;
+            if (c >= kw) continue;
+            const int q = em.col[c];
+            if (em.side[c] == 1) {
+                wi[c] = w;
+                ci[c] = q;
+            } else if (em.conv[c] == 1) {
+                wrank += w;
+            } else if (em.conv[c] == 2) {   // (of output column 0)
+                wlead = w;
+                qlead = q;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) wo[k] += q == k ? w : 0;
+            }
+            w *= D;
+        }
+    }
+    const bool inner_lead = a.by_bucket && wi[0];
+    u32 n = (u32)em.n, it = 0, cand = 0;
+    u64 written = 0, joined = 0;
+    bool too_many = false;
+    for (u32 r = t; r < n; r += SB) va[r] = (u32)dx[r];
+    for (u32 i = t; nb > 1 && i < D; i += SB) s_bucket[i] = a.bucket[i];
+    if (t < nb) {
+        s_seq[t] = a.seq[t];
+        s_run[t] = 0;
+    }
+    __syncthreads();
+    while (it < a.max_iters && n) {
+        // each row's inner run and the digits it gives: consecutive rows a
+        // thread, so that threads in order are rows in order
+        const u32 per = (n + SB - 1) / SB, r0 = t * per;
+        u32 base[IT], run[IT];   // run: first inner row, then in the top bits how many
+        u32 cnt = 0;
+#pragma unroll
+        for (int k0 = 0; k0 < IT; k0 += MLP) {
+            u32 f[MLP], e[MLP];
+#pragma unroll
+            for (int q = 0; q < MLP; q++) base[k0 + q] = run[k0 + q] = f[q] = e[q] = 0;
+            if ((u32)k0 >= per) continue;
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                // (past the last row: row 0 again, counted as none)
+                const bool in = (u32)(k0 + q) < per && r0 + k0 + q < n;
+                u32 digit[4] = {0, 0, 0, 0}, x = va[in ? r0 + k0 + q : 0];
+#pragma unroll
+                for (int c = 3; c > 0; c--)
+                    if (c < kw) x = pra_split32(x, D, M, &digit[c]);
+                digit[0] = x;
+                f[q] = first[x];
+                e[q] = first[in ? x + 1 : x];
+                u32 b = 0;
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (c < kw) b += digit[c] * wo[c];
+                if (wrank) b += rank_of[digit[0]] * wrank;
+                if (wlead) {
+                    const u32 d = qlead == 0 ? digit[0] : qlead == 1 ? digit[1] : qlead == 2 ? digit[2] : digit[3];
+                    b += lead_of[d] * wlead;
+                }
+                base[k0 + q] = b;
+            }
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                run[k0 + q] = f[q] | (e[q] - f[q]) << PRA_LOOP_RUN_SHIFT;
+                cnt += e[q] - f[q];
+            }
+        }
+        if (t < PRA_LOOP_SBS / 32) dirty[t] = 0;
+        if (t == 0) s_nd = 0;
+        u32 tot, p = pra_block_prefix<SW>(cnt, lds, &tot);
+        if (tot > a.max_cand || (long long)tot > em.thresh) {
+            too_many = true;
+            break;
+        }
+        if (written + tot > a.room) break;
+        // the candidates in arrival order: outer digits and inner row
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            if ((u32)k >= per) continue;
+            const u32 len = run[k] >> PRA_LOOP_RUN_SHIFT, i0 = run[k] & ((1u << PRA_LOOP_RUN_SHIFT) - 1);
+            for (u32 j = 0; j < len; j++, p++) {
+                va[p] = i0 + j;
+                vb[p] = base[k];
+            }
+        }
+        __syncthreads();
+        // claims: the candidates' bits
+        for (u32 p0 = t; p0 < tot; p0 += SB * MLP) {
+            u32 x[MLP];
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                const u32 pq = p0 + q * SB < tot ? p0 + q * SB : p0;   // (past the last: its own first again)
+                const u64* w = words + (u64)va[pq] * ia;
+                x[q] = vb[pq];
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (wi[c]) {
+                        const u64 e = w[ci[c]];
+                        x[q] += (c == 0 && inner_lead ? (u32)(e >> 32) : (u32)e - 1) * wi[c];
+                    }
+            }
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                const u32 pq = p0 + q * SB, sb = x[q] >> PRA_SB_BITS;
+                if (pq >= tot) continue;
+                __hip_atomic_fetch_or(fresh + (x[q] >> 5), 1u << (x[q] & 31), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (!(*(volatile u32*)(dirty + (sb >> 5)) >> (sb & 31) & 1)) atomicOr(dirty + (sb >> 5), 1u << (sb & 31));
+                va[pq] = ~0u;
+                vb[pq] = x[q];
+            }
+        }
+        __syncthreads();
+        // a wave to each dirty superblock, in four steps of whole lines: its
+        // new keys, into the members, and their places
+        if (t < a.sbs) {
+            sbpre[t] = 0;
+            if (dirty[t >> 5] >> (t & 31) & 1) list[atomicAdd(&s_nd, 1u)] = (unsigned short)t;
+        }
+        __syncthreads();
+        const u32 nd = s_nd;
+        for (u32 j = wave; j < nd; j += SW) {
+            const u32 sb = list[j];
+            uint4* const fw = (uint4*)fresh + (u64)sb * 256 + lane;
+            uint4* const mw = (uint4*)a.member + (u64)sb * 256 + lane;
+            uint4 v[4], m[4];
+            u32 c[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = fw[k * 64];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                c[k] = v[k].x | v[k].y | v[k].z | v[k].w;
+                m[k] = make_uint4(0, 0, 0, 0);
+                if (c[k]) m[k] = mw[k * 64];
+            }
+            u32 x01, x23;   // counts of the steps, two to a register: a step's 64 lanes hold at most 8,192 bits
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (c[k]) {
+                    fw[k * 64] = make_uint4(0, 0, 0, 0);
+                    v[k].x &= ~m[k].x;
+                    v[k].y &= ~m[k].y;
+                    v[k].z &= ~m[k].z;
+                    v[k].w &= ~m[k].w;
+                    mw[k * 64] = make_uint4(m[k].x | v[k].x, m[k].y | v[k].y, m[k].z | v[k].z, m[k].w | v[k].w);
+                }
+            }
+            u32 cnt4[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                cnt4[k] = (u32)(__popc(v[k].x) + __popc(v[k].y) + __popc(v[k].z) + __popc(v[k].w));
+            x01 = cnt4[0] | cnt4[1] << 16;
+            x23 = cnt4[2] | cnt4[3] << 16;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const u32 y01 = __shfl_up(x01, d, 64), y23 = __shfl_up(x23, d, 64);
+                if (lane >= d) {
+                    x01 += y01;
+                    x23 += y23;
+                }
+            }
+            const u32 t01 = __shfl(x01, 63, 64), t23 = __shfl(x23, 63, 64);
+            const u32 s1 = t01 & 0xFFFF, s2 = s1 + (t01 >> 16), s3 = s2 + (t23 & 0xFFFF);
+            const u32 o[4] = {(x01 & 0xFFFF) - cnt4[0], s1 + (x01 >> 16) - cnt4[1], s2 + (x23 & 0xFFFF) - cnt4[2],
+                              s3 + (x23 >> 16) - cnt4[3]};
+            uint4* const pw = (uint4*)places + ((u64)sb * 256 + lane) * 2;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (c[k]) {
+                    const u32 o1 = o[k] + (u32)__popc(v[k].x), o2 = o1 + (u32)__popc(v[k].y),
+                              o3 = o2 + (u32)__popc(v[k].z);
+                    pw[k * 128] = make_uint4(v[k].x, o[k], v[k].y, o1);
+                    pw[k * 128 + 1] = make_uint4(v[k].z, o2, v[k].w, o3);
+                }
+            if (lane == 0) sbpre[sb] = s3 + (t23 >> 16);
+        }
+        __syncthreads();
+        u32 fresh_rows;
+        const u32 sbex = pra_block_prefix<SW>(t < a.sbs ? sbpre[t] : 0u, lds, &fresh_rows);
+        if (t < a.sbs) sbpre[t] = sbex;
+        __syncthreads();
+        // the earliest arrival of each key: consecutive candidates a wave
+        const u32 items = (tot + SB - 1) / SB, p1 = (u32)wave * 64 * items + lane;
+        u32 xk[IT], pos[IT];
+#pragma unroll
+        for (int k0 = 0; k0 < IT; k0 += 2 * MLP) {
+            uint2 w[2 * MLP];
+#pragma unroll
+            for (int q = 0; q < 2 * MLP; q++) xk[k0 + q] = pos[k0 + q] = ~0u;
+            if ((u32)k0 >= items) continue;
+#pragma unroll
+            for (int q = 0; q < 2 * MLP; q++) {
+                w[q] = make_uint2(0, 0);
+                const u32 pk = p1 + (k0 + q) * 64;
+                if ((u32)(k0 + q) < items && pk < tot) {
+                    xk[k0 + q] = vb[pk];
+                    w[q] = ((const uint2*)places)[xk[k0 + q] >> 5];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 2 * MLP; q++) {
+                const u32 x = xk[k0 + q], bit = 1u << (x & 31);
+                if (w[q].x & bit) {   // (else a member, or no candidate)
+                    pos[k0 + q] = sbpre[x >> PRA_SB_BITS] + w[q].y + (u32)__popc(w[q].x & (bit - 1));
+                    atomicMin(va + pos[k0 + q], p1 + (k0 + q) * 64);
+                }
+            }
+        }
+        for (u32 i = lane; i < nb; i += 64) wh[wave][i] = 0;
+        __syncthreads();
+        // seq offsets of the kept candidates: per wave in arrival order, then
+        // over the waves
+        u32 dl[IT];   // bucket, and the kept candidates of it before this one in the wave
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            dl[k] = ~0u;
+            if ((u32)k >= items) continue;
+            if (pos[k] != ~0u && va[pos[k]] == p1 + k * 64) {
+                dl[k] = 0;
+                if (nb > 1) {
+                    u32 x = xk[k], rest;
+#pragma unroll
+                    for (int c = 3; c > 0; c--)
+                        if (c < kw) x = pra_split32(x, D, M, &rest);
+                    dl[k] = s_bucket[x];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            if ((u32)k >= items) continue;
+            const bool kept = dl[k] != ~0u;
+            u64 peers = __ballot(kept);
+            for (int b = 0; b < dbits; b++) {
+                const u64 set = __ballot(dl[k] >> b & 1);
+                peers &= dl[k] >> b & 1 ? set : ~set;
+            }
+            if (kept) {
+                const u32 d = dl[k], before = wh[wave][d];
+                dl[k] = d | (before + (u32)__popcll(peers & lt)) << 8;
+                if ((peers >> lane) == 1ULL) wh[wave][d] = before + (u32)__popcll(peers);
+            }
+        }
+        __syncthreads();
+        if (t < nb) {
+            u32 c[SW], acc = s_run[t];
+#pragma unroll
+            for (int v = 0; v < SW; v++) c[v] = wh[v][t];
+#pragma unroll
+            for (int v = 0; v < SW; v++) {
+                wh[v][t] = acc;
+                acc += c[v];
+            }
+            s_run[t] = acc;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < IT; k++)
+            if (dl[k] != ~0u) {
+                va[pos[k]] = xk[k];
+                vb[pos[k]] = wh[wave][dl[k] & 255] + (dl[k] >> 8);
+            }
+        __syncthreads();
+        // the new rows, in order
+        for (u32 rr = t; rr < fresh_rows; rr += SB * MLP) {
+            u32 lead[MLP];
+            u64 row[MLP][4];
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                const u32 r = rr + q * SB;
+                u32 y = va[r < fresh_rows ? r : 0];   // (past the last: row 0 again, not written)
+#pragma unroll
+                for (int c = 3; c > 0; c--)
+                    if (c < kw) {
+                        u32 d;
+                        y = pra_split32(y, D, M, &d);
+                        row[q][c] = vals[d];
+                    }
+                lead[q] = y;
+                row[q][0] = lead_vals[y];
+            }
+#pragma unroll
+            for (int q = 0; q < MLP; q++) {
+                const u32 r = rr + q * SB;
+                if (r >= fresh_rows) continue;
+                const u32 d = nb > 1 ? s_bucket[lead[q]] : 0;
+                u64* dst = a.rows + (written + r) * wn;
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (c < kw) dst[c] = row[q][c];
+                dst[kw] = ((u64)a.tag << 46) | ((u64)d << 28) | (s_seq[d] + vb[r]);
+            }
+        }
+        written += fresh_rows;
+        joined += tot;
+        cand = tot;
+        n = fresh_rows;
+        if (t == 0) ((u32*)(a.out + 4))[it] = n;
+        it++;
+    }
+    // the last iteration's rank indexes are in `va`
+    __syncthreads();
+    if (it)
+        for (u32 r = t; r < n; r += SB) dx[r] = va[r];
+    if (t < nb) a.seq[t] = s_seq[t] + s_run[t];
+    if (t == 0) {
+        a.out[0] = it;
+        a.out[1] = written;
+        a.out[2] = n;
+        a.out[3] = (u64)too_many << 32 | cand;
+        if (joined) atomicAdd((unsigned long long*)em.joined, (unsigned long long)joined);
+    }
+    if (!a.host) return;
+    __syncthreads();
+    if (t == 0) a.host[a.host_words] = *a.err;
+    pra_publish_words(a.out, 4 + (it + 1) / 2, a.err, a.host, a.host_seq);
+}
+
+__global__ __launch_bounds__(PRA_LOOP_BLOCK) void k_rank_loop(LoopArgs a) { pra_rank_loop(a); }
+__global__ __launch_bounds__(PRA_LOOP_BLOCK) void k_rank_loop_many(const LoopArgs* jobs) { pra_rank_loop(jobs[blockIdx.x]); }
+
 // Several outputs in one launch each: `jobs` (device memory) holds njobs
 // RankArgs, then five tables of njobs + 1 first blocks, one a step (outputs
 // that emit have no claim blocks, the others no emission tiles).
@@ -4207,6 +4624,16 @@ void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* 
         hipLaunchKernelGGL(k_rank_place, dim3(pra_tiles(cap)), dim3(PRA_PLACE_BLOCK), 0, st, a, status, ctr, epoch,
                            flags);
     }
+}
+
+void pra_launch_rank_loop(hipStream_t st, const LoopArgs& a)
+{
+    hipLaunchKernelGGL(k_rank_loop, dim3(1), dim3(PRA_LOOP_BLOCK), 0, st, a);
+}
+
+void pra_launch_rank_loop_many(hipStream_t st, const LoopArgs* jobs, int njobs)
+{
+    hipLaunchKernelGGL(k_rank_loop_many, dim3(njobs), dim3(PRA_LOOP_BLOCK), 0, st, jobs);
 }
 
 void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,

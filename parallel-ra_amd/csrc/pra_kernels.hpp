@@ -271,6 +271,38 @@ void pra_launch_rank(hipStream_t st, int step, const RankArgs& a, u64 cap, u64* 
 void pra_launch_rank_many(hipStream_t st, int step, const RankArgs* jobs, int njobs, u32 blocks, u64* status, u32* ctr,
                           u32 epoch, u32* flags);
 
+// Iterations of a ranked output by one block each (k_rank_loop): up to
+// PRA_LOOP_ROWS delta rows and candidates an iteration, rank spaces of up to
+// PRA_LOOP_SBS superblocks.
+#define PRA_LOOP_BLOCK 1024
+#define PRA_LOOP_ROWS 16384
+#define PRA_LOOP_SBS 1024
+#define PRA_LOOP_ITERS 256   // iterations a launch
+#define PRA_LOOP_LEADS 5824  // leading digits with a bucket
+#define PRA_LOOP_RUN_SHIFT 26   // inner rows < 2^26, runs of less than 64
+struct LoopArgs {
+    EmitArgs emit;          // dx: the delta's rank indexes, overwritten by the last iteration's; n: its rows
+    const u64 *vals, *lead_vals;
+    const unsigned char* bucket;   // of each leading digit (several buckets)
+    u32 *member, *fresh;
+    u64* places;            // per 32 bits of a dirty superblock: its new bits, and (above) their count before them
+    u64* rows;              // the new rows of one iteration after another, `room` of them
+    u64* seq;               // per-bucket seq counters, advanced in place
+    u64* out;               // PRA_LOOP_OUT words: iterations, rows written, rows of the last, its candidates (and
+                            // bit 32: the next iteration is not for one block), then the new rows of each, two a word
+    u64* host;              // the results go to the host from here (null: they do not)
+    u64 host_seq;
+    const u32* err;
+    u64 D, room;
+    double inv;
+    u32 host_words;         // where the error flags go
+    u32 sbs, nb, tag, max_iters, max_cand;
+    int kw, wn, by_bucket;
+};
+#define PRA_LOOP_OUT (4 + PRA_LOOP_ITERS / 2)
+void pra_launch_rank_loop(hipStream_t st, const LoopArgs& a);
+void pra_launch_rank_loop_many(hipStream_t st, const LoopArgs* jobs, int njobs);
+
 // job tables (device memory) of the batched launches of a lock-step iteration
 struct BinSortJob {
     const u64* bin_keys;
