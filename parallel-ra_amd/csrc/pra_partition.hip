@@ -91,10 +91,14 @@ __global__ __launch_bounds__(kScanBlock) void k_part_scan(u32* __restrict__ H, u
 // lane's own row would touch several.  Tiles run from the last one back: the
 // rows the histogram read last are still in the last-level cache.
 // W: the row width, 0 = any (w).  NT: non-temporal stores.
-// 24 M rows of 3 words into 8 buckets: 488 -> 377 us; 12 M rows of 6 words into
-// 64: 738 -> 463; 30 M of 2 into 200: 801 -> 561, into 3: 361 -> 346.  With
-// the histogram's read these move 24 bytes a word at 4.6 TB/s of the card's
-// copy rate, so 375 us is the first one's bound.
+// Whole partitions, a lane to each row's words / this without the prefetch /
+// with it: 24 M rows of 3 words into 8 buckets 482 / 360 / 343 us, 12 M of 6
+// into 64 739 / 463 / 419, 30 M of 2 into 200 800 / 560 / 558, into 3 359 / 345
+// / 327, 300,000 of 5 into 3 42.4 / 45.4 / 39.9, 1 M of 3 into 200 34.3 / 35.4
+// / 31.9.  Large ones are bound by memory (the histogram reads every line, the
+// scatter again: 24 bytes a word), those of less than a few tiles a compute
+// unit by a tile's own chain of loads, ranks and stores, which the prefetch
+// shortens.
 // NT against plain stores: 377 / 402 us (8 buckets, runs of 1.5 KB), 483 / 463
 // (64, 384 bytes), 854 / 561 (200, 41 bytes): kStreamRun lies in between.
 template <int W, int SUB, bool NT>
@@ -136,13 +140,34 @@ __global__ __launch_bounds__(kPartBlock) void k_part_scatter(const u64* __restri
     next[tid] = tid < nb ? st + H[(u64)tid * ntiles + tile] : 0;
     const u64 t0 = (u64)tile * PRA_PART_TILE;
     const u32 trows = (u32)min((u64)PRA_PART_TILE, n - t0);
+    // of a known width, the next sub-tile's words are loaded while this one's
+    // rows are ranked and written
+    constexpr int PF = W ? SUB * W / kPartBlock : 1;
+    u64 pre[PF];
+    auto fetch = [&](u32 s0) {
+        const u32 words = s0 < trows ? min((u32)SUB, trows - s0) * W : 0;
+        const u64* src = rows + (t0 + s0) * W;
+#pragma unroll
+        for (int k = 0; k < PF; k++) {
+            const u32 i = tid + k * kPartBlock;
+            pre[k] = i < words ? src[i] : 0;
+        }
+    };
+    if (W) fetch(0);
     for (u32 s0 = 0; s0 < trows; s0 += SUB) {
         const u32 m = min((u32)SUB, trows - s0);
-        const u64* src = rows + (t0 + s0) * (u64)w;
-        for (u32 i = tid; i < m * w; i += kPartBlock) stage[i] = src[i];
+        if (W) {
+#pragma unroll
+            for (int k = 0; k < PF; k++)
+                if (tid + k * kPartBlock < m * W) stage[tid + k * kPartBlock] = pre[k];
+        } else {
+            const u64* src = rows + (t0 + s0) * (u64)w;
+            for (u32 i = tid; i < m * w; i += kPartBlock) stage[i] = src[i];
+        }
 #pragma unroll
         for (int q = 0; q < PRA_WAVES; q++) wc[q][tid] = 0;
         __syncthreads();
+        if (W) fetch(s0 + SUB);
         // rows in input order: wave v holds rows [v * 64 * IT, (v + 1) * 64 * IT)
         u32 b[IT], rank[IT];
 #pragma unroll
@@ -245,6 +270,8 @@ void pra_launch_partition(hipStream_t st, const u64* rows, u64 n, int w, int jcc
     case 2: launch_scatter<2, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
     case 3: launch_scatter<3, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
     case 4: launch_scatter<4, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    case 5: launch_scatter<5, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
+    case 6: launch_scatter<6, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds); break;
     default:
         if (w <= 8)
             launch_scatter<0, 512>(st, rows, n, w, jcc, nb, H, T, ntiles, out, bounds);
