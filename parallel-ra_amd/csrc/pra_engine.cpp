@@ -3977,17 +3977,20 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         LoopArgs a;
         memset(&a, 0, sizeof(a));
         // room for what the rank space can still hold, or as much again twice
-        // over; an iteration stops by its candidates, so their most on top
+        // over (once under a budget, as the appends' growth would); an
+        // iteration stops by its candidates, so their most on top
         u64 bits = 1;
         for (int i = 0; i < R->arity; i++) bits *= G.dict_n;
         const u64 have = F.n + D.n;
-        a.room = std::min<u64>(bits - std::min(bits, have), std::max<u64>(1 << 18, 2 * have)) + PRA_LOOP_ROWS;
+        a.room = std::min<u64>(bits - std::min(bits, have), c->budget ? have : std::max<u64>(1 << 18, 2 * have)) + PRA_LOOP_ROWS;
         try {
             F.buf.reserve((have + a.room) * R->w * 8, c->st, (size_t)F.n * R->w * 8);
             R->dx.reserve(PRA_LOOP_ROWS * 8, c->st, D.n * 8);
             R->places.reserve((R->sbs_use << (PRA_SB_BITS - 5)) * 8, c->st);
         } catch (const PraError& e) {
             if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+            R->places.release();
+            sccs[k]->loop_stop = 0;   // the general launches from here on
             continue;
         }
         appends.push_back(CopyJob{D.d(), F.d() + F.n * R->w, D.n * (u64)R->w});
