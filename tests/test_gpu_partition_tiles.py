@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n", [1, 511, 512, 513, 2047, 2049, 5000])
-@pytest.mark.parametrize("w,jcc,k", [(1, 1, 2), (2, 1, 200), (3, 1, 3), (4, 2, 8), (5, 3, 64), (9, 2, 7), (32, 4, 256)])
+@pytest.mark.parametrize("w,jcc,k", [(1, 1, 2), (2, 1, 200), (3, 1, 3), (4, 2, 8), (5, 3, 64), (6, 1, 64), (8, 2, 13), (9, 2, 7), (32, 4, 256)])
 def test_widths(w, jcc, k, n):
     import pra_amd
     print("case", n, w, jcc, k, flush=True)
