@@ -1932,35 +1932,64 @@ static void ensure_index(pra_ctx* c, pra_rel* R, int v)
     R->idx_valid[v] = true;
 }
 
-// The dictionary words of a sorted version's columns and the first row of each
-// leading digit, for emissions in digits.  False when a value has no rank or
-// there is no room for 8 bytes a column.
-static bool ensure_rank_rows(pra_ctx* c, pra_rel* R, int v)
+// The dictionary words of sorted versions' columns and the first row of each
+// leading digit, for emissions in digits, where they are missing.  A version
+// stays without (rk_gen) when a value has no rank or there is no room for 8
+// bytes a column.  One launch and one wait for all of them.
+static void ensure_rank_rows(pra_ctx* c, const std::vector<std::pair<pra_rel*, int>>& versions)
 {
-    const Group& G = grp(c, R->group);
-    Rows& r = R->ver[v];
-    if (R->rk_gen[v] == G.dict_gen) return true;
-    if (R->rk_no[v] || R->jcc != 1 || !r.sorted || r.n >= (1ULL << 32)) return false;
-    try {
-        R->rk_words[v].reserve(r.n * (u64)R->arity * 8, c->st);
-        R->rk_first[v].reserve((G.dict_n + 1) * 4, c->st);
-    } catch (const PraError& e) {
-        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
-        R->rk_words[v].release();
-        R->rk_no[v] = true;
-        return false;
+    std::vector<std::pair<pra_rel*, int>> made;
+    for (auto& rv : versions) {
+        pra_rel* R = rv.first;
+        const int v = rv.second;
+        const Group& G = grp(c, R->group);
+        Rows& r = R->ver[v];
+        if (R->rk_gen[v] == G.dict_gen || R->rk_no[v] || R->jcc != 1 || !r.sorted || r.n >= (1ULL << 32) ||
+            std::find(made.begin(), made.end(), rv) != made.end())
+            continue;
+        try {
+            R->rk_words[v].reserve(r.n * (u64)R->arity * 8, c->st);
+            R->rk_first[v].reserve((G.dict_n + 1) * 4, c->st);
+        } catch (const PraError& e) {
+            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+            R->rk_words[v].release();
+            R->rk_no[v] = true;
+            continue;
+        }
+        made.push_back(rv);
     }
-    c->orand.reserve(32 * 8, c->st);
-    pra_launch_fill_u64(c->st, c->orand.as<u64>(), 1, 0);
-    pra_launch_rank_rows(c->st, r.d(), r.n, R->w, R->arity, G.dict.as<u64>(), G.dict_cap, G.dict_n, c->nb > 1,
-                         R->rk_words[v].as<u64>(), R->rk_first[v].as<u32>(), c->orand.as<u64>());
+    if (made.empty()) return;
+    c->orand.reserve(std::max<size_t>(32, made.size()) * 8, c->st);
+    pra_launch_fill_u64(c->st, c->orand.as<u64>(), made.size(), 0);
+    const size_t n = made.size();
+    std::vector<char> table(n * sizeof(RankRowsArgs) + (n + 1) * 4);
+    RankRowsArgs* jobs = (RankRowsArgs*)table.data();
+    u32* base = (u32*)(jobs + n);
+    base[0] = 0;
+    for (size_t k = 0; k < n; k++) {
+        pra_rel* R = made[k].first;
+        const int v = made[k].second;
+        const Group& G = grp(c, R->group);
+        Rows& r = R->ver[v];
+        jobs[k] = RankRowsArgs{r.d(), G.dict.as<u64>(), r.n, G.dict_cap, G.dict_n, R->rk_words[v].as<u64>(),
+                               R->rk_first[v].as<u32>(), c->orand.as<u64>() + k, R->w, R->arity, c->nb > 1};
+        base[k + 1] = base[k] + (u32)((r.n + PRA_BLOCK - 1) / PRA_BLOCK);
+    }
+    if (n == 1)
+        pra_launch_rank_rows(c->st, jobs[0]);
+    else
+        pra_launch_rank_rows_many(c->st, (const RankRowsArgs*)stage_table(c, JOB_SETUP, table.data(), table.size()),
+                                  (int)n, base[n]);
     check_launch("rank_rows");
-    if (readback(c, c->orand.p, 1)[0]) {
-        R->rk_no[v] = true;
-        return false;
+    const u64* missing = readback(c, c->orand.p, made.size());
+    for (size_t k = 0; k < made.size(); k++) {
+        pra_rel* R = made[k].first;
+        const int v = made[k].second;
+        if (missing[k])
+            R->rk_no[v] = true;
+        else
+            R->rk_gen[v] = grp(c, R->group).dict_gen;
     }
-    R->rk_gen[v] = G.dict_gen;
-    return true;
 }
 
 // membership table of full u delta keyed on kw leading columns, with room for
@@ -2756,7 +2785,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     // than kEmitRun inner rows take the expansion that balances outputs.
     // -1: none.
     std::vector<char> emit_off(no, 0);
-    auto emit_rule_of = [&](size_t oi) {
+    auto emit_shape = [&](size_t oi) {   // but for the inner rows' ranks
+
         pra_rel* R = outs[oi];
         if (emit_off[oi] || !bits_in_trie_order(c, R)) return -1;
         int rule = -1;
@@ -2772,8 +2802,17 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             ra.outer->jcc != 1 || ra.inner->jcc != 1 || ra.outer->arity > 4 || ra.inner->view_of || ra.outer->view_of ||
             ra.inner->idx_maxlen[ra.inner_v] > kEmitRun || ra.n_outer >= (1ULL << 32))
             return -1;
-        if (!projects_data(ra)) return -1;   // an intern id
-        return ensure_rank_rows(c, ra.inner, ra.inner_v) ? rule : -1;
+        return projects_data(ra) ? rule : -1;   // no intern id
+    };
+    auto emit_ranked = [&](size_t oi, int rule) {
+        const RADesc& ra = S->ras[rule];
+        return ra.inner->rk_gen[ra.inner_v] == grp(c, outs[oi]->group).dict_gen ? rule : -1;
+    };
+    auto emit_rule_of = [&](size_t oi) {
+        const int rule = emit_shape(oi);
+        if (rule < 0) return -1;
+        ensure_rank_rows(c, {{S->ras[rule].inner, S->ras[rule].inner_v}});
+        return emit_ranked(oi, rule);
     };
     // taken per output; the rule an output emits (-1: the general expansions);
     // an emission that stopped left fresh bits that only another would set
@@ -2787,11 +2826,17 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
         }
     }
+    std::vector<std::pair<pra_rel*, int>> to_rank;
     for (size_t oi = 0; oi < no; oi++) {
         if (!cap[oi]) continue;
         choice[oi] = decide(oi, cap[oi], nactive >= 2 ? 1 : 0, reg[oi].rb);
-        if (choice[oi].mode == 2) emit_rule[oi] = emit_rule_of(oi);
+        if (choice[oi].mode != 2) continue;
+        emit_rule[oi] = emit_shape(oi);
+        if (emit_rule[oi] >= 0) to_rank.push_back({S->ras[emit_rule[oi]].inner, S->ras[emit_rule[oi]].inner_v});
     }
+    ensure_rank_rows(c, to_rank);
+    for (size_t oi = 0; oi < no; oi++)
+        if (emit_rule[oi] >= 0) emit_rule[oi] = emit_ranked(oi, emit_rule[oi]);
 
     // 2. per-RA output counts and their exclusive offsets (the arrival plan
     //    reads them at the source-bucket bounds); an output that emits in

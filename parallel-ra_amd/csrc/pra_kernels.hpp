@@ -493,8 +493,18 @@ void pra_launch_dict_bucket_rank(hipStream_t st, const u64* vals, u64 n, u64* ta
                                  u64 nb, unsigned char* bucket);
 // the dictionary words of rows' first a columns and the first row of every
 // leading digit (k_rank_rows)
-void pra_launch_rank_rows(hipStream_t st, const u64* rows, u64 n, int w, int a, const u64* dict, u64 dict_cap, u64 D,
-                          int by_bucket, u64* words, u32* first, u64* miss);
+struct RankRowsArgs {
+    const u64 *rows, *dict;
+    u64 n, dict_cap, D;
+    u64* words;
+    u32* first;
+    u64* miss;
+    int w, a, by_bucket;
+};
+void pra_launch_rank_rows(hipStream_t st, const RankRowsArgs& a);
+// jobs (device) = njobs RankRowsArgs, then njobs + 1 first blocks of PRA_BLOCK
+// rows; `blocks` = the last of them
+void pra_launch_rank_rows_many(hipStream_t st, const RankRowsArgs* jobs, int njobs, u32 blocks);
 void pra_launch_gather_rows(hipStream_t st, const u64* in, const u32* idx, u64 n, int w, u64* out);
 void pra_launch_key_bounds(hipStream_t st, const u64* keys, u64 n, u64 bmul, int ls, u64 nb, u64* bnd);
 // Keyed row sort of more rows than one block holds: word 0 of every row's key
