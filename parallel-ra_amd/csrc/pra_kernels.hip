@@ -1518,8 +1518,8 @@ __device__ inline int pra_row_cmp(const u64* a, const u64* b, int n)
     return 0;
 }
 
-// First row of the sorted rows [a, z) whose first n columns are >= key (upper:
-// > key).  Three probes a step, their loads in flight together, so a search
+// First row of the sorted rows [a, z) whose first n > 0 columns are >= key
+// (upper: > key).  Three probes a step, their loads in flight together, so a search
 // takes half the dependent loads of a binary one; rows that differ from the
 // key in column 0 need no more than that.  With one row a thread and runs
 // found by four parallel compares, the points-to analysis' counts took 21 us a
@@ -1565,6 +1565,10 @@ __device__ inline u64 pra_sorted_run(const u64* key, int jcc, const u64* inner, 
 {
     u64 b = nb == 1 ? 0 : pra_bucket(pra_fnv(key, jcc), nb);
     u64 lo = ibnd[b], hi = ibnd[b + 1];
+    if (jcc == 0) {   // every row matches
+        *first_out = lo;
+        return hi - lo;
+    }
     const u64 first = pra_row_bound(inner, wi, key, jcc, lo, hi, false);   // first row >= key
     // first row > key: most runs end within four rows, whose loads go out
     // together; the others are searched for
