@@ -4163,7 +4163,7 @@ static bool record(pra_scc* S, u32* b, const std::vector<u64>& rows)
         S->hist.push_back(n);
         if (!S->fixpoint || n == 0) return true;
     }
-    if (*b == 0 || rows.back() != 0 || !S->ras[0].out->loops || S->ras.size() != 1) return false;
+    if (*b == 0 || rows.back() != 0 || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
     grp(c, S->group).iterations += c->batch_size - *b;
     *b = 0;
     S->hist.push_back(0);
