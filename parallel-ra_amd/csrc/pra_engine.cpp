@@ -4151,10 +4151,11 @@ static void advance(pra_ctx* c, const std::vector<pra_scc*>& members, u32 max, s
 
 // The batches that some iterations of S complete, *b of whose current batch
 // are made: records the delta after each.  True when S ends: after its one
-// iteration, or after a batch that leaves its delta at zero.  Iterations that
-// one block made end at an empty one, and those left of its batch would find
+// iteration, or after a batch that leaves its delta at zero.  With `whole`
+// (the caller takes more than one iteration at a time) an empty iteration ends
+// the batch of an SCC that one block can run: those left of it would find
 // nothing either.
-static bool record(pra_scc* S, u32* b, const std::vector<u64>& rows)
+static bool record(pra_scc* S, u32* b, const std::vector<u64>& rows, bool whole)
 {
     pra_ctx* c = S->ctx;
     for (u64 n : rows) {
@@ -4163,7 +4164,7 @@ static bool record(pra_scc* S, u32* b, const std::vector<u64>& rows)
         S->hist.push_back(n);
         if (!S->fixpoint || n == 0) return true;
     }
-    if (*b == 0 || rows.back() != 0 || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
+    if (!whole || *b == 0 || rows.back() != 0 || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
     grp(c, S->group).iterations += c->batch_size - *b;
     *b = 0;
     S->hist.push_back(0);
@@ -4288,7 +4289,7 @@ static void scc_run(pra_scc* S)
     std::vector<std::vector<u64>> rows;
     u32 b = 0;
     do advance(S->ctx, {S}, PRA_LOOP_ITERS, rows);
-    while (!record(S, &b, rows[0]));
+    while (!record(S, &b, rows[0], true));
     scc_end(S);
 }
 
@@ -4333,7 +4334,7 @@ static u64 lockstep_step(pra_ctx* c, u32 max = 1)
     u64 left = 0;
     for (size_t k = 0; k < members.size(); k++) {
         Group& G = grp(c, members[k]->group);
-        if (record(members[k], &G.batch_it, rows[k])) {
+        if (record(members[k], &G.batch_it, rows[k], max > 1)) {
             scc_end(members[k], false);
             G.running = nullptr;
         }
