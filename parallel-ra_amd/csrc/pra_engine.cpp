@@ -76,14 +76,24 @@ void hip_block_free(void* p, void*) { (void)hipFree(p); }
 const pra::BlockAllocator kHipBlocks{hip_block_alloc, hip_block_free, nullptr};
 
 // Device bytes held by each context, keyed by its stream (every buffer of a
-// context is ordered on the context's stream): live bytes, their peak, and the
-// context's cap (0 = none).
+// context is ordered on the context's stream): live bytes, their peak, the
+// context's cap (0 = none), and the stream's device.
 struct MemAcct {
     long long live = 0, peak = 0;
     u64 budget = 0;
+    int device = 0;
 };
 std::mutex g_acct_mu;
 std::map<hipStream_t, MemAcct> g_acct;
+
+// the device whose memory a stream's buffers are in; the calling thread's
+// current device may be another one
+int stream_device(hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(g_acct_mu);
+    auto it = g_acct.find(s);
+    return it == g_acct.end() ? 0 : it->second.device;
+}
 
 // charge `bytes` more to the context of stream s (fails past its budget while
 // `check`), or credit them back when negative
@@ -111,8 +121,7 @@ void small_idle_flush(int dev, hipStream_t st);
 
 void* big_get(size_t bytes, hipStream_t st, size_t* got)
 {
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
+    const int dev = stream_device(st);
     void* p = g_big.get(dev, st, bytes, got, kHipBlocks);
     if (!p) {
         small_idle_flush(dev, st);
@@ -128,9 +137,7 @@ void* big_get(size_t bytes, hipStream_t st, size_t* got)
 
 void big_put(void* p, size_t size, hipStream_t st)
 {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    g_big.put(dev, st, p, size);
+    g_big.put(stream_device(st), st, p, size);
 }
 
 // every piece of work enqueued on st so far has completed
@@ -187,8 +194,7 @@ size_t small_class(size_t bytes)
 
 void* small_take(hipStream_t st, size_t cls)
 {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
+    const int dev = stream_device(st);
     std::lock_guard<std::mutex> lk(g_small_mu);
     auto it = g_small.find(st);
     void* p = it == g_small.end() ? nullptr : it->second.take(cls);
@@ -223,9 +229,7 @@ void small_idle_flush(int dev, hipStream_t st)
 // free the small blocks kept for a stream and the device's idle ones, on it
 void small_flush(hipStream_t st)
 {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    small_idle_flush(dev, st);
+    small_idle_flush(stream_device(st), st);
     SmallFree f;
     {
         std::lock_guard<std::mutex> lk(g_small_mu);
@@ -243,8 +247,7 @@ void small_flush(hipStream_t st)
 // the same to free and to make again whatever its size.
 void small_retire(hipStream_t st)
 {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
+    const int dev = stream_device(st);
     const size_t limit = g_small_idle_limit;
     std::vector<void*> drop;
     {
@@ -464,9 +467,8 @@ struct DBuf {
                 np = big_get(want, s, &nc);
                 acct_charge(s, (long long)nc - (long long)want, false);   // a cached block of the next class
             } else if (!(np = small_take(s, nc)) && hipMallocAsync(&np, nc, s) != hipSuccess) {
-                int dev = 0;
+                const int dev = stream_device(s);
                 (void)hipGetLastError();
-                HIPCHK(hipGetDevice(&dev));
                 small_flush(s);
                 g_big.flush(dev, kHipBlocks, nc);
                 if (hipMallocAsync(&np, nc, s) != hipSuccess) {
@@ -4357,9 +4359,34 @@ static int fail(pra_ctx* c, int code, const std::string& m)
     return code;
 }
 
+// The context's device is the current one inside a call (allocations and
+// launches go by it).  API_BEGIN puts the caller's back at its end; the calls
+// that run programs or move an exchange's rows (API_BEGIN_ON) leave the
+// context's current.
+struct DeviceScope {
+    int prev = -1;
+    explicit DeviceScope(int device)
+    {
+        int cur = 0;
+        HIPCHK(hipGetDevice(&cur));
+        if (cur == device) return;
+        HIPCHK(hipSetDevice(device));
+        prev = cur;
+    }
+    ~DeviceScope()
+    {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+};
+
 #define API_BEGIN(ctxexpr)                                                                         \
     pra_ctx* ctx_ = (ctxexpr);                                                                     \
-    try {
+    try {                                                                                          \
+        DeviceScope device_scope_(ctx_->device);
+#define API_BEGIN_ON(ctxexpr)                                                                      \
+    pra_ctx* ctx_ = (ctxexpr);                                                                     \
+    try {                                                                                          \
+        HIPCHK(hipSetDevice(ctx_->device));
 #define API_END                                                                                    \
     }                                                                                              \
     catch (const PraError& e) { return fail(ctx_, e.code, e.what()); }                           \
@@ -4404,7 +4431,9 @@ int pra_ctx_create(int device, int nbuckets, uint64_t hbm_budget, pra_ctx** out)
         c->st = stream_get(device);
         {
             std::lock_guard<std::mutex> lk(g_acct_mu);
-            g_acct[c->st].budget = hbm_budget;
+            MemAcct& a = g_acct[c->st];
+            a.budget = hbm_budget;
+            a.device = device;
         }
         c->nb = nbuckets;
         c->budget = hbm_budget;
@@ -4522,8 +4551,7 @@ int pra_partition_rows(pra_ctx* ctx, const uint64_t* rows, uint64_t n, uint32_t 
 {
     const int rc = partition_args(ctx, rows, n, w, jcc, out_rows, bucket_bounds);
     if (rc != PRA_OK) return rc;
-    API_BEGIN(ctx)
-    HIPCHK(hipSetDevice(ctx->device));
+    API_BEGIN_ON(ctx)
     ctx->part_scratch.reserve(pra_partition_scratch_words(n, (u32)ctx->nb) * 4 + 256, ctx->st);
     pra_launch_partition(ctx->st, rows, n, (int)w, (int)jcc, (u32)ctx->nb, out_rows, bucket_bounds,
                          ctx->part_scratch.as<u32>());
@@ -4539,8 +4567,7 @@ int pra_partition_rows_noalloc(pra_ctx* ctx, const uint64_t* rows, uint64_t n, u
                                         " rows, got " + std::to_string(n));
     const int rc = partition_args(ctx, rows, n, w, jcc, out_rows, bucket_bounds);
     if (rc != PRA_OK) return rc;
-    API_BEGIN(ctx)
-    HIPCHK(hipSetDevice(ctx->device));
+    API_BEGIN_ON(ctx)
     u32* scratch = pra_partition_scratch(ctx->device);
     if (!scratch) throw PraError(PRA_E_STATE, "allocation-free scratch of this device was not set up");
     pra_launch_partition(ctx->st, rows, n, (int)w, (int)jcc, (u32)ctx->nb, out_rows, bucket_bounds, scratch);
@@ -4569,8 +4596,7 @@ int pra_ctx_group_joined(pra_ctx* ctx, int group, uint64_t* out)
 int pra_ctx_step(pra_ctx* ctx, uint64_t* active)
 {
     if (!ctx || !active) return PRA_E_ARG;
-    API_BEGIN(ctx)
-    HIPCHK(hipSetDevice(ctx->device));
+    API_BEGIN_ON(ctx)
     *active = lockstep_step(ctx);
     if (!*active) sync_check(ctx);
     API_END
@@ -4639,8 +4665,7 @@ int pra_autotune_report(char* buf, uint64_t cap, uint64_t* len)
 int pra_ctx_trim(pra_ctx* ctx)
 {
     if (!ctx) return PRA_E_ARG;
-    API_BEGIN(ctx)
-    HIPCHK(hipSetDevice(ctx->device));
+    API_BEGIN_ON(ctx)
     // written before they are read inside every iteration that uses them;
     // released on the context's stream, so reuse stays ordered behind the
     // work already enqueued
@@ -4959,8 +4984,7 @@ int pra_scc_add_dependency(pra_scc* before, pra_scc* after)
 int pra_scc_run(pra_scc* scc, uint64_t* delta_hist, uint64_t cap, uint64_t* nbatches)
 {
     if (!scc) return PRA_E_ARG;
-    API_BEGIN(scc->ctx)
-    HIPCHK(hipSetDevice(scc->ctx->device));
+    API_BEGIN_ON(scc->ctx)
     size_t before = scc->hist.size();
     scc_run(scc);
     size_t nb = scc->hist.size() - before;
@@ -4972,8 +4996,7 @@ int pra_scc_run(pra_scc* scc, uint64_t* delta_hist, uint64_t cap, uint64_t* nbat
 int pra_scc_begin(pra_scc* scc, int move_full_to_delta)
 {
     if (!scc) return PRA_E_ARG;
-    API_BEGIN(scc->ctx)
-    HIPCHK(hipSetDevice(scc->ctx->device));
+    API_BEGIN_ON(scc->ctx)
     scc_begin(scc, move_full_to_delta != 0);
     API_END
 }
@@ -4981,8 +5004,7 @@ int pra_scc_begin(pra_scc* scc, int move_full_to_delta)
 int pra_scc_step(pra_scc* scc, uint64_t* delta)
 {
     if (!scc) return PRA_E_ARG;
-    API_BEGIN(scc->ctx)
-    HIPCHK(hipSetDevice(scc->ctx->device));
+    API_BEGIN_ON(scc->ctx)
     u64 d = scc_step(scc);
     if (delta) *delta = d;
     API_END
@@ -4991,8 +5013,7 @@ int pra_scc_step(pra_scc* scc, uint64_t* delta)
 int pra_scc_end(pra_scc* scc)
 {
     if (!scc) return PRA_E_ARG;
-    API_BEGIN(scc->ctx)
-    HIPCHK(hipSetDevice(scc->ctx->device));
+    API_BEGIN_ON(scc->ctx)
     scc_end(scc);
     API_END
 }
@@ -5008,8 +5029,7 @@ int pra_scc_history(pra_scc* scc, uint64_t* out, uint64_t cap, uint64_t* n)
 int pra_execute(pra_ctx* ctx)
 {
     if (!ctx) return PRA_E_ARG;
-    API_BEGIN(ctx)
-    HIPCHK(hipSetDevice(ctx->device));
+    API_BEGIN_ON(ctx)
     if (ctx->groups.size() > 1) {
         execute_lockstep(ctx);
     } else {
