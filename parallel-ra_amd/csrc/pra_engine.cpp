@@ -953,13 +953,20 @@ struct ProfPerCand {
     }
 };
 
+// room for a job table of up to `bytes`
+static char* reserve_table(pra_ctx* c, int slot, size_t bytes)
+{
+    char* hs = c->job_stage_buf(slot, bytes);
+    c->jobtab[slot].reserve(bytes, c->st);
+    return hs;
+}
+
 // A batched launch's job table: through its pinned staging slot into device
 // memory, ordered on the context stream; returns the device copy.
 static char* stage_table(pra_ctx* c, int slot, const void* data, size_t bytes)
 {
-    char* hs = c->job_stage_buf(slot, bytes);
+    char* hs = reserve_table(c, slot, bytes);
     memcpy(hs, data, bytes);
-    c->jobtab[slot].reserve(bytes, c->st);
     HIPCHK(hipMemcpyAsync(c->jobtab[slot].p, hs, bytes, hipMemcpyHostToDevice, c->st));
     return c->jobtab[slot].as<char>();
 }
@@ -4034,6 +4041,8 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
             F.buf.reserve((have + a.room) * R->w * 8, c->st, (size_t)F.n * R->w * 8);
             R->dx.reserve(PRA_LOOP_ROWS * 8, c->st, D.n * 8);
             R->places.reserve((R->sbs_use << (PRA_SB_BITS - 5)) * 8, c->st);
+            // the delta that an iteration may leave: new keys of its candidates
+            D.buf.reserve(std::min<u64>(bits - std::min(bits, have), max_cand) * R->w * 8, c->st, (size_t)D.n * R->w * 8);
         } catch (const PraError& e) {
             if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
             R->places.release();
@@ -4065,8 +4074,19 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         of.push_back(k);
     }
     if (jobs.empty()) return;
+    // from the launch on nothing is allocated, so nothing can be refused
+    // between the rows that it writes and the counts that take them in
+    try {
+        c->tmp64a.reserve(jobs.size() * PRA_LOOP_OUT * 8, c->st);
+        if (jobs.size() > 1 || c->pub_open)
+            for (int slot : {JOB_LOOP_FULL, JOB_LOOP_DELTA, JOB_LOOP})
+                reserve_table(c, slot, jobs.size() * std::max(sizeof(LoopArgs), sizeof(CopyJob) + 4) + 4);
+    } catch (const PraError& e) {
+        if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+        for (pra_scc* S : sccs) S->loop_stop = 0;
+        return;
+    }
     copy_ranges(c, JOB_LOOP_FULL, appends);
-    c->tmp64a.reserve(jobs.size() * PRA_LOOP_OUT * 8, c->st);
     for (size_t k = 0; k < jobs.size(); k++) jobs[k].out = c->tmp64a.as<u64>() + k * PRA_LOOP_OUT;
     const u64* out;
     if (jobs.size() == 1 && !c->pub_open) {
@@ -4107,10 +4127,7 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         D.sorted = true;
         R->touched(PRA_DELTA);
         R->dx_gen = G.dict_gen;
-        if (last) {
-            D.buf.reserve((size_t)last * R->w * 8, c->st);
-            deltas.push_back(CopyJob{F.d() + F.n * R->w, D.d(), last * (u64)R->w});
-        }
+        if (last) deltas.push_back(CopyJob{F.d() + F.n * R->w, D.d(), last * (u64)R->w});
         R->jhint = (u32)out[3];
         R->mt_entries += written;
         G.iterations += its;
