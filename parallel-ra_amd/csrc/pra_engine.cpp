@@ -665,7 +665,7 @@ struct Group {
     DBuf dict, vals, lead_vals, rank_of, lead_of, lead_bucket;
     u64 dict_cap = 0, dict_n = 0;
     int dict_state = 0, dict_rebuilds = 0;   // state: 0 stale, 1 valid, 2 disabled
-    u64 dict_gen = 0;                        // dictionary builds so far
+    u64 dict_gen = 0;                        // dictionary builds begun so far
     DBuf joined;                             // join pairs so far (one device word)
     u64 iterations = 0;
     // lock-step execution: the instance's SCC in progress and the iterations
@@ -1622,6 +1622,7 @@ static bool small_dictionary_args(pra_ctx* c, int gi, DictSmallArgs* args)
             a.arity[a.k++] = R->arity;
         }
     if (total == 0) return false;
+    G.dict_gen++;   // the tables of the last build end here
     const u64 room = std::min<u64>(total, PRA_DICT_SMALL);
     a.cap = pow2_at_least(std::max<u64>(64, 2 * room));
     a.nb = (u64)c->nb;
@@ -1701,7 +1702,6 @@ static void build_dictionaries(pra_ctx* c, const std::vector<int>& groups)
             G.dict_cap = jobs[k].cap;
             G.dict_n = n[k];
             G.dict_state = 1;
-            G.dict_gen++;
         }
     }
     for (int gi : general) build_dictionary(c, gi);
@@ -1717,6 +1717,7 @@ static void build_dictionary(pra_ctx* c, int gi)
         if (R->group == gi && !R->view_of)
             for (int v : {PRA_FULL, PRA_DELTA}) total += R->ver[v].n * (u64)R->arity;
     if (total == 0) return;
+    G.dict_gen++;   // the tables of the last build end here, whether or not this one comes to its end
     Rows V;
     V.buf.reserve(total * 8, c->st);
     u64 off = 0;
@@ -1753,7 +1754,6 @@ static void build_dictionary(pra_ctx* c, int gi)
     G.dict_cap = cap;
     G.dict_n = V.n;
     G.dict_state = 1;
-    G.dict_gen++;
 }
 
 // The bits of a dense output's rank indexes put rows in trie order when a
