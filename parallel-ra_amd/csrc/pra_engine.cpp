@@ -32,11 +32,15 @@
 
 namespace {
 
+static bool yield_tables(pra_ctx* c);
+
 enum { RA_COPY = 0, RA_COPY_FILTER = 1, RA_ACOPY = 3, RA_JOIN = 4 };
 
 struct PraError : std::runtime_error {
     int code;
     PraError(int c, const std::string& m) : std::runtime_error(m), code(c) {}
+    // device memory, or the context's share of it, is used up
+    bool refused() const { return code == PRA_E_BUDGET || code == PRA_E_NOMEM; }
 };
 
 #define HIPCHK(x)                                                                                  \
@@ -77,14 +81,27 @@ const pra::BlockAllocator kHipBlocks{hip_block_alloc, hip_block_free, nullptr};
 
 // Device bytes held by each context, keyed by its stream (every buffer of a
 // context is ordered on the context's stream): live bytes, their peak, the
-// context's cap (0 = none), and the stream's device.
+// context's cap (0 = none), the stream's device, and the context.
 struct MemAcct {
     long long live = 0, peak = 0;
     u64 budget = 0;
     int device = 0;
+    pra_ctx* owner = nullptr;
 };
 std::mutex g_acct_mu;
 std::map<hipStream_t, MemAcct> g_acct;
+
+// the context of a stream gives back what it can do without
+bool yield_for(hipStream_t s)
+{
+    pra_ctx* c;
+    {
+        std::lock_guard<std::mutex> lk(g_acct_mu);
+        auto it = g_acct.find(s);
+        c = it == g_acct.end() ? nullptr : it->second.owner;
+    }
+    return c && yield_tables(c);
+}
 
 // the device whose memory a stream's buffers are in; the calling thread's
 // current device may be another one
@@ -108,6 +125,15 @@ void acct_charge(hipStream_t s, long long bytes, bool check)
                                          std::to_string(bytes) + " requested > budget " + std::to_string(a.budget));
     a.live += bytes;
     if (a.live > a.peak) a.peak = a.live;
+}
+
+// refuses when the context of stream s has not `bytes` left of its budget
+void acct_need(hipStream_t s, long long bytes)
+{
+    std::lock_guard<std::mutex> lk(g_acct_mu);
+    auto it = g_acct.find(s);
+    if (it != g_acct.end() && it->second.budget && (u64)(it->second.live + bytes) > it->second.budget)
+        throw PraError(PRA_E_BUDGET, "device memory budget exceeded: less than " + std::to_string(bytes) + " bytes left");
 }
 
 // the stream-ordered pool keeps freed memory for reuse; give it back
@@ -449,10 +475,20 @@ struct DBuf {
         cap = 0;
         big = false;
     }
-    // grow to at least `bytes`, preserving the first `used` bytes
+    // grow to at least `bytes`, preserving the first `used` bytes; a refusal
+    // is final only without the memory that the context can do without
     void reserve(size_t bytes, hipStream_t s, size_t used = 0)
     {
         if (bytes <= cap) return;
+        try {
+            grow(bytes, s, used);
+        } catch (const PraError& e) {
+            if (!e.refused() || !yield_for(s)) throw;
+            grow(bytes, s, used);
+        }
+    }
+    void grow(size_t bytes, hipStream_t s, size_t used)
+    {
         // grow by doubling (fewer growth copies than growing by half, which
         // measured slower); the quarter-octave block classes keep the
         // rounding on top of that within 25 %
@@ -727,6 +763,12 @@ struct pra_ctx {
     bool dense_on = true;        // dense membership for outputs that allow it
     bool tune_on = true;         // autotuned knobs (PRA_AUTOTUNE=0: the fixed defaults)
     bool loop_on = true;         // whole iterations in one block for small outputs (PRA_RANK_LOOP=0: never)
+    // how often memory was refused since the last SCC began (yield_tables): from
+    // once on no one-block iterations and second full buffers, from twice on no
+    // ranked membership
+    int lean = 0;
+    int no_yield = 0;            // they are in use by launches under way (NoYield)
+    bool merges_open = false;    // second full buffers are named by merges not yet launched
     bool seg_sort_on = true;     // segmented sort of newts too large for the bins (PRA_SEG_SORT=0: byte passes)
     u64 bin_cap_test = 0;        // PRA_SORT_TEST_BIN_CAP: a lower bin capacity, so tests reach the large-newt paths
     int dense_epoch_bits = 16;   // PRA_DENSE_EPOCH_BITS: at most this many epoch bits in claim slots (0: none)
@@ -923,6 +965,48 @@ static Group& grp(pra_ctx* c, int g)
     while ((int)c->groups.size() <= g) c->groups.emplace_back(new Group());
     return *c->groups[(size_t)g];
 }
+
+// Device memory that only speed needs -- the tables of ranked membership,
+// emission in digits and one-block iterations, claim tables, second full
+// buffers, tables that are out of date -- given back when a buffer that a
+// program cannot do without is refused.  All of it is at rest, or used only by
+// work already enqueued, outside of a NoYield's life.
+static bool yield_tables(pra_ctx* c)
+{
+    if (c->no_yield) return false;
+    bool any = false;
+    auto drop = [&](DBuf& b) {
+        any = any || b.p;
+        b.release();
+    };
+    for (pra_rel* R : c->rels) {
+        for (DBuf* b : {&R->fresh, &R->dirty, &R->sbpre, &R->linep, &R->places, &R->dtab, &R->rk_words[0],
+                        &R->rk_words[1], &R->rk_first[0], &R->rk_first[1]})
+            drop(*b);
+        R->fresh_sbs = R->dtab_cap = 0;
+        for (int v : {PRA_DELTA, PRA_FULL}) R->rk_gen[v] = ~0ULL;
+        if (!c->merges_open) drop(R->merged);
+        if (!R->mt_valid) drop(R->mt);
+        if (!R->bm_valid) drop(R->bm);
+    }
+    drop(c->first);
+    c->first_words = 0;
+    c->lean++;
+    return any;
+}
+
+struct NoYield {
+    pra_ctx* c;
+    explicit NoYield(pra_ctx* c_) : c(c_) { c->no_yield++; }
+    ~NoYield() { end(); }
+    void end()
+    {
+        if (c) c->no_yield--;
+        c = nullptr;
+    }
+    NoYield(const NoYield&) = delete;
+    NoYield& operator=(const NoYield&) = delete;
+};
 
 struct Prof {
     pra_ctx* c;
@@ -2219,6 +2303,7 @@ struct Merges {
     u64 rank_words = 0;
     double bytes = 0;
     explicit Merges(pra_ctx* c_) : c(c_) { memset(&b, 0, sizeof(b)); }
+    ~Merges() { c->merges_open = false; }
 
     void add(pra_rel* R)
     {
@@ -2230,15 +2315,19 @@ struct Merges {
             F.sorted = sorted;
             return;
         }
-        bool own = true;
-        try {
-            R->merged.reserve((F.n + D.n) * R->w * 8, c->st);
-        } catch (const PraError& e) {
-            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
-            R->merged.release();
-            own = false;
-            run();
+        bool own = !c->lean;
+        if (own) {
+            NoYield hold(c);
+            try {
+                R->merged.reserve((F.n + D.n) * R->w * 8, c->st);
+            } catch (const PraError& e) {
+                if (!e.refused()) throw;
+                R->merged.release();
+                own = false;
+            }
         }
+        if (own) c->merges_open = true;
+        if (!own) run();
         MergeJob& m = b.job[b.njobs];
         m.F = F.d();
         m.nf = F.n;
@@ -2284,6 +2373,7 @@ struct Merges {
         }
         rels.clear();
         memset(&b, 0, sizeof(b));
+        c->merges_open = false;
         rank_words = 0;
         bytes = 0;
     }
@@ -2779,7 +2869,10 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         // shares the partition and sort launches they need anyway: two
         // launches more, where ranked membership is four (points-to
         // analysis, 62 iterations: 15.04 against 15.60 ms)
-        if (phase == 1 && mixed && C < kMixedRankedCandidates) ch.mode = 1;
+        if (c->lean > 1 || (phase == 1 && mixed && C < kMixedRankedCandidates)) {
+            ch.mode = 1;
+            ch.rtime = false;
+        }
         if (ch.mode == 2 && !ensure_ranked(c, R, bits, rb, C, phase == 0)) {
             ch.mode = 1;
             ch.rtime = false;
@@ -2828,24 +2921,107 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     std::vector<Choice> choice(no);
     std::vector<int> emit_rule(no, -1);
     std::vector<char> use_dense(no, 0), fresh_left(no, 0);
-    if (nactive >= 2) {
-        try {
-            reserve_first(c, region_rows);
-        } catch (const PraError& e) {
-            if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
+    // the bins of an output's packed-key sort
+    auto reserve_bins = [&](size_t oi, u64 C) {
+        pra_rel* R = outs[oi];
+        // bins of twice the average top-byte share (a fuller bin sends
+        // the sort to its byte-pass fallback)
+        const u32 bcap = (u32)std::min<u64>(PRA_BIN_CAP, pow2_at_least(std::max<u64>(256, 2 * C / 256 + 1)));
+        if (bcap > R->bin_cap) {
+            R->bin_keys.reserve((size_t)PRA_RADIX * bcap * 8, c->st);
+            R->bin_idx.reserve((size_t)PRA_RADIX * bcap * 4, c->st);
+            R->bin_cap = bcap;
         }
-    }
-    std::vector<std::pair<pra_rel*, int>> to_rank;
-    for (size_t oi = 0; oi < no; oi++) {
-        if (!cap[oi]) continue;
-        choice[oi] = decide(oi, cap[oi], nactive >= 2 ? 1 : 0, reg[oi].rb);
-        if (choice[oi].mode != 2) continue;
-        emit_rule[oi] = emit_shape(oi);
-        if (emit_rule[oi] >= 0) to_rank.push_back({S->ras[emit_rule[oi]].inner, S->ras[emit_rule[oi]].inner_v});
-    }
-    ensure_rank_rows(c, to_rank);
-    for (size_t oi = 0; oi < no; oi++)
-        if (emit_rule[oi] >= 0) emit_rule[oi] = emit_ranked(oi, emit_rule[oi]);
+        if (!R->bin_cur.p) {
+            R->bin_cur.reserve(PRA_RADIX * 4, c->st);
+            pra_launch_fill_u64(c->st, R->bin_cur.as<u64>(), PRA_RADIX / 2, 0);
+        }
+        R->nkeys.reserve(C * 8, c->st);
+    };
+    // Room for what the launches of some outputs write, all of it before the
+    // first of them: a refusal here can still be answered without the memory
+    // that only speed needs, one between the launches could not.
+    auto reserve_outputs = [&](const std::vector<size_t>& ois, const std::vector<Choice>& ch,
+                               const std::vector<int>& er) {
+        u64 ct = 0, rows = 0, ht = 0, ranked_tiles = 0;
+        for (size_t oi : ois) {
+            const u64 C = cap[oi];
+            const int kw = out_intern[oi] == 1 ? outs[oi]->arity : outs[oi]->arity + 1;
+            pra_rel* R = outs[oi];
+            R->ver[PRA_NEWT].buf.reserve(C * R->w * 8, c->st);
+            rows += C;
+            if (er[oi] < 0) ct += C * (u64)kw;
+            if (ch[oi].mode == 2) {
+                ranked_tiles += pra_tiles(C);
+                continue;
+            }
+            ht += (u64)nb * pra_tiles(C) + 2;
+            if (packed[oi]) reserve_bins(oi, C);
+            if (ch[oi].mode == 0) R->bm_valid = false, ensure_member_table(c, R, kw, C);
+        }
+        if (ct || ois.size() > 1) {
+            c->cand.reserve(std::max<u64>(ct, 1) * 8, c->st);
+            c->dest.reserve(rows * 4, c->st);
+        }
+        c->slot_of.reserve(rows * 8, c->st);
+        c->keep.reserve(rows * 4, c->st);
+        c->hist.reserve(ht * 4, c->st);
+        c->offs.reserve(ht * 4 + 8, c->st);
+        if (ranked_tiles) prepare_lookback(c, ranked_tiles * PRA_TILE);
+        for (auto& ra : S->ras) {
+            const size_t oi = std::find(outs.begin(), outs.end(), ra.out) - outs.begin();
+            if (!ra.active || std::find(ois.begin(), ois.end(), oi) == ois.end() || er[oi] >= 0) continue;
+            ra.off.reserve((ra.n_outer + 1) * 8, c->st);
+            ra.istart.reserve(std::max<u64>(1, ra.n_outer) * 8, c->st);
+        }
+        // (job tables, counters and bounds, a few KB, have their room below)
+        if (c->lean < 2) acct_need(c->st, 64 << 10);
+    };
+    // f, and while it is refused memory, f again with less to speed it up
+    // (nothing that f makes is named by a launch before it returns)
+    auto or_lean = [&](bool first_pass, auto f) {
+        for (;;) {
+            try {
+                NoYield hold(c);
+                return f();
+            } catch (const PraError& e) {
+                if (!e.refused() || c->lean > 1) throw;
+            }
+            yield_tables(c);
+            for (pra_rel* R : c->rels) {
+                if (first_pass) R->nx.release();   // (else the new rows' indexes)
+                if (c->lean < 2) continue;
+                R->dx.release();
+                R->dx_gen = ~0ULL;
+            }
+        }
+    };
+    or_lean(true, [&]() {
+        choice.assign(no, Choice());
+        emit_rule.assign(no, -1);
+        if (nactive >= 2 && c->lean < 2) {
+            try {
+                reserve_first(c, region_rows);
+            } catch (const PraError& e) {
+                if (!e.refused()) throw;
+            }
+        }
+        std::vector<std::pair<pra_rel*, int>> to_rank;
+        std::vector<size_t> active;
+        for (size_t oi = 0; oi < no; oi++) {
+            if (!cap[oi]) continue;
+            active.push_back(oi);
+            choice[oi] = decide(oi, cap[oi], nactive >= 2 ? 1 : 0, reg[oi].rb);
+            if (choice[oi].mode != 2) continue;
+            emit_rule[oi] = emit_shape(oi);
+            if (emit_rule[oi] >= 0) to_rank.push_back({S->ras[emit_rule[oi]].inner, S->ras[emit_rule[oi]].inner_v});
+        }
+        ensure_rank_rows(c, to_rank);
+        for (size_t oi = 0; oi < no; oi++)
+            if (emit_rule[oi] >= 0) emit_rule[oi] = emit_ranked(oi, emit_rule[oi]);
+        reserve_outputs(active, choice, emit_rule);
+    });
+    NoYield tables_in_use(c);
 
     // 2. per-RA output counts and their exclusive offsets (the arrival plan
     //    reads them at the source-bucket bounds); an output that emits in
@@ -3318,24 +3494,12 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             a.tag = R->tag;
             a.rep_words = rep0;
             if (pk) {
-                // bins of twice the average top-byte share (a fuller bin sends
-                // the sort to its byte-pass fallback)
-                const u32 bcap = (u32)std::min<u64>(PRA_BIN_CAP, pow2_at_least(std::max<u64>(256, 2 * C / 256 + 1)));
-                if (bcap > R->bin_cap) {
-                    R->bin_keys.reserve((size_t)PRA_RADIX * bcap * 8, c->st);
-                    R->bin_idx.reserve((size_t)PRA_RADIX * bcap * 4, c->st);
-                    R->bin_cap = bcap;
-                }
-                if (!R->bin_cur.p) {
-                    R->bin_cur.reserve(PRA_RADIX * 4, c->st);
-                    pra_launch_fill_u64(c->st, R->bin_cur.as<u64>(), PRA_RADIX / 2, 0);
-                }
+                reserve_bins(oi, C);
                 a.bin_cap = R->bin_cap;
                 a.bin_keys = R->bin_keys.as<u64>();
                 a.bin_idx = R->bin_idx.as<u32>();
                 a.bin_cur = R->bin_cur.as<u32>();
                 f.bin_cur = a.bin_cur;
-                R->nkeys.reserve(C * 8, c->st);
                 Group& G = grp(c, R->group);
                 a.dict = G.dict.as<u64>();
                 a.dict_cap = G.dict_cap;
@@ -3723,6 +3887,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     // pass 1 redoes outputs whose candidates overflowed their capacity (now
     // sized exactly) or whose dense claims met a value without a dictionary
     // rank (now the general way); pass 2 the few that needed both
+    tables_in_use.end();
     for (int pass = 0; pass < 3; pass++) {
         u64* h = publish_begin(c, c->stage2.as<u64>(), no * SW, pass == 0 && have_last_fold ? &last_fold : nullptr,
                                pass == 0 && place_publishes);
@@ -3762,6 +3927,14 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             // an emission over the join threshold: by the arrival plan
             if (st2[oi * SW + 5] == 4) emit_off[oi] = 1;
             cap[oi] = st2[oi * SW + 4];
+            or_lean(false, [&]() {
+                std::vector<Choice> ch(no);
+                std::vector<int> er(no, -1);
+                ch[oi] = decide(oi, cap[oi], 0, 0);
+                if (ch[oi].mode == 2) er[oi] = emit_rule_of(oi);
+                reserve_outputs({oi}, ch, er);
+            });
+            NoYield in_use(c);
             run_output(oi, nullptr);
         }
     }
@@ -3987,7 +4160,7 @@ static RADesc* loop_rule(pra_scc* S)
 // general iterations before have made them).
 static bool loop_ready(pra_ctx* c, pra_scc* S, u32 max_cand)
 {
-    if (!c->loop_on || !S->running || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
+    if (!c->loop_on || c->lean || !S->running || S->ras.size() != 1 || !S->ras[0].out->loops) return false;
     RADesc* ra = loop_rule(S);
     if (!ra) return false;
     pra_rel* R = ra->out;
@@ -4020,6 +4193,7 @@ static bool loop_ready(pra_ctx* c, pra_scc* S, u32 max_cand)
 static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u32 max_cand,
                       std::vector<std::vector<u32>>& rows)
 {
+    NoYield hold(c);
     std::vector<LoopArgs> jobs;
     std::vector<size_t> of;
     std::vector<CopyJob> appends;
@@ -4030,19 +4204,28 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         Rows &F = R->ver[PRA_FULL], &D = R->ver[PRA_DELTA];
         LoopArgs a;
         memset(&a, 0, sizeof(a));
-        // room for what the rank space can still hold, or as much again twice
-        // over (once under a budget, as the appends' growth would); an
-        // iteration stops by its candidates, so their most on top
+        // room for what the rank space can still hold, or as much again as
+        // there is, as the appends' growth would make; an iteration stops by
+        // its candidates, so their most on top.  Under a budget the room that
+        // the general iterations have left in the log and the delta, and as
+        // many candidates: what they hold is never larger than they make it.
         u64 bits = 1;
         for (int i = 0; i < R->arity; i++) bits *= G.dict_n;
         const u64 have = F.n + D.n;
-        a.room = std::min<u64>(bits - std::min(bits, have), c->budget ? have : std::max<u64>(1 << 18, 2 * have)) + PRA_LOOP_ROWS;
+        const u64 more = c->budget ? 0 : std::min<u64>(bits - std::min(bits, have), std::max<u64>(1 << 18, have)) + PRA_LOOP_ROWS;
         try {
-            F.buf.reserve((have + a.room) * R->w * 8, c->st, (size_t)F.n * R->w * 8);
-            R->dx.reserve(PRA_LOOP_ROWS * 8, c->st, D.n * 8);
+            F.buf.reserve((have + more) * R->w * 8, c->st, (size_t)F.n * R->w * 8);
+            a.room = F.buf.cap / ((size_t)R->w * 8) - have;
+            if (a.room < R->jhint) continue;   // not for another iteration like the last
             R->places.reserve((R->sbs_use << (PRA_SB_BITS - 5)) * 8, c->st);
             // the delta that an iteration may leave: new keys of its candidates
-            D.buf.reserve(std::min<u64>(bits - std::min(bits, have), max_cand) * R->w * 8, c->st, (size_t)D.n * R->w * 8);
+            const u64 left = std::min<u64>(bits - std::min(bits, have), max_cand);
+            if (!c->budget) {
+                R->dx.reserve(left * 8, c->st, D.n * 8);
+                D.buf.reserve(left * R->w * 8, c->st, (size_t)D.n * R->w * 8);
+            }
+            a.max_cand = (u32)std::min<u64>(max_cand, std::min(R->dx.cap, D.buf.cap / (size_t)R->w) / 8);
+            if (left <= a.max_cand) a.max_cand = max_cand;
         } catch (const PraError& e) {
             if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
             R->places.release();
@@ -4066,7 +4249,6 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         a.nb = (u32)c->nb;
         a.tag = R->tag;
         a.max_iters = std::min<u32>(max, PRA_LOOP_ITERS);
-        a.max_cand = max_cand;
         a.kw = R->arity;
         a.wn = R->w;
         a.by_bucket = by_bucket(c, R);
@@ -4267,6 +4449,7 @@ static void scc_begin(pra_scc* S, bool move_status)
         for (size_t i = 0; i < S->rels.size(); i++)
             if (S->status[i]) full_to_delta(c, S->rels[i]);
     S->running = true;
+    c->lean = 0;
     S->loop_stop = ~0ULL;
     for (pra_rel* R : S->rels) R->loops = false;
     if (RADesc* ra = c->loop_on ? loop_rule(S) : nullptr) ra->out->loops = true;
@@ -4451,6 +4634,7 @@ int pra_ctx_create(int device, int nbuckets, uint64_t hbm_budget, pra_ctx** out)
             MemAcct& a = g_acct[c->st];
             a.budget = hbm_budget;
             a.device = device;
+            a.owner = c.get();
         }
         c->nb = nbuckets;
         c->budget = hbm_budget;
@@ -4679,20 +4863,46 @@ int pra_autotune_report(char* buf, uint64_t cap, uint64_t* len)
     return PRA_OK;
 }
 
-int pra_ctx_trim(pra_ctx* ctx)
+// the scratch of a context between steps: written before it is read inside
+// every iteration that uses it; released on the context's stream, so reuse
+// stays ordered behind the work already enqueued
+static void release_scratch(pra_ctx* ctx)
 {
-    if (!ctx) return PRA_E_ARG;
-    API_BEGIN_ON(ctx)
-    // written before they are read inside every iteration that uses them;
-    // released on the context's stream, so reuse stays ordered behind the
-    // work already enqueued
     for (DBuf* b : {&ctx->sort_tmp, &ctx->stage, &ctx->stage2, &ctx->tmp64a, &ctx->tmp64b, &ctx->tmp64c, &ctx->cand,
                     &ctx->dest, &ctx->slot_of, &ctx->keep, &ctx->hist, &ctx->offs, &ctx->ktmp, &ctx->idxa, &ctx->idxb,
                     &ctx->posadj_dev, &ctx->ttab, &ctx->kp, &ctx->lb_status, &ctx->first})
         b->release();
     ctx->first_words = 0;
     ctx->lb_zeroed = 0;   // look-back words are zeroed again on next use
+}
+
+int pra_ctx_trim(pra_ctx* ctx)
+{
+    if (!ctx) return PRA_E_ARG;
+    API_BEGIN_ON(ctx)
+    release_scratch(ctx);
     API_END
+}
+
+// a version in trie order, between steps: refused memory, again without the
+// scratch, tables, sort bins and empty versions of the iterations before
+static void sorted_between_steps(pra_ctx* c, pra_rel* R, int v)
+{
+    try {
+        ensure_sorted(c, R, v);
+    } catch (const PraError& e) {
+        if (!e.refused()) throw;
+        release_scratch(c);
+        yield_tables(c);
+        for (pra_rel* r : c->rels) {
+            for (DBuf* b : {&r->nkeys, &r->bin_keys, &r->bin_idx, &r->nx, &r->dx}) b->release();
+            r->bin_cap = 0;
+            r->dx_gen = ~0ULL;
+            for (int x : {PRA_DELTA, PRA_NEWT})
+                if (!r->ver[x].n) r->ver[x].buf.release();
+        }
+        ensure_sorted(c, R, v);
+    }
 }
 
 int pra_ctx_device_bytes(pra_ctx* ctx, uint64_t* live, uint64_t* peak)
@@ -4808,7 +5018,7 @@ int pra_rel_device_rows(pra_rel* rel, int version, const uint64_t** rows, uint64
     if (!rel || !rows || !nrows || !valid_ver(version)) return PRA_E_ARG;
     API_BEGIN(rel->ctx)
     pra_ctx* c = rel->ctx;
-    if (version != PRA_NEWT) ensure_sorted(c, rel, version);
+    if (version != PRA_NEWT) sorted_between_steps(c, rel, version);
     HIPCHK(hipStreamSynchronize(c->st));
     *rows = rel->ver[version].d();
     *nrows = rel->ver[version].n;
@@ -4820,7 +5030,7 @@ int pra_rel_checksum(pra_rel* rel, int version, uint64_t* out)
     if (!rel || !out || !valid_ver(version)) return PRA_E_ARG;
     API_BEGIN(rel->ctx)
     pra_ctx* c = rel->ctx;
-    if (version != PRA_NEWT) ensure_sorted(c, rel, version);
+    if (version != PRA_NEWT) sorted_between_steps(c, rel, version);
     Rows& r = rel->ver[version];
     c->orand.reserve(32 * 8, c->st);
     pra_launch_fill_u64(c->st, c->orand.as<u64>(), 1, 0);
@@ -4835,7 +5045,7 @@ int pra_rel_download(pra_rel* rel, int version, uint64_t* rows, uint64_t cap, ui
     if (!rel || !nrows || !valid_ver(version)) return PRA_E_ARG;
     API_BEGIN(rel->ctx)
     pra_ctx* c = rel->ctx;
-    if (version != PRA_NEWT) ensure_sorted(c, rel, version);
+    if (version != PRA_NEWT) sorted_between_steps(c, rel, version);
     Rows& r = rel->ver[version];
     *nrows = r.n;
     u64 m = std::min<u64>(cap, r.n);
