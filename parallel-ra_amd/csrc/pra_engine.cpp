@@ -781,15 +781,15 @@ struct pra_ctx {
         u64 cap;
     };
     std::vector<TuneSample> tune_pending;
-    // a claim-table sample of the ranked-membership choice still to be joined
-    // by its sort (ranked membership needs none): its time so far, then the
-    // sort's events
+    // samples whose events may not have completed when the iteration's summary
+    // arrives (the placement publishes it before it ends), with their
+    // candidates in `cap`.
+    // A claim-table sample of the ranked-membership choice also has the events
+    // of its sort, which ranked membership needs none of.
     struct LateSample {
-        int band;
-        size_t oi;
-        u64 n;
-        double ms;
-        hipEvent_t a, b;
+        TuneSample s;
+        bool sorts;
+        hipEvent_t sort_a, sort_b;
     };
     std::vector<LateSample> tune_late;
     size_t lb_zeroed = 0;        // words of lb_status known to be zero-initialised
@@ -834,7 +834,7 @@ struct pra_ctx {
         else if (st)
             small_flush(st);
         for (auto& t : tune_late)
-            for (hipEvent_t e : {t.a, t.b})
+            for (hipEvent_t e : {t.s.a, t.s.b, t.sort_a, t.sort_b})
                 if (e) evpool.push_back(e);
         for (auto e : evpool) (void)hipEventDestroy(e);
         if (st) {
@@ -3022,6 +3022,11 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         reserve_outputs(active, choice, emit_rule);
     });
     NoYield tables_in_use(c);
+    // both variants of the ranked-membership choice are timed from here:
+    // emission in digits does the counts' and expansions' work too
+    hipEvent_t rank_from = nullptr;
+    for (size_t oi = 0; oi < no; oi++)
+        if (cap[oi] && choice[oi].rtime) rank_from = c->tune_begin(true);
 
     // 2. per-RA output counts and their exclusive offsets (the arrival plan
     //    reads them at the source-bucket bounds); an output that emits in
@@ -3152,8 +3157,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         else if (!rs)
             ch = decide(oi, C, 0, 0);
         const int mode = ch.mode, dvar = ch.dvar;
-        const bool dtime = ch.dtime, rtime = ch.rtime;
-        hipEvent_t tr = nullptr;   // opens the claim table's share of the choice
+        const bool dtime = ch.dtime;
         const bool dn = mode != 0, ranked = mode == 2;
         use_dense[oi] = (char)mode;
         if (phase >= 2 && ranked) return;   // its new rows are in place
@@ -3357,7 +3361,6 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 }
                 const u64 etiles = er >= 0 ? (ra.emit.n + PRA_EMIT_BLOCK - 1) / PRA_EMIT_BLOCK : 0;
                 prepare_lookback(c, std::max<u64>(C, (etiles + PRA_RADIX - 1) / PRA_RADIX * PRA_TILE));
-                hipEvent_t ta = c->tune_begin(rtime);
                 for (int step = 0; step < PRA_RANK_STEPS; step++) {
                     if (step == (er >= 0 ? PRA_RANK_CLAIM : PRA_RANK_EMIT)) continue;
                     const u32 ep = next_sort_epoch(c);
@@ -3365,7 +3368,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                     pra_launch_rank(c->st, step, ra, C, c->lb_status.as<u64>(), c->lb_ctr.as<u32>(), ep, c->dflags());
                     check_launch("rank");
                 }
-                c->tune_end(ta, TUNE_RANKED, band_of(C), 1, oi, C);
+                if (planned) c->tune_end(rank_from, TUNE_RANKED, band_of(C), 1, oi, C);
                 fresh_left[oi] = er >= 0;
                 return;
             }
@@ -3403,7 +3406,6 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                     dense_jobs.emplace_back(da, oi);
                     return;
                 }
-                tr = c->tune_begin(rtime);
                 hipEvent_t ta = c->tune_begin(dtime);
                 {
                     ProfPerCand p(c, K_DEDUP_CLAIM, 8.0 * (kw + 1), oi);
@@ -3544,7 +3546,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
                 pra_launch_dedup_scatter(c->st, a, wide);
                 check_launch("dedup_scatter");
                 c->tune_end(ta, TUNE_SCATTER_WIDE, sband, wide, oi, C);
-                c->tune_end(tr, TUNE_RANKED, band_of(C), 0, oi, C);
+                if (planned) c->tune_end(rank_from, TUNE_RANKED, band_of(C), 0, oi, C);
             }
         }
         if (!fold_here && planned && oi == last_oi) {
@@ -3883,7 +3885,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     std::vector<u64> st2(no * SW, 0);
     // deltas of relations whose full version no rule of the SCC reads go to
     // their full logs while the host waits for the first readback
-    std::vector<char> early(S->rels.size(), 0);
+    std::vector<char> early(S->rels.size(), 0), redone(no, 0);
     // pass 1 redoes outputs whose candidates overflowed their capacity (now
     // sized exactly) or whose dense claims met a value without a dictionary
     // rank (now the general way); pass 2 the few that needed both
@@ -3927,6 +3929,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             // an emission over the join threshold: by the arrival plan
             if (st2[oi * SW + 5] == 4) emit_off[oi] = 1;
             cap[oi] = st2[oi * SW + 4];
+            redone[oi] = 1;
             or_lean(false, [&]() {
                 std::vector<Choice> ch(no);
                 std::vector<int> er(no, -1);
@@ -3952,28 +3955,36 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         if (std::get<0>(pc) < c->pending.size())
             c->pending[std::get<0>(pc)].bytes += std::get<1>(pc) * (double)st2[std::get<2>(pc) * SW + 4];
     c->per_candidate.clear();
-    // tuned launches: cost per candidate; a launch whose candidates passed
-    // its capacity did part of the work and is not counted
-    for (auto& t : c->tune_late) {
-        float ms = 0;
-        if (t.b && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess &&
-            g_tune.record(c->device, TUNE_RANKED, t.band, 0, (t.ms + ms) / (double)t.n, kTuneVariants[TUNE_RANKED]))
+    // tuned launches: cost per candidate, read at the next iteration (the
+    // launches may still be running); one whose candidates passed its capacity
+    // did part of the work and is not counted
+    std::vector<pra_ctx::LateSample> samples;
+    samples.swap(c->tune_late);
+    for (auto& l : samples) {
+        const auto& t = l.s;
+        float ms = 0, sort_ms = 0;
+        hipError_t e = l.sorts && !l.sort_b ? hipErrorInvalidValue : hipEventElapsedTime(&ms, t.a, t.b);
+        if (e == hipSuccess && l.sorts) e = hipEventElapsedTime(&sort_ms, l.sort_a, l.sort_b);
+        if (e == hipErrorNotReady) {
+            c->tune_late.push_back(l);
+            continue;
+        }
+        if (e == hipSuccess && g_tune.record(c->device, t.knob, t.band, t.var, (double)(ms + sort_ms) / (double)t.cap,
+                                             kTuneVariants[t.knob]))
             tune_save();
-        for (hipEvent_t e : {t.a, t.b})
-            if (e) c->evpool.push_back(e);
+        for (hipEvent_t x : {t.a, t.b, l.sort_a, l.sort_b})
+            if (x) c->evpool.push_back(x);
     }
-    c->tune_late.clear();
+    const size_t waiting = c->tune_late.size();   // samples of earlier iterations
     for (auto& t : c->tune_pending) {
         const u64 n = st2[t.oi * SW + 4];
-        float ms = 0;
-        const bool timed = n > 0 && n <= t.cap && hipEventElapsedTime(&ms, t.a, t.b) == hipSuccess;
-        if (timed && t.knob == TUNE_RANKED && t.var == 0)
-            c->tune_late.push_back({t.band, t.oi, n, (double)ms, nullptr, nullptr});
-        else if (timed &&
-            g_tune.record(c->device, t.knob, t.band, t.var, (double)ms / (double)n, kTuneVariants[t.knob]))
-            tune_save();
-        c->evpool.push_back(t.a);
-        c->evpool.push_back(t.b);
+        if (n > 0 && n <= t.cap && !in_rounds[t.oi] && !redone[t.oi]) {
+            t.cap = n;
+            c->tune_late.push_back({t, t.knob == TUNE_RANKED && t.var == 0, nullptr, nullptr});
+        } else {
+            c->evpool.push_back(t.a);
+            c->evpool.push_back(t.b);
+        }
     }
     c->tune_pending.clear();
     for (size_t oi = 0; oi < no; oi++) {
@@ -4058,16 +4069,16 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         }
         if (packed[oi] && !in_rounds[oi] && st2[oi * SW + 3] == 0) {
             BinSortJob job;
-            auto late = std::find_if(c->tune_late.begin(), c->tune_late.end(),
-                                     [&](const pra_ctx::LateSample& t) { return t.oi == oi && !t.a; });
-            if (late != c->tune_late.end()) late->a = c->tune_begin(true);
+            auto late = std::find_if(c->tune_late.begin() + (long)waiting, c->tune_late.end(),
+                                     [&](const pra_ctx::LateSample& l) { return l.sorts && l.s.oi == oi; });
+            if (late != c->tune_late.end()) late->sort_a = c->tune_begin(true);
             if (sort_by_packed_key(c, R, st2[oi * SW + 1], st2[oi * SW + 2], st2[oi * SW + 6], pk_mul[oi], pk_ls[oi],
                                    bnd, n_packed_sorts > 1 ? &job : nullptr, &R->ver[PRA_DELTA].buf)) {
                 bin_jobs.push_back(job);
                 bin_out.push_back(oi);
                 bins_max = std::max<u64>(bins_max, st2[oi * SW + 6]);
             }
-            if (late != c->tune_late.end()) late->b = c->tune_begin(true);
+            if (late != c->tune_late.end()) late->sort_b = c->tune_begin(true);
             bnd_ok[oi] = 1;
             continue;
         }
