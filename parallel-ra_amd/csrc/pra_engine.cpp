@@ -2737,6 +2737,8 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
     for (auto& ra : S->ras)
         if (std::find(outs.begin(), outs.end(), ra.out) == outs.end()) outs.push_back(ra.out);
     const size_t no = outs.size();
+    std::vector<size_t> out_of((size_t)nra);   // each rule's output
+    for (int r = 0; r < nra; r++) out_of[(size_t)r] = std::find(outs.begin(), outs.end(), S->ras[r].out) - outs.begin();
     std::vector<int> out_intern(no, 1);
     std::vector<u64> ub(no, 0), cap(no, 0);
     for (size_t oi = 0; oi < no; oi++) {
@@ -2968,9 +2970,11 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         c->hist.reserve(ht * 4, c->st);
         c->offs.reserve(ht * 4 + 8, c->st);
         if (ranked_tiles) prepare_lookback(c, ranked_tiles * PRA_TILE);
-        for (auto& ra : S->ras) {
-            const size_t oi = std::find(outs.begin(), outs.end(), ra.out) - outs.begin();
-            if (!ra.active || std::find(ois.begin(), ois.end(), oi) == ois.end() || er[oi] >= 0) continue;
+        std::vector<char> in(no, 0);
+        for (size_t oi : ois) in[oi] = er[oi] < 0;
+        for (int r = 0; r < nra; r++) {
+            RADesc& ra = S->ras[r];
+            if (!ra.active || !in[out_of[(size_t)r]]) continue;
             ra.off.reserve((ra.n_outer + 1) * 8, c->st);
             ra.istart.reserve(std::max<u64>(1, ra.n_outer) * 8, c->st);
         }
@@ -3091,7 +3095,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
         bucket_bounds(c, ra.outer, ra.outer_v);
     };
     for (int r = 0; r < nra; r++)
-        if (emit_rule[std::find(outs.begin(), outs.end(), S->ras[r].out) - outs.begin()] != r) count_rule(r);
+        if (emit_rule[out_of[(size_t)r]] != r) count_rule(r);
     flush_count_scans();
 
     // 3+4. per output: arrival plan, emit candidates, deduplicate, partition
@@ -3612,8 +3616,7 @@ static void run_iteration(pra_ctx* c, const std::vector<pra_scc*>& members)
             RADesc& ra = S->ras[r];
             pl.rout[r] = 0xFF;
             if (!ra.active || !counted[(size_t)r]) continue;
-            const size_t oi = std::find(outs.begin(), outs.end(), ra.out) - outs.begin();
-            pl.rout[r] = (unsigned char)oi;
+            pl.rout[r] = (unsigned char)out_of[(size_t)r];
             pl.is_join[r] = ra.type == RA_JOIN;
             pl.off[r] = ra.off.as<u64>();
             pl.bnd[r] = ra.outer->bnd[ra.outer_v].as<u64>();
@@ -4255,7 +4258,6 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         Group::Seq& sq = seq_counters(c, R->group, R->tag);
         a.seq = sq.buf.as<u64>() + sq.now * c->nb;
         a.D = G.dict_n;
-        a.inv = a.emit.inv;
         a.sbs = (u32)R->sbs_use;
         a.nb = (u32)c->nb;
         a.tag = R->tag;

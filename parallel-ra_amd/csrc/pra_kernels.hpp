@@ -294,7 +294,6 @@ struct LoopArgs {
     u64 host_seq;
     const u32* err;
     u64 D, room;
-    double inv;
     u32 host_words;         // where the error flags go
     u32 sbs, nb, tag, max_iters, max_cand;
     int kw, wn, by_bucket;
