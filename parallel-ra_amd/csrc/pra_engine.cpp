@@ -4215,13 +4215,13 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         RADesc& ra = *loop_rule(sccs[k]);
         pra_rel* R = ra.out;
         Group& G = grp(c, R->group);
-        Rows &F = R->ver[PRA_FULL], &D = R->ver[PRA_DELTA];
+        Rows &F = R->ver[PRA_FULL], &D = R->ver[PRA_DELTA], &N = R->ver[PRA_NEWT];
         LoopArgs a;
         memset(&a, 0, sizeof(a));
         // room for what the rank space can still hold, or as much again as
         // there is, as the appends' growth would make; an iteration stops by
         // its candidates, so their most on top.  Under a budget the room that
-        // the general iterations have left in the log and the delta, and as
+        // the general iterations have left in the log and newt, and as
         // many candidates: what they hold is never larger than they make it.
         u64 bits = 1;
         for (int i = 0; i < R->arity; i++) bits *= G.dict_n;
@@ -4232,13 +4232,14 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
             a.room = F.buf.cap / ((size_t)R->w * 8) - have;
             if (a.room < R->jhint) continue;   // not for another iteration like the last
             R->places.reserve((R->sbs_use << (PRA_SB_BITS - 5)) * 8, c->st);
-            // the delta that an iteration may leave: new keys of its candidates
+            // the delta that an iteration may leave (new keys of its candidates),
+            // in newt's buffer, which is empty
             const u64 left = std::min<u64>(bits - std::min(bits, have), max_cand);
             if (!c->budget) {
                 R->dx.reserve(left * 8, c->st, D.n * 8);
-                D.buf.reserve(left * R->w * 8, c->st, (size_t)D.n * R->w * 8);
+                N.buf.reserve(left * R->w * 8, c->st);
             }
-            a.max_cand = (u32)std::min<u64>(max_cand, std::min(R->dx.cap, D.buf.cap / (size_t)R->w) / 8);
+            a.max_cand = (u32)std::min<u64>(max_cand, std::min(R->dx.cap, N.buf.cap / (size_t)R->w) / 8);
             if (left <= a.max_cand) a.max_cand = max_cand;
         } catch (const PraError& e) {
             if (e.code != PRA_E_BUDGET && e.code != PRA_E_NOMEM) throw;
@@ -4322,6 +4323,7 @@ static void run_loops(pra_ctx* c, const std::vector<pra_scc*>& sccs, u32 max, u3
         D.sorted = true;
         R->touched(PRA_DELTA);
         R->dx_gen = G.dict_gen;
+        D.buf.swap(R->ver[PRA_NEWT].buf);
         if (last) deltas.push_back(CopyJob{F.d() + F.n * R->w, D.d(), last * (u64)R->w});
         R->jhint = (u32)out[3];
         R->mt_entries += written;
