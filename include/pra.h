@@ -95,8 +95,8 @@ int pra_ctx_release_group(pra_ctx* ctx, int group);
 int pra_ctx_trim(pra_ctx* ctx);
 /* Autotuner (no counterpart in the reference): variants of a step that give
  * identical results -- the dense claim table's size (2, 4 or 8 slots per
- * candidate of capacity) and the newt scatter's block width (256 or 1,024
- * threads) -- are timed on live single-output iterations, per device and band
+ * candidate of capacity), the newt scatter's block width (256 or 1,024
+ * threads), and the claim table or ranked membership -- are timed on live single-output iterations, per device and band
  * of log2(work), three times each, and the cheapest is kept for the process.
  * PRA_AUTOTUNE=0 in the environment keeps the fixed defaults.  With
  * PRA_AUTOTUNE_FILE=<path>, the choices settled in earlier processes are read

@@ -91,11 +91,12 @@ __global__ __launch_bounds__(kScanBlock) void k_part_scan(u32* __restrict__ H, u
 // lane's own row would touch several.  Tiles run from the last one back: the
 // rows the histogram read last are still in the last-level cache.
 // W: the row width, 0 = any (w).  NT: non-temporal stores.
-// Whole partitions, a lane to each row's words / this without the prefetch /
-// with it: 24 M rows of 3 words into 8 buckets 482 / 360 / 343 us, 12 M of 6
-// into 64 739 / 463 / 419, 30 M of 2 into 200 800 / 560 / 558, into 3 359 / 345
-// / 327, 300,000 of 5 into 3 42.4 / 45.4 / 39.9, 1 M of 3 into 200 34.3 / 35.4
-// / 31.9.  Large ones are bound by memory (the histogram reads every line, the
+// Whole partitions, queued one behind another, a lane to each row's words /
+// this without the prefetch / with it: 24 M rows of 3 words into 8 buckets 482 /
+// 360 / 345 us, 12 M of 6 into 64 739 / 463 / 419, 30 M of 2 into 200 800 / 560
+// / 560, into 3 359 / 345 / 328, 1 M of 3 into 200 34.3 / 35.4 / 32.6; waited
+// for, 300,000 of 5 into 3 42.4 / 45.4 / 36.5.  (A caller that waits for each
+// has 10 us more: 356 us for the first.)  Large ones are bound by memory (the histogram reads every line, the
 // scatter again: 24 bytes a word), those of less than a few tiles a compute
 // unit by a tile's own chain of loads, ranks and stores, which the prefetch
 // shortens.
